@@ -101,6 +101,33 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The ``_dlb_host`` module: native fast paths of the operators' common calls, bound to the
+    library :func:`load` opened.  Each returns None for arguments it does not cover, and its
+    wrapper goes through the general path (conversions, errors) then."""
+    global _host
+    if _host is not None:
+        return _host
+    import importlib.machinery
+    import importlib.util
+
+    import torch  # noqa: F401  (the module links against torch's libraries)
+
+    lib = load()
+    path = _PKG_DIR / "lib" / "_dlb_host.so"
+    if not path.exists():
+        raise ImportError(f"{path} not found: build it with `python -m dlcompiler_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("_dlb_host", str(path))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_dlb_host", loader))
+    loader.exec_module(module)
+    module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in module.names()})
+    _host = module
+    return module
+
+
 def check(status: int, what: str) -> None:
     if status != DLB_OK:
         msg = load().dlb_status_string(status).decode()

@@ -29,6 +29,9 @@ LIB_PATH = LIB_DIR / "libdlblas_hip.so"
 # measurement kernels that bench.py times; a library of their own, not part of the operator ABI
 PROBE_SRC = CSRC_DIR / "bench" / "probe.hip"
 PROBE_LIB_PATH = LIB_DIR / "libdlblas_bench_probe.so"
+# CPython module with the host side of the common calls (plain C++ against the torch headers)
+HOST_SRC = CSRC_DIR / "host" / "host_path.cpp"
+HOST_LIB_PATH = LIB_DIR / "_dlb_host.so"
 INCLUDE_DIR = PKG_DIR.parent / "include"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -163,8 +166,32 @@ def build_library(force: bool = False, verbose: bool = False, jobs: int | None =
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
+    build_host_module(force)
     build_probe_library(force)
     return LIB_PATH
+
+
+def build_host_module(force: bool = False) -> Path:
+    """Build ``_dlb_host.so``.  Host code only: no kernel and no HIP call of its own, so it goes
+    through the host compiler; HIP's headers (which torch's stream header includes) want the
+    platform named."""
+    if force or _stale(HOST_LIB_PATH, [HOST_SRC, *_headers()]):
+        import sysconfig
+
+        import torch
+
+        torch_dir = Path(torch.__file__).resolve().parent
+        LIB_DIR.mkdir(parents=True, exist_ok=True)
+        cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+               "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{INCLUDE_DIR}", f"-I{torch_dir / 'include'}",
+               f"-I{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+               f"-I{Path(HIPCC).resolve().parent.parent / 'include'}",
+               f"-I{sysconfig.get_paths()['include']}", str(HOST_SRC), "-o", str(HOST_LIB_PATH),
+               f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"{cmd[0]} failed for {HOST_SRC.name}:\n{proc.stderr}")
+    return HOST_LIB_PATH
 
 
 def build_probe_library(force: bool = False) -> Path:

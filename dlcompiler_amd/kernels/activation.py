@@ -14,6 +14,9 @@ def silu_and_mul(gate_up: torch.Tensor, out: torch.Tensor = None):
     ``gate_up.new_empty((M, N))`` when not given, and the result tensor is returned.  The
     kernel needs unit stride in the last dimension (rows may be strided).
     """
+    done = _lib.host().silu_and_mul(gate_up, out)
+    if done is not None:
+        return done
     assert gate_up.dim() == 2
     _lib.require_cuda(gate_up, out)
     M = gate_up.size(0)

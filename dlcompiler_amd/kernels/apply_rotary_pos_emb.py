@@ -22,6 +22,9 @@ def apply_rotary_pos_emb(
     token (any shape with ``numel == tokens * D``); ``q_embed``/``k_embed`` may be ``q``/``k``.
     Returns ``(q_embed, k_embed)``.
     """
+    done = _lib.host().apply_rotary_pos_emb(q, k, cos, sin, q_embed, k_embed)
+    if done is not None:
+        return done
     _lib.require_cuda(q, k)
     if cos.device != q.device:
         cos = cos.to(device=q.device)

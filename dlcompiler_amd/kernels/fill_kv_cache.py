@@ -20,6 +20,9 @@ def fill_kv_cache(
     block_offsets: Tensor,
 ):
     """fill key/value state to cache for paged attention (in place; returns None)."""
+    if _lib.host().fill_kv_cache(k_states, v_states, k_caches, v_caches, q_start_loc, q_seq_length,
+                                 kv_seq_length, block_offsets):
+        return
     _lib.require_cuda(k_states, v_states, k_caches, v_caches, block_offsets)
     if block_offsets.stride(-1) != 1:
         block_offsets = block_offsets.contiguous()

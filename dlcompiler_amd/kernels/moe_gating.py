@@ -115,19 +115,19 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     return sorted_ids, expert_ids, num_post
 
 
-_FUSED_PLANS = {}   # (T, E, k, block) -> (piece sizes, total words) of the result buffer
-_FUSED_MAX_TOKENS = 32768  # beyond this the fused entry point declines (DLB_ERR_UNSUPPORTED)
-
-
 def moe_topk_softmax_align(logits: torch.Tensor, k: int, block_size: int, num_experts: int = None,
                            renormalize: bool = True, return_counts: bool = False):
     """:func:`moe_topk_softmax` followed by :func:`moe_align_block_size` on its ids, as one
     native call of two launches (the router also produces the alignment's per-chunk expert
     counts).  Returns ``(weights, ids, sorted_token_ids, expert_ids, num_tokens_post_padded)``,
     bit for bit what the two functions return (plus the per-expert ``counts`` with
-    ``return_counts``).  More than 32768 tokens, or ``num_experts`` different from the router's
-    expert count, take the two separate calls.
+    ``return_counts``).  More than 32768 tokens, no tokens at all, or ``num_experts``
+    different from the router's expert count take the two separate calls.
     """
+    if num_experts is None or num_experts == logits.shape[-1]:
+        done = _lib.host().moe_topk_softmax_align(logits, k, block_size, renormalize)
+        if done is not None:
+            return done if return_counts else done[:5]
     assert logits.dim() == 2
     _lib.require_cuda(logits)
     T, E = logits.shape
@@ -137,43 +137,12 @@ def moe_topk_softmax_align(logits: torch.Tensor, k: int, block_size: int, num_ex
         raise ValueError(f"need 1 <= k <= num_experts, got k={k}, E={E}")
     if block_size < 1:
         raise ValueError("block_size must be positive")
-    if T > _FUSED_MAX_TOKENS or num_experts != E or k > 16 or E > 256:
-        weights, ids = moe_topk_softmax(logits, k, renormalize)
-        return (weights, ids) + tuple(moe_align_block_size(ids, block_size, num_experts,
-                                                           return_counts=return_counts))
     logits = _router_logits(logits)
-    dev = logits.device
-    numel = T * k
-    cap = numel + E * (block_size - 1)
-    nblk = max(1, -(-cap // block_size))
-    lib = _lib.load()
-    plan = _FUSED_PLANS.get((T, E, k, block_size))
-    if plan is None:
-        ws_words = max((lib.dlb_moe_topk_softmax_align_ws_bytes(T, E) + 3) // 4, 1)
-        # one allocation of 4-byte words, carved into the results and the scratch; every piece
-        # is rounded up to 16 bytes so that the next one starts aligned, and a piece that was
-        # rounded is trimmed afterwards (the one-word total goes last and needs neither)
-        sizes = (numel, numel, cap, nblk, ws_words, E, 1)
-        pieces = [n + (-n & 3) for n in sizes[:-1]] + [1]
-        if len(_FUSED_PLANS) > 64:
-            _FUSED_PLANS.clear()
-        trims = tuple(None if n == p else n for n, p in zip(sizes, pieces))
-        plan = _FUSED_PLANS[(T, E, k, block_size)] = (trims, pieces, sum(pieces))
-    trims, pieces, total = plan
-    buf = torch.empty((total,), dtype=torch.int32, device=dev)
-    parts = [t if n is None else t.narrow(0, 0, n) for t, n in zip(buf.split(pieces), trims)]
-    w_raw, ids, sorted_ids, expert_ids, ws, counts, num_post = parts
-    weights = w_raw.view(torch.float32).view(T, k)
-    ids = ids.view(T, k)
-    with _lib.device_guard(dev):
-        st = lib.dlb_moe_topk_softmax_align_f32(
-            logits.data_ptr(), weights.data_ptr(), ids.data_ptr(), T, E, k,
-            logits.stride(0) if T > 1 else E, _lib.torch_dtype_code(logits.dtype), int(bool(renormalize)),
-            block_size,
-            sorted_ids.data_ptr(), cap, expert_ids.data_ptr(), nblk, counts.data_ptr(),
-            num_post.data_ptr(),
-            ws.data_ptr(), ws.numel() * 4, _lib.current_stream_ptr(dev))
-    _lib.check(st, "dlb_moe_topk_softmax_align_f32")
-    if return_counts:
-        return weights, ids, sorted_ids, expert_ids, num_post, counts
-    return weights, ids, sorted_ids, expert_ids, num_post
+    done = None
+    if num_experts == E:
+        with _lib.device_guard(logits.device):
+            done = _lib.host().moe_topk_softmax_align(logits, k, block_size, renormalize)
+    if done is None:
+        weights, ids = moe_topk_softmax(logits, k, renormalize)
+        done = (weights, ids) + tuple(moe_align_block_size(ids, block_size, num_experts, return_counts=True))
+    return done if return_counts else done[:5]

@@ -33,6 +33,9 @@ def paged_attention_fwd(
     (paged_attention.py:560-607): the last ``q_seqlens[s]`` context positions of sequence
     ``s`` are its queries.  Sliding window and logit soft-capping apply to both.
     """
+    if _lib.host().paged_attention_fwd(q, k, v, o, block_offsets, q_start_loc, q_seqlens, kv_seqlens, max_seqlen,
+                                       window_size, sm_scale, logit_softcapping):
+        return
     _lib.require_cuda(q, k, v, o, block_offsets, kv_seqlens)
     if window_size is None:
         window_size = -1

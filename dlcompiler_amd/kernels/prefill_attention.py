@@ -14,6 +14,8 @@ def context_attention_fwd(q, k, v, o, b_start_loc, b_seq_len, max_input_len):
     ``Hq > Hkv``); sequence ``i`` owns rows ``b_start_loc[i] .. + b_seq_len[i]``.  As in the
     reference the softmax scale is ``1 / sqrt(D)`` and the function returns ``None``.
     """
+    if _lib.host().context_attention_fwd(q, k, v, o, b_start_loc, b_seq_len, max_input_len):
+        return
     _lib.require_cuda(q, k, v, o, b_start_loc, b_seq_len)
     Lq, Lk, Lv = q.shape[-1], k.shape[-1], v.shape[-1]
     assert Lq == Lk and Lk == Lv

@@ -19,6 +19,9 @@ def rms_norm(
 ):
     """rms norm; with ``residual`` returns ``(out, out_residual)`` where
     ``out_residual = hidden_states + residual`` is what gets normalised."""
+    done = _lib.host().rms_norm(hidden_states, weight, eps, residual, out, out_residual)
+    if done is not None:
+        return done
     _lib.require_cuda(hidden_states, weight, residual, out, out_residual)
     if not hidden_states.is_contiguous():
         hidden_states = hidden_states.contiguous()
