@@ -16,9 +16,12 @@
 //              start[chunk][e] + (number of earlier i' in the chunk with the same e), the rank
 //              coming from wave ballots, which makes the sort stable (ascending i per expert).
 // Integer work only; no float or order-dependent atomics, so the output is bit-reproducible.
+//
+// Up to kOneSlots routing slots (a decode step) all of it runs in ONE workgroup and one launch,
+// after the router itself where the caller asks for both.
 #include <mutex>
 
-#include "common.h"
+#include "moe_route.h"
 #include "quant_fp8.h"
 
 namespace dlb {
@@ -29,7 +32,6 @@ constexpr int kWaves = kThreads / kWave;
 constexpr int kChunk = 2048;  // flat ids per workgroup (large inputs)
 constexpr int kMaxE = 256;
 constexpr int kFusedChunks = 256;  // rows of the count table the fused placement kernel reduces
-static_assert(kFusedChunks == kRouteMaxChunks, "the fused router sizes its chunks for this table");
 
 // Flat ids per chunk (= per workgroup of the counting and the placement pass).  Inputs of up to
 // kFusedChunks * kChunk ids are cut into as many chunks as the fused placement kernel takes (256),
@@ -47,10 +49,364 @@ __host__ __device__ inline int64_t num_chunks(int64_t numel) {
   return numel > 0 ? (numel + c - 1) / c : 1;
 }
 
+// sets p[0 .. n) to v, as thread t of nt; 16 bytes per store where p is aligned
+__device__ __forceinline__ void fill_words(int32_t* __restrict__ p, int64_t n, int32_t v, int64_t t, int64_t nt) {
+  int64_t done = 0;
+  if ((reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
+    typedef __attribute__((ext_vector_type(4))) int i32x4;
+    const i32x4 q = {v, v, v, v};
+    for (int64_t i = t; i < n / 4; i += nt) ((i32x4*)p)[i] = q;
+    done = n / 4 * 4;
+  }
+  for (int64_t i = done + t; i < n; i += nt) p[i] = v;
+}
+
+// lanes of the wave holding the same expert, from ballots over the 9 key bits (bit 8 separates
+// the dropped entries, e = -1 -> key 0x1ff)
+__device__ __forceinline__ uint64_t same_expert(int32_t e) {
+  const uint32_t key = (uint32_t)e & 0x1ffu;
+  uint64_t peers = ~0ull;
+#pragma unroll
+  for (int b = 0; b < 9; ++b) {
+    const bool bit = (key >> b) & 1u;
+    const uint64_t m = __ballot(bit);
+    peers &= bit ? m : ~m;
+  }
+  return peers;
+}
+
+// totals (0 past E, 16-byte aligned) -> padded expert bases base_s[0 .. E], by one wave: four
+// experts per lane
+__device__ __forceinline__ void scan_bases(const int32_t* total_s, int32_t* base_s, int E, int block, int lane) {
+  typedef __attribute__((ext_vector_type(4))) int i32x4;
+  const i32x4 total = ((const i32x4*)total_s)[lane];
+  int32_t pad[4], sum = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    pad[c] = (int32_t)(((uint32_t)total[c] + (uint32_t)block - 1u) / (uint32_t)block * (uint32_t)block);
+    sum += pad[c];
+  }
+  int32_t run = wave_inclusive_scan(sum) - sum;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    if (4 * lane + c < E) base_s[4 * lane + c] = run;
+    run += pad[c];
+  }
+  if (lane == 63) base_s[E] = run;
+}
+
+// expert whose padded run holds position p (base_s[E] > p): the last one that starts at or before p
+__device__ __forceinline__ int expert_at(const int32_t* base_s, int E, int32_t p) {
+  int lo = 0, hi = E;  // base_s[lo] <= p < base_s[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (base_s[mid] <= p) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+struct AlignOut {
+  int32_t* sorted_ids;
+  int64_t sorted_cap;
+  int32_t* expert_ids;
+  int64_t expert_ids_cap;
+  int32_t* counts;  // may be null
+  int32_t* num_post_pad;
+  int64_t numel;
+  int E, block;
+};
+// block -> expert ids (-1 past the last block) and the padded total, as thread t of nt
+__device__ __forceinline__ void write_block_experts(const AlignOut& o, const int32_t* base_s, int t, int nt) {
+  const int32_t total_padded = base_s[o.E];
+  if (t == 0) *o.num_post_pad = total_padded;
+  for (int64_t b = t; b < o.expert_ids_cap; b += nt) {
+    const int64_t p = b * o.block;
+    o.expert_ids[b] = p < total_padded ? expert_at(base_s, o.E, (int32_t)p) : -1;
+  }
+}
+
+// ---- everything in one workgroup ------------------------------------------------------------
+// A launch costs more than the work of a few thousand slots, so up to kOneSlots of them are
+// counted, scanned and placed by one workgroup.  A wave takes consecutive slots, 64 at a time; its
+// running per-expert counts give every slot its rank inside the wave, one scan over the waves and
+// one over the experts turn ranks into positions.  The pad value is written everywhere first,
+// while the ids are on their way.  Router and alignment of 48 tokens x 6 of 64 experts (block 128):
+// 14.6 us a call in two launches, 5.8 us in this one; of 45 tokens x 8 of 256 experts, where the
+// pads used to be written by one workgroup expert by expert, 35.7 -> 11.0 us.
+constexpr int kOneThreads = 1024;
+constexpr int kOneWaves = kOneThreads / kWave;
+constexpr int kOneGroups = 4;  // slots per lane
+constexpr int kOneSlots = kOneThreads * kOneGroups;
+
+struct OneShared {
+  int32_t wave_cnt[kOneWaves][kMaxE];  // running counts of a wave, then its exclusive prefix
+  __attribute__((aligned(16))) int32_t total[kMaxE];
+  int32_t base[kMaxE + 1];
+};
+__device__ __forceinline__ void align_one_begin(const AlignOut& o, OneShared& s) {
+  fill_words(o.sorted_ids, o.sorted_cap, (int32_t)o.numel, threadIdx.x, kOneThreads);
+  for (int i = threadIdx.x; i < kOneWaves * kMaxE; i += kOneThreads) (&s.wave_cnt[0][0])[i] = 0;
+}
+// get(i): expert of slot i, or -1.  Between align_one_begin and this call lies a barrier.
+template <typename Get>
+__device__ __forceinline__ void align_one_workgroup(const AlignOut& o, OneShared& s, Get get) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int numel = (int)o.numel, E = o.E;
+  const int per = (numel + kOneThreads - 1) / kOneThreads * kWave;  // slots per wave
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int32_t e[kOneGroups], rank[kOneGroups];
+#pragma unroll
+  for (int g = 0; g < kOneGroups; ++g) {
+    const int i = wave * per + g * kWave + lane;
+    e[g] = (g * kWave < per && i < numel) ? get(i) : -1;
+    rank[g] = 0;
+  }
+#pragma unroll
+  for (int g = 0; g < kOneGroups; ++g) {
+    if (g * kWave < per) {
+      const uint64_t peers = same_expert(e[g]);
+      const int r = __popcll(peers & lt_mask);
+      if (e[g] >= 0) {
+        const int32_t before = s.wave_cnt[wave][e[g]];
+        rank[g] = before + r;
+        // (the wave's own row: its LDS operations complete in order)
+        if (r == 0) s.wave_cnt[wave][e[g]] = before + __popcll(peers);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  __syncthreads();
+  if (tid < kMaxE) {  // (nothing was counted past E)
+    int32_t run = 0;
+#pragma unroll
+    for (int w = 0; w < kOneWaves; ++w) {
+      const int32_t c = s.wave_cnt[w][tid];
+      s.wave_cnt[w][tid] = run;
+      run += c;
+    }
+    s.total[tid] = run;
+    if (tid < E && o.counts) o.counts[tid] = run;
+  }
+  __syncthreads();
+  if (wave == 0) scan_bases(s.total, s.base, E, o.block, lane);
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < kOneGroups; ++g)
+    if (e[g] >= 0)
+      o.sorted_ids[s.base[e[g]] + s.wave_cnt[wave][e[g]] + rank[g]] = wave * per + g * kWave + lane;
+  write_block_experts(o, s.base, tid, kOneThreads);
+}
+
+__device__ __forceinline__ void align_one_ids(const AlignOut& o, const IdxArray ids) {
+  __shared__ OneShared s;
+  align_one_begin(o, s);
+  __syncthreads();
+  align_one_workgroup(o, s, [&](int i) {
+    const int32_t e = ids[i];
+    return (e >= 0 && e < o.E) ? e : -1;
+  });
+}
+__global__ __launch_bounds__(kOneThreads) void align_one_kernel(const AlignOut o, const IdxArray ids) {
+  align_one_ids(o, ids);
+}
+// ... with the fp8 activation quantiser on the other workgroups (see align_place_quant_kernel)
+static_assert(kOneThreads % kQuantThreads == 0, "whole quantiser blocks per workgroup");
+constexpr int kOneQuantBlocks = kOneThreads / kQuantThreads;
+template <int DT>
+__global__ __launch_bounds__(kOneThreads) void align_one_quant_kernel(const AlignOut o, const IdxArray ids,
+                                                                      const QuantParams q) {
+  if (blockIdx.x == 0) align_one_ids(o, ids);
+  else
+    quant_fp8_group128_block<DT>(q, ((int64_t)blockIdx.x - 1) * kOneQuantBlocks + threadIdx.x / kQuantThreads,
+                                 threadIdx.x % kQuantThreads);
+}
+
+// ---- router and alignment -------------------------------------------------------------------
+struct RouteParams {
+  const void* logits;
+  float* weights;
+  int32_t* ids;
+  int64_t T;
+  int E, K;
+  int64_t ld;
+  int renorm, vec_ok;
+};
+
+// Router, then the alignment of its own selections, in one workgroup: 64 tokens per pass.
+constexpr int kOneTokens = 256;
+template <int VPL, int LT>
+__global__ __launch_bounds__(kOneThreads) void route_align_one_kernel(const RouteParams p, const AlignOut o) {
+  __shared__ OneShared s;
+  __shared__ int32_t ids_s[kOneSlots];
+  const int row = threadIdx.x >> 4;
+  float v[VPL];
+  load_token_logits<VPL, LT>(p.logits, row, row < p.T, p.E, p.ld, p.vec_ok, v);
+  align_one_begin(o, s);
+  for (int64_t first = 0; first < p.T; first += 64) {
+    const int64_t token = first + row;
+    float next[VPL];
+    load_token_logits<VPL, LT>(p.logits, token + 64, token + 64 < p.T, p.E, p.ld, p.vec_ok, next);
+    const int32_t e = route_token<VPL, LT>(v, p.weights, p.ids, token, token < p.T, p.E, p.K, p.renorm);
+    if (e >= 0) ids_s[token * p.K + (threadIdx.x & 15)] = e;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) v[j] = next[j];
+  }
+  __syncthreads();
+  align_one_workgroup(o, s, [&](int i) { return ids_s[i]; });
+}
+
+// More tokens: two launches.  First the router, 64 * PASSES tokens per workgroup, which also
+// writes a row of the [chunks, E] count table: the experts selected by exactly those tokens.  A
+// token selects an expert at most once, so a count fits a byte, and the table the second launch
+// reduces in every workgroup is a quarter of what 32-bit counts take.  The pad value goes
+// everywhere meanwhile (the second launch scatters the slots over it).  Both launches are bound by
+// latency: 16384 tokens x 6 of 64 experts 15.7 -> 12.8 us a call, 9336 x 8 of 256 43.9 -> 16.6 us.
+template <int VPL, int PASSES, int LT>
+__global__ __launch_bounds__(kOneThreads) void route_count_kernel(const RouteParams p, const AlignOut o,
+                                                                  uint32_t* __restrict__ table) {
+  static_assert(64 * PASSES < 256, "counts are bytes");
+  __shared__ int32_t hist[kMaxE];
+  if (threadIdx.x < kMaxE) hist[threadIdx.x] = 0;
+  const int64_t first = (int64_t)blockIdx.x * (64 * PASSES);
+  float v[PASSES][VPL];
+#pragma unroll
+  for (int pass = 0; pass < PASSES; ++pass) {  // all loads first: one memory round trip
+    const int64_t token = first + pass * 64 + (threadIdx.x >> 4);
+    load_token_logits<VPL, LT>(p.logits, token, token < p.T, p.E, p.ld, p.vec_ok, v[pass]);
+  }
+  fill_words(o.sorted_ids, o.sorted_cap, (int32_t)o.numel, (int64_t)blockIdx.x * kOneThreads + threadIdx.x,
+             (int64_t)gridDim.x * kOneThreads);
+  __syncthreads();
+#pragma unroll
+  for (int pass = 0; pass < PASSES; ++pass) {
+    const int64_t token = first + pass * 64 + (threadIdx.x >> 4);
+    const int32_t e = route_token<VPL, LT>(v[pass], p.weights, p.ids, token, token < p.T, p.E, p.K, p.renorm);
+    if (e >= 0) atomicAdd(&hist[e], 1);  // integer add: order-insensitive
+  }
+  __syncthreads();
+  const int words = (p.E + 3) / 4;
+  if (threadIdx.x < words) {
+    const int e = 4 * threadIdx.x;  // (entries past E are zero)
+    table[(int64_t)blockIdx.x * words + threadIdx.x] = (uint32_t)hist[e] | (uint32_t)hist[e + 1] << 8 |
+                                                       (uint32_t)hist[e + 2] << 16 | (uint32_t)hist[e + 3] << 24;
+  }
+}
+
+// Second launch: every workgroup reduces the count table itself (expert totals and the part of
+// them in earlier chunks) and places its chunk.  The ranks inside the chunk need nothing from the
+// table, so they are worked out while its rows are on their way.
+constexpr int kRouteGroups = 8;  // slots per lane: chunks of up to 128 tokens x 16
+__global__ __launch_bounds__(kThreads) void route_place_kernel(const IdxArray ids, const AlignOut o,
+                                                               const uint32_t* __restrict__ table, int chunks,
+                                                               int chunk_ids) {
+  __shared__ int32_t wave_cnt[kWaves][kMaxE];
+  __shared__ __attribute__((aligned(16))) int32_t total_s[kMaxE];
+  __shared__ int32_t before_s[kMaxE];
+  __shared__ int32_t base_s[kMaxE + 1];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int E = o.E, me = blockIdx.x;
+  const int64_t begin = (int64_t)me * chunk_ids;
+  const int count = (int)(begin + chunk_ids < o.numel ? chunk_ids : o.numel - begin);
+  const int per = (count + kThreads - 1) / kThreads * kWave;  // slots per wave
+  int32_t e[kRouteGroups], rank[kRouteGroups];
+#pragma unroll
+  for (int g = 0; g < kRouteGroups; ++g) {
+    const int i = wave * per + g * kWave + lane;
+    e[g] = (g * kWave < per && i < count) ? ids[begin + i] : -1;
+    rank[g] = 0;
+  }
+  // table columns of four experts: thread = (column tid % W, rows tid / W, + 256 / W, ...)
+  const int words = (E + 3) / 4, W = words <= 16 ? 16 : words <= 32 ? 32 : 64;
+  const int col = tid % W, slices = kThreads / W;
+  const bool live = col < words;
+  uint32_t tot_lo = 0, tot_hi = 0, bef_lo = 0, bef_hi = 0;  // 16-bit sums of experts 0, 2 and 1, 3 of the column
+  constexpr int kRowsInFlight = 16;
+  uint32_t n[kRowsInFlight];
+  auto request = [&](int r0) {
+#pragma unroll
+    for (int u = 0; u < kRowsInFlight; ++u)
+      n[u] = (live && r0 + u * slices < chunks) ? table[(int64_t)(r0 + u * slices) * words + col] : 0u;
+  };
+  auto collect = [&](int r0) {
+#pragma unroll
+    for (int u = 0; u < kRowsInFlight; ++u) {
+      const uint32_t lo = n[u] & 0x00ff00ffu, hi = (n[u] >> 8) & 0x00ff00ffu;
+      tot_lo += lo;
+      tot_hi += hi;
+      if (r0 + u * slices < me) {
+        bef_lo += lo;
+        bef_hi += hi;
+      }
+    }
+  };
+  request(tid / W);
+  for (int i = tid; i < kWaves * kMaxE; i += kThreads) (&wave_cnt[0][0])[i] = 0;
+  total_s[tid] = 0;
+  before_s[tid] = 0;
+  __syncthreads();
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int g = 0; g < kRouteGroups; ++g) {
+    if (g * kWave < per) {
+      const uint64_t peers = same_expert(e[g]);
+      const int r = __popcll(peers & lt_mask);
+      if (e[g] >= 0) {
+        const int32_t before = wave_cnt[wave][e[g]];
+        rank[g] = before + r;
+        if (r == 0) wave_cnt[wave][e[g]] = before + __popcll(peers);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  collect(tid / W);
+  for (int r0 = tid / W + kRowsInFlight * slices; r0 < chunks; r0 += kRowsInFlight * slices) {
+    request(r0);
+    collect(r0);
+  }
+  if (live) {
+    const int e0 = 4 * col;
+    atomicAdd(&total_s[e0], (int)(tot_lo & 0xffffu));
+    atomicAdd(&total_s[e0 + 1], (int)(tot_hi & 0xffffu));
+    atomicAdd(&total_s[e0 + 2], (int)(tot_lo >> 16));
+    atomicAdd(&total_s[e0 + 3], (int)(tot_hi >> 16));
+    atomicAdd(&before_s[e0], (int)(bef_lo & 0xffffu));
+    atomicAdd(&before_s[e0 + 1], (int)(bef_hi & 0xffffu));
+    atomicAdd(&before_s[e0 + 2], (int)(bef_lo >> 16));
+    atomicAdd(&before_s[e0 + 3], (int)(bef_hi >> 16));
+  }
+  __syncthreads();
+  if (wave == 0) scan_bases(total_s, base_s, E, o.block, lane);
+  __syncthreads();
+  if (tid < E) {  // first position of each wave's slots of expert tid
+    int32_t run = base_s[tid] + before_s[tid];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int32_t c = wave_cnt[w][tid];
+      wave_cnt[w][tid] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < kRouteGroups; ++g)
+    if (e[g] >= 0)
+      o.sorted_ids[wave_cnt[wave][e[g]] + rank[g]] = (int32_t)(begin + wave * per + g * kWave + lane);
+  if (me == chunks - 1) {  // the last chunk is the shortest
+    if (tid < E && o.counts) o.counts[tid] = total_s[tid];
+    write_block_experts(o, base_s, tid, kThreads);
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void align_count_kernel(const IdxArray ids,
                                                                int64_t numel, int E, int chunk_ids,
-                                                               int32_t* __restrict__ chunk_counts) {
+                                                               int32_t* __restrict__ chunk_counts,
+                                                               int32_t* __restrict__ sorted_ids,
+                                                               int64_t sorted_cap) {
   __shared__ int32_t hist[kMaxE];
+  // (the pad value goes everywhere here; the placement scatters the slots over it)
+  fill_words(sorted_ids, sorted_cap, (int32_t)numel, (int64_t)blockIdx.x * kThreads + threadIdx.x,
+             (int64_t)gridDim.x * kThreads);
   for (int e = threadIdx.x; e < E; e += kThreads) hist[e] = 0;
   __syncthreads();
   const int64_t begin = (int64_t)blockIdx.x * chunk_ids;
@@ -69,12 +425,10 @@ __global__ __launch_bounds__(kThreads) void align_count_kernel(const IdxArray id
 constexpr int kScanThreads = 1024;
 
 __global__ __launch_bounds__(kScanThreads) void align_scan_kernel(
-    int32_t* __restrict__ chunk_counts /* in: counts, out: start offsets */, int64_t chunks, int E,
-    int block, int32_t numel, int32_t* __restrict__ sorted_ids, int64_t sorted_cap,
-    int32_t* __restrict__ expert_ids, int64_t expert_ids_cap, int32_t* __restrict__ counts,
-    int32_t* __restrict__ num_post_pad) {
+    int32_t* __restrict__ chunk_counts /* in: counts, out: start offsets */, int64_t chunks, const AlignOut o) {
+  const int E = o.E, block = o.block;
   __shared__ int32_t part_s[kScanThreads];  // [group][expert'] slice totals -> slice bases
-  __shared__ int32_t total_s[kMaxE];
+  __shared__ __attribute__((aligned(16))) int32_t total_s[kMaxE];
   __shared__ int32_t base_s[kMaxE + 1];
   const int tid = threadIdx.x;
   const int ep = (E + 63) & ~63;           // experts rounded up to a whole wave
@@ -97,29 +451,12 @@ __global__ __launch_bounds__(kScanThreads) void align_scan_kernel(
       run += v;
     }
     total_s[tid] = run;
+  } else if (tid < kMaxE) {
+    total_s[tid] = 0;
   }
   __syncthreads();
-  if (tid < 64) {  // padded totals -> expert bases: wave scan over up to 256 experts
-    int32_t run = 0;
-    for (int i0 = 0; i0 < E; i0 += 64) {
-      const int i = i0 + tid;
-      const int32_t padded = (i < E) ? (int32_t)(ceil_div(total_s[i], block) * block) : 0;
-      int32_t incl = padded;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int32_t up = __shfl_up(incl, d);
-        if (tid >= d) incl += up;
-      }
-      if (i < E) base_s[i] = run + incl - padded;
-      run += __shfl(incl, 63);
-    }
-    if (tid == 0) {
-      base_s[E] = run;
-      *num_post_pad = run;
-    }
-  }
+  if (tid < 64) scan_bases(total_s, base_s, E, block, tid);
   __syncthreads();
-  const int32_t total_padded = base_s[E];
   if (live) {
     // chunk start offsets of this slice for the placement pass
     int32_t run = base_s[e] + part_s[q * ep + e];
@@ -129,16 +466,8 @@ __global__ __launch_bounds__(kScanThreads) void align_scan_kernel(
       run += n;
     }
   }
-  if (tid < E) {
-    const int32_t base = base_s[tid], total = total_s[tid], next = base_s[tid + 1];
-    if (counts) counts[tid] = total;
-    for (int32_t p = base + total; p < next; ++p) sorted_ids[p] = numel;   // pad slots
-    for (int32_t b = base / block; b < next / block; ++b) expert_ids[b] = tid;
-  }
-  // tails beyond the padded total
-  for (int64_t p = (int64_t)total_padded + tid; p < sorted_cap; p += kScanThreads) sorted_ids[p] = numel;
-  for (int64_t b = (int64_t)total_padded / block + tid; b < expert_ids_cap; b += kScanThreads)
-    expert_ids[b] = -1;
+  if (tid < E && o.counts) o.counts[tid] = total_s[tid];
+  write_block_experts(o, base_s, tid, kScanThreads);
 }
 
 __global__ __launch_bounds__(kThreads) void align_place_kernel(
@@ -162,16 +491,7 @@ __global__ __launch_bounds__(kThreads) void align_place_kernel(
       e = ids[i];
       if (e < 0 || e >= E) e = -1;
     }
-    // lanes of this wave holding the same expert: intersect ballots over the 9 key bits
-    // (bit 8 separates the dropped entries, e = -1 -> key 0x1ff).
-    const uint32_t key = (uint32_t)e & 0x1ffu;
-    uint64_t peers = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 9; ++b) {
-      const bool bit = (key >> b) & 1u;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
+    const uint64_t peers = same_expert(e);
     const int rank_in_wave = __popcll(peers & lt_mask);
     const int peer_count = __popcll(peers);
     if (e >= 0 && rank_in_wave == 0) wave_cnt[wave][e] = peer_count;
@@ -198,36 +518,24 @@ __global__ __launch_bounds__(kThreads) void align_place_kernel(
 // Scan and placement in one launch, for inputs of up to kFusedChunks chunks: every workgroup
 // reduces the (small) [chunks, E] count table itself -- expert totals, padded expert bases and
 // the offsets of its own chunk -- instead of waiting for a separate one-workgroup scan kernel;
-// one extra workgroup emits what the scan kernel emits (counts, block -> expert ids, pad slots,
-// tails, padded total).  The table is only read here.
+// one extra workgroup emits what the scan kernel emits (counts, block -> expert ids, padded total).  The table is only read here.
 struct PlaceParams {
   IdxArray ids;  // int32 or int64 (the routing ids as torch.topk returns them)
-  int64_t numel;
-  int E, block;
   const int32_t* chunk_counts;
   int chunks, chunk_ids;
-  int32_t* sorted_ids;
-  int64_t sorted_cap;
-  int32_t* expert_ids;
-  int64_t expert_ids_cap;
-  int32_t* counts;
-  int32_t* num_post_pad;
+  AlignOut out;
 };
 
 // the work of workgroup `me` (0 .. chunks) of the fused scan + placement
 __device__ __forceinline__ void align_place_fused_block(const PlaceParams& pp, const int me) {
   const IdxArray ids = pp.ids;
-  const int64_t numel = pp.numel;
-  const int E = pp.E, block = pp.block, chunks = pp.chunks, chunk_ids = pp.chunk_ids;
+  const int64_t numel = pp.out.numel;
+  const int E = pp.out.E, chunks = pp.chunks, chunk_ids = pp.chunk_ids;
   const int32_t* __restrict__ chunk_counts = pp.chunk_counts;
-  int32_t* __restrict__ sorted_ids = pp.sorted_ids;
-  const int64_t sorted_cap = pp.sorted_cap, expert_ids_cap = pp.expert_ids_cap;
-  int32_t* __restrict__ expert_ids = pp.expert_ids;
-  int32_t* __restrict__ counts = pp.counts;
-  int32_t* __restrict__ num_post_pad = pp.num_post_pad;
+  int32_t* __restrict__ sorted_ids = pp.out.sorted_ids;
   __shared__ int32_t cursor[kMaxE];            // next free slot per expert for this chunk
   __shared__ int32_t wave_cnt[kWaves][kMaxE];  // per-tile, per-wave counts
-  __shared__ int32_t total_s[kMaxE];
+  __shared__ __attribute__((aligned(16))) int32_t total_s[kMaxE];
   __shared__ int32_t base_s[kMaxE + 1];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -292,41 +600,18 @@ __device__ __forceinline__ void align_place_fused_block(const PlaceParams& pp, c
       before += part[kThreads + q * ep + tid];
     }
     total_s[tid] = total;
+  } else {
+    total_s[tid] = 0;
   }
   __syncthreads();
   for (int i = tid; i < kWaves * kMaxE; i += kThreads) (&wave_cnt[0][0])[i] = 0;
   __syncthreads();
-  if (tid < 64) {  // padded totals -> expert bases: wave scan over up to 256 experts
-    int32_t run = 0;
-    for (int i0 = 0; i0 < E; i0 += 64) {
-      const int i = i0 + tid;
-      const int32_t padded = (i < E) ? (int32_t)(ceil_div(total_s[i], block) * block) : 0;
-      int32_t incl = padded;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int32_t up = __shfl_up(incl, d);
-        if (tid >= d) incl += up;
-      }
-      if (i < E) base_s[i] = run + incl - padded;
-      run += __shfl(incl, 63);
-    }
-    if (tid == 0) base_s[E] = run;
-  }
+  if (tid < 64) scan_bases(total_s, base_s, E, pp.out.block, tid);
   __syncthreads();
   if (tid < E) cursor[tid] = base_s[tid] + before;
   if (me == chunks) {  // the extra workgroup: what the scan kernel emits besides offsets
-    const int32_t total_padded = base_s[E];
-    if (tid == 0) *num_post_pad = total_padded;
-    if (tid < E) {
-      const int32_t base = base_s[tid], total = total_s[tid], next = base_s[tid + 1];
-      if (counts) counts[tid] = total;
-      for (int32_t q = base + total; q < next; ++q) sorted_ids[q] = (int32_t)numel;  // pad slots
-      for (int32_t b = base / block; b < next / block; ++b) expert_ids[b] = tid;
-    }
-    for (int64_t q = (int64_t)total_padded + tid; q < sorted_cap; q += kThreads)
-      sorted_ids[q] = (int32_t)numel;
-    for (int64_t b = (int64_t)total_padded / block + tid; b < expert_ids_cap; b += kThreads)
-      expert_ids[b] = -1;
+    if (tid < E && pp.out.counts) pp.out.counts[tid] = total_s[tid];
+    write_block_experts(pp.out, base_s, tid, kThreads);
     return;
   }
   __syncthreads();
@@ -336,15 +621,7 @@ __device__ __forceinline__ void align_place_fused_block(const PlaceParams& pp, c
     const int64_t i = tile + tid;
     const int32_t e = e_next;
     e_next = load_expert(tile + kThreads);
-    // lanes of this wave holding the same expert: intersect ballots over the 9 key bits
-    const uint32_t key = (uint32_t)e & 0x1ffu;
-    uint64_t peers = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 9; ++b) {
-      const bool bit = (key >> b) & 1u;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
+    const uint64_t peers = same_expert(e);
     const int rank_in_wave = __popcll(peers & lt_mask);
     const int peer_count = __popcll(peers);
     if (e >= 0 && rank_in_wave == 0) wave_cnt[wave][e] = peer_count;
@@ -381,7 +658,7 @@ __global__ __launch_bounds__(kThreads) void align_place_quant_kernel(const Place
                                                                      const QuantParams q) {
   const int nplace = pp.chunks + 1;
   if ((int)blockIdx.x < nplace) align_place_fused_block(pp, blockIdx.x);
-  else quant_fp8_group128_block<DT>(q, (int64_t)blockIdx.x - nplace);
+  else quant_fp8_group128_block<DT>(q, (int64_t)blockIdx.x - nplace, threadIdx.x);
 }
 
 }  // namespace
@@ -415,15 +692,27 @@ int launch_align(const IdxArray topk_ids, int64_t numel, int E, int block, int32
                  int64_t sorted_cap, int32_t* expert_ids, int64_t expert_ids_cap, int32_t* counts,
                  int32_t* num_post_pad, int32_t* chunk_counts, hipStream_t s,
                  const QuantParams* quant = nullptr, int quant_dtype = DLB_DTYPE_BF16) {
+  const AlignOut out = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block};
+  if (numel <= kOneSlots) {
+    if (quant && quant->total_groups > 0) {
+      const uint32_t grid = (uint32_t)(1 + ceil_div(quant->total_groups, kQuantGroupsPerBlock * kOneQuantBlocks));
+      if (quant_dtype == DLB_DTYPE_BF16)
+        hipLaunchKernelGGL(align_one_quant_kernel<DLB_DTYPE_BF16>, dim3(grid), dim3(kOneThreads), 0, s, out,
+                           topk_ids, *quant);
+      else
+        hipLaunchKernelGGL(align_one_quant_kernel<DLB_DTYPE_F16>, dim3(grid), dim3(kOneThreads), 0, s, out,
+                           topk_ids, *quant);
+    } else {
+      hipLaunchKernelGGL(align_one_kernel, dim3(1), dim3(kOneThreads), 0, s, out, topk_ids);
+    }
+    return launch_status();
+  }
   const int64_t chunks = num_chunks(numel);
   const int chunk_ids = chunk_ids_for(numel);
   hipLaunchKernelGGL(align_count_kernel, dim3((uint32_t)chunks), dim3(kThreads), 0, s, topk_ids,
-                     numel, E, chunk_ids, chunk_counts);
+                     numel, E, chunk_ids, chunk_counts, sorted_ids, sorted_cap);
   if (chunks <= kFusedChunks) {
-    // (with numel = 0 the single chunk is empty: the extra workgroup still writes pads, tails and totals)
-    const PlaceParams pp = {topk_ids,   numel,      E,          block,          chunk_counts, (int)chunks,
-                            chunk_ids,  sorted_ids, sorted_cap, expert_ids,     expert_ids_cap,
-                            counts,     num_post_pad};
+    const PlaceParams pp = {topk_ids, chunk_counts, (int)chunks, chunk_ids, out};
     if (quant && quant->total_groups > 0) {
       const uint32_t grid = (uint32_t)(chunks + 1 + ceil_div(quant->total_groups, kQuantGroupsPerBlock));
       if (quant_dtype == DLB_DTYPE_BF16)
@@ -436,12 +725,9 @@ int launch_align(const IdxArray topk_ids, int64_t numel, int E, int block, int32
     return launch_status();
   }
   if (quant) return DLB_ERR_UNSUPPORTED;  // (the caller launches the quantiser on its own then)
-  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_counts, chunks, E, block,
-                     (int32_t)numel, sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts,
-                     num_post_pad);
-  if (numel > 0)
-    hipLaunchKernelGGL(align_place_kernel, dim3((uint32_t)chunks), dim3(kThreads), 0, s, topk_ids,
-                       numel, E, chunk_counts, sorted_ids);
+  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_counts, chunks, out);
+  hipLaunchKernelGGL(align_place_kernel, dim3((uint32_t)chunks), dim3(kThreads), 0, s, topk_ids, numel, E,
+                     chunk_counts, sorted_ids);
   return launch_status();
 }
 
@@ -543,14 +829,40 @@ extern "C" int dlb_moe_align_block_size_static(const void* topk_ids, int ids_int
 }
 
 // ---------------------------------------------------------------------------------------
-// Router and alignment as one pipeline of two launches: the router kernel also writes the
+// Router and alignment as one pipeline: one workgroup up to kOneTokens tokens, else the router with
 // per-chunk expert counts (a chunk = the K routing slots of route_chunk_tokens(T) consecutive
-// tokens), so the alignment's own counting pass over the ids is not needed.
+// tokens) and the placement.
 // ---------------------------------------------------------------------------------------
+namespace dlb {
+namespace {
+
+// tokens per workgroup of the router: 64 (one pass) while that keeps the count table within
+// kFusedChunks rows, else 128 (two passes)
+int route_chunk_tokens(int64_t T) { return (T + 63) / 64 <= kFusedChunks ? 64 : 128; }
+
+template <int VPL, int LT>
+void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table, hipStream_t s) {
+  if (p.T <= kOneTokens && o.numel <= kOneSlots) {
+    hipLaunchKernelGGL((route_align_one_kernel<VPL, LT>), dim3(1), dim3(kOneThreads), 0, s, p, o);
+    return;
+  }
+  const int chunk_tokens = route_chunk_tokens(p.T);
+  const int chunks = (int)ceil_div(p.T, chunk_tokens);
+  if (chunk_tokens == 64)
+    hipLaunchKernelGGL((route_count_kernel<VPL, 1, LT>), dim3(chunks), dim3(kOneThreads), 0, s, p, o, table);
+  else
+    hipLaunchKernelGGL((route_count_kernel<VPL, 2, LT>), dim3(chunks), dim3(kOneThreads), 0, s, p, o, table);
+  hipLaunchKernelGGL(route_place_kernel, dim3(chunks), dim3(kThreads), 0, s, IdxArray{p.ids, 0}, o, table, chunks,
+                     chunk_tokens * p.K);
+}
+
+}  // namespace
+}  // namespace dlb
+
 extern "C" size_t dlb_moe_topk_softmax_align_ws_bytes(int64_t T, int E) {
   if (T < 0 || E < 1) return 0;
   const int64_t chunks = T > 0 ? dlb::ceil_div(T, dlb::route_chunk_tokens(T)) : 1;
-  return (size_t)chunks * (size_t)E * sizeof(int32_t);
+  return (size_t)chunks * (size_t)((E + 3) / 4) * sizeof(uint32_t);
 }
 
 extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights, int32_t* ids,
@@ -578,19 +890,19 @@ extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights
   if (expert_ids_cap < ceil_div(sorted_cap, block)) return DLB_ERR_BAD_ARG;
   if (!ws || ws_bytes < dlb_moe_topk_softmax_align_ws_bytes(T, E)) return DLB_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
-  int32_t* chunk_counts = (int32_t*)ws;
-  if (T > 0) {
-    const int st = launch_topk_softmax_count(logits, logits_dtype, weights, ids, T, E, K, ld_logits,
-                                             renormalize, chunk_tokens, chunk_counts, s);
-    if (st != DLB_OK) return st;
-  } else {
-    // no tokens: the single chunk is empty, but its row of the table is still read
-    hipLaunchKernelGGL(align_count_kernel, dim3(1), dim3(kThreads), 0, s, IdxArray{ids, 0}, (int64_t)0, E,
-                       kChunk, chunk_counts);
-  }
-  const PlaceParams pp = {IdxArray{ids, 0}, numel, E, block, chunk_counts, (int)chunks,
-                          chunk_tokens * K, sorted_ids, sorted_cap, expert_ids, expert_ids_cap,
-                          counts,     num_post_pad};
-  hipLaunchKernelGGL(align_place_fused_kernel, dim3((uint32_t)chunks + 1), dim3(kThreads), 0, s, pp);
+  const RouteParams p = {logits, weights, ids, T, E, K, ld_logits, renormalize,
+                         (int)(logits_vector_ok(logits, logits_dtype, ld_logits) && (E == 64 || E == 128 || E == 256))};
+  const AlignOut o = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block};
+  uint32_t* table = (uint32_t*)ws;
+#define DLB_LAUNCH_ROUTE_ALIGN(VPL_)                                                                   \
+  do {                                                                                                 \
+    if (logits_dtype == DLB_DTYPE_F32) launch_route_align<VPL_, DLB_DTYPE_F32>(p, o, table, s);        \
+    else if (logits_dtype == DLB_DTYPE_BF16) launch_route_align<VPL_, DLB_DTYPE_BF16>(p, o, table, s); \
+    else launch_route_align<VPL_, DLB_DTYPE_F16>(p, o, table, s);                                      \
+  } while (0)
+  if (E <= 64) DLB_LAUNCH_ROUTE_ALIGN(4);
+  else if (E <= 128) DLB_LAUNCH_ROUTE_ALIGN(8);
+  else DLB_LAUNCH_ROUTE_ALIGN(16);
+#undef DLB_LAUNCH_ROUTE_ALIGN
   return launch_status();
 }

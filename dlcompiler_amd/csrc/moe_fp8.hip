@@ -49,7 +49,7 @@ constexpr float kWScaleFloor = 1e-12f;
 // ---------------------------------------------------------------------------------------
 template <int DT>
 __global__ __launch_bounds__(kQuantThreads) void quant_fp8_group128_kernel(const QuantParams q) {
-  quant_fp8_group128_block<DT>(q, blockIdx.x);
+  quant_fp8_group128_block<DT>(q, blockIdx.x, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------

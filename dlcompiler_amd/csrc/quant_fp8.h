@@ -34,18 +34,18 @@ struct QuantParams {
   int64_t ldx, ldq, lds;
 };
 
-// the work of workgroup `block` (kQuantThreads threads): one DPP row (16 lanes x 8 elements) per
+// the work of thread `tid` of block `block` (kQuantThreads threads): one DPP row (16 lanes x 8 elements) per
 // 128-element group, kQuantUnroll groups per row
 template <int DT>
-__device__ __forceinline__ void quant_fp8_group128_block(const QuantParams& q, int64_t block) {
-  const int lane16 = threadIdx.x & 15;
+__device__ __forceinline__ void quant_fp8_group128_block(const QuantParams& q, int64_t block, int tid) {
+  const int lane16 = tid & 15;
   int64_t row[kQuantUnroll];
   int gc[kQuantUnroll];
   bool live[kQuantUnroll];
   u32x4 raw[kQuantUnroll];
 #pragma unroll
   for (int u = 0; u < kQuantUnroll; ++u) {
-    const int64_t gidx = (block * kQuantUnroll + u) * 16 + (threadIdx.x >> 4);
+    const int64_t gidx = (block * kQuantUnroll + u) * 16 + (tid >> 4);
     live[u] = gidx < q.total_groups;
     row[u] = live[u] ? gidx / q.groups_per_row : 0;
     gc[u] = live[u] ? (int)(gidx - row[u] * q.groups_per_row) : 0;

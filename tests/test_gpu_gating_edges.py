@@ -1,0 +1,35 @@
+"""GPU parity of the router + alignment around the sizes where the launch changes: one workgroup up to
+256 tokens / 4096 slots, 64- and 128-token chunks beyond."""
+import pytest
+import torch
+
+from oracle import moe_gating as og
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,k,block", [(256, 256, 16, 128), (257, 256, 16, 128), (256, 13, 3, 16), (257, 13, 3, 16),
+                                         (192, 128, 8, 1), (16384, 255, 2, 128), (16448, 256, 16, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_and_alignment_at_launch_edges(dev, T, E, k, block, dtype):
+    from dlcompiler_amd.kernels.moe_gating import moe_topk_softmax_align
+
+    logits = torch.randn((T, E), generator=torch.Generator().manual_seed(T + E)).to(dtype)
+    w, ids, slots, experts, total, counts = moe_topk_softmax_align(logits.to(dev), k, block, return_counts=True)
+    rw, rids = og.topk_softmax(logits.float(), k)
+    rs, re_, rn, rc = og.align_block_size(rids, block, E)
+    assert torch.equal(ids.cpu(), rids) and torch.equal(slots.cpu(), rs) and torch.equal(experts.cpu(), re_)
+    assert int(total.item()) == int(rn.item()) and torch.equal(counts.cpu(), rc.to(torch.int32))
+    torch.testing.assert_close(w.cpu(), rw, rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("numel", [0, 1, 63, 1023, 1025, 4096, 4097])
+@pytest.mark.parametrize("E,block", [(256, 128), (5, 16)])
+def test_alignment_of_given_ids_at_launch_edges(dev, numel, E, block):
+    from dlcompiler_amd.kernels.moe_gating import moe_align_block_size
+
+    ids = torch.randint(-1, E + 1, (numel, 1), generator=torch.Generator().manual_seed(numel), dtype=torch.int32)
+    slots, experts, total, counts = moe_align_block_size(ids.to(dev), block, E, return_counts=True)
+    rs, re_, rn, rc = og.align_block_size(ids, block, E)
+    assert torch.equal(slots.cpu(), rs) and torch.equal(experts.cpu(), re_)
+    assert int(total.item()) == int(rn.item()) and torch.equal(counts.cpu(), rc.to(torch.int32))
