@@ -26,7 +26,7 @@
 // shared between waves); only the 128 x 128-byte activation chunk passes through LDS.
 #include <type_traits>
 
-#include "common.h"
+#include "moe_gemm.h"
 #include "quant_fp8.h"
 
 namespace dlb {
@@ -55,51 +55,6 @@ __global__ __launch_bounds__(kQuantThreads) void quant_fp8_group128_kernel(const
 // ---------------------------------------------------------------------------------------
 // grouped GEMM
 // ---------------------------------------------------------------------------------------
-struct MoeGemmParams {
-  const unsigned char* a;     // activations fp8 [rows, K] (or 16-bit: K = bytes per row)
-  const float* a_scale;       // [rows, K / 128]
-  const unsigned char* w;     // weights [E_local, N, K]
-  const float* w_scale;       // [E_local, N / 128, K / 128]
-  IdxArray sorted_ids;        // [num_mblocks * block_m] routing slots grouped by expert
-  IdxArray counts;            // [num_experts] routed slots per (global) expert
-  // launcher form of the routing (non-gated kernel only): the slot list is NOT padded per expert;
-  // expert e owns its positions seg_start[e] .. counts[e] - 1 (counts then holds the segment ENDS)
-  IdxArray seg_start;         // p == nullptr: block-aligned list
-  int64_t a_rows;             // rows of `a` when it is read in sorted order (reads are clamped to it)
-  int gather_a;               // non-gated kernel: rows of `a` are gathered by token (slot / topk)
-  int scatter_c;              // non-gated kernel: output row = routing slot (else the sorted position)
-  int num_experts;            // global expert count = length of counts
-  int num_mblocks;            // capacity of sorted_ids in blocks
-  int bm_shift;               // log2(block_m): 6 or 7
-  int num_ntiles;
-  int K, N, KC;               // K = bytes per activation / weight row, KC = K / 128
-  int topk, numel;            // flat slots = tokens * topk (also the pad sentinel)
-  int num_tokens;
-  int expert_offset;          // weights hold experts [expert_offset, expert_offset + E_local)
-  int num_local;              // E_local
-  // gate_up flavour
-  unsigned char* hq;          // [num_mblocks * block_m, I] fp8, or 16-bit when QT = 1
-  float* hs;                  // [num_mblocks * block_m, I / 128]
-  int I;
-  // down flavour
-  void* out;                  // [numel, N] bf16/f16
-  const float* topk_w;        // [numel]
-};
-
-__device__ __forceinline__ i32x8 cat8(const u32x4& lo, const u32x4& hi) {
-  return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
-               (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-}
-
-// exchange between the two lane halves: afterwards lane half 0 holds (its a, the partner's a)
-// and lane half 1 (the partner's b, its b), partner = the lane 32 away
-__device__ __forceinline__ void swap_halves(unsigned int& a, unsigned int& b) {
-  typedef __attribute__((ext_vector_type(2))) unsigned int u2;
-  const u2 r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  a = r[0];
-  b = r[1];
-}
-
 // One weight unit = the lane's operand pieces of one 64-byte half (HK) of a 128-byte K chunk for
 // the wave's two column tiles: 2 tiles x 2 pieces of 16 bytes, uniform base + 32-bit lane
 // offsets.  WL 1 (operand order): the half's pieces sit 512 bytes apart in the tile's 2 KB
@@ -134,12 +89,6 @@ __device__ __forceinline__ void wait_vm() {
 // The expert's first block and its row count come from the per-expert counts of the alignment
 // (block b of expert e starts at sum_{e' < e} ceil(count / block_m) + b): one load per lane
 // and two wave scans.  All results are wave-uniform.
-struct TileId {
-  int e;     // local expert
-  int row0;  // first position of the tile's rows in sorted_ids
-  int nt;    // column tile
-  int rows;  // real (unpadded) rows of the block, 1 .. block_m
-};
 __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, TileId& t) {
   const int bm = 1 << p.bm_shift;
   const bool segs = p.seg_start.p != nullptr;
@@ -794,6 +743,8 @@ int launch_moe_gemm(const MoeGemmParams& p, int dtype, int w_layout, hipStream_t
   // one workgroup per tile slot of the block capacity; a workgroup finds its tile from the
   // expert counts (or finds none and leaves), in the order described at find_tile
   if (w_layout && p.N % 16 != 0) return DLB_ERR_UNSUPPORTED;  // operand order comes in 16-row tiles
+  if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
+  if (moe_stream_case(p, QT == 0)) return launch_moe_stream(p, GATED, QT == 0, dtype, w_layout, s);
   const uint32_t grid = (uint32_t)(ceil_div((int64_t)p.num_mblocks * p.num_ntiles, 8) * 8);
 #define DLB_LAUNCH_GEMM(DT_)                                                                   \
   do {                                                                                       \
@@ -803,8 +754,7 @@ int launch_moe_gemm(const MoeGemmParams& p, int dtype, int w_layout, hipStream_t
       hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, QT, 0>), dim3(grid), dim3(256), 0, s, p); \
   } while (0)
   if (dtype == DLB_DTYPE_BF16) DLB_LAUNCH_GEMM(DLB_DTYPE_BF16);
-  else if (dtype == DLB_DTYPE_F16) DLB_LAUNCH_GEMM(DLB_DTYPE_F16);
-  else return DLB_ERR_UNSUPPORTED;
+  else DLB_LAUNCH_GEMM(DLB_DTYPE_F16);
 #undef DLB_LAUNCH_GEMM
   return launch_status();
 }

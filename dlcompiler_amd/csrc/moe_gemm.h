@@ -1,0 +1,74 @@
+// Operands and small device helpers shared by the two grouped MoE GEMMs: the tiled one for many
+// rows per expert (moe_fp8.hip) and the streaming one for few (moe_stream.hip).
+#pragma once
+#include <type_traits>
+
+#include "common.h"
+
+namespace dlb {
+
+struct MoeGemmParams {
+  const unsigned char* a;     // activations fp8 [rows, K] (or 16-bit: K = bytes per row)
+  const float* a_scale;       // [rows, K / 128]
+  const unsigned char* w;     // weights [E_local, N, K]
+  const float* w_scale;       // [E_local, N / 128, K / 128]
+  IdxArray sorted_ids;        // [num_mblocks * block_m] routing slots grouped by expert
+  IdxArray counts;            // [num_experts] routed slots per (global) expert
+  // launcher form of the routing (non-gated kernel only): the slot list is NOT padded per expert;
+  // expert e owns its positions seg_start[e] .. counts[e] - 1 (counts then holds the segment ENDS)
+  IdxArray seg_start;         // p == nullptr: block-aligned list
+  int64_t a_rows;             // rows of `a` when it is read in sorted order (reads are clamped to it)
+  int gather_a;               // non-gated kernel: rows of `a` are gathered by token (slot / topk)
+  int scatter_c;              // non-gated kernel: output row = routing slot (else the sorted position)
+  int num_experts;            // global expert count = length of counts
+  int num_mblocks;            // capacity of sorted_ids in blocks
+  int bm_shift;               // log2(block_m): 6 or 7
+  int num_ntiles;
+  int K, N, KC;               // K = bytes per activation / weight row, KC = K / 128
+  int topk, numel;            // flat slots = tokens * topk (also the pad sentinel)
+  int num_tokens;
+  int expert_offset;          // weights hold experts [expert_offset, expert_offset + E_local)
+  int num_local;              // E_local
+  // gate_up flavour
+  unsigned char* hq;          // [num_mblocks * block_m, I] fp8, or 16-bit when QT = 1
+  float* hs;                  // [num_mblocks * block_m, I / 128]
+  int I;
+  // down flavour
+  void* out;                  // [numel, N] bf16/f16
+  const float* topk_w;        // [numel]
+};
+
+__device__ __forceinline__ i32x8 cat8(const u32x4& lo, const u32x4& hi) {
+  return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
+               (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+}
+
+// exchange between the two lane halves: afterwards lane half 0 holds (its a, the partner's a)
+// and lane half 1 (the partner's b, its b), partner = the lane 32 away
+__device__ __forceinline__ void swap_halves(unsigned int& a, unsigned int& b) {
+  typedef __attribute__((ext_vector_type(2))) unsigned int u2;
+  const u2 r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// the tile of a workgroup
+struct TileId {
+  int e;     // local expert
+  int row0;  // first position of the tile's rows in sorted_ids
+  int nt;    // column tile
+  int rows;  // real (unpadded) rows of the tile
+};
+
+// Launches the streaming kernel.  gated / quantised as the entry points; N_out checks are done.
+int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dtype, int w_layout, hipStream_t s);
+// Up to this many rows per expert, on average over the routed slots, the streaming kernel is the faster
+// one: its time grows with every 64 rows of an expert, the tiled kernel's with every 128.  Measured
+// (64 experts, 2048 x 1408): fp8 at 38 rows 118 vs 123 us, at 48 rows 130 vs 127; 16-bit row-major at
+// 48 rows 243 vs 274, at 72 rows 319 vs 284.  Both weight layouts take the same kernel (their results
+// are bit-identical).
+inline bool moe_stream_case(const MoeGemmParams& p, bool quantised) {
+  return (int64_t)p.numel <= (quantised ? 42 : 56) * (int64_t)p.num_experts;
+}
+
+}  // namespace dlb

@@ -1,0 +1,494 @@
+// Grouped MoE GEMM for few rows per expert (decode steps and small mixed steps).
+//
+// With a few rows per expert the weights are read once for almost no arithmetic: the kernel is a stream
+// through them, and what counts is whole loads in flight on every CU.  The tiled kernel of
+// moe_fp8.hip (128 x 256 tiles, one barrier per chunk, two workgroups of four waves per CU) reads
+// them at 4.3 - 5.2 TB/s.  Here a wave owns 64 weight rows and every KW-th 128-byte chunk of them,
+// loads the weights straight into MFMA operands, two chunks ahead, and 8 - 16 waves per CU keep
+// 96 - 192 KB on their way: 5.3 - 6.2 TB/s (64 experts of 2048 x 1408 bf16, 300 tokens: layer
+// 265 -> 221 us; fp8, 32 tokens: 113 -> 101 us, 128 tokens 118 -> 109 us).
+//
+// Activations: up to 16 rows they go straight into operands too.  With 32 or 64 rows they would
+// pass through the CU once per wave, as many bytes as the weights (300 tokens: 255 us); there each
+// thread brings its share of the chunk, which goes on through LDS, two buffers, one barrier per chunk.
+//
+// MFMA mapping: 16 x 16 x 128 (fp8) or 2 x 16 x 16 x 32 (16 bit) per chunk; weight rows are the A
+// operand, token rows the B operand.  Lane (c = lane % 16, g = lane / 16) supplies for weight row /
+// token c the 16-byte pieces g of both 64-byte halves of the chunk -- the same pieces on both
+// sides, so the order of K inside the instruction does not matter -- and holds output columns
+// 4 g .. 4 g + 3 of token c.  In operand-order storage a load is a contiguous 1 KB, in row-major
+// storage 16 runs of 64 bytes whose lines the other half completes.
+//
+// fp8 block scales: a chunk's product is taken with a zero accumulator and added with its scale,
+// acc += P * (x_scale * w_scale); activation scales are per-lane loads beside the chunk, weight
+// block scales sit in a lane each and are read by lane index.
+#include "moe_gemm.h"
+#include "quant_fp8.h"
+
+namespace dlb {
+namespace {
+
+// As find_tile of the tiled kernel, with tiles of ROWS rows inside the alignment blocks.
+template <int ROWS>
+__device__ __forceinline__ bool find_stream_tile(const MoeGemmParams& p, int ntiles, int lane, TileId& t) {
+  const bool segs = p.seg_start.p != nullptr;
+  int cnt[4], nb[4], tl[4], st[4];
+  int nb_sum = 0, tl_sum = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int e = 4 * lane + c;
+    st[c] = (segs && e < p.num_experts) ? p.seg_start[e] : 0;
+    cnt[c] = e < p.num_experts ? max(p.counts[e] - st[c], 0) : 0;
+    nb[c] = (cnt[c] + (1 << p.bm_shift) - 1) >> p.bm_shift;
+    const bool local = e >= p.expert_offset && e < p.expert_offset + p.num_local;
+    tl[c] = local ? (cnt[c] + ROWS - 1) / ROWS * ntiles : 0;
+    nb_sum += nb[c];
+    tl_sum += tl[c];
+  }
+  const int nb_incl = wave_inclusive_scan(nb_sum);
+  const int tl_incl = wave_inclusive_scan(tl_sum);
+  const int total = __builtin_amdgcn_readlane(tl_incl, 63);
+  // an expert's tiles on one XCD: its row tiles then share its weights in that XCD's L2
+  const int per_xcd = (total + 7) >> 3;
+  const int i = blockIdx.x >> 3;
+  const int logical = (blockIdx.x & 7) * per_xcd + i;
+  if (i >= per_xcd || logical >= total) return false;
+  const int L = __builtin_ctzll(__ballot(tl_incl > logical));
+  int rem = logical - __builtin_amdgcn_readlane(tl_incl - tl_sum, L);
+  int mbase = __builtin_amdgcn_readlane(nb_incl - nb_sum, L);
+  int e = 4 * L, ce = 0, se = 0;
+  bool found = false;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int tc = __builtin_amdgcn_readlane(tl[c], L);
+    const int nc = __builtin_amdgcn_readlane(nb[c], L);
+    const int cc = __builtin_amdgcn_readlane(cnt[c], L);
+    const int sc = __builtin_amdgcn_readlane(st[c], L);
+    if (!found) {
+      if (rem < tc) {
+        found = true;
+        e = 4 * L + c;
+        ce = cc;
+        se = sc;
+      } else {
+        rem -= tc;
+        mbase += nc;
+      }
+    }
+  }
+  const int nrb = (ce + ROWS - 1) / ROWS;  // row tiles of a column tile follow each other
+  const int rb = rem % nrb;
+  t.e = e - p.expert_offset;
+  t.nt = rem / nrb;
+  t.row0 = (segs ? se : mbase << p.bm_shift) + rb * ROWS;
+  t.rows = min(ROWS, ce - rb * ROWS);
+  // (counts that do not fit the slot list: touch nothing)
+  return t.row0 + t.rows <= (segs ? p.numel : p.num_mblocks << p.bm_shift);
+}
+
+// max over the four lanes that hold a token's columns
+__device__ __forceinline__ float max_groups(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16));
+  return max_xor32(v);
+}
+
+// descriptor of `bytes` bytes at p (wave-uniform): raw buffer, no swizzle, loads past the end give 0
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(uniform_ptr((const unsigned char*)p)), 0,
+                                           (int)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+
+// CW waves side by side in the columns, KW in K.  GATED: a wave's 64 weight rows are 32 gate rows and
+// the 32 up rows that go with them (fp8: CW = 4, the workgroup then holds whole 128-column
+// quantisation groups of its rows); else 64 consecutive rows.
+constexpr int kWaveTiles = 4;  // MFMA tiles of 16 weight rows per wave
+template <bool GATED, int DT, int QT, int WL, int CW, int KW, int NT>
+__global__ __launch_bounds__(64 * CW * KW, NT == 1 ? 4 : NT == 2 ? 3 : 2) void moe_stream_kernel(const MoeGemmParams p, const int ntiles) {
+  static_assert(!GATED || QT == 1 || CW == 4, "fp8 intermediate: whole quantisation groups");
+  constexpr int NCT = kWaveTiles;
+  constexpr int kTileRows = 16 * NT;
+  constexpr int kWaveCols = GATED ? 8 * NCT : 16 * NCT;  // output columns of a wave
+  constexpr int kCols = kWaveCols * CW;                   // ... of the workgroup
+  constexpr int NSB = GATED ? 2 : 1;                      // 128-row blocks of weight scales a wave meets
+  constexpr bool XS = NT > 1;                             // activations through LDS
+  constexpr int kXRows = 16 * NT, NXL = XS ? 2 * NT / CW : 0;  // 16-byte pieces a thread brings per chunk
+  static_assert(!XS || (2 * NT % CW == 0 && kXRows <= 64 * CW), "whole pieces per thread");
+  __shared__ f32x4 part_lds[KW > 1 ? (KW - 1) * CW * NT * NCT * 64 : 1];
+  __shared__ float amax_lds[CW][kTileRows];
+  __shared__ __attribute__((aligned(16))) unsigned char x_lds[XS ? KW : 1][XS ? 2 : 1][XS ? kXRows * 128 : 16];
+  __shared__ float xs_lds[XS && QT == 0 ? KW : 1][2][XS && QT == 0 ? 64 * CW : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cw = wave % CW, kw = wave / CW;
+  const int c = lane & 15, g = lane >> 4;
+
+  TileId tile;
+  if (!find_stream_tile<kTileRows>(p, ntiles, lane, tile)) return;
+
+  const int K = p.K, KC = p.KC;
+  const int nk = (KC - kw + KW - 1) / KW;  // this wave's chunks: kw, kw + KW, ...
+  const int col0 = tile.nt * kCols + kWaveCols * cw;
+  // first weight row of MFMA tile ct
+  auto ncol = [&](int ct) { return GATED && ct >= NCT / 2 ? p.I + col0 + 16 * (ct - NCT / 2) : col0 + 16 * ct; };
+  const unsigned char* wbase = p.w + (int64_t)tile.e * p.N * K;
+  uint32_t woff[NCT];
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct)
+    woff[ct] = WL ? (uint32_t)min(ncol(ct) >> 4, (p.N >> 4) - 1) * (uint32_t)KC * 2048u + (uint32_t)lane * 16u
+                  : (uint32_t)min(ncol(ct) + c, p.N - 1) * (uint32_t)K + 16u * g;
+  u32x4 w[2][NCT][2];                     // [buffer][tile][half]
+  u32x4 x[2][XS ? 1 : NT][2];             // operands ...
+  u32x4 xp[2][XS ? NXL : 1];              // ... or this thread's pieces of the chunk, on their way to LDS
+  float xs[2][XS ? 1 : NT];
+  // Loads go through buffer descriptors: scalar base and chunk offset, 32-bit lane offset, no vector
+  // address arithmetic; a chunk past the wave's last one is read through an empty descriptor,
+  // which touches no memory, so the loop needs no condition around a load (where two paths
+  // meet, the compiler waits as if the loads of the longer one had not been sent).
+  const uint32_t wbytes = (uint32_t)p.N * (uint32_t)K, xbytes = (uint32_t)p.a_rows * (uint32_t)K;
+  // A wave starts somewhere in its chunks and wraps around: if all started at the first one, all would
+  // ask for the same offsets of rows whose distance is a multiple of the channels' period.
+  const int skew = (int)((uint32_t)(tile.e * 5 + tile.nt * 3) % (uint32_t)max(nk, 1));
+  auto chunk_of = [&](int i) {
+    const int j = i + skew;
+    return kw + (j < nk ? j : j - nk) * KW;
+  };
+  auto load_w = [&](auto buf, int i) {
+    constexpr int B = decltype(buf)::value;
+    const auto rsrc = buffer_of(wbase, i < nk ? wbytes : 0u);
+    const int soff = chunk_of(i) * (WL ? 2048 : 128);
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      // operand order: whole lines, non-temporal (8 - 10 % faster); row-major: half lines, kept for
+      // the load of the other half (non-temporal 8 - 10 % slower)
+      w[B][ct][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct], soff, WL ? 2 : 0);
+      w[B][ct][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct] + (WL ? 1024 : 64), soff, WL ? 2 : 0);
+    }
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  // Prologue: the loads go out in the order in which the loop waits for them (a wait in the loop
+  // serves both ways into it): everything that is needed once, then chunk by chunk weights,
+  // activations and their scales.
+  // rows whose activations this thread loads (rows past the tile repeat its last one): its operand
+  // rows, or the rows of its pieces and the row of its scale
+  const int xtid = threadIdx.x % (64 * CW);
+  constexpr int NR = XS ? NXL : NT;
+  auto row_of = [&](int t) { return min(XS ? (t * 64 * CW + xtid) >> 3 : 16 * t + c, tile.rows - 1); };
+  int sid[NR + 1];
+#pragma unroll
+  for (int t = 0; t < NR; ++t) sid[t] = p.sorted_ids[tile.row0 + row_of(t)];
+  sid[NR] = 0;
+  if (XS && QT == 0) sid[NR] = p.sorted_ids[tile.row0 + min(xtid % kXRows, tile.rows - 1)];
+  // block scales of the weight tiles: chunk kc in lane kc % 64 of register kc / 64
+  float ws[NSB][2];
+  if (QT == 0) {
+#pragma unroll
+    for (int b = 0; b < NSB; ++b) {
+      const int blk = min(ncol(b * NCT / 2) >> 7, (p.N >> 7) - 1);
+      const float* src = p.w_scale + ((int64_t)tile.e * (p.N >> 7) + blk) * KC;
+      ws[b][0] = src[min(lane, KC - 1)];
+      ws[b][1] = src[min(lane + 64, KC - 1)];
+    }
+  }
+  load_w(B0{}, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  auto src_row = [&](int sid, int row) -> uint32_t {
+    if (GATED || p.gather_a) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
+    return (uint32_t)min((int64_t)(tile.row0 + row), p.a_rows - 1);
+  };
+  uint32_t xoff[NR], soff[NR];
+#pragma unroll
+  for (int t = 0; t < NR; ++t) {
+    const uint32_t src = src_row(sid[t], row_of(t));
+    xoff[t] = src * (uint32_t)K + 16u * (XS ? xtid & 7 : g);
+    soff[t] = src * (uint32_t)KC * 4u;
+  }
+  if (XS && QT == 0) soff[0] = src_row(sid[NR], min(xtid % kXRows, tile.rows - 1)) * (uint32_t)KC * 4u;
+  auto load_x = [&](auto buf, int i) {
+    constexpr int B = decltype(buf)::value;
+    const auto rsrc = buffer_of(p.a, i < nk ? xbytes : 0u);
+    const auto srsrc = buffer_of(p.a_scale, i < nk ? xbytes / 32u : 0u);  // 4 bytes per 128
+    const int kc = chunk_of(i);
+    if constexpr (XS) {
+#pragma unroll
+      for (int q = 0; q < NXL; ++q) xp[B][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[q], kc * 128, 0);
+      if (QT == 0) xs[B][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[0], kc * 4, 0));
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        x[B][t][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t], kc * 128, 0);
+        x[B][t][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t] + 64, kc * 128, 0);
+        if (QT == 0) xs[B][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[t], kc * 4, 0));
+      }
+    }
+  };
+  // XS: piece (row, p) of a chunk sits at piece p ^ (row & 7) of its row, so that neither the
+  // writes (a row at a time) nor the operand reads (16 rows, one piece) meet in the banks
+  auto store_x = [&](auto buf) {
+    constexpr int B = decltype(buf)::value;
+    if constexpr (XS) {
+#pragma unroll
+      for (int q = 0; q < NXL; ++q) {
+        const int row = (q * 64 * CW + xtid) >> 3;
+        *(u32x4*)(x_lds[kw][B] + row * 128 + (((xtid ^ row) & 7) << 4)) = xp[B][q];
+      }
+      if (QT == 0) xs_lds[kw][B][xtid] = xs[B][0];  // (rows repeat past kXRows: no branch in the loop)
+    }
+  };
+  load_x(B0{}, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_w(B1{}, 1);
+  load_x(B1{}, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (XS) {
+    store_x(B0{});
+    load_x(B0{}, 2);
+    __syncthreads();
+  }
+
+  f32x4 acc[NT][NCT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) acc[t][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto operand = [&](auto buf, int t, u32x4& x0, u32x4& x1) {
+    constexpr int B = decltype(buf)::value;
+    if constexpr (XS) {
+      const unsigned char* row = x_lds[kw][B] + (16 * t + c) * 128;
+      x0 = *(const u32x4*)(row + (((g ^ c) & 7) << 4));
+      x1 = *(const u32x4*)(row + ((((g + 4) ^ c) & 7) << 4));
+    } else {
+      x0 = x[B][t][0];
+      x1 = x[B][t][1];
+    }
+  };
+  auto compute = [&](auto buf, int i) {
+    constexpr int B = decltype(buf)::value;
+    if constexpr (QT == 0) {
+      const int kc = chunk_of(i);
+      float sw[NSB];
+#pragma unroll
+      for (int b = 0; b < NSB; ++b)
+        sw[b] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kc < 64 ? ws[b][0] : ws[b][1]), kc & 63));
+      // (one row tile's products at a time: all of them together do not fit the registers)
+      u32x4 xo[2][2];
+      operand(buf, 0, xo[0][0], xo[0][1]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (t + 1 < NT) operand(buf, t + 1, xo[(t + 1) & 1][0], xo[(t + 1) & 1][1]);
+        if (XS) __builtin_amdgcn_sched_barrier(0);
+        const u32x4 x0 = xo[t & 1][0], x1 = xo[t & 1][1];
+        const float a = XS ? xs_lds[kw][B][16 * t + c] : xs[B][XS ? 0 : t];
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+          const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+          const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              cat8(w[B][ct][0], w[B][ct][1]), cat8(x0, x1), zero, 0, 0, 0, 0, 0, 0);
+          const float f = a * sw[GATED ? ct / (NCT / 2) : 0];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][ct][r] = fmaf(pr[r], f, acc[t][ct][r]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        u32x4 xo[2];
+        operand(buf, t, xo[0], xo[1]);
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int ct = 0; ct < NCT; ++ct) {
+            if constexpr (DT == DLB_DTYPE_BF16)
+              acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[B][ct][half]),
+                                                                   __builtin_bit_cast(bf16x8, xo[half]),
+                                                                   acc[t][ct], 0, 0, 0);
+            else
+              acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[B][ct][half]),
+                                                                  __builtin_bit_cast(f16x8, xo[half]),
+                                                                  acc[t][ct], 0, 0, 0);
+          }
+      }
+    }
+  };
+  // XS: while chunk i is multiplied from LDS buffer i % 2, chunk i + 1 goes from registers into the
+  // other one (whose readers passed the barrier that ended step i - 1), and chunk i + 3 is asked for.
+  auto step = [&](auto buf, int i) {
+    using Other = std::integral_constant<int, 1 - decltype(buf)::value>;
+    compute(buf, i);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(buf, i + 2);
+    if constexpr (XS) {
+      store_x(Other{});
+      load_x(Other{}, i + 3);
+      __syncthreads();
+    } else {
+      load_x(buf, i + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // (XS: all waves make the same number of steps; a wave past its last chunk multiplies zeros)
+  const int steps = XS ? (KC + KW - 1) / KW : nk;
+  int i = 0;
+#pragma nounroll
+  for (; i + 1 < steps; i += 2) {
+    step(B0{}, i);
+    step(B1{}, i + 1);
+  }
+  if (i < steps) compute(B0{}, i);
+
+  // ---- partial sums of the K split
+  if constexpr (KW > 1) {
+    f32x4* part = part_lds + ((kw - 1) * CW + cw) * (NT * NCT * 64);
+    if (kw > 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) part[(NCT * t + ct) * 64 + lane] = acc[t][ct];
+    }
+    __syncthreads();
+    if (kw == 0) {
+#pragma unroll
+      for (int q = 1; q < KW; ++q)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int ct = 0; ct < NCT; ++ct) 
+            acc[t][ct] += part_lds[(((q - 1) * CW + cw) * NT * NCT + NCT * t + ct) * 64 + lane];
+    }
+  }
+
+  // ---- epilogues: lane holds token row 16 t + c, columns ncol(ct) + 4 g + r
+  if constexpr (GATED && QT == 0) {
+    f32x4 v[NT][NCT / 2];
+    if (kw == 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int ct = 0; ct < NCT / 2; ++ct)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float gate = acc[t][ct][r], up = acc[t][ct + NCT / 2][r];
+            v[t][ct][r] = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;  // 1-ulp reciprocal
+            amax = fmaxf(amax, fabsf(v[t][ct][r]));
+          }
+        amax = max_groups(amax);
+        if (g == 0) amax_lds[cw][16 * t + c] = amax;
+      }
+    }
+    __syncthreads();
+    if (kw == 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        float m = amax_lds[0][16 * t + c];
+#pragma unroll
+        for (int q = 1; q < CW; ++q) m = fmaxf(m, amax_lds[q][16 * t + c]);
+        const float scale = fmaxf(m, kQuantEps) / kFp8Max;
+        const float inv = __builtin_amdgcn_rcpf(scale);  // the stored scale stays exact
+        if (16 * t + c < tile.rows) {
+          const int64_t row = tile.row0 + 16 * t + c;
+#pragma unroll
+          for (int ct = 0; ct < NCT / 2; ++ct)
+            *(unsigned int*)(p.hq + row * p.I + col0 + 16 * ct + 4 * g) =
+                pack4_fp8(v[t][ct][0] * inv, v[t][ct][1] * inv, v[t][ct][2] * inv, v[t][ct][3] * inv);
+          if (cw == 0 && g == 0) p.hs[row * (p.I >> 7) + tile.nt] = scale;
+        }
+      }
+    }
+  } else if constexpr (GATED) {
+    // rounding points of the reference pipeline (fused_moe.py:166,351-352): GEMM result,
+    // silu(gate) and the product are each rounded to the activation type
+    if (kw == 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int ct = 0; ct < NCT / 2; ++ct) {
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const unsigned int gu = Elem<DT>::pack(acc[t][ct][r], acc[t][ct + NCT / 2][r]);
+            const float gate = Elem<DT>::lo(gu), up = Elem<DT>::hi(gu);
+            v[r] = Elem<DT>::lo(Elem<DT>::pack(gate / (1.0f + __expf(-gate)), 0.0f)) * up;
+          }
+          // (the last column tile may be partial)
+          if (16 * t + c < tile.rows && col0 + 16 * ct < p.I)
+            *(u32x2*)((unsigned short*)p.hq + (int64_t)(tile.row0 + 16 * t + c) * p.I + col0 + 16 * ct + 4 * g) =
+                u32x2{Elem<DT>::pack(v[0], v[1]), Elem<DT>::pack(v[2], v[3])};
+        }
+    }
+  } else if (kw == 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (16 * t + c >= tile.rows) continue;
+      const int slot = p.sorted_ids[tile.row0 + 16 * t + c];
+      if (slot < 0 || slot >= p.numel) continue;
+      const float f = p.topk_w ? p.topk_w[slot] : 1.0f;
+      const int64_t dst = p.scatter_c ? slot : tile.row0 + 16 * t + c;
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct)
+        if (col0 + 16 * ct + 4 * g < p.N)
+          *(u32x2*)((unsigned short*)p.out + dst * p.N + col0 + 16 * ct + 4 * g) =
+              u32x2{Elem<DT>::pack(acc[t][ct][0] * f, acc[t][ct][1] * f),
+                    Elem<DT>::pack(acc[t][ct][2] * f, acc[t][ct][3] * f)};
+    }
+  }
+}
+
+template <bool GATED, int DT, int QT, int CW, int KW, int NT>
+void launch_shape(const MoeGemmParams& p, int w_layout, hipStream_t s) {
+  // at most one partial row tile per expert that holds slots
+  const int64_t row_tiles = (int64_t)p.numel / (16 * NT) + (p.numel < p.num_local ? p.numel : p.num_local);
+  const int ntiles = (int)ceil_div(GATED ? p.I : p.N, (GATED ? 8 : 16) * kWaveTiles * CW);
+  const uint32_t grid = (uint32_t)(ceil_div(row_tiles * ntiles, 8) * 8);
+  if (w_layout)
+    hipLaunchKernelGGL((moe_stream_kernel<GATED, DT, QT, 1, CW, KW, NT>), dim3(grid), dim3(64 * CW * KW), 0, s, p, ntiles);
+  else
+    hipLaunchKernelGGL((moe_stream_kernel<GATED, DT, QT, 0, CW, KW, NT>), dim3(grid), dim3(64 * CW * KW), 0, s, p, ntiles);
+}
+
+// Workgroup shape.  Four waves side by side share most of their activations; where that leaves fewer
+// workgroups than two per CU (256 CUs), the waves of a workgroup split K instead, and there are
+// twice or four times as many: 16-bit, 8 experts of 4096 x 4096, 16 tokens, 184 -> 151 us; one
+// token 142 -> 57 us.  (64 experts, 2048 x 1408, 300 tokens: side by side 221 us, split 232 us.)
+// The fp8 gate_up GEMM always holds whole quantisation groups; its K split doubles the waves.
+template <bool GATED, int DT, int QT, int NT>
+void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
+  constexpr int kCols4 = (GATED ? 8 : 16) * kWaveTiles * 4;
+  const int64_t tiles = ceil_div(GATED ? p.I : p.N, kCols4) * (p.numel < p.num_local ? p.numel : p.num_local);
+  if constexpr (GATED && QT == 0) {
+    if (NT == 1 && tiles < 128) launch_shape<GATED, DT, QT, 4, NT == 1 ? 2 : 1, NT>(p, w_layout, s);
+    else launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
+  } else {
+    if (tiles >= 512) launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
+    else if (NT == 1) launch_shape<GATED, DT, QT, NT == 1 ? 1 : 2, NT == 1 ? 4 : 2, NT>(p, w_layout, s);
+    else launch_shape<GATED, DT, QT, 2, 2, NT>(p, w_layout, s);
+  }
+}
+
+// Rows per tile from the mean rows per expert: enough that few experts need a second row tile, whose
+// weights come from L2 but pass through the CU again.
+template <bool GATED, int DT, int QT>
+void launch_gemm(const MoeGemmParams& p, int w_layout, hipStream_t s) {
+  if ((int64_t)p.numel <= 7 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 1>(p, w_layout, s);
+  else if ((int64_t)p.numel <= 19 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 2>(p, w_layout, s);
+  else launch_nt<GATED, DT, QT, 4>(p, w_layout, s);
+}
+
+template <int DT>
+void launch_dt(const MoeGemmParams& p, bool gated, int quantised, int w_layout, hipStream_t s) {
+  if (gated && quantised) launch_gemm<true, DLB_DTYPE_BF16, 0>(p, w_layout, s);
+  else if (gated) launch_gemm<true, DT, 1>(p, w_layout, s);
+  else if (quantised) launch_gemm<false, DT, 0>(p, w_layout, s);
+  else launch_gemm<false, DT, 1>(p, w_layout, s);
+}
+
+}  // namespace
+
+int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dtype, int w_layout, hipStream_t s) {
+  if (dtype == DLB_DTYPE_BF16) launch_dt<DLB_DTYPE_BF16>(p, gated, quantised, w_layout, s);
+  else launch_dt<DLB_DTYPE_F16>(p, gated, quantised, w_layout, s);
+  return launch_status();
+}
+
+}  // namespace dlb

@@ -278,11 +278,11 @@ int dlb_per_token_group_quant_fp8(const void* x, void* xq, float* xs, int64_t M,
  *     quant(silu(x_t W_gate^T) * (x_t W_up^T)) for the slot at sorted position r (rows of
  *     32-row groups that hold padding only are not written)
  * H % 128 == 0, I % 128 == 0, and the reduction length (H here, I in the down GEMM) at most
- * 16384.  Scales must be positive: activation scales below 1e-13 count as 1e-13 (the quantisation
- * rule above never produces less than 1e-10 / 448) and weight block scales below 1e-12 count as
+ * 16384.  Scales must be positive: activation scales below 1e-13 may count as 1e-13 (the quantisation
+ * rule above never produces less than 1e-10 / 448) and weight block scales below 1e-12 as
  * 1e-12 (an all-zero block may carry the scale 0).
- * One kernel serves both tile heights and both weight layouts: four-wave tiles of block_m rows
- * x 256 columns, weights streamed straight into operand registers, activations staged in LDS.
+ * Up to about 40 routed rows per expert a kernel that streams the weights runs, beyond it one with
+ * tiles of block_m rows x 256 columns; both take both tile heights and both weight layouts.
  * Outputs are stored 16 bytes at a time: hq, out and the 16-bit act must be 16-byte aligned;
  * other alignments return DLB_ERR_UNSUPPORTED.
  * w_layout selects how the fp8 weight bytes of both GEMMs are stored:
