@@ -65,6 +65,9 @@ SIGNATURES = {
                      + [c_float, c_int, c_void_p]),
     "dlb_apply_rotary_pos_emb": (c_int, [c_void_p] * 6 + [c_int64, c_int, c_int, c_int]
                                  + [c_int64] * 9 + [c_int, c_void_p]),
+    "dlb_fused_moe_ws_bytes": (c_size_t, [c_int, c_int, c_int64] + [c_int] * 6),
+    "dlb_fused_moe": (c_int, [c_int, c_void_p, c_int64] + [c_void_p] * 6 + [c_int, c_void_p, c_void_p, c_int64]
+                      + [c_int] * 10 + [c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
     "dlb_moe_topk_sum": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_void_p]),
 }
 

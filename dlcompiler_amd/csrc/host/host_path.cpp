@@ -36,7 +36,9 @@ namespace {
   X(dlb_prefill_attn_varlen)      \
   X(dlb_paged_prefill_attn)       \
   X(dlb_paged_decode_ws_bytes)    \
-  X(dlb_paged_decode_attn)
+  X(dlb_paged_decode_attn)         \
+  X(dlb_fused_moe_ws_bytes)       \
+  X(dlb_fused_moe)
 
 struct Abi {
 #define X(name) decltype(&::name) name = nullptr;
@@ -446,6 +448,80 @@ PyObject* paged_attention_fwd(PyObject*, PyObject* const* args, Py_ssize_t) {
   END_HANDLE_TH_ERRORS
 }
 
+// fused_moe(x, w1, w1_scale | None, w2, w2_scale | None, topk_weights, topk_ids, topk, expert_offset,
+//           num_experts | None, renormalize, operand_order, (sorted_ids, counts) | None, block) -> out
+PyObject* fused_moe(PyObject*, PyObject* const* args, Py_ssize_t) {
+  HANDLE_TH_ERRORS
+  const at::Tensor *x = tensor(args[0]), *w1 = tensor(args[1]), *w2 = tensor(args[3]);
+  const at::Tensor *tw = tensor(args[5]), *ids = tensor(args[6]);
+  const int dev = launch_device(x);
+  const bool fp8 = args[2] != Py_None;
+  const at::Tensor *s1 = fp8 ? tensor(args[2]) : nullptr, *s2 = fp8 ? tensor(args[4]) : nullptr;
+  if (dev < 0 || !on_gpu(w1, dev) || !on_gpu(w2, dev) || !on_gpu(tw, dev) || !on_gpu(ids, dev)) NOT_HANDLED;
+  if (fp8 && (!on_gpu(s1, dev) || !on_gpu(s2, dev))) NOT_HANDLED;
+  int64_t topk, offset, experts, block;
+  if (!as_int(args[7], topk) || !as_int(args[8], offset) || !as_int(args[13], block)) NOT_HANDLED;
+  const int renorm = PyObject_IsTrue(args[10]), order = PyObject_IsTrue(args[11]);
+  if (renorm < 0 || order < 0) return nullptr;
+  if (x->dim() != 2 || w1->dim() != 3 || w2->dim() != 3 || tw->dim() != 2 || ids->dim() != 2) NOT_HANDLED;
+  const int code = dtype_code(*x);
+  if (code != DLB_DTYPE_BF16 && code != DLB_DTYPE_F16) NOT_HANDLED;
+  const auto wtype = fp8 ? at::kFloat8_e4m3fn : x->scalar_type();
+  const int64_t T = x->size(0), H = x->size(1), E = w1->size(0), N2 = w1->size(1), I = N2 / 2, O = w2->size(1);
+  if (w1->scalar_type() != wtype || w2->scalar_type() != wtype || !w1->is_contiguous() || !w2->is_contiguous() ||
+      T == 0 || E == 0 || I == 0 || O == 0 || N2 != 2 * I || w1->size(2) != H || w2->size(0) != E ||
+      w2->size(2) != I || x->stride(1) != 1 || (!fp8 && T > 1 && x->stride(0) != H) || topk < 1 || topk > (1 << 20) ||
+      H > (1 << 24) || I > (1 << 24) || O > (1 << 24) || T > 0x7fffffff / topk)
+    NOT_HANDLED;
+  auto routing = [&](const at::Tensor* t) {
+    return t->is_contiguous() && t->size(0) == T && t->size(1) == topk;
+  };
+  if (!routing(tw) || !routing(ids) || tw->scalar_type() != at::kFloat ||
+      (ids->scalar_type() != at::kInt && ids->scalar_type() != at::kLong))
+    NOT_HANDLED;
+  if (fp8) {
+    auto scales = [&](const at::Tensor* t, int64_t rows, int64_t cols) {
+      return t->scalar_type() == at::kFloat && t->is_contiguous() && t->dim() == 3 && t->size(0) == E &&
+             t->size(1) == rows / 128 && t->size(2) == cols / 128;
+    };
+    if (H % 128 != 0 || !scales(s1, N2, H) || !scales(s2, O, I)) NOT_HANDLED;
+  }
+  if (args[9] == Py_None) experts = E;
+  else if (!as_int(args[9], experts)) NOT_HANDLED;
+  if (experts < 1 || experts > 256 || offset < 0 || offset + E > experts || (block != 64 && block != 128)) NOT_HANDLED;
+  const at::Tensor *sorted = nullptr, *counts = nullptr;
+  if (args[12] != Py_None) {
+    if (!PyTuple_Check(args[12]) || PyTuple_GET_SIZE(args[12]) != 2) NOT_HANDLED;
+    sorted = tensor(PyTuple_GET_ITEM(args[12], 0));
+    counts = tensor(PyTuple_GET_ITEM(args[12], 1));
+    auto list = [&](const at::Tensor* t) {
+      return on_gpu(t, dev) && t->scalar_type() == at::kInt && t->is_contiguous();
+    };
+    if (!list(sorted) || !list(counts) || sorted->numel() < T * topk + experts * (block - 1) ||
+        counts->numel() != experts)
+      NOT_HANDLED;
+  }
+  const size_t ws_bytes = abi.dlb_fused_moe_ws_bytes(fp8, sorted != nullptr, T, (int)topk, (int)H, (int)I, (int)O,
+                                                     (int)experts, (int)block);
+  const at::Tensor ws = empty({(int64_t)std::max<size_t>(ws_bytes, 16)}, at::kByte, dev);
+  const at::Tensor out = empty({T, O}, x->scalar_type(), dev);
+  int st;
+  {
+    NoGil nogil;
+    st = abi.dlb_fused_moe(fp8, x->data_ptr(), T > 1 ? x->stride(0) : H, w1->data_ptr(),
+                           fp8 ? (const float*)s1->data_ptr() : nullptr, w2->data_ptr(),
+                           fp8 ? (const float*)s2->data_ptr() : nullptr, (const float*)tw->data_ptr(),
+                           ids->data_ptr(), ids->scalar_type() == at::kLong,
+                           sorted ? (const int32_t*)sorted->data_ptr() : nullptr,
+                           counts ? (const int32_t*)counts->data_ptr() : nullptr, T, (int)topk, (int)H, (int)I,
+                           (int)O, (int)experts, (int)offset, (int)E, renorm, order, (int)block, out.data_ptr(),
+                           code, ws.data_ptr(), ws_bytes, stream_of(dev));
+  }
+  if (st != DLB_OK) NOT_HANDLED;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
 // bind({name: address}): the entry points of the library the ctypes loader opened
 PyObject* bind(PyObject*, PyObject* table) {
   if (!PyDict_Check(table)) {
@@ -510,6 +586,7 @@ PyMethodDef methods[] = {
     OP(moe_topk_softmax_align, 4),
     OP(context_attention_fwd, 7),
     OP(paged_attention_fwd, 12),
+    OP(fused_moe, 14),
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dlb_host", "host side of the operators' common calls", -1, methods};

@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
         const int sid = p.sorted_ids[row0 + tid];
         if (sid >= 0 && sid < p.numel) {
           dst = p.scatter_c ? sid : row0 + tid;
-          rwt = p.topk_w ? p.topk_w[sid] : 1.0f;
+          rwt = slot_weight(p, sid);
         }
       }
       sid_lds[tid] = dst;  // published by the barrier that opens the main loop
@@ -671,11 +671,17 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 // TOPK > 0: the slot count is a compile-time constant and all its loads are requested before the
 // first is used (the kernel is a pure stream: what counts is the number of bytes in flight);
 // TOPK = 0: any slot count, four loads at a time.
-template <int DT, int TOPK>
+// SHARD: only slots of experts [first, first + num_local) hold a value (the others were never
+// written and are not read).
+struct ShardIds {
+  IdxArray ids;
+  int first, num_local;
+};
+template <int DT, int TOPK, bool SHARD>
 __global__ __launch_bounds__(256) void moe_topk_sum_kernel(const u32x4* __restrict__ in,
                                                            u32x4* __restrict__ out,
                                                            int64_t total_vec, int vec_per_row,
-                                                           int topk) {
+                                                           int topk, const ShardIds shard) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total_vec) return;
   const int64_t t = i / vec_per_row;
@@ -691,7 +697,24 @@ __global__ __launch_bounds__(256) void moe_topk_sum_kernel(const u32x4* __restri
     }
   };
   const u32x4* row = in + t * (int64_t)(TOPK ? TOPK : topk) * vec_per_row + col;
-  if constexpr (TOPK > 0) {
+  if constexpr (SHARD) {
+    constexpr int U = TOPK ? TOPK : 4;
+    const int k = TOPK ? TOPK : topk;
+    for (int j0 = 0; j0 < k; j0 += U) {
+      bool have[U];
+      u32x4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        have[u] = j0 + u < k && (unsigned)(shard.ids[t * k + j0 + u] - shard.first) < (unsigned)shard.num_local;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        v[u] = u32x4{0u, 0u, 0u, 0u};
+        if (have[u]) v[u] = __builtin_nontemporal_load(row + (int64_t)(j0 + u) * vec_per_row);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) add(v[u]);
+    }
+  } else if constexpr (TOPK > 0) {
     u32x4 v[TOPK];
 #pragma unroll
     for (int j = 0; j < TOPK; ++j) v[j] = __builtin_nontemporal_load(row + (int64_t)j * vec_per_row);
@@ -952,20 +975,24 @@ extern "C" int dlb_moe_gemm_16bit_launcher(const void* a, const void* b, void* c
   return launch_moe_gemm<false, 1>(p, dtype, 0, (hipStream_t)stream);
 }
 
-extern "C" int dlb_moe_topk_sum(const void* in, void* out, int64_t num_tokens, int topk,
-                                int64_t N, int dtype, void* stream) {
-  using namespace dlb;
-  if (num_tokens < 0 || topk < 1 || N < 0) return DLB_ERR_BAD_ARG;
-  if (num_tokens == 0 || N == 0) return DLB_OK;
-  if (!in || !out) return DLB_ERR_BAD_ARG;
-  if (N % 8 != 0 || !aligned16(in) || !aligned16(out)) return DLB_ERR_UNSUPPORTED;
+namespace dlb {
+namespace {
+
+// in [num_tokens * topk, N] -> out [num_tokens, N]; arguments checked
+int launch_topk_sum(const void* in, void* out, int64_t num_tokens, int topk, int64_t N, int dtype,
+                    const ShardIds* shard, hipStream_t s) {
   const int64_t total = num_tokens * (N / 8);
   const dim3 grid((uint32_t)ceil_div(total, 256));
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
-#define DLB_LAUNCH_SUM(DT_, TK_)                                                                  \
-  hipLaunchKernelGGL((moe_topk_sum_kernel<DT_, TK_>), grid, dim3(256), 0, s, (const u32x4*)in, \
-                     (u32x4*)out, total, (int)(N / 8), topk)
+  const ShardIds none = {IdxArray{nullptr, 0}, 0, 0};
+#define DLB_LAUNCH_SUM(DT_, TK_)                                                                       \
+  do {                                                                                                 \
+    if (shard)                                                                                         \
+      hipLaunchKernelGGL((moe_topk_sum_kernel<DT_, TK_, true>), grid, dim3(256), 0, s, (const u32x4*)in, \
+                         (u32x4*)out, total, (int)(N / 8), topk, *shard);                              \
+    else                                                                                               \
+      hipLaunchKernelGGL((moe_topk_sum_kernel<DT_, TK_, false>), grid, dim3(256), 0, s,                \
+                         (const u32x4*)in, (u32x4*)out, total, (int)(N / 8), topk, none);              \
+  } while (0)
 #define DLB_DISPATCH_SUM(DT_)                 \
   switch (topk) {                             \
     case 1: DLB_LAUNCH_SUM(DT_, 1); break;    \
@@ -979,4 +1006,145 @@ extern "C" int dlb_moe_topk_sum(const void* in, void* out, int64_t num_tokens, i
 #undef DLB_DISPATCH_SUM
 #undef DLB_LAUNCH_SUM
   return launch_status();
+}
+
+}  // namespace
+}  // namespace dlb
+
+extern "C" int dlb_moe_topk_sum(const void* in, void* out, int64_t num_tokens, int topk,
+                                int64_t N, int dtype, void* stream) {
+  using namespace dlb;
+  if (num_tokens < 0 || topk < 1 || N < 0) return DLB_ERR_BAD_ARG;
+  if (num_tokens == 0 || N == 0) return DLB_OK;
+  if (!in || !out) return DLB_ERR_BAD_ARG;
+  if (N % 8 != 0 || !aligned16(in) || !aligned16(out)) return DLB_ERR_UNSUPPORTED;
+  if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
+  return launch_topk_sum(in, out, num_tokens, topk, N, dtype, nullptr, (hipStream_t)stream);
+}
+
+// ---------------------------------------------------------------------------------------
+// the whole layer
+// ---------------------------------------------------------------------------------------
+namespace dlb {
+namespace {
+
+// Scratch of a layer call, carved from one allocation (pieces 256-byte aligned).
+struct LayerScratch {
+  int64_t num_mblocks;   // whole alignment blocks the slot list can hold
+  int64_t used_mblocks;  // ... and that slots can occupy: what the intermediate is sized for
+  size_t sorted_ids, expert_ids, counts, num_post, align_ws, xq, xs, h, hs, slots, total;
+};
+LayerScratch layer_scratch(bool quantised, bool aligned, int64_t T, int topk, int H, int I, int O, int E, int block) {
+  LayerScratch l;
+  const int64_t numel = T * topk, cap = numel + (int64_t)E * (block - 1);
+  l.num_mblocks = cap / block;
+  l.used_mblocks = numel / block + (numel < E ? numel : E);
+  if (l.used_mblocks > l.num_mblocks) l.used_mblocks = l.num_mblocks;
+  const int64_t rows = l.used_mblocks * block;
+  size_t at = 0;
+  auto take = [&](int64_t bytes) {
+    const size_t mine = at;
+    at += (size_t)((bytes + 255) & ~(int64_t)255);
+    return mine;
+  };
+  l.sorted_ids = take(aligned ? 0 : 4 * cap);
+  l.expert_ids = take(aligned ? 0 : 4 * ceil_div(cap, block));
+  l.counts = take(aligned ? 0 : 4 * E);
+  l.num_post = take(aligned ? 0 : 4);
+  l.align_ws = take(aligned ? 0 : (int64_t)dlb_moe_align_ws_bytes(numel, E));
+  l.xq = take(quantised ? T * H : 0);
+  l.xs = take(quantised ? T * (H / 128) * 4 : 0);
+  l.h = take(rows * I * (quantised ? 1 : 2));
+  l.hs = take(quantised ? rows * (I / 128) * 4 : 0);
+  l.slots = take(numel * O * 2);
+  l.total = at;
+  return l;
+}
+
+bool layer_sizes_ok(int64_t T, int topk, int H, int I, int O, int E, int block) {
+  return T >= 0 && topk >= 1 && H >= 1 && I >= 1 && O >= 1 && E >= 1 && (block == 64 || block == 128) &&
+         T * topk + (int64_t)E * block < (int64_t)0x7fffffff;
+}
+
+}  // namespace
+}  // namespace dlb
+
+extern "C" size_t dlb_fused_moe_ws_bytes(int quantised, int aligned, int64_t T, int topk, int H, int I, int O,
+                                         int num_experts, int block) {
+  using namespace dlb;
+  if (!layer_sizes_ok(T, topk, H, I, O, num_experts, block)) return 0;
+  return layer_scratch(quantised != 0, aligned != 0, T, topk, H, I, O, num_experts, block).total;
+}
+
+extern "C" int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const void* w1, const float* w1s,
+                             const void* w2, const float* w2s, const float* topk_weights, const void* topk_ids,
+                             int ids_int64, const int32_t* sorted_ids, const int32_t* counts, int64_t T, int topk,
+                             int H, int I, int O, int num_experts, int expert_offset, int num_local_experts,
+                             int renormalize, int w_layout, int block, void* out, int dtype, void* ws,
+                             size_t ws_bytes, void* stream) {
+  using namespace dlb;
+  if (!layer_sizes_ok(T, topk, H, I, O, num_experts, block) || ld_x < H) return DLB_ERR_BAD_ARG;
+  if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
+  if (T == 0) return DLB_OK;
+  if (!x || !w1 || !w2 || !topk_weights || !topk_ids || !out || (!sorted_ids != !counts)) return DLB_ERR_BAD_ARG;
+  if (quantised && (!w1s || !w2s)) return DLB_ERR_BAD_ARG;
+  if (!quantised && T > 1 && ld_x != H) return DLB_ERR_UNSUPPORTED;
+  if (O % 8 != 0 || (quantised && (H % 128 != 0 || I % 128 != 0)) || !aligned16(out)) return DLB_ERR_UNSUPPORTED;
+  const bool aligned = sorted_ids != nullptr;
+  const LayerScratch l = layer_scratch(quantised != 0, aligned, T, topk, H, I, O, num_experts, block);
+  if (!ws || ws_bytes < l.total) return DLB_ERR_WORKSPACE;
+  if (!aligned16(ws)) return DLB_ERR_UNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  char* base = (char*)ws;
+  const int64_t numel = T * topk, cap = numel + (int64_t)num_experts * (block - 1);
+  void* xq = base + l.xq;
+  float* xs = (float*)(base + l.xs);
+  void* h = base + l.h;
+  float* hs = (float*)(base + l.hs);
+
+  // both GEMMs are checked before anything is launched
+  if (T >= (int64_t)0x7fffffff) return DLB_ERR_UNSUPPORTED;
+  int32_t* own_sorted = (int32_t*)(base + l.sorted_ids);
+  int32_t* own_counts = (int32_t*)(base + l.counts);
+  const int32_t* srt = aligned ? sorted_ids : own_sorted;
+  const int32_t* cnt = aligned ? counts : own_counts;
+  const int elem = quantised ? 1 : 2;
+  MoeGemmParams up, down;
+  int st = fill_gemm_params(up, true, elem, quantised ? xq : x, quantised ? xs : nullptr, w1, w1s, srt, cnt,
+                            num_experts, (int)l.used_mblocks, block, (int)T, topk, H, I, expert_offset,
+                            num_local_experts);
+  if (st != DLB_OK) return st;
+  st = fill_gemm_params(down, false, elem, h, quantised ? hs : nullptr, w2, w2s, srt, cnt, num_experts,
+                        (int)l.used_mblocks, block, (int)T, topk, O, I, expert_offset, num_local_experts);
+  if (st != DLB_OK) return st;
+  if (w_layout && (up.N % 16 != 0 || down.N % 16 != 0)) return DLB_ERR_UNSUPPORTED;
+  up.hq = (unsigned char*)h;
+  up.hs = hs;
+  down.out = base + l.slots;
+  down.topk_w = topk_weights;
+  down.renorm = renormalize ? 1 : 0;
+
+  int32_t* eids = (int32_t*)(base + l.expert_ids);
+  const int64_t eids_cap = ceil_div(cap, block);
+  int32_t* post = (int32_t*)(base + l.num_post);
+  const size_t align_bytes = dlb_moe_align_ws_bytes(numel, num_experts);
+  if (quantised && aligned)
+    st = dlb_per_token_group_quant_fp8(x, xq, xs, T, H, ld_x, H, H / 128, dtype, stream);
+  else if (quantised)
+    st = dlb_moe_align_quant_fp8(topk_ids, ids_int64, numel, num_experts, block, own_sorted, cap, eids, eids_cap,
+                                 own_counts, post, base + l.align_ws, align_bytes, x, xq, xs, T, H, ld_x, H,
+                                 H / 128, dtype, stream);
+  else if (!aligned)
+    st = dlb_moe_align_block_size(topk_ids, ids_int64, numel, num_experts, block, own_sorted, cap, eids, eids_cap,
+                                  own_counts, post, base + l.align_ws, align_bytes, stream);
+  if (st != DLB_OK) return st;
+  st = quantised ? launch_moe_gemm<true, 0>(up, DLB_DTYPE_BF16, w_layout, s)
+                 : launch_moe_gemm<true, 1>(up, dtype, w_layout, s);
+  if (st != DLB_OK) return st;
+  st = quantised ? launch_moe_gemm<false, 0>(down, dtype, w_layout, s)
+                 : launch_moe_gemm<false, 1>(down, dtype, w_layout, s);
+  if (st != DLB_OK) return st;
+  const ShardIds shard = {idx_array(topk_ids, ids_int64 ? 1 : 0, 0), expert_offset, num_local_experts};
+  const bool full = expert_offset == 0 && num_local_experts == num_experts;
+  return launch_topk_sum(base + l.slots, out, T, topk, O, dtype, full ? nullptr : &shard, s);
 }

@@ -36,7 +36,19 @@ struct MoeGemmParams {
   // down flavour
   void* out;                  // [numel, N] bf16/f16
   const float* topk_w;        // [numel]
+  int renorm;                 // weights are divided by the sum of their token's
 };
+
+// routing weight of a slot (1 without weights)
+__device__ __forceinline__ float slot_weight(const MoeGemmParams& p, int slot) {
+  if (!p.topk_w) return 1.0f;
+  const float w = p.topk_w[slot];
+  if (!p.renorm) return w;
+  const float* mine = p.topk_w + (slot - slot % p.topk);
+  float sum = 0.0f;
+  for (int j = 0; j < p.topk; ++j) sum += mine[j];
+  return w / sum;
+}
 
 __device__ __forceinline__ i32x8 cat8(const u32x4& lo, const u32x4& hi) {
   return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(64 * CW * KW, NT == 1 ? 4 : NT == 2 ? 3 : 2) void m
       if (16 * t + c >= tile.rows) continue;
       const int slot = p.sorted_ids[tile.row0 + 16 * t + c];
       if (slot < 0 || slot >= p.numel) continue;
-      const float f = p.topk_w ? p.topk_w[slot] : 1.0f;
+      const float f = slot_weight(p, slot);
       const int64_t dst = p.scatter_c ? slot : tile.row0 + 16 * t + c;
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct)

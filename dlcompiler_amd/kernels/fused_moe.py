@@ -194,6 +194,33 @@ def fused_moe_kernel_launcher(
     _lib.check(st, "dlb_moe_gemm_16bit_launcher")
 
 
+def _layer(x, w1, s1, w2, s2, topk_weights, topk_ids, topk, expert_offset, num_experts, renormalize, shuffled,
+           alignment):
+    """The layer as one native call; arguments of the types the C ABI takes (``s1`` None: 16-bit)."""
+    T, H = x.shape
+    E, N2, _ = w1.shape
+    I, O, dev, block = N2 // 2, w2.shape[1], x.device, _BLOCK_M
+    ids = routing_ids(topk_ids)
+    sorted_ids = counts = None
+    if alignment is not None:
+        sorted_ids, counts = _check_alignment(alignment, ids, block, num_experts)
+    lib = _lib.load()
+    quantised, aligned = int(s1 is not None), int(sorted_ids is not None)
+    ws_bytes = lib.dlb_fused_moe_ws_bytes(quantised, aligned, T, topk, H, I, O, num_experts, block)
+    ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=dev)
+    out = torch.empty((T, O), dtype=x.dtype, device=dev)
+    with _lib.device_guard(dev):
+        st = lib.dlb_fused_moe(
+            quantised, x.data_ptr(), x.stride(0) if T > 1 else H, w1.data_ptr(),
+            s1.data_ptr() if quantised else None, w2.data_ptr(), s2.data_ptr() if quantised else None,
+            topk_weights.data_ptr(), ids.data_ptr(), int(ids.dtype == torch.int64),
+            sorted_ids.data_ptr() if aligned else None, counts.data_ptr() if aligned else None, T, topk, H, I, O,
+            num_experts, expert_offset, E, int(bool(renormalize)), int(bool(shuffled)), block, out.data_ptr(),
+            _lib.torch_dtype_code(x.dtype), ws.data_ptr(), ws_bytes, _lib.current_stream_ptr(dev))
+    _lib.check(st, "dlb_fused_moe")
+    return out
+
+
 def fused_moe_fp8(hidden_states: torch.Tensor,
                   w1_q: torch.Tensor,
                   w1_s: torch.Tensor,
@@ -229,6 +256,12 @@ def fused_moe_fp8(hidden_states: torch.Tensor,
     call: the operand-order copies are made on the first call and reused while the weight tensors
     stay unmodified, at the price of holding the weights twice.
     """
+    cache = not weights_shuffled and _cache_requested(cache_operand_order)
+    if not cache:
+        out = _lib.host().fused_moe(hidden_states, w1_q, w1_s, w2_q, w2_s, topk_weights, topk_ids, topk,
+                                    expert_offset, num_experts, renormalize, weights_shuffled, alignment, _BLOCK_M)
+        if out is not None:
+            return out
     _lib.require_cuda(hidden_states, w1_q, w1_s, w2_q, w2_s, topk_weights, topk_ids)
     assert hidden_states.dim() == 2 and topk_ids.shape == topk_weights.shape
     T, H = hidden_states.shape
@@ -238,59 +271,22 @@ def fused_moe_fp8(hidden_states: torch.Tensor,
     assert H1 == H and w2_q.shape == (E, O, I) and topk_ids.shape == (T, topk)
     assert w1_q.dtype == torch.float8_e4m3fn and w2_q.dtype == torch.float8_e4m3fn
     assert w1_q.is_contiguous() and w2_q.is_contiguous()
-    if not weights_shuffled and _cache_requested(cache_operand_order) and O % 16 == 0:
+    if cache and O % 16 == 0:
         w1_q, w2_q, weights_shuffled = _operand_order_cached(w1_q), _operand_order_cached(w2_q), True
     assert w1_s.shape == (E, N2 // 128, H // 128) and w2_s.shape == (E, O // 128, I // 128)
     if num_experts is None:
         num_experts = E
-    dev = hidden_states.device
-    dt = hidden_states.dtype
     if T == 0:
         return hidden_states.new_empty((0, O))
-
-    if renormalize:
-        topk_weights = topk_weights / topk_weights.sum(dim=-1, keepdim=True)
-    topk_weights = topk_weights.to(torch.float32).contiguous()
-    w1_s = w1_s.to(torch.float32).contiguous()
-    w2_s = w2_s.to(torch.float32).contiguous()
-
-    block = _BLOCK_M
-    if alignment is None:
-        # alignment and activation quantisation: one native call, two launches
-        sorted_ids, counts, xq, xs = _align_and_quant(topk_ids, block, num_experts, hidden_states)
-    else:
-        sorted_ids, counts = _check_alignment(alignment, topk_ids, block, num_experts)
-        xq, xs = per_token_group_quant_fp8(hidden_states)
-    num_mblocks = sorted_ids.numel() // block  # whole blocks the slot list can hold
-
-    # one allocation for the intermediates: fp8 rows + their scales (fp32) + the slot outputs
-    rows = num_mblocks * block
-    full = (expert_offset == 0 and num_experts == E)
-    hq = torch.empty((rows, I), dtype=torch.float8_e4m3fn, device=dev)
-    hs = torch.empty((rows, I // 128), dtype=torch.float32, device=dev)
-    slots = (torch.empty if full else torch.zeros)((T * topk, O), dtype=dt, device=dev)
-    out = torch.empty((T, O), dtype=dt, device=dev)
-
-    lib = _lib.load()
-    stream = _lib.current_stream_ptr(dev)
-    with _lib.device_guard(dev):
-        st = lib.dlb_moe_gemm_fp8_gate_up(xq.data_ptr(), xs.data_ptr(), w1_q.data_ptr(),
-                                          w1_s.data_ptr(), sorted_ids.data_ptr(),
-                                          counts.data_ptr(), num_experts, num_mblocks, block, T,
-                                          topk, H, I, expert_offset, E, int(weights_shuffled),
-                                          hq.data_ptr(), hs.data_ptr(), stream)
-        _lib.check(st, "dlb_moe_gemm_fp8_gate_up")
-        st = lib.dlb_moe_gemm_fp8_down(hq.data_ptr(), hs.data_ptr(), w2_q.data_ptr(),
-                                       w2_s.data_ptr(), sorted_ids.data_ptr(),
-                                       counts.data_ptr(), num_experts, topk_weights.data_ptr(),
-                                       num_mblocks, block, T, topk, O, I, expert_offset, E,
-                                       int(weights_shuffled),
-                                       slots.data_ptr(), _lib.torch_dtype_code(dt), stream)
-        _lib.check(st, "dlb_moe_gemm_fp8_down")
-        st = lib.dlb_moe_topk_sum(slots.data_ptr(), out.data_ptr(), T, topk, O,
-                                  _lib.torch_dtype_code(dt), stream)
-        _lib.check(st, "dlb_moe_topk_sum")
-    return out
+    if H % 128 != 0:
+        raise ValueError("the hidden size must be a multiple of 128")
+    if hidden_states.stride(1) != 1:
+        hidden_states = hidden_states.contiguous()
+    if renormalize and topk_weights.dtype != torch.float32:
+        topk_weights, renormalize = topk_weights / topk_weights.sum(dim=-1, keepdim=True), False
+    return _layer(hidden_states, w1_q, w1_s.to(torch.float32).contiguous(), w2_q,
+                  w2_s.to(torch.float32).contiguous(), topk_weights.to(torch.float32).contiguous(), topk_ids, topk,
+                  expert_offset, num_experts, renormalize, weights_shuffled, alignment)
 
 
 def fused_moe(hidden_states: torch.Tensor,
@@ -312,6 +308,12 @@ def fused_moe(hidden_states: torch.Tensor,
     grouped GEMM applies the routing weight and the top-k slots are summed.
     ``weights_shuffled``, ``alignment`` and ``cache_operand_order`` are this package's extensions
     (see :func:`shuffle_moe_weight` and :func:`fused_moe_fp8`)."""
+    cache = not weights_shuffled and _cache_requested(cache_operand_order)
+    if not cache:
+        out = _lib.host().fused_moe(hidden_states, w1, None, w2, None, topk_weights, topk_ids, topk, expert_offset,
+                                    num_experts, renormalize, weights_shuffled, alignment, _BLOCK_M)
+        if out is not None:
+            return out
     _lib.require_cuda(hidden_states, w1, w2, topk_weights, topk_ids)
     M = hidden_states.size(0)
     E, N, _ = w1.shape
@@ -319,49 +321,17 @@ def fused_moe(hidden_states: torch.Tensor,
     I = N // 2
     O = w2.shape[1]  # output width, taken from w2 as in the reference (fused_moe.py:354-357)
     assert w1.shape == (E, 2 * I, H) and w2.shape == (E, O, I)
-    assert hidden_states.dtype == w1.dtype == w2.dtype
+    assert hidden_states.dtype == w1.dtype == w2.dtype and topk_ids.numel() == topk_weights.numel() == M * topk
     assert w1.is_contiguous() and w2.is_contiguous()
-    if not weights_shuffled and _cache_requested(cache_operand_order) and O % 16 == 0:
+    if cache and O % 16 == 0:
         w1, w2, weights_shuffled = _operand_order_cached(w1), _operand_order_cached(w2), True
     if num_experts is None:
         num_experts = E
-    dev, dt = hidden_states.device, hidden_states.dtype
     if M == 0:
         return hidden_states.new_empty((0, O))
     if hidden_states.stride(1) != 1 or hidden_states.stride(0) != H:
         hidden_states = hidden_states.contiguous()
-
-    if renormalize:
-        topk_weights = topk_weights / topk_weights.sum(dim=-1, keepdim=True)
-    topk_weights = topk_weights.to(torch.float32).contiguous()
-
-    block = _BLOCK_M
-    if alignment is None:
-        sorted_ids, _, _, counts = moe_align_block_size(topk_ids, block, num_experts,
-                                                        return_counts=True)
-    else:
-        sorted_ids, counts = _check_alignment(alignment, topk_ids, block, num_experts)
-    num_mblocks = sorted_ids.numel() // block  # whole blocks the slot list can hold
-    act = torch.empty((num_mblocks * block, I), dtype=dt, device=dev)
-    full = (expert_offset == 0 and num_experts == E)
-    slots = (torch.empty if full else torch.zeros)((M * topk, O), dtype=dt, device=dev)
-    out = torch.empty((M, O), dtype=dt, device=dev)
-    lib = _lib.load()
-    code = _lib.torch_dtype_code(dt)
-    stream = _lib.current_stream_ptr(dev)
-    with _lib.device_guard(dev):
-        st = lib.dlb_moe_gemm_16bit_gate_up(hidden_states.data_ptr(), w1.data_ptr(),
-                                            sorted_ids.data_ptr(), counts.data_ptr(),
-                                            num_experts, num_mblocks, block, M, topk, H, I,
-                                            expert_offset, E, int(weights_shuffled),
-                                            act.data_ptr(), code, stream)
-        _lib.check(st, "dlb_moe_gemm_16bit_gate_up")
-        st = lib.dlb_moe_gemm_16bit_down(act.data_ptr(), w2.data_ptr(), sorted_ids.data_ptr(),
-                                         counts.data_ptr(), num_experts,
-                                         topk_weights.data_ptr(), num_mblocks, block, M, topk,
-                                         O, I, expert_offset, E, int(weights_shuffled),
-                                         slots.data_ptr(), code, stream)
-        _lib.check(st, "dlb_moe_gemm_16bit_down")
-        st = lib.dlb_moe_topk_sum(slots.data_ptr(), out.data_ptr(), M, topk, O, code, stream)
-        _lib.check(st, "dlb_moe_topk_sum")
-    return out
+    if renormalize and topk_weights.dtype != torch.float32:
+        topk_weights, renormalize = topk_weights / topk_weights.sum(dim=-1, keepdim=True), False
+    return _layer(hidden_states, w1, None, w2, None, topk_weights.to(torch.float32).contiguous(), topk_ids, topk,
+                  expert_offset, num_experts, renormalize, weights_shuffled, alignment)

@@ -341,6 +341,24 @@ int dlb_moe_gemm_16bit_down(const void* act, const void* w2, const int32_t* sort
                             int num_local_experts, int w_layout, void* out, int dtype,
                             void* stream);
 
+/* The whole layer in one call: the routing is aligned by expert (unless sorted_ids / counts hand over
+ * an alignment of these topk_ids with this block over all num_experts experts), the activations are
+ * quantised (quantised != 0), then gate_up, down and the sum over the top-k slots.
+ *   x [T, H] of dtype (row stride ld_x; H where quantised == 0), topk_weights [T, topk] fp32,
+ *   topk_ids [T, topk] int32 or int64 (ids_int64); w1, w1s, w2, w2s, w_layout as above; out [T, O].
+ *   renormalize: routing weights are divided by the sum of their token's (kernels/fused_moe.py:322-323).
+ *   Slots of experts outside [expert_offset, expert_offset + num_local_experts) contribute nothing.
+ *   block in {64, 128}; ws: dlb_fused_moe_ws_bytes(quantised, sorted_ids != NULL, ...) bytes.
+ * Replaces fused_moe, kernels/fused_moe.py:296-376. */
+size_t dlb_fused_moe_ws_bytes(int quantised, int aligned, int64_t T, int topk, int H, int I, int O,
+                              int num_experts, int block);
+int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const void* w1, const float* w1s,
+                  const void* w2, const float* w2s, const float* topk_weights, const void* topk_ids,
+                  int ids_int64, const int32_t* sorted_ids, const int32_t* counts, int64_t T, int topk,
+                  int H, int I, int O, int num_experts, int expert_offset, int num_local_experts,
+                  int renormalize, int w_layout, int block, void* out, int dtype, void* ws,
+                  size_t ws_bytes, void* stream);
+
 /* The reference's grouped-GEMM launcher in its own argument form: replaces fused_moe_kernel +
  * fused_moe_kernel_launcher, kernels/fused_moe.py:82-235 (16-bit operands, fp32 accumulation).
  *   a [a_rows, K], b [num_local_experts, N, K] (row-major), c [rows, N], all of `dtype`

@@ -65,3 +65,18 @@ def test_fp8(dev, T, H, I, E, k, skew):
         assert err <= 3e-2, err
 
 
+@pytest.mark.parametrize("topk", [2, 3])
+def test_expert_shards_add_up(dev, topk):
+    """Two halves of an expert-parallel group: slots of experts held elsewhere are not read."""
+    from dlcompiler_amd.kernels.fused_moe import fused_moe
+
+    g = torch.Generator().manual_seed(topk)
+    T, H, I, E = 50, 256, 128, 8
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16)
+    w1, w2 = (torch.randn(s, generator=g).mul_(0.05).to(torch.bfloat16) for s in ((E, 2 * I, H), (E, H, I)))
+    tw, ids = og.topk_softmax(torch.randn((T, E), generator=g), topk, renormalize=False)
+    xd, tw, ids = x.to(dev), tw.to(dev), ids.to(dev)
+    halves = [fused_moe(xd, w1[o:o + 4].to(dev), w2[o:o + 4].to(dev), tw, ids, topk, o, E, True).double()
+              for o in (0, 4)]
+    whole = fused_moe(xd, w1.to(dev), w2.to(dev), tw, ids, topk, renormalize=True).double()
+    assert ((halves[0] + halves[1] - whole).norm() / whole.norm()).item() < 1e-2
