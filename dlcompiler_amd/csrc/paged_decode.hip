@@ -21,6 +21,9 @@
 //     registers ARE the B operand of O^T = V^T.P^T: P never moves between lanes.
 // The kernel is an HBM stream (4 FLOP/byte at GQA 4:1); everything else is sized to keep
 // tens of KB of loads in flight per CU.
+// Short contexts are bound by latency instead: there one workgroup of 4 or 8 wavefronts per (sequence,
+// kv-head unit) cuts the context among its wavefronts and merges their partials in LDS, in one
+// launch (paged_decode_direct_kernel).
 #include "common.h"
 
 namespace dlb {
@@ -94,58 +97,31 @@ constexpr int kVtRowBytes = 144;   // 64 keys * 2 B + 16 B pad
 // (The masked variant keeps a few more per-lane offsets alive: it is built for one wavefront per
 // SIMD instead of two rather than spilling them.)
 template <int DT, int D, bool POW2, bool RAGGED>
-__global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(const DecodeParams p) {
-  constexpr int KS = D / 32;   // MFMA k-steps over the head dim
-  constexpr int MT = D / 16;   // 16-row tiles of O^T
-  constexpr int DG = D / 8;    // 8-dim groups per key row
+struct DecodeSegment {
+  static constexpr int KS = D / 32;  // MFMA k-steps over the head dim
+  static constexpr int MT = D / 16;  // 16-row tiles of O^T
+  static constexpr int DG = D / 8;   // 8-dim groups per key row
+  static constexpr int kVtBytes = D * kVtRowBytes;
+  f32x4 o[MT];  // O^T: lane (g, c) holds dims 16 mt + 4 g .. + 3 of query head c
+  float m_run;  // running maximum of head c (base 2)
+  float l_run;  // softmax denominator of head c (complete after run())
 
-  // grid: x = (kv head, head chunk) unit, y = team.  The unit is the fastest index, so the
-  // wavefronts that start together read the 256-byte head slices of the SAME token rows at the
-  // same time: whole 2 KB cache rows are in flight together and DRAM pages are hit while open.
-  const int unit = blockIdx.x;
-  const int team = blockIdx.y;
-  const int kvh = unit / p.hchunks;
-  const int hchunk = unit - kvh * p.hchunks;
-
+  // Keys [k_begin, k_end) of sequence b (context ctx, keys before kv_min masked), for one kv-head
+  // unit; k_begin is a multiple of 32.  vt: this wavefront's V^T tile in LDS (kVtBytes).
+  __device__ __forceinline__ void run(const DecodeParams& p, unsigned char* vt, int b, int ctx, int kvh, int head,
+                                      bool head_ok, int k_begin, int k_end, int kv_min) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4;  // lane group 0..3
   const int c = lane & 15;  // column (query head) / row (key) inside a 16-tile
-
-  __shared__ __attribute__((aligned(16))) unsigned char vt[D * kVtRowBytes];  // this wave's V^T tile
-  __shared__ int32_t seg_lds[2][64];  // (first unit, units) of the 64 sequences being walked
-
   const unsigned short* qb = (const unsigned short*)p.q;
-  const int hq_local = hchunk * 16 + c;
-  const bool head_ok = hq_local < p.group;
-  const int head = kvh * p.group + hq_local;
-
-  // ---- this team's piece of the concatenated KV streams (32-key units) ----
-  auto units_of = [&](int bb) { return bb < p.B ? (max(p.kv_len[bb], 0) + 31) >> 5 : 0; };
-  int total = 0;
-  for (int b0 = 0; b0 < p.B; b0 += 64) {
-    int t = units_of(b0 + lane);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) t += __shfl_xor(t, d);
-    total += t;
-  }
-  // (the reduction leaves the same value in every lane; say so, or every address derived from
-  // it is treated as lane-dependent and the block-table lookups become vector loads that
-  // share the in-order return queue of the K/V stream)
-  total = __builtin_amdgcn_readfirstlane(total);
-  const int upt = max((total + p.num_teams - 1) / p.num_teams, p.min_units);  // units per team
-  const int lo = team * upt;
-  if (lo >= total) return;
-  const int hi = min(lo + upt, total);
-
-  // one sequence segment [k_begin, k_end) of sequence b -> partial number `piece` of b
-  auto process_segment = [&](int b, int k_begin, int k_end, int piece) {
   // everything that shapes the walk is wave-uniform; saying so keeps the loops and the page
   // arithmetic on the scalar unit
   b = __builtin_amdgcn_readfirstlane(b);
-  const int ctx = __builtin_amdgcn_readfirstlane(p.kv_len[b]);
+  ctx = __builtin_amdgcn_readfirstlane(ctx);
+  kvh = __builtin_amdgcn_readfirstlane(kvh);
+  k_begin = __builtin_amdgcn_readfirstlane(k_begin);
   k_end = __builtin_amdgcn_readfirstlane(min(k_end, ctx));
-  const int kv_min = p.window > 0 ? max(ctx - 1 - p.window, 0) : 0;  // first visible key
-  k_begin = __builtin_amdgcn_readfirstlane(max(k_begin, kv_min & ~31));  // the half tile holding kv_min
+  kv_min = __builtin_amdgcn_readfirstlane(kv_min);
   const int32_t* bt = p.block_table.p + (((int64_t)b * p.bt_stride) << p.block_table.sh);
   const int bt_sh = p.block_table.sh;
 
@@ -158,11 +134,10 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
       qf[ks] = *(const u32x4*)(qb + (int64_t)b * p.q_sb + (int64_t)head * p.q_sh + 32 * ks + 8 * g);
   }
 
-  f32x4 o[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -__builtin_inff();
-  float l_run = 0.0f;  // per-lane partial of the softmax denominator
+  m_run = -__builtin_inff();
+  l_run = 0.0f;  // per-lane partial of the softmax denominator
 
   // Addressing: a 16-key sub-tile never straddles a page (page % 16 == 0), so its physical
   // page comes from ONE wave-uniform block-table entry (a scalar load) and every lane adds a
@@ -172,7 +147,7 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   const uint32_t k_tok_bytes = (uint32_t)p.k_st * 2u, v_tok_bytes = (uint32_t)p.v_st * 2u;
   constexpr int VL = 64 / DG < 4 ? 64 / DG : 4;  // 4-key groups of a sub-tile staged per pass
   constexpr int VPASS = 4 / VL;                  // passes per 16-key sub-tile
-  const int dg = lane % DG, kgl = lane / DG;     // lanes with kgl >= VL idle (D < 128)
+  const int dg = lane % DG, kgl = lane / DG;     // lanes with kgl >= VL idle
   // byte offsets of this lane's 16-byte pieces inside a key / value row
   uint32_t kdim_off[KS];
 #pragma unroll
@@ -378,28 +353,66 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   l_run += __shfl_xor(l_run, 16);
   l_run += __shfl_xor(l_run, 32);
 
-  if (head_ok) {
-    const int64_t slot = ((int64_t)b * p.Hq + head) * p.nsplit_max + piece;
-    float* wo = p.ws_o + slot * D;
+  }  // run
+};
+
+// first visible key of a context
+__device__ __forceinline__ int first_visible(const DecodeParams& p, int ctx) {
+  return p.window > 0 ? max(ctx - 1 - p.window, 0) : 0;
+}
+
+template <int DT, int D, bool POW2, bool RAGGED>
+__global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(const DecodeParams p) {
+  // grid: x = (kv head, head chunk) unit, y = team.  The unit is the fastest index, so the
+  // wavefronts that start together read the 256-byte head slices of the SAME token rows at the
+  // same time: whole 2 KB cache rows are in flight together and DRAM pages are hit while open.
+  using Segment = DecodeSegment<DT, D, POW2, RAGGED>;
+  const int unit = blockIdx.x;
+  const int team = blockIdx.y;
+  const int kvh = unit / p.hchunks;
+  const int hchunk = unit - kvh * p.hchunks;
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, c = lane & 15;
+
+  __shared__ __attribute__((aligned(16))) unsigned char vt[Segment::kVtBytes];
+  __shared__ int32_t seg_lds[3][64];  // (first unit, units, context) of the 64 sequences being walked
+
+  const int hq_local = hchunk * 16 + c;
+  const bool head_ok = hq_local < p.group;
+  const int head = kvh * p.group + hq_local;
+
+  // ---- this team's piece of the concatenated KV streams (32-key units, visible keys only: with a
+  // sliding window the teams share what the windows leave, not the whole contexts) ----
+  auto context_of = [&](int bb) { return bb < p.B ? max(p.kv_len[bb], 0) : 0; };
+  auto units_of = [&](int ctx) { return ((ctx + 31) >> 5) - (first_visible(p, ctx) >> 5); };
+  int total = 0;
+  for (int b0 = 0; b0 < p.B; b0 += 64) {
+    int t = units_of(context_of(b0 + lane));
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) *(f32x4*)(wo + 16 * mt + 4 * g) = o[mt];
-    if (g == 0) {
-      p.ws_ml[slot * 2 + 0] = m_run;  // -inf with l = 0 for an empty segment: weight 0 in the combine
-      p.ws_ml[slot * 2 + 1] = l_run;
-    }
+    for (int d = 32; d >= 1; d >>= 1) t += __shfl_xor(t, d);
+    total += t;
   }
-  };  // process_segment
+  // (the reduction leaves the same value in every lane; say so, or every address derived from
+  // it is treated as lane-dependent and the block-table lookups become vector loads that
+  // share the in-order return queue of the K/V stream)
+  total = __builtin_amdgcn_readfirstlane(total);
+  const int upt = max((total + p.num_teams - 1) / p.num_teams, p.min_units);  // units per team
+  const int lo = team * upt;
+  if (lo >= total) return;
+  const int hi = min(lo + upt, total);
 
   // ---- walk the sequences this piece overlaps ----
   int carry = 0;  // units of all sequences before b0
   for (int b0 = 0; b0 < p.B; b0 += 64) {
-    const int t = units_of(b0 + lane);
+    const int ctx_mine = context_of(b0 + lane);
+    const int t = units_of(ctx_mine);
     const int incl = wave_inclusive_scan(t);
     const int excl = carry + incl - t;
     uint64_t hit = __ballot(t > 0 && excl < hi && excl + t > lo);
     // park the per-sequence values in LDS: nothing per-lane stays live across a segment
     seg_lds[0][lane] = excl;
     seg_lds[1][lane] = t;
+    seg_lds[2][lane] = ctx_mine;
     carry = __builtin_amdgcn_readfirstlane(carry + __shfl(incl, 63));
     while (hit) {  // wave-uniform
       const int l = __builtin_ctzll(hit);
@@ -407,55 +420,189 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
       const int b = b0 + l;
       const int pb = __builtin_amdgcn_readfirstlane(seg_lds[0][l]);
       const int tb = __builtin_amdgcn_readfirstlane(seg_lds[1][l]);
+      const int ctx = __builtin_amdgcn_readfirstlane(seg_lds[2][l]);
       const int first_team = pb / upt;
       if (team == first_team && unit == 0 && lane == 0)
         p.ws_np[b] = (pb + tb - 1) / upt - first_team + 1;
-      process_segment(b, (max(lo, pb) - pb) * 32, (min(hi, pb + tb) - pb) * 32, team - first_team);
+      // one segment of sequence b -> partial number team - first_team of b
+      const int kv_min = first_visible(p, ctx), k0 = kv_min & ~31;
+      Segment seg;
+      seg.run(p, vt, b, ctx, kvh, head, head_ok, k0 + (max(lo, pb) - pb) * 32, k0 + (min(hi, pb + tb) - pb) * 32,
+              kv_min);
+      if (head_ok) {
+        const int64_t slot = ((int64_t)b * p.Hq + head) * p.nsplit_max + (team - first_team);
+        float* wo = p.ws_o + slot * D;
+#pragma unroll
+        for (int mt = 0; mt < Segment::MT; ++mt) *(f32x4*)(wo + 16 * mt + 4 * g) = seg.o[mt];
+        if (g == 0) {
+          p.ws_ml[slot * 2 + 0] = seg.m_run;
+          p.ws_ml[slot * 2 + 1] = seg.l_run;
+        }
+      }
     }
     if (carry >= hi) break;
   }
 }
 
 // Combine the partials of one (sequence, head): O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s
-// (paged_attention.py:238-285 with the exponent in base 2).  Lane s of every wave fetches
-// (m_s, l_s) so the weights come from two wave reductions; the O_s rows are then read with all
-// loads of a group of four in flight.
+// (paged_attention.py:238-285 with the exponent in base 2).  A row of D floats is read by D / 4 lanes
+// and the rows are spread over the workgroup, so up to 8 - 16 rows are in flight per round; the
+// kernel is a chain of memory latencies, so what does not depend on the number of partials (the
+// first 64 (m, l) pairs and the first round of rows: inside the scratch whether written or not,
+// and masked) is requested together with it.
+constexpr int kCombineThreads = 256;
 template <int DT, int D>
-__global__ __launch_bounds__(D) void paged_decode_combine_kernel(const DecodeParams p) {
-  const int head = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
-  const int lane = d & 63;
+__global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(const DecodeParams p) {
+  constexpr int RL = D / 4;                    // lanes per row
+  constexpr int RG = kCombineThreads / RL;     // rows per round
+  __shared__ float acc_lds[RG][D];
+  __shared__ float w_lds[kCombineThreads / 64][64];
+  const int head = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int d4 = tid % RL, rg = tid / RL;
+  const bool row_lane = rg < RG;  // (D = 96: the last lanes have no row)
+  const int64_t slot0 = ((int64_t)b * p.Hq + head) * p.nsplit_max;
   const int ctx = p.kv_len[b];
-  float acc = 0.0f;
-  if (ctx > 0) {
-    const int ns = p.ws_np[b];  // pieces of this sequence (empty ones carry m = -inf, l = 0)
-    const int64_t slot0 = ((int64_t)b * p.Hq + head) * p.nsplit_max;
-    float m = -__builtin_inff();
-    for (int s0 = 0; s0 < ns; s0 += 64) {
-      float ms = (s0 + lane < ns) ? p.ws_ml[(slot0 + s0 + lane) * 2] : -__builtin_inff();
+  int ns = p.ws_np[b];  // partials of this sequence (unset if it is empty)
+  float m0 = -__builtin_inff(), l0 = 0.0f;
+  if (lane < p.nsplit_max) {
+    m0 = p.ws_ml[(slot0 + lane) * 2];
+    l0 = p.ws_ml[(slot0 + lane) * 2 + 1];
+  }
+  f32x4 v0 = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (row_lane && rg < p.nsplit_max) v0 = *(const f32x4*)(p.ws_o + (slot0 + rg) * D + 4 * d4);
+  if (ctx <= 0) ns = 0;
+  if (lane >= ns) {
+    m0 = -__builtin_inff();
+    l0 = 0.0f;
+  }
+  auto wave_max = [](float v) {
 #pragma unroll
-      for (int x = 32; x >= 1; x >>= 1) ms = fmaxf(ms, __shfl_xor(ms, x));
-      m = fmaxf(m, ms);
+    for (int x = 32; x >= 1; x >>= 1) v = fmaxf(v, __shfl_xor(v, x));
+    return v;
+  };
+  float m = m0;
+  for (int s0 = 64; s0 < ns; s0 += 64) m = fmaxf(m, s0 + lane < ns ? p.ws_ml[(slot0 + s0 + lane) * 2] : m);
+  m = wave_max(m);
+  float den = 0.0f;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < ns; s0 += 64) {
+    float ms = m0, ls = l0;
+    if (s0 > 0) {
+      ms = s0 + lane < ns ? p.ws_ml[(slot0 + s0 + lane) * 2] : -__builtin_inff();
+      ls = s0 + lane < ns ? p.ws_ml[(slot0 + s0 + lane) * 2 + 1] : 0.0f;
     }
-    float den = 0.0f;
-    for (int s0 = 0; s0 < ns; s0 += 64) {
-      const bool live = s0 + lane < ns;
-      const float w = live ? __builtin_amdgcn_exp2f(p.ws_ml[(slot0 + s0 + lane) * 2] - m) : 0.0f;
-      float wl = live ? w * p.ws_ml[(slot0 + s0 + lane) * 2 + 1] : 0.0f;
+    const float w = ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(ms - m);
+    den += w * ls;
+    w_lds[wave][lane] = w;  // (each wave its own copy: no barrier)
+    const int n = min(64, ns - s0);
+    for (int r0 = rg; r0 < n && row_lane; r0 += 4 * RG) {
+      f32x4 v[4];
 #pragma unroll
-      for (int x = 32; x >= 1; x >>= 1) wl += __shfl_xor(wl, x);
-      den += wl;
-      const int n = min(64, ns - s0);
-      for (int s = 0; s < n; s += 4) {
-        float v[4];
+      for (int u = 0; u < 4; ++u) {
+        const int r = r0 + u * RG;
+        v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (s0 == 0 && r0 == rg && u == 0) v[u] = v0;
+        else if (r < n) v[u] = *(const f32x4*)(p.ws_o + (slot0 + s0 + r) * D + 4 * d4);
+      }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = (s + u < n) ? p.ws_o[(slot0 + s0 + s + u) * D + d] : 0.0f;
+      for (int u = 0; u < 4; ++u) {
+        const int r = r0 + u * RG;
+        const float wr = r < n ? w_lds[wave][r] : 0.0f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc += __shfl(w, min(s + u, 63)) * v[u];
+        for (int i = 0; i < 4; ++i) acc[i] += wr * v[u][i];
       }
     }
-    acc /= den;
   }
-  if (d < p.dv) Elem<DT>::store1(p.o, (int64_t)b * p.o_sb + (int64_t)head * p.o_sh + d, acc);
+#pragma unroll
+  for (int x = 32; x >= 1; x >>= 1) den += __shfl_xor(den, x);
+  if (row_lane) *(f32x4*)&acc_lds[rg][4 * d4] = acc;
+  __syncthreads();
+  if (tid < p.dv) {
+    float out = 0.0f;
+#pragma unroll
+    for (int r = 0; r < RG; ++r) out += acc_lds[r][tid];
+    Elem<DT>::store1(p.o, (int64_t)b * p.o_sb + (int64_t)head * p.o_sh + tid, ns > 0 ? out / den : 0.0f);
+  }
+}
+
+// One workgroup per (kv-head unit, sequence): its W wavefronts take equal runs of the context's
+// visible 32-key units and merge their partials in LDS.  No scratch, no second launch.
+template <int DT, int D, bool POW2, bool RAGGED, int W>
+__global__ __launch_bounds__(64 * W, RAGGED ? 1 : 2) void paged_decode_direct_kernel(const DecodeParams p) {
+  using Segment = DecodeSegment<DT, D, POW2, RAGGED>;
+  constexpr int kPitch = D + 4;  // floats between the O rows of two heads: spreads them over the banks
+  static_assert(16 * kPitch * 4 <= Segment::kVtBytes, "a wavefront's O rows fit its V^T tile");
+  __shared__ __attribute__((aligned(16))) unsigned char vt[W][Segment::kVtBytes];
+  __shared__ float ml_lds[2][W][16];
+  const int unit = blockIdx.x, b = blockIdx.y;
+  const int kvh = unit / p.hchunks;
+  const int hchunk = unit - kvh * p.hchunks;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int hq_local = hchunk * 16 + c;
+  const bool head_ok = hq_local < p.group;
+
+  const int ctx = __builtin_amdgcn_readfirstlane(max(p.kv_len[b], 0));
+  const int kv_min = first_visible(p, ctx), k0 = kv_min & ~31;
+  const int units = (ctx - k0 + 31) >> 5;
+  const int u0 = units * wave / W, u1 = units * (wave + 1) / W;
+  Segment seg;
+  seg.run(p, vt[wave], b, ctx, kvh, kvh * p.group + hq_local, head_ok, k0 + 32 * u0, k0 + 32 * u1, kv_min);
+  // O rows into this wavefront's own tile (its LDS operations complete in order)
+  float* rows = (float*)vt[wave];
+#pragma unroll
+  for (int mt = 0; mt < Segment::MT; ++mt) *(f32x4*)(rows + c * kPitch + 16 * mt + 4 * g) = seg.o[mt];
+  if (g == 0) {
+    ml_lds[0][wave][c] = seg.m_run;
+    ml_lds[1][wave][c] = seg.l_run;
+  }
+  __syncthreads();
+  const int heads = min(16, p.group - hchunk * 16);
+  for (int i = threadIdx.x; i < heads * (D / 4); i += 64 * W) {
+    const int h = i / (D / 4), d4 = i % (D / 4);
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int w = 0; w < W; ++w) m = fmaxf(m, ml_lds[0][w][h]);
+    float den = 0.0f;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float mw = ml_lds[0][w][h];
+      const float f = mw == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mw - m);  // (no keys: weight 0)
+      den += f * ml_lds[1][w][h];
+      const f32x4 v = *(const f32x4*)((const float*)vt[w] + h * kPitch + 4 * d4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] += f * v[j];
+    }
+    const float inv = ctx > 0 ? 1.0f / den : 0.0f;
+    const int64_t out = (int64_t)b * p.o_sb + (int64_t)(kvh * p.group + hchunk * 16 + h) * p.o_sh;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (!RAGGED || 4 * d4 + j < p.dv) Elem<DT>::store1(p.o, out + 4 * d4 + j, acc[j] * inv);
+  }
+}
+
+// Wavefronts per workgroup of the one-launch kernel, 0: the split kernel.
+// One workgroup per (sequence, kv-head unit) reads a CU's share of the bandwidth at best, so with few
+// workgroups the split is the faster one from about 700 keys of 128 dims on (one sequence, 8 kv
+// heads: 100 keys 17.1 -> 4.7 us, 300 keys 17.1 -> 6.8, 700 keys 10.1 either way, 1400 keys 15.7
+// against 10.4).  With most CUs busy it wins up to the lengths where one long context among short
+// ones would be the whole time (20 sequences of 16 kv heads, 64 - 1024 keys: 22.7 -> 22.0 us; 250
+// of one kv head 23.9 -> 16.3; 128 x 100 keys 20.1 -> 13.4); past 1024 keys mixed lengths cost 3 - 6 %.
+// What a sliding window leaves is about the same for every sequence.
+// Eight wavefronts pay where the rows are short and a few CUs read many keys (1000 keys of 64 dims,
+// one sequence: 9.2 us, with four 10.7).
+int direct_waves(int B, int units, int max_ctx, int window, int D) {
+  if (D > 128) return 0;
+  const bool windowed = window > 0 && window + 32 < max_ctx;
+  const int keys = windowed ? window + 32 : max_ctx;
+  const int64_t wgs = (int64_t)B * units;
+  const bool few_keys = (int64_t)keys * D <= 700 * 128;
+  const bool busy = keys <= (windowed ? 2048 : 1024) && wgs >= (windowed ? 128 : 192);
+  if (!few_keys && !busy) return 0;
+  return D <= 64 && keys > 512 && wgs < 256 ? 8 : 4;
 }
 
 // smallest piece a team may get, in 32-key units: 512 keys, less for small problems so that
@@ -474,9 +621,17 @@ int partial_slots(int max_ctx, int min_units) {
   return t / min_units + 2;
 }
 
-// teams that are resident together: 8 wavefronts per CU (2 per SIMD) / wavefronts per team
-int pick_num_teams(int units_per_team) {
-  return max(1, current_device_cu_count() * 8 / units_per_team);
+// teams that are resident together: wavefronts per CU (2 per SIMD, 1 in the masked variant) /
+// wavefronts per team
+int pick_num_teams(int units_per_team, bool ragged) {
+  return max(1, current_device_cu_count() * (ragged ? 4 : 8) / units_per_team);
+}
+
+// head size the kernel instance is built for; past 128 one instance, for 256, takes every size on
+// its masked path
+int padded_head_size(int D, int Dv) {
+  const int d = D > Dv ? D : Dv;
+  return d <= 64 ? 64 : d <= 96 ? 96 : d <= 128 ? 128 : 256;
 }
 
 }  // namespace
@@ -485,7 +640,7 @@ int pick_num_teams(int units_per_team) {
 extern "C" size_t dlb_paged_decode_ws_bytes(int B, int Hq, int Hkv, int D, int page,
                                             int max_blocks) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || D > 256 || page <= 0 || max_blocks <= 0) return 0;
-  D = D <= 64 ? 64 : D <= 128 ? 128 : 256;  // the head size the kernels are built for
+  D = dlb::padded_head_size(D, D);
   const int group = Hq / Hkv;
   const int hchunks = (group + 15) / 16;
   const int64_t max_ctx = (int64_t)page * max_blocks;
@@ -510,9 +665,7 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
   if (B == 0) return DLB_OK;
   if (!q || !k_cache || !v_cache || !o || !block_table || !kv_len) return DLB_ERR_BAD_ARG;
   if (D % 8 != 0 || Dv % 8 != 0 || D > 256 || Dv > 256) return DLB_ERR_UNSUPPORTED;
-  // head size the kernel instance is built for; past 128 one instance, for 256, takes every size
-  // on its ragged path
-  const int Dp = (D <= 64 && Dv <= 64) ? 64 : (D <= 128 && Dv <= 128) ? 128 : 256;
+  const int Dp = padded_head_size(D, Dv);
   const bool ragged = D != Dp || Dv != Dp || Dp == 256;
   if (page % 16 != 0) return DLB_ERR_UNSUPPORTED;
   if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
@@ -573,40 +726,52 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
 
   hipStream_t s = (hipStream_t)stream;
   const int units = Hkv * p.hchunks;
-  p.num_teams = pick_num_teams(units);
-  if (units > 65535 || p.num_teams > 65535) return DLB_ERR_UNSUPPORTED;
+  p.num_teams = pick_num_teams(units, ragged);
+  if (units > 65535 || p.num_teams > 65535 || B > 65535) return DLB_ERR_UNSUPPORTED;
   const dim3 grid1((uint32_t)units, (uint32_t)p.num_teams);
-  const dim3 grid2((uint32_t)Hq, (uint32_t)B);
-#define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_) \
-  hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_>), grid1, dim3(64), 0, s, p)
-#define DLB_LAUNCH_DECODE(DT_, D_)                                                        \
-  do {                                                                                    \
-    if (p.page_shift >= 0) {                                                              \
-      if (ragged) DLB_LAUNCH_SPLIT(DT_, D_, true, true);                                  \
-      else DLB_LAUNCH_SPLIT(DT_, D_, true, false);                                        \
-    } else {                                                                              \
-      if (ragged) DLB_LAUNCH_SPLIT(DT_, D_, false, true);                                 \
-      else DLB_LAUNCH_SPLIT(DT_, D_, false, false);                                       \
-    }                                                                                     \
-    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_>), grid2, dim3(D_), 0, s, p); \
+  const dim3 grid2((uint32_t)Hq, (uint32_t)B), grid_direct((uint32_t)units, (uint32_t)B);
+  const int direct = direct_waves(B, units, max_ctx, window_size, Dp);
+#define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_)                                                                       \
+  do {                                                                                                            \
+    if (direct == 4)                                                                                              \
+      hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, D_, P2_, RG_, 4>), grid_direct, dim3(256), 0, s, p);    \
+    else if (D_ == 64 && direct == 8)                                                                             \
+      hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, 64, P2_, RG_, 8>), grid_direct, dim3(512), 0, s, p);    \
+    else                                                                                                          \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_>), grid1, dim3(64), 0, s, p);               \
   } while (0)
-#define DLB_LAUNCH_DECODE_256(DT_)                                                         \
-  do {                                                                                    \
-    if (p.page_shift >= 0) DLB_LAUNCH_SPLIT(DT_, 256, true, true);                        \
-    else DLB_LAUNCH_SPLIT(DT_, 256, false, true);                                         \
-    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, 256>), grid2, dim3(256), 0, s, p); \
+#define DLB_LAUNCH_DECODE(DT_, D_)                                                                           \
+  do {                                                                                                       \
+    if (p.page_shift >= 0) {                                                                                 \
+      if (ragged) DLB_LAUNCH_SPLIT(DT_, D_, true, true);                                                     \
+      else DLB_LAUNCH_SPLIT(DT_, D_, true, false);                                                           \
+    } else {                                                                                                 \
+      if (ragged) DLB_LAUNCH_SPLIT(DT_, D_, false, true);                                                    \
+      else DLB_LAUNCH_SPLIT(DT_, D_, false, false);                                                          \
+    }                                                                                                        \
+    if (!direct)                                                                                             \
+      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_>), grid2, dim3(kCombineThreads), 0, s, p);      \
   } while (0)
-  if (dtype == DLB_DTYPE_BF16) {
-    if (Dp == 256) DLB_LAUNCH_DECODE_256(DLB_DTYPE_BF16);
-    else if (Dp == 128) DLB_LAUNCH_DECODE(DLB_DTYPE_BF16, 128);
-    else DLB_LAUNCH_DECODE(DLB_DTYPE_BF16, 64);
-  } else {
-    if (Dp == 256) DLB_LAUNCH_DECODE_256(DLB_DTYPE_F16);
-    else if (Dp == 128) DLB_LAUNCH_DECODE(DLB_DTYPE_F16, 128);
-    else DLB_LAUNCH_DECODE(DLB_DTYPE_F16, 64);
-  }
+#define DLB_LAUNCH_DECODE_256(DT_)                                                                           \
+  do {                                                                                                       \
+    if (p.page_shift >= 0)                                                                                   \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, true, true>), grid1, dim3(64), 0, s, p);        \
+    else                                                                                                     \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, false, true>), grid1, dim3(64), 0, s, p);       \
+    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, 256>), grid2, dim3(kCombineThreads), 0, s, p);       \
+  } while (0)
+#define DLB_DISPATCH_DECODE(DT_)                        \
+  do {                                                  \
+    if (Dp == 256) DLB_LAUNCH_DECODE_256(DT_);          \
+    else if (Dp == 128) DLB_LAUNCH_DECODE(DT_, 128);    \
+    else if (Dp == 96) DLB_LAUNCH_DECODE(DT_, 96);      \
+    else DLB_LAUNCH_DECODE(DT_, 64);                    \
+  } while (0)
+  if (dtype == DLB_DTYPE_BF16) DLB_DISPATCH_DECODE(DLB_DTYPE_BF16);
+  else DLB_DISPATCH_DECODE(DLB_DTYPE_F16);
+#undef DLB_DISPATCH_DECODE
 #undef DLB_LAUNCH_DECODE_256
-#undef DLB_LAUNCH_SPLIT
 #undef DLB_LAUNCH_DECODE
+#undef DLB_LAUNCH_SPLIT
   return launch_status();
 }
