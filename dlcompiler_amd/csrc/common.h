@@ -136,6 +136,12 @@ __device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char*
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
   return (const unsigned char*)(uintptr_t)(((uint64_t)hi << 32) | lo);
 }
+// descriptor of `bytes` bytes at p (wave-uniform): raw buffer, no swizzle, loads past the end give 0
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(uniform_ptr((const unsigned char*)p)), 0,
+                                           (int)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+
 // wave-uniform LDS byte address of a pointer into __shared__ memory, in a scalar register
 __device__ __forceinline__ unsigned int lds_addr(const void* p) {
   typedef const __attribute__((address_space(3))) void* lds_ptr_t;

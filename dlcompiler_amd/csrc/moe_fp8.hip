@@ -86,11 +86,15 @@ __device__ __forceinline__ void wait_vm() {
 // dispatcher starts them.  At any moment an XCD therefore works on a handful of experts: an
 // expert's weights are streamed once while its few row blocks run side by side, and its
 // activation rows stay in that XCD's L2 across all its column tiles.
-// The expert's first block and its row count come from the per-expert counts of the alignment
-// (block b of expert e starts at sum_{e' < e} ceil(count / block_m) + b): one load per lane
-// and two wave scans.  All results are wave-uniform.
+// An expert's first position and its row count come from the per-expert counts of the alignment
+// (its rows start at block sum_{e' < e} ceil(count / block_m)): one load per lane and two wave scans.
+// Its rows are cut into as few tiles of up to 128 as hold them, equal to within one 32-row group: 268
+// rows make three tiles of 96, not 128 + 128 + 12 (which runs as 64), so the matrix work follows
+// the rows in steps of 32 and no workgroup outlasts its neighbours (fp8 layer, 64 experts of 2048 x
+// 1408: 72 rows each 143.5 -> 134.1 us, 192 rows 210 -> 203.6; 268 rows of 3840 x 512 246 -> 230.5).  All results are wave-uniform.
 __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, TileId& t) {
   const int bm = 1 << p.bm_shift;
+  constexpr int kMaxRows = 128;
   const bool segs = p.seg_start.p != nullptr;
   int cnt[4], nb[4], tl[4], st[4];
   int nb_sum = 0, tl_sum = 0;
@@ -101,7 +105,7 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
     cnt[c] = e < p.num_experts ? max(p.counts[e] - st[c], 0) : 0;
     nb[c] = (cnt[c] + bm - 1) >> p.bm_shift;
     const bool local = e >= p.expert_offset && e < p.expert_offset + p.num_local;
-    tl[c] = local ? nb[c] * p.num_ntiles : 0;
+    tl[c] = local ? (cnt[c] + kMaxRows - 1) / kMaxRows * p.num_ntiles : 0;
     nb_sum += nb[c];
     tl_sum += tl[c];
   }
@@ -116,7 +120,7 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
   const int L = __builtin_ctzll(hit);  // the lane whose four experts hold the tile
   int rem = logical - __builtin_amdgcn_readlane(tl_incl - tl_sum, L);
   int mbase = __builtin_amdgcn_readlane(nb_incl - nb_sum, L);
-  int e = 4 * L, nbe = 1, ce = 0, se = 0;
+  int e = 4 * L, ce = 0, se = 0;
   bool found = false;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -128,7 +132,6 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
       if (rem < tc) {
         found = true;
         e = 4 * L + c;
-        nbe = nc;
         ce = cc;
         se = sc;
       } else {
@@ -137,15 +140,17 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
       }
     }
   }
+  const int nbe = (ce + kMaxRows - 1) / kMaxRows;  // row tiles of this expert
   const int nt = rem / nbe;
   const int rb = rem - nt * nbe;
+  const int groups = (ce + 31) >> 5, base = groups / nbe, extra = groups - base * nbe;  // 32-row groups
+  const int r0 = 32 * (rb * base + min(rb, extra));
   t.e = e - p.expert_offset;
-  // block-aligned list: block mbase + rb; launcher form: the expert's own segment
-  t.row0 = segs ? se + (rb << p.bm_shift) : (mbase + rb) << p.bm_shift;
+  t.row0 = (segs ? se : mbase << p.bm_shift) + r0;  // block-aligned list / launcher form: its own segment
   t.nt = nt;
-  t.rows = min(bm, ce - (rb << p.bm_shift));
+  t.rows = min(32 * (base + (rb < extra ? 1 : 0)), ce - r0);
   // (counts that do not fit the slot list: touch nothing)
-  return segs ? t.row0 + t.rows <= p.numel : (mbase + rb) < p.num_mblocks;
+  return t.row0 + t.rows <= (segs ? p.numel : p.num_mblocks << p.bm_shift);
 }
 
 // QT = 0: fp8 operands with block scales; QT = 1: 16-bit operands of type DT, no scales.
@@ -154,7 +159,7 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
 // GATED = false: down GEMM, tile = 256 cols, epilogue * routing weight -> out[slot, n].
 // WL = weight layout (0 row-major, 1 operand order).
 //
-// Tile = one alignment block (up to 128 routing slots = four 32-row tiles) x 256 output columns,
+// Tile = up to 128 routing slots of one expert (two to four 32-row tiles) x 256 output columns,
 // four waves, two workgroups per CU.  A wave owns 64 output columns (two 32-column tiles; gated:
 // 32 gate + the matching 32 up columns) x all the rows: 4 x 2 accumulator tiles of the 32x32x64
 // (fp8) / 32x32x16 (16 bit) MFMA.  Lane (j = lane % 32, h = lane / 32) supplies, for weight
@@ -214,10 +219,9 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 
   TileId tile;
   if (!find_tile(p, lane, tile)) return;
-  // The rest of the kernel exists twice, for tiles of four and of two 32-row tiles (blocks with
-  // more / at most 64 real rows), each with its loops fully unrolled: row tiles of padding are
-  // skipped at that granularity without a run-time condition inside the main loop, and the two
-  // versions share no live values (each ends the kernel), so neither costs the other registers.
+  // The rest of the kernel exists three times, for tiles of four, three and two 32-row tiles, each
+  // with its loops fully unrolled: no run-time condition inside the main loop, and the versions
+  // share no live values (each ends the kernel), so none costs the others registers.
   auto run = [&](auto nrt_tag) {
   constexpr int NRT = decltype(nrt_tag)::value;
   const int e = tile.e, nt = tile.nt;
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   wait_vm<12 + D>();  // X(0) landed
   __syncthreads();
 
-  u32x4 xa[2], xb[2];  // fragment buffers: row tiles 0 and 2 use xa, 1 and 3 use xb
+  u32x4 xa[2], xb[2];  // fragment buffers, taken in turn by the 2 * NRT steps of a chunk
   read_x(0, 0, 0, xa);
   // s(k) / s(k + 1), k and k + 1 being the chunks in slots `cur` and `nxt` (both chunks' scales
   // are in LDS), split by operand: the activation part of row tile rt is computed where it is
@@ -444,8 +448,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
-      // even row tiles compute from xa, odd ones from xb; the next step's fragments are fetched
-      // into the other buffer before this step's MFMAs ((row tile 0, half 1) after the last)
+      // a step computes from one buffer while the next step's fragments are fetched into the
+      // other ((row tile 0, half 1) after the last)
       u32x4(&xc)[2] = (rt & 1) ? xb : xa;
       u32x4(&xn)[2] = (rt & 1) ? xa : xb;
       if (rt + 1 < NRT) read_x(x_cur, rt + 1, 0, xn);
@@ -471,8 +475,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
-      u32x4(&xc)[2] = (rt & 1) ? xb : xa;
-      u32x4(&xn)[2] = (rt & 1) ? xa : xb;
+      u32x4(&xc)[2] = ((NRT + rt) & 1) ? xb : xa;
+      u32x4(&xn)[2] = ((NRT + rt) & 1) ? xa : xb;
       if (rt + 1 < NRT) read_x(x_cur, rt + 1, 1, xn);
       else if (more) read_x(x_nxt, 0, 0, xn);
       __builtin_amdgcn_sched_barrier(0);
@@ -559,7 +563,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {  // 128 rows x 16 pieces of 16 bytes
       const int r = (tid_e >> 4) + 16 * i, pc = tid_e & 15;
-      if (r < 32 * NRT && nt * 128 + 8 * pc < p.I)  // (the last column tile may be partial)
+      if (r < tile.rows && nt * 128 + 8 * pc < p.I)  // (the last column tile may be partial)
         *(u32x4*)((unsigned short*)p.hq + (int64_t)(row0 + r) * p.I + nt * 128 + 8 * pc) =
             *(const u32x4*)(x_lds + r * kActPitch + 16 * pc);
     }
@@ -600,14 +604,14 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
         unsigned char* dst = x_lds + r * kGatedPitch + wave * 32 + 8 * h_e;
         *(u32x2*)(dst) = u32x2{q[0], q[1]};
         *(u32x2*)(dst + 16) = u32x2{q[2], q[3]};
-        if (wave == 0 && h_e == 0) p.hs[(int64_t)(row0 + r) * (p.I >> 7) + nt] = scale;
+        if (wave == 0 && h_e == 0 && r < tile.rows) p.hs[(int64_t)(row0 + r) * (p.I >> 7) + nt] = scale;
       }
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // 128 rows x 8 pieces of 16 bytes
       const int r = (tid_e >> 3) + 32 * i, pc = tid_e & 7;
-      if (r < 32 * NRT)
+      if (r < tile.rows)  // (the rows after them are another tile's)
         *(u32x4*)(p.hq + (int64_t)(row0 + r) * p.I + nt * 128 + 16 * pc) =
             *(const u32x4*)(x_lds + r * kGatedPitch + 16 * pc);
     }
@@ -618,12 +622,12 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     const int ncols = min(256, p.N - nt * 256);
     __syncthreads();  // every wave has left the main loop
 #pragma unroll
-    for (int half = 0; half < NRT / 2; ++half) {
+    for (int half = 0; half < (NRT + 1) / 2; ++half) {
       {
 #pragma unroll
         for (int rr = 0; rr < 2; ++rr) {
           const int rt = 2 * half + rr;
-          {
+          if (rt < NRT) {
             const float rwt = rw_lds[32 * rt + j_e];
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct) {
@@ -658,12 +662,13 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
                 *(const u32x4*)(x_lds + r * kPitch + 16 * pc),
                 (u32x4*)((unsigned short*)p.out + (int64_t)sid * p.N + nt * 256 + 8 * pc));
         }
-        if (half + 1 < NRT / 2) __syncthreads();  // the second half reuses the staging rows
+        if (half + 1 < (NRT + 1) / 2) __syncthreads();  // the second half reuses the staging rows
       }
     }
   }
   };  // run
-  if (tile.rows > 64) run(std::integral_constant<int, 4>{});
+  if (tile.rows > 96) run(std::integral_constant<int, 4>{});
+  else if (tile.rows > 64) run(std::integral_constant<int, 3>{});
   else run(std::integral_constant<int, 2>{});
 }
 
@@ -698,18 +703,24 @@ __global__ __launch_bounds__(256) void moe_topk_sum_kernel(const u32x4* __restri
   };
   const u32x4* row = in + t * (int64_t)(TOPK ? TOPK : topk) * vec_per_row + col;
   if constexpr (SHARD) {
+    // A slot held elsewhere is read at an offset past the descriptor's end: it gives zeros and touches
+    // no memory, and the loads of all slots go out behind each other.  (The descriptor starts at
+    // the workgroup's first row, so its offsets stay small whatever the size of `in`.)
     constexpr int U = TOPK ? TOPK : 4;
     const int k = TOPK ? TOPK : topk;
+    const int64_t t0 = (int64_t)blockIdx.x * 256 / vec_per_row;
+    const auto rsrc = buffer_of(in + t0 * k * vec_per_row, 0x7ffffff0u);
+    const uint32_t first = ((uint32_t)(t - t0) * k * (uint32_t)vec_per_row + col) * 16u;
     for (int j0 = 0; j0 < k; j0 += U) {
-      bool have[U];
+      int id[U];
       u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        have[u] = j0 + u < k && (unsigned)(shard.ids[t * k + j0 + u] - shard.first) < (unsigned)shard.num_local;
+      for (int u = 0; u < U; ++u) id[u] = shard.ids[t * k + min(j0 + u, k - 1)];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        v[u] = u32x4{0u, 0u, 0u, 0u};
-        if (have[u]) v[u] = __builtin_nontemporal_load(row + (int64_t)(j0 + u) * vec_per_row);
+        const bool have = j0 + u < k && (unsigned)(id[u] - shard.first) < (unsigned)shard.num_local;
+        const uint32_t off = first + (uint32_t)(j0 + u) * (uint32_t)vec_per_row * 16u;
+        v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, have ? (int)off : -1, 0, 2 /* non-temporal */);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) add(v[u]);
@@ -763,12 +774,13 @@ namespace {
 
 template <bool GATED, int QT>
 int launch_moe_gemm(const MoeGemmParams& p, int dtype, int w_layout, hipStream_t s) {
-  // one workgroup per tile slot of the block capacity; a workgroup finds its tile from the
-  // expert counts (or finds none and leaves), in the order described at find_tile
+  // one workgroup per tile there can be (at most one partial row tile per expert that holds slots); a
+  // workgroup finds its tile from the expert counts (or finds none and leaves), see find_tile
   if (w_layout && p.N % 16 != 0) return DLB_ERR_UNSUPPORTED;  // operand order comes in 16-row tiles
   if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
   if (moe_stream_case(p, QT == 0)) return launch_moe_stream(p, GATED, QT == 0, dtype, w_layout, s);
-  const uint32_t grid = (uint32_t)(ceil_div((int64_t)p.num_mblocks * p.num_ntiles, 8) * 8);
+  const int64_t row_tiles = (int64_t)p.numel / 128 + (p.numel < p.num_local ? p.numel : p.num_local);
+  const uint32_t grid = (uint32_t)(ceil_div(row_tiles * p.num_ntiles, 8) * 8);
 #define DLB_LAUNCH_GEMM(DT_)                                                                   \
   do {                                                                                       \
     if (w_layout)                                                                            \

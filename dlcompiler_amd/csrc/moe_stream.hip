@@ -92,12 +92,6 @@ __device__ __forceinline__ float max_groups(float v) {
   return max_xor32(v);
 }
 
-// descriptor of `bytes` bytes at p (wave-uniform): raw buffer, no swizzle, loads past the end give 0
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(uniform_ptr((const unsigned char*)p)), 0,
-                                           (int)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
-}
-
 // CW waves side by side in the columns, KW in K.  GATED: a wave's 64 weight rows are 32 gate rows and
 // the 32 up rows that go with them (fp8: CW = 4, the workgroup then holds whole 128-column
 // quantisation groups of its rows); else 64 consecutive rows.

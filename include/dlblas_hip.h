@@ -266,7 +266,7 @@ int dlb_per_token_group_quant_fp8(const void* x, void* xq, float* xs, int64_t M,
  *   w1q [num_local_experts, 2I, H] fp8 (gate rows first), w1s [num_local_experts, 2I/128, H/128]
  *   sorted_ids [num_mblocks * block_m] and expert_counts [num_experts]: the sorted slot list and
  *     the per-expert counts written by dlb_moe_align_block_size with block = block_m over all
- *     num_experts (global) experts; block_m in {64, 128} = rows per workgroup tile; flat slot =
+ *     num_experts (global) experts; block_m in {64, 128}; flat slot =
  *     token * topk + j, sentinel num_tokens * topk.  num_mblocks = whole blocks sorted_ids
  *     holds (it has at least num_mblocks * block_m entries; floor(sorted_cap / block_m) of the
  *     alignment call is always >= sum over experts of ceil(count / block_m), the blocks in use;
@@ -276,13 +276,13 @@ int dlb_per_token_group_quant_fp8(const void* x, void* xq, float* xs, int64_t M,
  *     [expert_offset, expert_offset + num_local_experts) are skipped.  num_experts <= 256.
  *   hq [num_mblocks * block_m, I] fp8 and hs [num_mblocks * block_m, I/128]: row r holds
  *     quant(silu(x_t W_gate^T) * (x_t W_up^T)) for the slot at sorted position r (rows of
- *     32-row groups that hold padding only are not written)
+ *     padding are not written)
  * H % 128 == 0, I % 128 == 0, and the reduction length (H here, I in the down GEMM) at most
  * 16384.  Scales must be positive: activation scales below 1e-13 may count as 1e-13 (the quantisation
  * rule above never produces less than 1e-10 / 448) and weight block scales below 1e-12 as
  * 1e-12 (an all-zero block may carry the scale 0).
  * Up to about 40 routed rows per expert a kernel that streams the weights runs, beyond it one with
- * tiles of block_m rows x 256 columns; both take both tile heights and both weight layouts.
+ * tiles of up to 128 rows x 256 columns; both take both tile heights and both weight layouts.
  * Outputs are stored 16 bytes at a time: hq, out and the 16-bit act must be 16-byte aligned;
  * other alignments return DLB_ERR_UNSUPPORTED.
  * w_layout selects how the fp8 weight bytes of both GEMMs are stored:
