@@ -226,6 +226,16 @@ __device__ __forceinline__ float max_xor32(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// tanh for the logit soft-cap, relative error below 4e-7: odd polynomial near 0, 1 - 2 / (e^2x + 1)
+// elsewhere (saturates to +-1).  A third of tanhf's instructions, and no branch.
+__device__ __forceinline__ float softcap_tanh(float x) {
+  const float x2 = x * x;
+  const float poly = x * (1.0f + x2 * (-1.0f / 3.0f + x2 * (2.0f / 15.0f + x2 * (-17.0f / 315.0f + x2 * (62.0f / 2835.0f)))));
+  const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);
+  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+  return fabsf(x) < 0.25f ? poly : big;
+}
+
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) {
   return (a + b - 1) / b;
 }

@@ -265,7 +265,7 @@ struct DecodeSegment {
       for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          s[sub][i] = p.softcap * tanhf(s[sub][i] * p.sm_scale / p.softcap) * 1.4426950408889634f;
+          s[sub][i] = p.softcap * softcap_tanh(s[sub][i] * p.sm_scale / p.softcap) * 1.4426950408889634f;
     } else {
 #pragma unroll
       for (int sub = 0; sub < 2; ++sub)

@@ -78,7 +78,6 @@ struct Mma32<DLB_DTYPE_F16> {
   }
 };
 
-constexpr int kBlockM = 128;  // query rows per workgroup
 constexpr int kTileN = 64;    // keys per LDS tile
 constexpr int kThreads = 256;
 
@@ -90,7 +89,7 @@ struct Smem {
   static constexpr int stage = kBytes + vBytes;
 };
 
-// D is the padded head size the kernel is built for (64 or 128).  RAGGED: the real key size dk
+// D is the padded head size the kernel is built for (64, 96, 128 or 256).  RAGGED: the real key size dk
 // and / or value size dv is smaller (any multiple of 8): the query dims past dk are loaded as
 // zeros, so the key bytes staged for those dims do not count -- their copies are redirected to
 // the row's first 16 bytes to stay inside the tensor -- and value dims past dv (redirected
@@ -101,14 +100,22 @@ struct Smem {
 // with pages that are whole multiples of the 64-key tile: a tile lies in one page, so its page
 // number is one wave-uniform look-up and the copies are addressed as in the packed layout (a
 // scalar base per tile plus constant lane offsets).
-template <int DT, int D, int PAGED, bool RAGGED>
-__global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel(const PrefillParams p) {
+// RW: row waves, KG = 4 / RW key groups of a workgroup's four waves.  RW = 4: 128 query rows.  RW = 2: 64
+// rows, and two pairs of waves that work on every second key tile each, with LDS buffers of their
+// own; their partial results meet in LDS at the end.  A wave keeps its SIMD busy by itself, so a
+// launch with fewer 128-row workgroups than CUs is as fast as one workgroup's chain of tiles: this
+// shape gives it twice the workgroups and half the chain (one sequence of 512 tokens, 32 heads of
+// 128: 13.6 -> 11.2 us, of 1125 tokens, 8 heads: 21.7 -> 16.0; eight waves on 128 rows: 13.6 and 19.5).
+template <int DT, int D, int PAGED, bool RAGGED, int RW>
+__global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefill_attn_kernel(const PrefillParams p) {
+  constexpr int KG = 4 / RW;
+  constexpr int kBlockM = 32 * RW;  // query rows per workgroup
   constexpr int KS = D / 16;  // MFMA k-steps over the head dim for S^T
   constexpr int MT = D / 32;  // 32-row tiles of O^T
   constexpr int DG = D / 8;
   using SM = Smem<D>;
 
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * SM::stage];
+  __shared__ __attribute__((aligned(16))) unsigned char smem_all[KG * 2 * SM::stage];
 
   // The grid runs over (head, query tile, sequence), tile index reversed: what an XCD holds at
   // any time is the query tiles of ONE sequence's heads of ONE KV group (see the head remap
@@ -139,13 +146,14 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
     __syncthreads();
     seq = __builtin_amdgcn_readfirstlane(rank_seq);
   }
-  const int L = p.seq_len[seq];
+  // (vector loads of wave-uniform values: saying that they are keeps loops and conditions scalar)
+  const int L = __builtin_amdgcn_readfirstlane(p.seq_len[seq]);
   const int qtile = gridDim.y - 1 - blockIdx.y;  // heaviest first
   const int q0 = qtile * kBlockM;
   if (q0 >= L) return;
-  const int64_t tok0 = p.start_loc[seq];
+  const int64_t tok0 = __builtin_amdgcn_readfirstlane(p.start_loc[seq]);
   // context seen by this sequence: kv_total keys, the queries are its last L positions
-  const int kv_total = PAGED ? p.kv_len[seq] : L;
+  const int kv_total = PAGED ? __builtin_amdgcn_readfirstlane(p.kv_len[seq]) : L;
   const int hist = kv_total - L;
   if (PAGED && hist < 0) return;  // inconsistent lengths: nothing sensible to compute
   int head = blockIdx.x;
@@ -153,8 +161,10 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   const int kvh = head / p.group;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane((tid >> 6) / RW) : 0;
+  const int wave = (tid >> 6) % RW;  // row wave
   const int lane = tid & 63;
+  unsigned char* const smem = smem_all + grp * (2 * SM::stage);
   const int col = lane & 31;  // query column / operand row
   const int hh = lane >> 5;   // lane half
 
@@ -181,12 +191,13 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   // (only the paged entry point exposes them; the packed kernel compiles them out)
   const int window = PAGED ? p.window : -1;
   const float softcap = PAGED ? p.softcap : -1.0f;
-  const bool generic = (window > 0) || (softcap > 0.0f);
   // tiles below this index lie entirely under the diagonal for every wave of the workgroup
   // (all 64 keys <= position of row q0): no mask, no clamping of key rows
-  const int nfull = generic ? 0 : (hist + q0 + 1) / kTileN;
-  // first tile that can hold a visible key (sliding window)
+  const int nfull = softcap > 0.0f ? 0 : (hist + q0 + 1) / kTileN;
+  // first tile that can hold a visible key (sliding window), and the first whose keys every query
+  // of the workgroup sees
   const int jfirst = window > 0 ? max(hist + q0 - window, 0) / kTileN : 0;
+  const int jopen = window > 0 ? max(hist + q0 + kBlockM - 1 - window + kTileN - 1, 0) / kTileN : 0;
   const int qpos = hist + qrow;                          // context position of this lane's query
   const int wave_last_pos = hist + q0 + 32 * wave + 31;
 
@@ -200,28 +211,32 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   // row r reads position c ^ swz(r).  K: swz(r) = r mod DG (128-bit fragment reads, one row
   // per lane).  V: swz(r) spreads the 4 (or 8) rows that one transposing read touches over
   // all banks.
-  constexpr int KRPI = 1024 / (2 * D);            // rows per wave instruction
-  constexpr int KINS = kTileN / KRPI / 4;         // instructions per wave, tile and operand
-  const int k_lrow = lane / DG;                   // row inside an instruction
-  const int k_pos = lane % DG;                    // 16-byte position inside the row
+  constexpr int KINS = kTileN * DG / (64 * RW);  // instructions per wave, tile and operand
+  // copy i of a wave brings the tile's 16-byte pieces 64 * (RW i + wave) + lane, counted row by row
+  auto copy_row = [&](int i) -> int { return ((RW * i + wave) * 64 + lane) / DG; };
+  auto copy_pos = [&](int i) -> int { return ((RW * i + wave) * 64 + lane) % DG; };
   const unsigned char* kbytes = (const unsigned char*)kb;
   const unsigned char* vbytes = (const unsigned char*)vb;
   const int64_t k_row_bytes = p.k_st * 2, v_row_bytes = p.v_st * 2;
   const IdxArray bt = {PAGED ? p.block_table.p + (((int64_t)seq * p.bt_stride) << p.block_table.sh) : nullptr,
                        p.block_table.sh};
+  // K chunk swizzle of row r.  (Rows of 96 elements start 48 banks apart: four rows fill all 64
+  // banks, the swizzle separates the four groups of four that a fragment read touches.)
+  auto k_swz = [](int r) -> int { return D == 96 ? (r >> 2) & 3 : r & (DG - 1); };
   // V chunk swizzle of row r (depends on r mod 8 only)
   auto v_swz = [](int r) -> int {
+    if (D == 96) return 0;
     return D == 128 ? (((r & 3) << 2) | (((r >> 2) & 1) << 1))
                     : ((((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1));
   };
-  // byte offset inside its source row of the 16-byte chunk this lane copies into position k_pos
-  // of row r (the swizzle undone; chunks past the real head size fetch the row's first chunk)
-  auto k_chunk = [&](int r) -> unsigned int {
-    const int c = k_pos ^ (r & (DG - 1));
+  // byte offset inside its source row of the 16-byte chunk that copy i of this lane brings (the
+  // swizzle undone; chunks past the real head size fetch the row's first chunk)
+  auto k_chunk = [&](int i) -> unsigned int {
+    const int c = copy_pos(i) ^ k_swz(copy_row(i));
     return (unsigned int)((RAGGED && 8 * c >= p.dk) ? 0 : c) << 4;
   };
-  auto v_chunk = [&](int r) -> unsigned int {
-    const int c = k_pos ^ v_swz(r);
+  auto v_chunk = [&](int i) -> unsigned int {
+    const int c = copy_pos(i) ^ v_swz(copy_row(i));
     return (unsigned int)((RAGGED && 8 * c >= p.dv) ? 0 : c) << 4;
   };
   // paged layout: the page ids of the rows this lane copies are fetched one tile ahead of the
@@ -236,11 +251,11 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
     }
 #pragma unroll
     for (int i = 0; i < KINS; ++i) {
-      const int key = min(t0 + (4 * i + wave) * KRPI + k_lrow, kv_total - 1);
+      const int key = min(t0 + copy_row(i), kv_total - 1);
       pg_next[i] = bt[p.page_shift >= 0 ? (key >> p.page_shift) : (key / p.page)];
     }
   };
-  const unsigned int smem_base = lds_addr(smem) + wave * 1024;  // + q * 1024 with q = 4*i + wave
+  const unsigned int smem_base = lds_addr(smem_all) + grp * (2 * SM::stage) + wave * 1024;  // + q * 1024 with q = RW*i + wave
   // source addresses and LDS targets of the copies of the tile being staged: prepare_tile
   // computes them, issue_copy(n) sends copy n of 2 * KINS (K and V slices alternate)
   // Packed layout: a copy's address is a tile base in scalar registers plus a 32-bit lane
@@ -254,9 +269,8 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   const unsigned char* vbase = nullptr;
 #pragma unroll
   for (int i = 0; i < KINS; ++i) {
-    const int r = (4 * i + wave) * KRPI + k_lrow;
-    koff0[i] = (unsigned int)(r * k_row_bytes) + k_chunk(r);
-    voff0[i] = (unsigned int)(r * v_row_bytes) + v_chunk(r);
+    koff0[i] = (unsigned int)(copy_row(i) * k_row_bytes) + k_chunk(i);
+    voff0[i] = (unsigned int)(copy_row(i) * v_row_bytes) + v_chunk(i);
   }
   unsigned int stage_dst = 0;
   auto prepare_tile = [&](auto clamp_tag, int t0, int buf) {
@@ -277,28 +291,28 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
     }
 #pragma unroll
     for (int i = 0; i < KINS; ++i) {
-      const int r = (4 * i + wave) * KRPI + k_lrow;  // key row inside the tile
+      const int r = copy_row(i);  // key row inside the tile
       if (PAGED == 1) {
         int key = t0 + r;
         if (CLAMP) key = min(key, kv_total - 1);
         const int pi = p.page_shift >= 0 ? (key >> p.page_shift) : (key / p.page);
         const int64_t slot = key - pi * p.page;
-        ksrc[i] = kbytes + ((int64_t)pg_next[i] * p.k_sp + slot * p.k_st) * 2 + k_chunk(r);
-        vsrc[i] = vbytes + ((int64_t)pg_next[i] * p.v_sp + slot * p.v_st) * 2 + v_chunk(r);
+        ksrc[i] = kbytes + ((int64_t)pg_next[i] * p.k_sp + slot * p.k_st) * 2 + k_chunk(i);
+        vsrc[i] = vbytes + ((int64_t)pg_next[i] * p.v_sp + slot * p.v_st) * 2 + v_chunk(i);
       } else if (CLAMP) {
         const int rc = min(r, kv_total - 1 - t0);  // >= 0: a staged tile starts inside the context
-        koff[i] = (unsigned int)(rc * k_row_bytes) + k_chunk(r);
-        voff[i] = (unsigned int)(rc * v_row_bytes) + v_chunk(r);
+        koff[i] = (unsigned int)(rc * k_row_bytes) + k_chunk(i);
+        voff[i] = (unsigned int)(rc * v_row_bytes) + v_chunk(i);
       } else {
         koff[i] = koff0[i];
         voff[i] = voff0[i];
       }
     }
-    if (PAGED) fetch_pages(t0 + kTileN);  // consumed by the next prepare_tile
+    if (PAGED) fetch_pages(t0 + KG * kTileN);  // consumed by the next prepare_tile
   };
   auto issue_copy = [&](int n) {
-    const int i = n >> 1;  // 1 KB slice 4*i + wave of the tile
-    const unsigned int dst = stage_dst + (n & 1) * SM::kBytes + i * 4096;
+    const int i = n >> 1;  // 1 KB slice RW*i + wave of the tile
+    const unsigned int dst = stage_dst + (n & 1) * SM::kBytes + i * (RW * 1024);
     if (PAGED == 1) dma16_global_to_lds((n & 1) ? vsrc[i] : ksrc[i], dst);
     else if (n & 1) dma16_global_to_lds(vbase, voff[i], dst);
     else dma16_global_to_lds(kbase, koff[i], dst);
@@ -335,16 +349,17 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   }
 
   // one K/V tile against this wave's 32 queries; MASK: apply the causal mask
-  // COPY: the copies of the tile prepared by prepare_tile go out between the S^T MFMAs, one per
-  // k-step, instead of as one burst that would hold up this wave's instruction stream
-  auto process_tile = [&](auto mask_tag, auto copy_tag, int j) {
+  // COPY: the copies of the tile prepared by prepare_tile go out between the S^T MFMAs, one or two
+  // per k-step, instead of as one burst that would hold up this wave's instruction stream
+  auto process_tile = [&](auto mask_tag, auto copy_tag, int j, int buf) __attribute__((always_inline)) {
     constexpr bool MASK = decltype(mask_tag)::value;
     constexpr bool COPY = decltype(copy_tag)::value;
-    static_assert(2 * KINS == KS, "one copy per k-step");
+    constexpr int kCopies = 2 * KINS / KS;  // per k-step
+    static_assert(kCopies * KS == 2 * KINS, "whole copies per k-step");
     const int t0 = j * kTileN;
     if (MASK && t0 > wave_last_pos) return;  // wave-uniform: tile entirely above the diagonal
     if (MASK && window > 0 && t0 + kTileN - 1 < wave_last_pos - 31 - window) return;  // below the window
-    const unsigned char* ks = smem + (j & 1) * SM::stage;
+    const unsigned char* ks = smem + buf * SM::stage;
     const unsigned char* vs = ks + SM::kBytes;
 
     // ---- S^T = K . Q^T : two 32-key tiles x 32 queries (raw scores)
@@ -361,7 +376,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
     {
       const unsigned char* krow0 = ks + col * SM::kRowBytes;
       const unsigned char* krow1 = ks + (32 + col) * SM::kRowBytes;
-      const int ksw = col & (DG - 1);  // (32 + col) & (DG - 1) is the same
+      const int ksw = k_swz(col);  // (row 32 + col has the same)
       auto ldk = [&](int kstep, u32x4 (&a)[2]) {
         const int off = ((2 * kstep + hh) ^ ksw) << 4;
         a[0] = *(const u32x4*)(krow0 + off);
@@ -374,7 +389,10 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
 #pragma unroll
       for (int kstep = 0; kstep < KS; ++kstep) {
         if (kstep + kAhead < KS) ldk(kstep + kAhead, ka[(kstep + kAhead) % (kAhead + 1)]);
-        if (COPY) issue_copy(kstep);
+        if (COPY) {
+#pragma unroll
+          for (int n = 0; n < kCopies; ++n) issue_copy(kCopies * kstep + n);
+        }
         __builtin_amdgcn_sched_barrier(0);  // keep the fetch ahead of the MFMAs (it would be sunk)
         s[0] = Mma32<DT>::run(ka[kstep % (kAhead + 1)][0], qf[kstep], s[0]);
         s[1] = Mma32<DT>::run(ka[kstep % (kAhead + 1)][1], qf[kstep], s[1]);
@@ -384,6 +402,18 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
 
     __builtin_amdgcn_s_setprio(0);
     // ---- causal mask and tile maximum of the raw scores (scale > 0 commutes with max)
+    // (opaque: a condition on a value the compiler knows to be constant in the loop makes it split the
+    // loop by it, and the copies' accumulators do not share registers)
+    float cap = softcap;
+    if (MASK && PAGED) asm volatile("" : "+s"(cap));
+    if (MASK && cap > 0.0f) {  // cap * tanh(x * scale / cap), kept in raw-score units
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          s[nt][i] = softcap_tanh(s[nt][i] * (p.sm_scale / cap)) * (cap / p.sm_scale);
+    }
+    const int oldest = MASK && window > 0 ? qpos - window : 0;  // first key this lane's query sees
     float mpart[2] = {-__builtin_inff(), -__builtin_inff()};  // two independent chains
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -391,12 +421,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
       for (int i = 0; i < 16; ++i) {
         if (MASK) {
           const int key = t0 + 32 * nt + 8 * (i >> 2) + 4 * hh + (i & 3);
-          float x = s[nt][i];
-          if (softcap > 0.0f)  // cap * tanh(x * scale / cap), kept in raw-score units
-            x = tanhf(x * (p.sm_scale / softcap)) * (softcap / p.sm_scale);
-          bool vis = key <= qpos;
-          if (window > 0) vis = vis && (key >= qpos - window);
-          s[nt][i] = vis ? x : -__builtin_inff();
+          s[nt][i] = key <= qpos && key >= oldest ? s[nt][i] : -__builtin_inff();
         }
         mpart[nt] = fmaxf(mpart[nt], s[nt][i]);
       }
@@ -460,31 +485,91 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void prefill_attn_kernel
   // vmcnt(0): the direct-to-LDS loads of this wave have landed before the barrier publishes
   // the buffer (encoding: vmcnt = 0, expcnt / lgkmcnt left at their maxima)
   auto wait_dma = [&]() { __builtin_amdgcn_s_waitcnt(0x0F70); };
-  int j = jfirst;
-  if (PAGED) fetch_pages(j * kTileN);
-  if (j < nfull) load_tile(NoClamp{}, j * kTileN, j & 1); else load_tile(Clamp{}, j * kTileN, j & 1);
+  using Yes = std::integral_constant<bool, true>;
+  using No = std::integral_constant<bool, false>;
+  // Group grp takes tiles jfirst + grp, + KG, ...; both groups make the same number of steps, one barrier
+  // each.  A wave whose rows all lie past the sequence only copies.
+  const bool wave_rows = q0 + 32 * __builtin_amdgcn_readfirstlane(wave) < L;
+  int jb = jfirst;  // the step's first tile
+  // (the step's LDS buffer, worked out where it is used: carried along as a variable it costs the paged
+  // kernels 50 registers)
+  auto buf = [&]() -> int { return ((jb - jfirst) / KG) & 1; };
+  auto stage_tile = [&](int j, int to) __attribute__((always_inline)) {
+    if (j >= ntiles) return;
+    if (j < nfull) load_tile(NoClamp{}, j * kTileN, to); else load_tile(Clamp{}, j * kTileN, to);
+  };
+  if (PAGED) fetch_pages((jb + grp) * kTileN);
+  stage_tile(jb + grp, 0);
   wait_dma();
   __syncthreads();
 
-  // tiles under the diagonal whose successor is also under it: nothing to mask or clamp
-  using Yes = std::integral_constant<bool, true>;
-  using No = std::integral_constant<bool, false>;
-  for (; j + 1 < nfull; ++j) {
-    prepare_tile(NoClamp{}, (j + 1) * kTileN, (j + 1) & 1);
-    process_tile(No{}, Yes{}, j);
+  auto end_step = [&]() __attribute__((always_inline)) {
     wait_dma();
     __syncthreads();
+    jb += KG;
+  };
+  // a step whose tiles may be masked, or whose successors may run past the sequence: at the window's edge,
+  // the last unmasked tiles, the diagonal
+  auto edge_step = [&]() __attribute__((always_inline)) {
+    const int j = jb + grp;
+    stage_tile(j + KG, buf() ^ 1);
+    // a diagonal tile still lies entirely under the diagonal for the waves further down (and a tile at
+    // the window's edge entirely inside it for some)
+    const bool wave_full = softcap <= 0.0f && (j + 1) * kTileN - 1 <= hist + q0 + 32 * wave &&
+                           (window <= 0 || j * kTileN >= wave_last_pos - window);
+    if (j < ntiles) {
+      if (wave_full) process_tile(No{}, No{}, j, buf());
+      else process_tile(Yes{}, No{}, j, buf());
+    }
+    end_step();
+  };
+  if (!wave_rows) {
+    while (jb < ntiles) {
+      stage_tile(jb + grp + KG, buf() ^ 1);
+      end_step();
+    }
+  } else {
+    if (PAGED)
+      while (jb < min(jopen, ntiles)) edge_step();
+    // tiles under the diagonal (and inside every query's window) whose successor is also under it:
+    // nothing to mask or clamp
+    while (jb + 2 * KG - 1 < nfull) {
+      prepare_tile(NoClamp{}, (jb + grp + KG) * kTileN, buf() ^ 1);
+      process_tile(No{}, Yes{}, jb + grp, buf());
+      end_step();
+    }
+    while (jb < ntiles) edge_step();
   }
-  // last unmasked tile (its successor may run past the sequence), then the diagonal tiles
-  for (; j < ntiles; ++j) {
-    const bool more = (j + 1 < ntiles);
-    if (more) load_tile(Clamp{}, (j + 1) * kTileN, (j + 1) & 1);
-    // a diagonal tile still lies entirely under the diagonal for the waves further down
-    const bool wave_full = !generic && (j + 1) * kTileN - 1 <= hist + q0 + 32 * wave;
-    if (j < nfull || wave_full) process_tile(No{}, No{}, j);
-    else process_tile(Yes{}, No{}, j);
-    wait_dma();
+
+  if constexpr (KG > 1) {
+    // the second group's partial results, by lane: its rows are the first group's
+    float* part = (float*)smem_all + wave * ((16 * MT + 2) * 64);
+    if (grp == 1) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(f32x4*)(part + ((4 * mt + q) * 64 + lane) * 4) =
+              f32x4{o[mt][4 * q], o[mt][4 * q + 1], o[mt][4 * q + 2], o[mt][4 * q + 3]};
+      part[16 * MT * 64 + lane] = m_run;
+      part[16 * MT * 64 + 64 + lane] = l_run;
+    }
     __syncthreads();
+    if (grp == 1) return;
+    const float m1 = part[16 * MT * 64 + lane], l1 = part[16 * MT * 64 + 64 + lane];
+    const float m = fmaxf(m_run, m1);
+    // (a group without a visible key: weight 0)
+    const float a0 = m_run == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
+    const float a1 = m1 == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
+    l_run = l_run * a0 + l1 * a1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = *(const f32x4*)(part + ((4 * mt + q) * 64 + lane) * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[mt][4 * q + i] = o[mt][4 * q + i] * a0 + v[i] * a1;
+      }
   }
 
   // ---- epilogue: normalise and store O (lane holds 4 consecutive dims per register quad)
@@ -514,12 +599,13 @@ namespace {
 // Shared argument checks and launch of both entry points; the paged fields of `p` are already
 // filled in (or zeroed) by the caller.
 int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk, int Dv, int max_len,
-                   float sm_scale, int dtype, void* stream) {
+                   int64_t max_keys, float sm_scale, int dtype, void* stream) {
   if (Dk % 8 != 0 || Dv % 8 != 0 || Dk > 256 || Dv > 256) return DLB_ERR_UNSUPPORTED;
   // head size the kernel instance is built for; past 128 there is one instance, for 256, that
   // takes every size on its ragged path (one workgroup per CU, one wave per SIMD: the 128 output
   // accumulators and the 64 query registers of a lane leave no room for a second wave)
-  const int D = (Dk <= 64 && Dv <= 64) ? 64 : (Dk <= 128 && Dv <= 128) ? 128 : 256;
+  const int Dm = Dk > Dv ? Dk : Dv;
+  const int D = Dm <= 64 ? 64 : Dm <= 96 ? 96 : Dm <= 128 ? 128 : 256;
   const bool ragged = Dk != D || Dv != D || D == 256;
   p.dk = Dk;
   p.dv = Dv;
@@ -545,37 +631,50 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.sm_scale = sm_scale;
 
   hipStream_t s = (hipStream_t)stream;
-  const uint32_t qtiles = (uint32_t)ceil_div(max_len, kBlockM);
+  // 64-row workgroups where 128-row ones would leave CUs without any (of 256), unless there are so few
+  // keys that the merge costs more than it saves (40 heads, 4 x 49 tokens: 5.4 against 6.9 us)
+  const bool small = D <= 128 && Hq * ceil_div(max_len, 128) * B <= 240 && max_keys > 128;
+  const uint32_t qtiles = (uint32_t)ceil_div(max_len, small ? 64 : 128);
   if (qtiles > 65535) return DLB_ERR_UNSUPPORTED;
   const dim3 grid = dim3((uint32_t)Hq, qtiles, (uint32_t)B);
-#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                                                          \
-  do {                                                                                            \
-    if (ragged)                                                                                   \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, true>), grid, dim3(kThreads), 0, s, p);  \
-    else                                                                                          \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, false>), grid, dim3(kThreads), 0, s, p); \
+#define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_)                                                               \
+  do {                                                                                                         \
+    if (ragged)                                                                                                \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, true, RW_>), grid, dim3(kThreads), 0, s, p);        \
+    else                                                                                                       \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, false, RW_>), grid, dim3(kThreads), 0, s, p);       \
   } while (0)
-#define DLB_DISPATCH_PREFILL(PG_)                                                                \
-  if (dtype == DLB_DTYPE_BF16) {                                                                 \
-    if (D == 256)                                                                                \
-      hipLaunchKernelGGL((prefill_attn_kernel<DLB_DTYPE_BF16, 256, PG_, true>), grid,            \
-                         dim3(kThreads), 0, s, p);                                               \
-    else if (D == 128) DLB_LAUNCH_PREFILL(DLB_DTYPE_BF16, 128, PG_);                              \
-    else DLB_LAUNCH_PREFILL(DLB_DTYPE_BF16, 64, PG_);                                             \
-  } else {                                                                                       \
-    if (D == 256)                                                                                \
-      hipLaunchKernelGGL((prefill_attn_kernel<DLB_DTYPE_F16, 256, PG_, true>), grid,             \
-                         dim3(kThreads), 0, s, p);                                               \
-    else if (D == 128) DLB_LAUNCH_PREFILL(DLB_DTYPE_F16, 128, PG_);                               \
-    else DLB_LAUNCH_PREFILL(DLB_DTYPE_F16, 64, PG_);                                              \
-  }
+#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                 \
+  do {                                                   \
+    if (small) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 2);   \
+    else DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4);         \
+  } while (0)
+#define DLB_DISPATCH_PREFILL_DT(DT_, PG_)                                                               \
+  do {                                                                                                  \
+    if (D == 256)                                                                                       \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, 256, PG_, true, 4>), grid, dim3(kThreads), 0, s, p); \
+    else if (D == 128) DLB_LAUNCH_PREFILL(DT_, 128, PG_);                                               \
+    else if (D == 96) DLB_LAUNCH_PREFILL(DT_, 96, PG_);                                                 \
+    else DLB_LAUNCH_PREFILL(DT_, 64, PG_);                                                              \
+  } while (0)
+#define DLB_DISPATCH_PREFILL(PG_)                                               \
+  if (dtype == DLB_DTYPE_BF16) DLB_DISPATCH_PREFILL_DT(DLB_DTYPE_BF16, PG_);    \
+  else DLB_DISPATCH_PREFILL_DT(DLB_DTYPE_F16, PG_)
   // pages that hold whole 64-key tiles take the kernel with one page look-up per tile (the lane
   // offsets inside a page are 32-bit)
   const bool tile_pages = paged && p.page % kTileN == 0 &&
                           (int64_t)p.page * p.k_st * 2 <= 0x7fffffff && (int64_t)p.page * p.v_st * 2 <= 0x7fffffff;
-  if (tile_pages) { DLB_DISPATCH_PREFILL(2) } else if (paged) { DLB_DISPATCH_PREFILL(1) } else { DLB_DISPATCH_PREFILL(0) }
+  if (tile_pages) {
+    DLB_DISPATCH_PREFILL(2);
+  } else if (paged) {
+    DLB_DISPATCH_PREFILL(1);
+  } else {
+    DLB_DISPATCH_PREFILL(0);
+  }
 #undef DLB_DISPATCH_PREFILL
+#undef DLB_DISPATCH_PREFILL_DT
 #undef DLB_LAUNCH_PREFILL
+#undef DLB_LAUNCH_PREFILL_RW
   return launch_status();
 }
 
@@ -615,7 +714,7 @@ extern "C" int dlb_prefill_attn_varlen(const void* q, const void* k, const void*
   p.page_shift = 0;
   p.window = -1;
   p.softcap = -1.0f;
-  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, sm_scale, dtype, stream);
+  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, max_len, sm_scale, dtype, stream);
 }
 
 extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const void* v_cache,
@@ -662,5 +761,5 @@ extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const 
   p.page_shift = (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1;
   p.window = window_size;
   p.softcap = logit_softcapping;
-  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, sm_scale, dtype, stream);
+  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, (int64_t)page * max_blocks, sm_scale, dtype, stream);
 }
