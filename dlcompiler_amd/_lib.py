@@ -48,6 +48,9 @@ SIGNATURES = {
                                 + [c_float, c_int, c_void_p]),
     "dlb_paged_prefill_attn": (c_int, [c_void_p] * 8 + [c_int] * 9 + [c_int64] * 11
                                + [c_float, c_int, c_float, c_int, c_void_p]),
+    "dlb_paged_prefill_attn_ws": (c_int, [c_void_p] * 8 + [c_int] * 9 + [c_int64] * 11
+                               + [c_float, c_int, c_float, c_int, c_int64, c_void_p, c_size_t, c_void_p]),
+    "dlb_paged_prefill_ws_bytes": (c_size_t, [c_int64] + [c_int] * 9),
     "dlb_per_token_group_quant_fp8": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                               c_int64, c_int64, c_int64, c_int, c_void_p]),
     "dlb_moe_gemm_fp8_gate_up": (c_int, [c_void_p] * 6 + [c_int] * 10 + [c_void_p] * 3),

@@ -34,7 +34,8 @@ namespace {
   X(dlb_moe_topk_softmax_align_ws_bytes) \
   X(dlb_moe_topk_softmax_align_f32) \
   X(dlb_prefill_attn_varlen)      \
-  X(dlb_paged_prefill_attn)       \
+  X(dlb_paged_prefill_ws_bytes)   \
+  X(dlb_paged_prefill_attn_ws)    \
   X(dlb_paged_decode_ws_bytes)    \
   X(dlb_paged_decode_attn)         \
   X(dlb_fused_moe_ws_bytes)       \
@@ -424,13 +425,17 @@ PyObject* paged_attention_fwd(PyObject*, PyObject* const* args, Py_ssize_t) {
     if (!index_table(bt, dev, 0, mask) || !index_array(start, dev, 1, mask) || !index_array(qlen, dev, 2, mask) ||
         !index_array(kvlen, dev, 3, mask) || !as_int(args[8], max_len) || max_len < 0 || max_len > 0x7fffffff)
       NOT_HANDLED;
+    const size_t ws_bytes = abi.dlb_paged_prefill_ws_bytes(q->size(0), (int)B, (int)Hq, Hkv, (int)D, (int)Dv, page,
+                                                           max_blocks, (int)max_len, (int)window);
+    at::Tensor ws;
+    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, dev);
     NoGil nogil;
-    st = abi.dlb_paged_prefill_attn(
+    st = abi.dlb_paged_prefill_attn_ws(
         q->data_ptr(), k->data_ptr(), v->data_ptr(), o->data_ptr(), bt->data_ptr(), start->data_ptr(),
         qlen->data_ptr(), kvlen->data_ptr(), mask, (int)B, (int)Hq, Hkv, (int)D, (int)Dv, page, max_blocks,
         (int)max_len, q->stride(0), q->stride(1), k->stride(0), k->stride(1), k->stride(2), v->stride(0),
         v->stride(1), v->stride(2), o->stride(0), o->stride(1), bt->stride(0), (float)scale, (int)window, (float)cap,
-        code, stream_of(dev));
+        code, q->size(0), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream_of(dev));
   } else {
     if (page % 16 != 0 || !index_table(bt, dev, 0, mask) || !index_array(kvlen, dev, 1, mask)) NOT_HANDLED;
     const size_t ws_bytes =

@@ -34,7 +34,16 @@ struct PrefillParams {
   IdxArray seq_len;
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;  // token / head strides (elements)
   int Hq, Hkv, group;
-  int xcd_heads;  // != 0: remap blockIdx.x so the heads of a KV group share an XCD
+  int xcd_heads;  // heads (head groups) per XCD, != 0: remap blockIdx.x so a KV group's share an XCD
+  // PACK kernels: a workgroup's rows are those of 1 << pack_shift query heads of a KV group, the rows of
+  // each being (kBlockM >> pack_shift) queries
+  int pack_shift;
+  // nsplit > 1: a workgroup takes one of nsplit equal runs of its key tiles and leaves unnormalised
+  // rows in ws_o [nsplit][tokens][Hq][ws_d] and (maximum, denominator) in ws_ml [nsplit][tokens][Hq][2]
+  int nsplit, ws_d;
+  int64_t tokens;
+  float* ws_o;
+  float* ws_ml;
   float scale_log2e;
   // paged K/V (PAGED kernels): k/v point at caches [pages, page, Hkv, D]; *_st is the slot
   // stride, *_sp the page stride; sequence s reads pages block_table[s][.] and its queries sit
@@ -106,7 +115,10 @@ struct Smem {
 // launch with fewer 128-row workgroups than CUs is as fast as one workgroup's chain of tiles: this
 // shape gives it twice the workgroups and half the chain (one sequence of 512 tokens, 32 heads of
 // 128: 13.6 -> 11.2 us, of 1125 tokens, 8 heads: 21.7 -> 16.0; eight waves on 128 rows: 13.6 and 19.5).
-template <int DT, int D, int PAGED, bool RAGGED, int RW>
+// PACK: short query runs over a history (every run fits a fraction of the rows): the heads of a KV
+// group share a workgroup, so the rows are filled and K/V is staged once for all of them; and the
+// key tiles may be split over workgroups.
+template <int DT, int D, int PAGED, bool RAGGED, int RW, bool PACK>
 __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefill_attn_kernel(const PrefillParams p) {
   constexpr int KG = 4 / RW;
   constexpr int kBlockM = 32 * RW;  // query rows per workgroup
@@ -148,16 +160,20 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   }
   // (vector loads of wave-uniform values: saying that they are keeps loops and conditions scalar)
   const int L = __builtin_amdgcn_readfirstlane(p.seq_len[seq]);
-  const int qtile = gridDim.y - 1 - blockIdx.y;  // heaviest first
-  const int q0 = qtile * kBlockM;
+  const int pack = PACK ? p.pack_shift : 0;
+  const int kBlockQ = kBlockM >> pack;  // queries of a workgroup
+  const int qy = PACK ? blockIdx.y / p.nsplit : blockIdx.y, split = PACK ? blockIdx.y - qy * p.nsplit : 0;
+  const int qtile = (PACK ? gridDim.y / p.nsplit : gridDim.y) - 1 - qy;  // heaviest first
+  const int q0 = qtile * kBlockQ;
   if (q0 >= L) return;
   const int64_t tok0 = __builtin_amdgcn_readfirstlane(p.start_loc[seq]);
   // context seen by this sequence: kv_total keys, the queries are its last L positions
   const int kv_total = PAGED ? __builtin_amdgcn_readfirstlane(p.kv_len[seq]) : L;
   const int hist = kv_total - L;
   if (PAGED && hist < 0) return;  // inconsistent lengths: nothing sensible to compute
-  int head = blockIdx.x;
-  if (p.xcd_heads) head = (blockIdx.x & 7) * (p.Hq >> 3) + (blockIdx.x >> 3);
+  int head = blockIdx.x;  // PACK: first of the workgroup's heads
+  if (p.xcd_heads) head = (blockIdx.x & 7) * p.xcd_heads + (blockIdx.x >> 3);
+  if (PACK) head <<= pack;
   const int kvh = head / p.group;
 
   const int tid = threadIdx.x;
@@ -173,7 +189,9 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   const unsigned short* vb = (const unsigned short*)p.v + (int64_t)kvh * p.v_sh;
 
   // ---- Q^T as B operand: lane (n = query, k = dims 16*ks + 8*hh .. +8), kept in registers
-  const int qrow = q0 + 32 * wave + col;
+  const int brow = 32 * wave + col;  // row of the workgroup
+  const int qrow = q0 + (PACK ? brow & (kBlockQ - 1) : brow);
+  if (PACK) head += brow / kBlockQ;  // (by lane from here on)
   u32x4 qf[KS];
   {
     const unsigned short* qp =
@@ -185,21 +203,30 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
     }
   }
 
-  const int kv_end = min(kv_total, hist + q0 + kBlockM);  // keys this workgroup needs
-  const int ntiles = (kv_end + kTileN - 1) / kTileN;
+  const int kv_end = min(kv_total, hist + q0 + kBlockQ);  // keys this workgroup needs
+  int ntiles = (kv_end + kTileN - 1) / kTileN;
   // window / soft-cap requests take the masked path for every tile
   // (only the paged entry point exposes them; the packed kernel compiles them out)
   const int window = PAGED ? p.window : -1;
   const float softcap = PAGED ? p.softcap : -1.0f;
   // tiles below this index lie entirely under the diagonal for every wave of the workgroup
   // (all 64 keys <= position of row q0): no mask, no clamping of key rows
-  const int nfull = softcap > 0.0f ? 0 : (hist + q0 + 1) / kTileN;
+  int nfull = softcap > 0.0f ? 0 : (hist + q0 + 1) / kTileN;
   // first tile that can hold a visible key (sliding window), and the first whose keys every query
   // of the workgroup sees
-  const int jfirst = window > 0 ? max(hist + q0 - window, 0) / kTileN : 0;
-  const int jopen = window > 0 ? max(hist + q0 + kBlockM - 1 - window + kTileN - 1, 0) / kTileN : 0;
+  int jfirst = window > 0 ? max(hist + q0 - window, 0) / kTileN : 0;
+  const int jopen = window > 0 ? max(hist + q0 + kBlockQ - 1 - window + kTileN - 1, 0) / kTileN : 0;
   const int qpos = hist + qrow;                          // context position of this lane's query
-  const int wave_last_pos = hist + q0 + 32 * wave + 31;
+  // context positions of the wave's first and last query
+  const int wave_q0 = PACK ? (32 * wave) & (kBlockQ - 1) : 32 * wave;
+  const int wave_first_pos = hist + q0 + wave_q0;
+  const int wave_last_pos = wave_first_pos + (PACK ? min(32, kBlockQ) : 32) - 1;
+  if (PACK && p.nsplit > 1) {  // this workgroup's run of the tiles
+    const int per = (ntiles - jfirst + p.nsplit - 1) / p.nsplit;
+    jfirst += split * per;
+    ntiles = min(ntiles, jfirst + per);
+    nfull = min(nfull, ntiles);
+  }
 
   // ---- global -> LDS staging of one K/V tile.  Per-thread base pointers are formed once; a
   // tile adds a workgroup-uniform offset.  CLAMP (tiles that may run past the sequence)
@@ -358,7 +385,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
     static_assert(kCopies * KS == 2 * KINS, "whole copies per k-step");
     const int t0 = j * kTileN;
     if (MASK && t0 > wave_last_pos) return;  // wave-uniform: tile entirely above the diagonal
-    if (MASK && window > 0 && t0 + kTileN - 1 < wave_last_pos - 31 - window) return;  // below the window
+    if (MASK && window > 0 && t0 + kTileN - 1 < wave_first_pos - window) return;  // below the window
     const unsigned char* ks = smem + buf * SM::stage;
     const unsigned char* vs = ks + SM::kBytes;
 
@@ -489,7 +516,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   using No = std::integral_constant<bool, false>;
   // Group grp takes tiles jfirst + grp, + KG, ...; both groups make the same number of steps, one barrier
   // each.  A wave whose rows all lie past the sequence only copies.
-  const bool wave_rows = q0 + 32 * __builtin_amdgcn_readfirstlane(wave) < L;
+  const bool wave_rows = q0 + __builtin_amdgcn_readfirstlane(wave_q0) < L;
   int jb = jfirst;  // the step's first tile
   // (the step's LDS buffer, worked out where it is used: carried along as a variable it costs the paged
   // kernels 50 registers)
@@ -515,7 +542,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
     stage_tile(j + KG, buf() ^ 1);
     // a diagonal tile still lies entirely under the diagonal for the waves further down (and a tile at
     // the window's edge entirely inside it for some)
-    const bool wave_full = softcap <= 0.0f && (j + 1) * kTileN - 1 <= hist + q0 + 32 * wave &&
+    const bool wave_full = softcap <= 0.0f && (j + 1) * kTileN - 1 <= wave_first_pos &&
                            (window <= 0 || j * kTileN >= wave_last_pos - window);
     if (j < ntiles) {
       if (wave_full) process_tile(No{}, No{}, j, buf());
@@ -574,6 +601,24 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
 
   // ---- epilogue: normalise and store O (lane holds 4 consecutive dims per register quad)
   l_run += __shfl_xor(l_run, 32);
+  if (PACK && p.nsplit > 1) {
+    if (qrow < L) {
+      const int64_t row = ((int64_t)split * p.tokens + tok0 + qrow) * p.Hq + head;
+      float* wo = p.ws_o + row * p.ws_d;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd)
+          if (!RAGGED || 32 * mt + 8 * qd + 4 * hh < p.dv)
+            *(f32x4*)(wo + 32 * mt + 8 * qd + 4 * hh) =
+                f32x4{o[mt][4 * qd], o[mt][4 * qd + 1], o[mt][4 * qd + 2], o[mt][4 * qd + 3]};
+      if (hh == 0) {
+        p.ws_ml[2 * row] = m_run;
+        p.ws_ml[2 * row + 1] = l_run;
+      }
+    }
+    return;
+  }
   if (qrow < L) {
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     unsigned short* op = (unsigned short*)p.o + (tok0 + qrow) * p.o_st + (int64_t)head * p.o_sh;
@@ -590,16 +635,80 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   }
 }
 
+// Merge of the nsplit partial rows of every (query, head) of a sequence (blockIdx.y): one wave per row,
+// four rows per workgroup.  Rows without a visible key in any part become 0.
+template <int DT>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillParams p) {
+  const int seq = blockIdx.y;
+  const int idx = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int qrow = idx / p.Hq, head = idx - qrow * p.Hq;
+  const int lane = threadIdx.x & 63;
+  const int L = p.seq_len[seq];
+  if (qrow >= L || p.kv_len[seq] < L) return;
+  const int64_t rows = p.tokens * p.Hq, tok = p.start_loc[seq] + qrow, row = tok * p.Hq + head;
+  float m = -__builtin_inff();
+  for (int s = 0; s < p.nsplit; ++s) m = fmaxf(m, p.ws_ml[2 * (s * rows + row)]);
+  float den = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < p.nsplit; ++s) {
+    const float ms = p.ws_ml[2 * (s * rows + row)];
+    const float w = ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(ms - m);
+    den += w * p.ws_ml[2 * (s * rows + row) + 1];
+    if (4 * lane < p.dv && w > 0.0f) {
+      const f32x4 v = *(const f32x4*)(p.ws_o + (s * rows + row) * p.ws_d + 4 * lane);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += w * v[i];
+    }
+  }
+  const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+  if (4 * lane < p.dv)
+    *(u32x2*)((unsigned short*)p.o + tok * p.o_st + head * p.o_sh + 4 * lane) =
+        u32x2{Mma32<DT>::pack2(acc[0] * inv, acc[1] * inv), Mma32<DT>::pack2(acc[2] * inv, acc[3] * inv)};
+}
+
 }  // namespace
 }  // namespace dlb
 
 namespace dlb {
 namespace {
 
+// How a paged launch is cut.
+// Query runs that fill a fraction of 128 rows share a workgroup by heads of their KV group.  Where that
+// leaves few workgroups (up to 128, of 512 slots at two per CU) their key tiles are split, from 32
+// tiles on, eight tiles per part at least; with more workgroups or fewer tiles the partial rows cost
+// more than the split saves (256 workgroups, 34 tiles: 43 us, split in two 49; 129 tiles: 156
+// against 110).  Where nothing is split, heads share a workgroup only while every CU still has one.
+// 32 heads (8 kv) of 128: 32 queries over 16000 keys 240 -> 38.6 us, 2 x 100 over 10000 156 -> 42.7,
+// 16 x 8 - 32 over up to 8000 174 -> 94.
+struct PackPlan {
+  int pack_shift, nsplit;
+  bool use;
+};
+PackPlan pack_plan(int B, int Hq, int Hkv, int D, int max_len, int64_t max_keys, int window) {
+  PackPlan plan = {0, 1, false};
+  if (D > 128) return plan;
+  const int group = Hq / Hkv;
+  const int64_t seen = window > 0 && window + max_len < max_keys ? window + max_len : max_keys;
+  const int64_t tiles = ceil_div(seen, kTileN);
+  auto workgroups = [&](int shift) { return (int64_t)(Hq >> shift) * ceil_div(max_len, 128 >> shift) * B; };
+  while (group % (2 << plan.pack_shift) == 0 && (int64_t)max_len << (plan.pack_shift + 1) <= 128 &&
+         (tiles >= 32 || workgroups(plan.pack_shift + 1) >= 256))
+    ++plan.pack_shift;
+  const int64_t wgs = workgroups(plan.pack_shift);
+  if (wgs <= 128 ? tiles >= 32 : wgs <= 256 && tiles >= 96) {
+    const int64_t most = tiles / 8;
+    plan.nsplit = (int)(512 / wgs < most ? 512 / wgs : most);
+  }
+  plan.use = plan.pack_shift > 0 || plan.nsplit > 1;
+  return plan;
+}
+size_t split_ws_bytes(int64_t tokens, int Hq, int Dv, int nsplit) {
+  return nsplit > 1 ? (size_t)tokens * Hq * nsplit * ((Dv + 3) / 4 * 4 + 2) * sizeof(float) : 0;
+}
+
 // Shared argument checks and launch of both entry points; the paged fields of `p` are already
 // filled in (or zeroed) by the caller.
 int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk, int Dv, int max_len,
-                   int64_t max_keys, float sm_scale, int dtype, void* stream) {
+                   int64_t max_keys, float sm_scale, int dtype, void* ws, size_t ws_bytes, void* stream) {
   if (Dk % 8 != 0 || Dv % 8 != 0 || Dk > 256 || Dv > 256) return DLB_ERR_UNSUPPORTED;
   // head size the kernel instance is built for; past 128 there is one instance, for 256, that
   // takes every size on its ragged path (one workgroup per CU, one wave per SIMD: the 128 output
@@ -623,36 +732,51 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.Hq = Hq;
   p.Hkv = Hkv;
   p.group = Hq / Hkv;
-  // workgroups are dealt round-robin to the 8 XCDs by linear id; with Hq % 8 == 0 the
-  // remap in the kernel puts heads {x, x+8, ...} -> consecutive heads on one XCD so a KV
-  // group's four query heads hit the same L2.
-  p.xcd_heads = (Hq % 8 == 0 && Hq >= 16) ? 1 : 0;
   p.scale_log2e = sm_scale * 1.4426950408889634f;
   p.sm_scale = sm_scale;
 
   hipStream_t s = (hipStream_t)stream;
   // 64-row workgroups where 128-row ones would leave CUs without any (of 256), unless there are so few
   // keys that the merge costs more than it saves (40 heads, 4 x 49 tokens: 5.4 against 6.9 us)
-  const bool small = D <= 128 && Hq * ceil_div(max_len, 128) * B <= 240 && max_keys > 128;
-  const uint32_t qtiles = (uint32_t)ceil_div(max_len, small ? 64 : 128);
-  if (qtiles > 65535) return DLB_ERR_UNSUPPORTED;
-  const dim3 grid = dim3((uint32_t)Hq, qtiles, (uint32_t)B);
-#define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_)                                                               \
+  PackPlan plan = {0, 1, false};
+  if (paged) plan = pack_plan(B, Hq, Hkv, D, max_len, max_keys, p.window);
+  if (plan.nsplit > 1) {
+    const size_t need = split_ws_bytes(p.tokens, Hq, Dv, plan.nsplit);
+    if (!ws) plan.nsplit = 1;  // (a caller without scratch)
+    else if (ws_bytes < need || !aligned16(ws)) return DLB_ERR_WORKSPACE;
+    plan.use = plan.pack_shift > 0 || plan.nsplit > 1;
+  }
+  p.pack_shift = plan.pack_shift;
+  p.nsplit = plan.nsplit;
+  p.ws_d = (Dv + 3) / 4 * 4;
+  p.ws_o = (float*)ws;
+  p.ws_ml = p.ws_o ? p.ws_o + (size_t)p.tokens * Hq * p.nsplit * p.ws_d : nullptr;
+  const bool small = !plan.use && D <= 128 && Hq * ceil_div(max_len, 128) * B <= 240 && max_keys > 128;
+  const int64_t qtiles = ceil_div(max_len, small ? 64 : 128 >> p.pack_shift);
+  if (qtiles * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
+  const int head_groups = Hq >> p.pack_shift;
+  // workgroups are dealt round-robin to the 8 XCDs by linear id; with Hq % 8 == 0 the
+  // remap in the kernel puts heads {x, x+8, ...} -> consecutive heads on one XCD so a KV
+  // group's four query heads hit the same L2.
+  p.xcd_heads = head_groups % 8 == 0 && head_groups >= 16 ? head_groups >> 3 : 0;
+  const dim3 grid = dim3((uint32_t)head_groups, (uint32_t)(qtiles * p.nsplit), (uint32_t)B);
+#define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_, PK_)                                                          \
   do {                                                                                                         \
     if (ragged)                                                                                                \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, true, RW_>), grid, dim3(kThreads), 0, s, p);        \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, true, RW_, PK_>), grid, dim3(kThreads), 0, s, p);   \
     else                                                                                                       \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, false, RW_>), grid, dim3(kThreads), 0, s, p);       \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, false, RW_, PK_>), grid, dim3(kThreads), 0, s, p);  \
   } while (0)
-#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                 \
-  do {                                                   \
-    if (small) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 2);   \
-    else DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4);         \
+#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                                          \
+  do {                                                                            \
+    if (PG_ != 0 && plan.use) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, (PG_ != 0)); \
+    else if (small) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 2, false);                \
+    else DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, false);                           \
   } while (0)
 #define DLB_DISPATCH_PREFILL_DT(DT_, PG_)                                                               \
   do {                                                                                                  \
     if (D == 256)                                                                                       \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, 256, PG_, true, 4>), grid, dim3(kThreads), 0, s, p); \
+      hipLaunchKernelGGL((prefill_attn_kernel<DT_, 256, PG_, true, 4, false>), grid, dim3(kThreads), 0, s, p); \
     else if (D == 128) DLB_LAUNCH_PREFILL(DT_, 128, PG_);                                               \
     else if (D == 96) DLB_LAUNCH_PREFILL(DT_, 96, PG_);                                                 \
     else DLB_LAUNCH_PREFILL(DT_, 64, PG_);                                                              \
@@ -675,6 +799,13 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
 #undef DLB_DISPATCH_PREFILL_DT
 #undef DLB_LAUNCH_PREFILL
 #undef DLB_LAUNCH_PREFILL_RW
+  if (p.nsplit > 1) {
+    const dim3 rows((uint32_t)ceil_div((int64_t)max_len * Hq, 4), (uint32_t)B);
+    if (dtype == DLB_DTYPE_BF16)
+      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_BF16>, rows, dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_F16>, rows, dim3(256), 0, s, p);
+  }
   return launch_status();
 }
 
@@ -714,21 +845,46 @@ extern "C" int dlb_prefill_attn_varlen(const void* q, const void* k, const void*
   p.page_shift = 0;
   p.window = -1;
   p.softcap = -1.0f;
-  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, max_len, sm_scale, dtype, stream);
+  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, max_len, sm_scale, dtype, nullptr, 0, stream);
 }
 
-extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const void* v_cache,
-                                      void* o, const void* block_table,
-                                      const void* q_start_loc, const void* q_len,
-                                      const void* kv_len, int index64_mask, int B, int Hq, int Hkv, int D,
-                                      int Dv, int page, int max_blocks, int max_q_len,
-                                      int64_t q_stride_tok, int64_t q_stride_head,
-                                      int64_t k_stride_page, int64_t k_stride_tok,
-                                      int64_t k_stride_head, int64_t v_stride_page,
-                                      int64_t v_stride_tok, int64_t v_stride_head,
-                                      int64_t o_stride_tok, int64_t o_stride_head,
-                                      int64_t bt_stride, float sm_scale, int window_size,
-                                      float logit_softcapping, int dtype, void* stream) {
+extern "C" size_t dlb_paged_prefill_ws_bytes(int64_t tokens, int B, int Hq, int Hkv, int D, int Dv, int page,
+                                             int max_blocks, int max_q_len, int window_size) {
+  using namespace dlb;
+  if (tokens < 1 || B < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || page < 1 || max_blocks < 1 || max_q_len < 1 ||
+      D < 1 || Dv < 1)
+    return 0;
+  const PackPlan plan =
+      pack_plan(B, Hq, Hkv, D > Dv ? D : Dv, max_q_len, (int64_t)page * max_blocks, window_size);
+  return split_ws_bytes(tokens, Hq, Dv, plan.nsplit);
+}
+
+extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const void* v_cache, void* o,
+                                      const void* block_table, const void* q_start_loc, const void* q_len,
+                                      const void* kv_len, int index64_mask, int B, int Hq, int Hkv, int D, int Dv,
+                                      int page, int max_blocks, int max_q_len, int64_t q_stride_tok,
+                                      int64_t q_stride_head, int64_t k_stride_page, int64_t k_stride_tok,
+                                      int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_tok,
+                                      int64_t v_stride_head, int64_t o_stride_tok, int64_t o_stride_head,
+                                      int64_t bt_stride, float sm_scale, int window_size, float logit_softcapping,
+                                      int dtype, void* stream) {
+  return dlb_paged_prefill_attn_ws(q, k_cache, v_cache, o, block_table, q_start_loc, q_len, kv_len, index64_mask, B,
+                                   Hq, Hkv, D, Dv, page, max_blocks, max_q_len, q_stride_tok, q_stride_head,
+                                   k_stride_page, k_stride_tok, k_stride_head, v_stride_page, v_stride_tok,
+                                   v_stride_head, o_stride_tok, o_stride_head, bt_stride, sm_scale, window_size,
+                                   logit_softcapping, dtype, 0, nullptr, 0, stream);
+}
+
+extern "C" int dlb_paged_prefill_attn_ws(const void* q, const void* k_cache, const void* v_cache, void* o,
+                                         const void* block_table, const void* q_start_loc, const void* q_len,
+                                         const void* kv_len, int index64_mask, int B, int Hq, int Hkv, int D, int Dv,
+                                         int page, int max_blocks, int max_q_len, int64_t q_stride_tok,
+                                         int64_t q_stride_head, int64_t k_stride_page, int64_t k_stride_tok,
+                                         int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_tok,
+                                         int64_t v_stride_head, int64_t o_stride_tok, int64_t o_stride_head,
+                                         int64_t bt_stride, float sm_scale, int window_size,
+                                         float logit_softcapping, int dtype, int64_t tokens, void* ws,
+                                         size_t ws_bytes, void* stream) {
   using namespace dlb;
   if (B < 0 || Hq < 1 || Hkv < 1 || D < 1 || Dv < 1 || max_q_len < 0 || page < 1 || max_blocks < 0)
     return DLB_ERR_BAD_ARG;
@@ -747,6 +903,7 @@ extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const 
   p.seq_len = idx_array(q_len, index64_mask, 2);
   p.kv_len = idx_array(kv_len, index64_mask, 3);
   p.bt_stride = bt_stride;
+  p.tokens = tokens;
   p.q_st = q_stride_tok;
   p.q_sh = q_stride_head;
   p.k_sp = k_stride_page;
@@ -761,5 +918,6 @@ extern "C" int dlb_paged_prefill_attn(const void* q, const void* k_cache, const 
   p.page_shift = (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1;
   p.window = window_size;
   p.softcap = logit_softcapping;
-  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, (int64_t)page * max_blocks, sm_scale, dtype, stream);
+  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, (int64_t)page * max_blocks, sm_scale, dtype, ws,
+                        ws_bytes, stream);
 }

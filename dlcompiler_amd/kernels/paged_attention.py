@@ -68,16 +68,19 @@ def paged_attention_fwd(
         assert q.dim() == 3 and o.dim() == 3
         (block_offsets, q_start_loc, q_seqlens, kv_seqlens), mask = _lib.index_arrays(
             block_offsets, q_start_loc.contiguous(), q_seqlens.contiguous(), kv_seqlens.contiguous())
+        ws_bytes = lib.dlb_paged_prefill_ws_bytes(q.size(0), batch, head, num_kv_heads, Lq, Lv, page, max_blocks,
+                                                  int(max_seqlen), int(window_size))
+        ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=q.device)
         with _lib.device_guard(q.device):
-            st = lib.dlb_paged_prefill_attn(
+            st = lib.dlb_paged_prefill_attn_ws(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), block_offsets.data_ptr(),
                 q_start_loc.data_ptr(), q_seqlens.data_ptr(), kv_seqlens.data_ptr(), mask, batch, head,
                 num_kv_heads, Lq, Lv, page, max_blocks, int(max_seqlen), q.stride(0), q.stride(1),
                 k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
                 o.stride(0), o.stride(1), block_offsets.stride(0), float(sm_scale),
                 int(window_size), float(logit_softcapping), _lib.torch_dtype_code(q.dtype),
-                _lib.current_stream_ptr(q.device))
-        _lib.check(st, "dlb_paged_prefill_attn")
+                q.size(0), ws.data_ptr(), ws_bytes, _lib.current_stream_ptr(q.device))
+        _lib.check(st, "dlb_paged_prefill_attn_ws")
         return
 
     if page % 16 != 0:

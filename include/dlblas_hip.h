@@ -245,6 +245,23 @@ int dlb_paged_prefill_attn(const void* q, const void* k_cache, const void* v_cac
                            int64_t bt_stride, float sm_scale, int window_size,
                            float logit_softcapping, int dtype, void* stream);
 
+/* The same with scratch, which lets a launch of few, long workgroups split their keys: tokens = rows of q
+ * and o; ws (16-byte aligned) holds dlb_paged_prefill_ws_bytes bytes (0: nothing is needed, ws may
+ * be NULL). */
+size_t dlb_paged_prefill_ws_bytes(int64_t tokens, int B, int Hq, int Hkv, int D, int Dv, int page,
+                                  int max_blocks, int max_q_len, int window_size);
+int dlb_paged_prefill_attn_ws(const void* q, const void* k_cache, const void* v_cache, void* o,
+                              const void* block_table, const void* q_start_loc, const void* q_len,
+                              const void* kv_len, int index64_mask, int B, int Hq, int Hkv,
+                              int D, int Dv, int page, int max_blocks, int max_q_len,
+                              int64_t q_stride_tok,
+                              int64_t q_stride_head, int64_t k_stride_page, int64_t k_stride_tok,
+                              int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_tok,
+                              int64_t v_stride_head, int64_t o_stride_tok, int64_t o_stride_head,
+                              int64_t bt_stride, float sm_scale, int window_size,
+                              float logit_softcapping, int dtype, int64_t tokens, void* ws,
+                              size_t ws_bytes, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * fp8 fused-MoE building blocks (OCP e4m3fn, fp32 scales per 128 along K; weights carry one
  * scale per 128 x 128 block).  Pipeline shape follows fused_moe, kernels/fused_moe.py:296-376

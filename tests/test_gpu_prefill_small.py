@@ -24,7 +24,8 @@ def test_packed(dev, lens, Hq, Hkv, D, dtype):
     torch.testing.assert_close(o.cpu().float(), ref.float(), rtol=2e-2, atol=2e-2)
 
 
-@pytest.mark.parametrize("new,history", [([16, 3], [300, 0]), ([1, 130, 64], [900, 63, 2000]), ([300], [1500]), ([40] * 9, [500] * 9)])
+@pytest.mark.parametrize("new,history", [([16, 3], [300, 0]), ([1, 130, 64], [900, 63, 2000]), ([300], [1500]), ([40] * 9, [500] * 9),
+                                         ([100], [3000]), ([33, 7], [2500, 10]), ([1, 2], [1300, 0])])
 @pytest.mark.parametrize("page", [16, 64])
 @pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 96), (8, 1, 128), (4, 4, 64)])
 @pytest.mark.parametrize("window,cap", [(None, None), (200, None), (64, 15.0), (None, 15.0)])
