@@ -98,11 +98,20 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
   const bool segs = p.seg_start.p != nullptr;
   int cnt[4], nb[4], tl[4], st[4];
   int nb_sum = 0, tl_sum = 0;
+  // (clamped instead of masked: behind a branch each load would be waited for before the next one)
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    cnt[c] = p.counts[min(4 * lane + c, p.num_experts - 1)];
+    st[c] = 0;
+  }
+  if (segs) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) st[c] = p.seg_start[min(4 * lane + c, p.num_experts - 1)];
+  }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int e = 4 * lane + c;
-    st[c] = (segs && e < p.num_experts) ? p.seg_start[e] : 0;
-    cnt[c] = e < p.num_experts ? max(p.counts[e] - st[c], 0) : 0;
+    cnt[c] = e < p.num_experts ? max(cnt[c] - st[c], 0) : 0;
     nb[c] = (cnt[c] + bm - 1) >> p.bm_shift;
     const bool local = e >= p.expert_offset && e < p.expert_offset + p.num_local;
     tl[c] = local ? (cnt[c] + kMaxRows - 1) / kMaxRows * p.num_ntiles : 0;
@@ -271,31 +280,17 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   // fetches.  Down: thread t < 128 keeps slot and routing weight of row t for the epilogue.
   int sid_x[4] = {0, 0, 0, 0};
   int sid_s = 0;
-  // (positions past the tile's real rows hold the pad sentinel in a block-aligned list and another
-  // expert's slots in the launcher form: they are not read)
-  auto slot_at = [&](int r) -> int { return r < tile.rows ? p.sorted_ids[row0 + r] : p.numel; };
+  // (positions past the tile's real rows hold the pad sentinel or another tile's slots: the last real
+  // row is read instead, unconditionally -- behind a branch each load would be waited for)
+  auto slot_at = [&](int r) -> int { return p.sorted_ids[row0 + min(r, tile.rows - 1)]; };
   const bool gather = GATED || p.gather_a;
   if (gather && stager) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) sid_x[i] = slot_at(32 * wave + 8 * i + drow);
     if (QT == 0) sid_s = slot_at(32 * wave + j);
   }
-  if (!GATED) {
-    if (tid < 128) {
-      // destination row of the tile's row `tid` (-1: none) and its routing weight
-      int dst = -1;
-      float rwt = 0.0f;
-      if (tid < tile.rows) {
-        const int sid = p.sorted_ids[row0 + tid];
-        if (sid >= 0 && sid < p.numel) {
-          dst = p.scatter_c ? sid : row0 + tid;
-          rwt = slot_weight(p, sid);
-        }
-      }
-      sid_lds[tid] = dst;  // published by the barrier that opens the main loop
-      rw_lds[tid] = rwt;
-    }
-  }
+  int sid_out = -1;  // down: slot of the tile's row `tid`
+  if (!GATED) sid_out = slot_at(tid & 127);
   // source row of the tile's row r whose routing slot is sid (gated: the slot's token; pad
   // slots read a valid row)
   auto src_row_of = [&](int sid, int r) -> uint32_t {
@@ -416,6 +411,15 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   issue_w(H0{}, 1, wr[1][0]);
   issue_x(1, 1);
   issue_w(H1{}, 1, wr[1][1]);
+  if (!GATED) {
+    // destination row of the tile's row `tid` (-1: none) and its routing weight, published by the
+    // barrier that opens the main loop; here, behind the loads that the first chunks wait for
+    if (tid < 128) {
+      const bool real = tid < tile.rows && sid_out >= 0 && sid_out < p.numel;
+      sid_lds[tid] = !real ? -1 : p.scatter_c ? sid_out : row0 + tid;
+      rw_lds[tid] = real ? slot_weight(p, sid_out) : 0.0f;
+    }
+  }
   wait_vm<12 + D>();  // X(0) landed
   __syncthreads();
 

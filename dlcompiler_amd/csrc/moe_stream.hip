@@ -34,11 +34,20 @@ __device__ __forceinline__ bool find_stream_tile(const MoeGemmParams& p, int nti
   const bool segs = p.seg_start.p != nullptr;
   int cnt[4], nb[4], tl[4], st[4];
   int nb_sum = 0, tl_sum = 0;
+  // (clamped instead of masked: behind a branch each load would be waited for before the next one)
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    cnt[c] = p.counts[min(4 * lane + c, p.num_experts - 1)];
+    st[c] = 0;
+  }
+  if (segs) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) st[c] = p.seg_start[min(4 * lane + c, p.num_experts - 1)];
+  }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int e = 4 * lane + c;
-    st[c] = (segs && e < p.num_experts) ? p.seg_start[e] : 0;
-    cnt[c] = e < p.num_experts ? max(p.counts[e] - st[c], 0) : 0;
+    cnt[c] = e < p.num_experts ? max(cnt[c] - st[c], 0) : 0;
     nb[c] = (cnt[c] + (1 << p.bm_shift) - 1) >> p.bm_shift;
     const bool local = e >= p.expert_offset && e < p.expert_offset + p.num_local;
     tl[c] = local ? (cnt[c] + ROWS - 1) / ROWS * ntiles : 0;
