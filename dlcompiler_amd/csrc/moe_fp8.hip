@@ -15,8 +15,8 @@
 // counterpart there; its nearest precedent is the int8 per-token quantisation and
 // scale-in-epilogue GEMM of python/dlBLAS/dlblas/kernels/w8a8.py:102-106,275-335.
 //
-// The same kernel also runs unquantised bf16/f16 operands (QT = 1): the reference's own
-// fused_moe, with 32x32x16 MFMAs and no scales.
+// Unquantised bf16/f16 operands (the reference's own fused_moe) and fp8 with few rows per expert
+// run the kernel of moe_stream.hip.
 //
 // GEMM mapping.  The MFMA runs "transposed": weight rows are the A operand (M index = output
 // column n), activations the B operand (N index = token row), so a lane's sixteen accumulator
@@ -95,23 +95,15 @@ __device__ __forceinline__ void wait_vm() {
 __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, TileId& t) {
   const int bm = 1 << p.bm_shift;
   constexpr int kMaxRows = 128;
-  const bool segs = p.seg_start.p != nullptr;
-  int cnt[4], nb[4], tl[4], st[4];
+  int cnt[4], nb[4], tl[4];
   int nb_sum = 0, tl_sum = 0;
   // (clamped instead of masked: behind a branch each load would be waited for before the next one)
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    cnt[c] = p.counts[min(4 * lane + c, p.num_experts - 1)];
-    st[c] = 0;
-  }
-  if (segs) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) st[c] = p.seg_start[min(4 * lane + c, p.num_experts - 1)];
-  }
+  for (int c = 0; c < 4; ++c) cnt[c] = p.counts[min(4 * lane + c, p.num_experts - 1)];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int e = 4 * lane + c;
-    cnt[c] = e < p.num_experts ? max(cnt[c] - st[c], 0) : 0;
+    cnt[c] = e < p.num_experts ? max(cnt[c], 0) : 0;
     nb[c] = (cnt[c] + bm - 1) >> p.bm_shift;
     const bool local = e >= p.expert_offset && e < p.expert_offset + p.num_local;
     tl[c] = local ? (cnt[c] + kMaxRows - 1) / kMaxRows * p.num_ntiles : 0;
@@ -129,20 +121,18 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
   const int L = __builtin_ctzll(hit);  // the lane whose four experts hold the tile
   int rem = logical - __builtin_amdgcn_readlane(tl_incl - tl_sum, L);
   int mbase = __builtin_amdgcn_readlane(nb_incl - nb_sum, L);
-  int e = 4 * L, ce = 0, se = 0;
+  int e = 4 * L, ce = 0;
   bool found = false;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int tc = __builtin_amdgcn_readlane(tl[c], L);
     const int nc = __builtin_amdgcn_readlane(nb[c], L);
     const int cc = __builtin_amdgcn_readlane(cnt[c], L);
-    const int sc = __builtin_amdgcn_readlane(st[c], L);
     if (!found) {
       if (rem < tc) {
         found = true;
         e = 4 * L + c;
         ce = cc;
-        se = sc;
       } else {
         rem -= tc;
         mbase += nc;
@@ -155,14 +145,13 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
   const int groups = (ce + 31) >> 5, base = groups / nbe, extra = groups - base * nbe;  // 32-row groups
   const int r0 = 32 * (rb * base + min(rb, extra));
   t.e = e - p.expert_offset;
-  t.row0 = (segs ? se : mbase << p.bm_shift) + r0;  // block-aligned list / launcher form: its own segment
+  t.row0 = (mbase << p.bm_shift) + r0;
   t.nt = nt;
   t.rows = min(32 * (base + (rb < extra ? 1 : 0)), ce - r0);
   // (counts that do not fit the slot list: touch nothing)
-  return t.row0 + t.rows <= (segs ? p.numel : p.num_mblocks << p.bm_shift);
+  return t.row0 + t.rows <= p.num_mblocks << p.bm_shift;
 }
 
-// QT = 0: fp8 operands with block scales; QT = 1: 16-bit operands of type DT, no scales.
 // GATED = true : gate_up GEMM (N = 2I), tile = 128 gate cols + the matching 128 up cols,
 //                epilogue silu(gate) * up -> fp8 + per-128 scale, rows kept in sorted order.
 // GATED = false: down GEMM, tile = 256 cols, epilogue * routing weight -> out[slot, n].
@@ -171,10 +160,10 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
 // Tile = up to 128 routing slots of one expert (two to four 32-row tiles) x 256 output columns,
 // four waves, two workgroups per CU.  A wave owns 64 output columns (two 32-column tiles; gated:
 // 32 gate + the matching 32 up columns) x all the rows: 4 x 2 accumulator tiles of the 32x32x64
-// (fp8) / 32x32x16 (16 bit) MFMA.  Lane (j = lane % 32, h = lane / 32) supplies, for weight
+// MFMA.  Lane (j = lane % 32, h = lane / 32) supplies, for weight
 // row / token j, the four 16-byte pieces q = 0..3 of a 128-byte K chunk at chunk offset
-// 32 q + 16 h; the fp8 MFMA of chunk half m consumes pieces 2m and 2m + 1, the 16-bit MFMA q
-// consumes piece q.  Its 16 accumulators of a tile are token j, columns 8 (r / 4) + 4 h + r % 4.
+// 32 q + 16 h; the fp8 MFMA of chunk half m consumes pieces 2m and 2m + 1.
+// Its 16 accumulators of a tile are token j, columns 8 (r / 4) + 4 h + r % 4.
 // Row tiles made of padding only are skipped (wave-uniform), so the matrix work follows the
 // routed rows in steps of 32.
 //
@@ -203,14 +192,14 @@ __device__ __forceinline__ bool find_tile(const MoeGemmParams& p, int lane, Tile
 //     clamped addresses, waves whose row tile is padding copy one dummy line);
 //   * the block scales of the wave's two column tiles are parked in LDS once per tile.
 // None of this may go through scratch memory: the build checks that the kernel spills nothing.
-template <bool GATED, int DT, int QT, int WL>
+template <bool GATED, int DT, int WL>
 __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p) {
   constexpr int NX = 3;                 // activation chunk slots in LDS
   constexpr int kXSlot = 128 * 128;     // bytes of one slot
   constexpr int kScWave = 128;          // scale strip of a wave per slot: its 32 activation scales
   constexpr int kMaxKC = kMoeMaxKChunks;  // chunks of block scales parked in LDS (K <= 16384 bytes)
   constexpr int kScSlot = 4 * kScWave;
-  constexpr int D = QT == 0 ? 5 : 4;    // direct-to-LDS operations per wave and chunk
+  constexpr int D = 5;                  // direct-to-LDS operations per wave and chunk
   __shared__ __attribute__((aligned(1024))) unsigned char x_lds[NX * kXSlot];
   __shared__ __attribute__((aligned(16))) unsigned char sc_lds[NX * kScSlot];
   __shared__ float ws_lds[4][2][kMaxKC];  // block scales of wave w's column tile ct, by chunk
@@ -283,18 +272,17 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   // (positions past the tile's real rows hold the pad sentinel or another tile's slots: the last real
   // row is read instead, unconditionally -- behind a branch each load would be waited for)
   auto slot_at = [&](int r) -> int { return p.sorted_ids[row0 + min(r, tile.rows - 1)]; };
-  const bool gather = GATED || p.gather_a;
-  if (gather && stager) {
+  if (GATED && stager) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) sid_x[i] = slot_at(32 * wave + 8 * i + drow);
-    if (QT == 0) sid_s = slot_at(32 * wave + j);
+    sid_s = slot_at(32 * wave + j);
   }
   int sid_out = -1;  // down: slot of the tile's row `tid`
   if (!GATED) sid_out = slot_at(tid & 127);
   // source row of the tile's row r whose routing slot is sid (gated: the slot's token; pad
   // slots read a valid row)
   auto src_row_of = [&](int sid, int r) -> uint32_t {
-    if (gather) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
+    if (GATED) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
     return (uint32_t)min((int64_t)(row0 + r), p.a_rows - 1);
   };
   // ---- activation staging: per chunk 16 instructions of 8 rows x 128 bytes, four per wave
@@ -315,7 +303,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   // the scale of the wave's staging row l.  The block scales of the wave's two column tiles for
   // all chunks are fetched once, here, and parked in LDS.
   uint32_t sc_voff = 0;
-  if (QT == 0) {
+  {
     if (stager && lane < 32) sc_voff = src_row_of(sid_s, 32 * wave + j) * (uint32_t)KC * 4u;
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) {
@@ -338,10 +326,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       dma16_global_to_lds(p.a, xo[i] + koff, x_dst0 + slot * kXSlot + i * 1024);
-    if constexpr (QT == 0) {
-      dma4_global_to_lds_masked<0xffffffffull>(p.a_scale, sc_voff + (uint32_t)min(kc, KC - 1) * 4u,
-                                               sc_dst0 + slot * kScSlot);
-    }
+    dma4_global_to_lds_masked<0xffffffffull>(p.a_scale, sc_voff + (uint32_t)min(kc, KC - 1) * 4u,
+                                             sc_dst0 + slot * kScSlot);
   };
 
   // ---- fragment reads of the activations: lane (j, h), row tile rt, pieces 2q + h at
@@ -377,22 +363,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[rt][ct][r] = 0.0f;
 
-  // both MFMAs (fp8: one per column tile; 16 bit: two per column tile) of one (row tile, half)
   auto mma = [&](f32x16& a, const u32x4 (&b)[2], const u32x4 (&x)[2]) {
-    if constexpr (QT == 0) {
-      a = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cat8(b[0], b[1]), cat8(x[0], x[1]), a, 0, 0,
-                                                          0, 0, 0, 0);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        if constexpr (DT == DLB_DTYPE_BF16)
-          a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, b[q]),
-                                                      __builtin_bit_cast(bf16x8, x[q]), a, 0, 0, 0);
-        else
-          a = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, b[q]),
-                                                     __builtin_bit_cast(f16x8, x[q]), a, 0, 0, 0);
-      }
-    }
+    a = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cat8(b[0], b[1]), cat8(x[0], x[1]), a, 0, 0, 0, 0, 0, 0);
   };
   auto scale_tile = [&](f32x16& a, float f) {
 #pragma unroll
@@ -416,7 +388,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     // barrier that opens the main loop; here, behind the loads that the first chunks wait for
     if (tid < 128) {
       const bool real = tid < tile.rows && sid_out >= 0 && sid_out < p.numel;
-      sid_lds[tid] = !real ? -1 : p.scatter_c ? sid_out : row0 + tid;
+      sid_lds[tid] = real ? sid_out : -1;
       rw_lds[tid] = real ? slot_weight(p, sid_out) : 0.0f;
     }
   }
@@ -461,17 +433,17 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
       __builtin_amdgcn_sched_barrier(0);
       // (the previous chunk's scales sit in the slot that is refilled after this chunk's barrier)
       float al = 1.0f;
-      if (QT == 0 && rt == 0 && !first) al = ratio_a(x_tgt, x_cur, NRT - 1);
+      if (rt == 0 && !first) al = ratio_a(x_tgt, x_cur, NRT - 1);
       mma(acc[rt][0], wr[P][0][0], xc);
-      if (QT == 0 && rt == 0 && !first) scale_tile(acc[NRT - 1][0], al * __uint_as_float(rw_in[0]));
+      if (rt == 0 && !first) scale_tile(acc[NRT - 1][0], al * __uint_as_float(rw_in[0]));
       mma(acc[rt][1], wr[P][0][1], xc);
-      if (QT == 0 && rt == 0 && !first) scale_tile(acc[NRT - 1][1], al * __uint_as_float(rw_in[1]));
+      if (rt == 0 && !first) scale_tile(acc[NRT - 1][1], al * __uint_as_float(rw_in[1]));
       __builtin_amdgcn_sched_barrier(0);
     }
     issue_w(H0{}, k + 2, wr[P][0]);
     wait_vm<8>();     // this wave's part of X(k + 1) landed
     __syncthreads();  // X(k + 1) complete; every wave is done reading X(k - 1)
-    if (QT == 0 && more) {
+    if (more) {
       rw_out[0] = ratio_w(k, 0);
       rw_out[1] = ratio_w(k, 1);
     }
@@ -485,11 +457,11 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
       else if (more) read_x(x_nxt, 0, 0, xn);
       __builtin_amdgcn_sched_barrier(0);
       float ap = 1.0f;
-      if (QT == 0 && rt > 0 && more) ap = ratio_a(x_cur, x_nxt, rt - 1);
+      if (rt > 0 && more) ap = ratio_a(x_cur, x_nxt, rt - 1);
       mma(acc[rt][0], wr[P][1][0], xc);
-      if (QT == 0 && rt > 0 && more) scale_tile(acc[rt - 1][0], ap * __uint_as_float(rw_out[0]));
+      if (rt > 0 && more) scale_tile(acc[rt - 1][0], ap * __uint_as_float(rw_out[0]));
       mma(acc[rt][1], wr[P][1][1], xc);
-      if (QT == 0 && rt > 0 && more) scale_tile(acc[rt - 1][1], ap * __uint_as_float(rw_out[1]));
+      if (rt > 0 && more) scale_tile(acc[rt - 1][1], ap * __uint_as_float(rw_out[1]));
       __builtin_amdgcn_sched_barrier(0);
     }
     issue_w(H1{}, k + 2, wr[P][1]);
@@ -518,7 +490,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   // the accumulators hold sum / s(last chunk), whose scales are still in their LDS slot (x_tgt
   // after the last rotation): final scale of tile (rt, ct)
   auto final_scale = [&](int rt, int ct) -> float {
-    return QT == 0 ? read_as(x_tgt, rt) * read_ws(KC - 1, ct) : 1.0f;
+    return read_as(x_tgt, rt) * read_ws(KC - 1, ct);
   };
 
   // The lane coordinates are derived afresh for the epilogue: carried across the main loop they
@@ -530,48 +502,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   // A swap between the lane halves turns two 4-column runs into one 8-column run per lane.
   // Output tiles leave through LDS (the activation slots, free once every wave has left the
   // main loop and drained its copies) as whole rows, adjacent lanes on adjacent 16-byte pieces.
-  if (GATED && QT == 1) {
-    // rounding points of the reference pipeline (fused_moe.py:166,351-352): GEMM result,
-    // silu(gate) and the product are each rounded to the activation type
-    constexpr int kActPitch = 256 + 16;
-    static_assert(128 * kActPitch <= NX * kXSlot, "output staging fits the activation slots");
-    __syncthreads();
-#pragma unroll
-    for (int rt = 0; rt < NRT; ++rt) {
-      {
-        unsigned short* dst = (unsigned short*)(x_lds + (32 * rt + j_e) * kActPitch) + wave * 32 + 8 * h_e;
-#pragma unroll
-        for (int pr = 0; pr < 2; ++pr) {
-          unsigned int o[2][2];
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int r = 4 * (2 * pr + s) + i;
-              const unsigned int gu = Elem<DT>::pack(acc[rt][0][r], acc[rt][1][r]);
-              const float gate = Elem<DT>::lo(gu), up = Elem<DT>::hi(gu);
-              const float sg = Elem<DT>::lo(Elem<DT>::pack(gate / (1.0f + __expf(-gate)), 0.0f));
-              v[i] = sg * up;
-            }
-            o[s][0] = Elem<DT>::pack(v[0], v[1]);
-            o[s][1] = Elem<DT>::pack(v[2], v[3]);
-          }
-          swap_halves(o[0][0], o[1][0]);
-          swap_halves(o[0][1], o[1][1]);
-          *(u32x4*)(dst + 16 * pr) = u32x4{o[0][0], o[0][1], o[1][0], o[1][1]};
-        }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {  // 128 rows x 16 pieces of 16 bytes
-      const int r = (tid_e >> 4) + 16 * i, pc = tid_e & 15;
-      if (r < tile.rows && nt * 128 + 8 * pc < p.I)  // (the last column tile may be partial)
-        *(u32x4*)((unsigned short*)p.hq + (int64_t)(row0 + r) * p.I + nt * 128 + 8 * pc) =
-            *(const u32x4*)(x_lds + r * kActPitch + 16 * pc);
-    }
-  } else if (GATED) {
+  if (GATED) {
     constexpr int kGatedPitch = 128 + 16;  // staging row pitch of the fp8 output tile
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
@@ -776,25 +707,29 @@ extern "C" int dlb_per_token_group_quant_fp8(const void* x, void* xq, float* xs,
 namespace dlb {
 namespace {
 
+// dtype: of the outputs (and, 16-bit, of the operands)
 template <bool GATED, int QT>
 int launch_moe_gemm(const MoeGemmParams& p, int dtype, int w_layout, hipStream_t s) {
-  // one workgroup per tile there can be (at most one partial row tile per expert that holds slots); a
-  // workgroup finds its tile from the expert counts (or finds none and leaves), see find_tile
   if (w_layout && p.N % 16 != 0) return DLB_ERR_UNSUPPORTED;  // operand order comes in 16-row tiles
   if (dtype != DLB_DTYPE_BF16 && dtype != DLB_DTYPE_F16) return DLB_ERR_UNSUPPORTED;
-  if (moe_stream_case(p, QT == 0)) return launch_moe_stream(p, GATED, QT == 0, dtype, w_layout, s);
-  const int64_t row_tiles = (int64_t)p.numel / 128 + (p.numel < p.num_local ? p.numel : p.num_local);
-  const uint32_t grid = (uint32_t)(ceil_div(row_tiles * p.num_ntiles, 8) * 8);
-#define DLB_LAUNCH_GEMM(DT_)                                                                   \
-  do {                                                                                       \
-    if (w_layout)                                                                            \
-      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, QT, 1>), dim3(grid), dim3(256), 0, s, p); \
-    else                                                                                     \
-      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, QT, 0>), dim3(grid), dim3(256), 0, s, p); \
+  if (QT == 1 || (int64_t)p.numel <= (int64_t)kStreamMeanRows * p.num_experts)
+    return launch_moe_stream(p, GATED, QT == 0, dtype, w_layout, s);
+  if constexpr (QT == 0) {
+    // one workgroup per tile there can be (at most one partial row tile per expert that holds slots); a
+    // workgroup finds its tile from the expert counts (or finds none and leaves), see find_tile
+    const int64_t row_tiles = (int64_t)p.numel / 128 + (p.numel < p.num_local ? p.numel : p.num_local);
+    const uint32_t grid = (uint32_t)(ceil_div(row_tiles * p.num_ntiles, 8) * 8);
+#define DLB_LAUNCH_GEMM(DT_)                                                               \
+  do {                                                                                   \
+    if (w_layout)                                                                        \
+      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, 1>), dim3(grid), dim3(256), 0, s, p); \
+    else                                                                                 \
+      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, 0>), dim3(grid), dim3(256), 0, s, p); \
   } while (0)
-  if (dtype == DLB_DTYPE_BF16) DLB_LAUNCH_GEMM(DLB_DTYPE_BF16);
-  else DLB_LAUNCH_GEMM(DLB_DTYPE_F16);
+    if (dtype == DLB_DTYPE_BF16) DLB_LAUNCH_GEMM(DLB_DTYPE_BF16);
+    else DLB_LAUNCH_GEMM(DLB_DTYPE_F16);
 #undef DLB_LAUNCH_GEMM
+  }
   return launch_status();
 }
 

@@ -1,5 +1,5 @@
 // Operands and small device helpers shared by the two grouped MoE GEMMs: the tiled one for many
-// rows per expert (moe_fp8.hip) and the streaming one for few (moe_stream.hip).
+// rows per expert (moe_fp8.hip, fp8) and the streaming one (moe_stream.hip).
 #pragma once
 #include <type_traits>
 
@@ -74,13 +74,9 @@ struct TileId {
 
 // Launches the streaming kernel.  gated / quantised as the entry points; N_out checks are done.
 int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dtype, int w_layout, hipStream_t s);
-// Up to this many rows per expert, on average over the routed slots, the streaming kernel is the faster
-// one: its time grows with every 64 rows of an expert, the tiled kernel's with every 128.  Measured
-// (64 experts, 2048 x 1408): fp8 at 38 rows 118 vs 123 us, at 48 rows 130 vs 127; 16-bit row-major at
-// 48 rows 243 vs 274, at 72 rows 319 vs 284.  Both weight layouts take the same kernel (their results
-// are bit-identical).
-inline bool moe_stream_case(const MoeGemmParams& p, bool quantised) {
-  return (int64_t)p.numel <= (quantised ? 42 : 56) * (int64_t)p.num_experts;
-}
+// fp8: up to this many rows per expert, on average over the routed slots, the streaming kernel is the
+// faster one (64 experts, 2048 x 1408: at 38 rows 118 vs 123 us, at 48 rows 130 vs 127).  16-bit
+// operands always take it.
+constexpr int kStreamMeanRows = 42;
 
 }  // namespace dlb

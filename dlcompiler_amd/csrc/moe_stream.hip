@@ -1,4 +1,4 @@
-// Grouped MoE GEMM for few rows per expert (decode steps and small mixed steps).
+// Grouped MoE GEMM: fp8 with few rows per expert (decode steps and small mixed steps), 16-bit with any.
 //
 // With a few rows per expert the weights are read once for almost no arithmetic: the kernel is a stream
 // through them, and what counts is whole loads in flight on every CU.  The tiled kernel of
@@ -8,9 +8,16 @@
 // 96 - 192 KB on their way: 5.3 - 6.2 TB/s (64 experts of 2048 x 1408 bf16, 300 tokens: layer
 // 265 -> 221 us; fp8, 32 tokens: 113 -> 101 us, 128 tokens 118 -> 109 us).
 //
-// Activations: up to 16 rows they go straight into operands too.  With 32 or 64 rows they would
-// pass through the CU once per wave, as many bytes as the weights (300 tokens: 255 us); there each
-// thread brings its share of the chunk, which goes on through LDS, two buffers, one barrier per chunk.
+// Activations: up to 16 rows they go straight into operands too.  With more rows they would pass
+// through the CU once per wave, as many bytes as the weights (300 tokens: 255 us); there each thread
+// brings its share of the chunk, which goes on through LDS, two buffers, one barrier per chunk.
+//
+// With many rows the matrix cores are the bound, and 16-bit operands stay here all the same: a 16-row
+// operand of row-major weights takes 16 cache lines per load, a 32-row one (which the tiled kernel
+// used for both types) 32, and the lines, not the bytes, limit the CU's load path.  64 experts,
+// 2048 x 1408, 4096 tokens: row-major 694 -> 623 us, operand order 504 -> 494; 768 tokens 277 -> 228.
+// (fp8 through this shape: products with a zero accumulator leave nothing to overlap the scaling
+// with, gate_up 201 against 171 us.)
 //
 // MFMA mapping: 16 x 16 x 128 (fp8) or 2 x 16 x 16 x 32 (16 bit) per chunk; weight rows are the A
 // operand, token rows the B operand.  Lane (c = lane % 16, g = lane / 16) supplies for weight row /
@@ -28,7 +35,7 @@
 namespace dlb {
 namespace {
 
-// As find_tile of the tiled kernel, with tiles of ROWS rows inside the alignment blocks.
+// As find_tile of the tiled kernel, with tiles of ROWS rows; also for the launcher form of the routing.
 template <int ROWS>
 __device__ __forceinline__ bool find_stream_tile(const MoeGemmParams& p, int ntiles, int lane, TileId& t) {
   const bool segs = p.seg_start.p != nullptr;
@@ -89,8 +96,15 @@ __device__ __forceinline__ bool find_stream_tile(const MoeGemmParams& p, int nti
   const int rb = rem % nrb;
   t.e = e - p.expert_offset;
   t.nt = rem / nrb;
-  t.row0 = (segs ? se : mbase << p.bm_shift) + rb * ROWS;
-  t.rows = min(ROWS, ce - rb * ROWS);
+  // (tiles of up to 128 rows: equal ones, to within a 32-row group, as in the tiled kernel)
+  int r0 = rb * ROWS, rows = ROWS;
+  if (ROWS == 128) {
+    const int groups = (ce + 31) >> 5, base = groups / nrb, extra = groups - base * nrb;
+    r0 = 32 * (rb * base + min(rb, extra));
+    rows = 32 * (base + (rb < extra ? 1 : 0));
+  }
+  t.row0 = (segs ? se : mbase << p.bm_shift) + r0;
+  t.rows = min(rows, ce - r0);
   // (counts that do not fit the slot list: touch nothing)
   return t.row0 + t.rows <= (segs ? p.numel : p.num_mblocks << p.bm_shift);
 }
@@ -105,21 +119,30 @@ __device__ __forceinline__ float max_groups(float v) {
 // the 32 up rows that go with them (fp8: CW = 4, the workgroup then holds whole 128-column
 // quantisation groups of its rows); else 64 consecutive rows.
 constexpr int kWaveTiles = 4;  // MFMA tiles of 16 weight rows per wave
-template <bool GATED, int DT, int QT, int WL, int CW, int KW, int NT>
-__global__ __launch_bounds__(64 * CW * KW, NT == 1 ? 4 : NT == 2 ? 3 : 2) void moe_stream_kernel(const MoeGemmParams p, const int ntiles) {
+// MAXNT: 16-row tiles of the largest row tile; 8 runs tiles of at most 64 or 96 rows on smaller copies of
+// the body (which share no registers).
+template <bool GATED, int DT, int QT, int WL, int CW, int KW, int MAXNT>
+__global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) void moe_stream_kernel(const MoeGemmParams p, const int ntiles) {
   static_assert(!GATED || QT == 1 || CW == 4, "fp8 intermediate: whole quantisation groups");
   constexpr int NCT = kWaveTiles;
-  constexpr int kTileRows = 16 * NT;
+  constexpr int kTileRows = 16 * MAXNT;
   constexpr int kWaveCols = GATED ? 8 * NCT : 16 * NCT;  // output columns of a wave
   constexpr int kCols = kWaveCols * CW;                   // ... of the workgroup
   constexpr int NSB = GATED ? 2 : 1;                      // 128-row blocks of weight scales a wave meets
-  constexpr bool XS = NT > 1;                             // activations through LDS
-  constexpr int kXRows = 16 * NT, NXL = XS ? 2 * NT / CW : 0;  // 16-byte pieces a thread brings per chunk
-  static_assert(!XS || (2 * NT % CW == 0 && kXRows <= 64 * CW), "whole pieces per thread");
-  __shared__ f32x4 part_lds[KW > 1 ? (KW - 1) * CW * NT * NCT * 64 : 1];
+  constexpr int kNonTemporal = WL && MAXNT < 8 ? 2 : 0;
+  constexpr bool XS = MAXNT > 1;                          // activations through LDS
+  constexpr int XD = MAXNT == 8 ? 1 : 2;                  // chunks of activations on their way there
+  __shared__ f32x4 part_lds[KW > 1 ? (KW - 1) * CW * MAXNT * NCT * 64 : 1];
   __shared__ float amax_lds[CW][kTileRows];
-  __shared__ __attribute__((aligned(16))) unsigned char x_lds[XS ? KW : 1][XS ? 2 : 1][XS ? kXRows * 128 : 16];
+  // (128-row tiles also stage their output there, 32 rows at a time in two buffers)
+  constexpr int kOutPitch = 2 * kCols + 16;
+  constexpr int kXBuf = MAXNT == 8 && 32 * kOutPitch > kTileRows * 128 ? 32 * kOutPitch : XS ? kTileRows * 128 : 16;
+  __shared__ __attribute__((aligned(16))) unsigned char x_lds[XS ? KW : 1][XS ? 2 : 1][kXBuf];
   __shared__ float xs_lds[XS && QT == 0 ? KW : 1][2][XS && QT == 0 ? 64 * CW : 1];
+  // down GEMM, 128-row tiles: destination row (-1: none) and routing weight of the tile's rows
+  constexpr bool kRowTable = !GATED && MAXNT == 8;
+  __shared__ int32_t dst_lds[kRowTable ? kTileRows : 1];
+  __shared__ float rw_lds[kRowTable ? kTileRows : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cw = wave % CW, kw = wave / CW;
@@ -128,313 +151,393 @@ __global__ __launch_bounds__(64 * CW * KW, NT == 1 ? 4 : NT == 2 ? 3 : 2) void m
   TileId tile;
   if (!find_stream_tile<kTileRows>(p, ntiles, lane, tile)) return;
 
-  const int K = p.K, KC = p.KC;
-  const int nk = (KC - kw + KW - 1) / KW;  // this wave's chunks: kw, kw + KW, ...
-  const int col0 = tile.nt * kCols + kWaveCols * cw;
-  // first weight row of MFMA tile ct
-  auto ncol = [&](int ct) { return GATED && ct >= NCT / 2 ? p.I + col0 + 16 * (ct - NCT / 2) : col0 + 16 * ct; };
-  const unsigned char* wbase = p.w + (int64_t)tile.e * p.N * K;
-  uint32_t woff[NCT];
+  auto run = [&](auto nt_tag) __attribute__((always_inline)) {
+    constexpr int NT = decltype(nt_tag)::value;
+    constexpr int kXRows = 16 * NT, NXL = XS ? 2 * NT / CW : 0;  // 16-byte pieces a thread brings per chunk
+    static_assert(!XS || (2 * NT % CW == 0 && kXRows <= 64 * CW), "whole pieces per thread");
+    const int K = p.K, KC = p.KC;
+    const int nk = (KC - kw + KW - 1) / KW;  // this wave's chunks: kw, kw + KW, ...
+    const int col0 = tile.nt * kCols + kWaveCols * cw;
+    // first weight row of MFMA tile ct
+    auto ncol = [&](int ct) { return GATED && ct >= NCT / 2 ? p.I + col0 + 16 * (ct - NCT / 2) : col0 + 16 * ct; };
+    const unsigned char* wbase = p.w + (int64_t)tile.e * p.N * K;
+    uint32_t woff[NCT];
 #pragma unroll
-  for (int ct = 0; ct < NCT; ++ct)
-    woff[ct] = WL ? (uint32_t)min(ncol(ct) >> 4, (p.N >> 4) - 1) * (uint32_t)KC * 2048u + (uint32_t)lane * 16u
-                  : (uint32_t)min(ncol(ct) + c, p.N - 1) * (uint32_t)K + 16u * g;
-  u32x4 w[2][NCT][2];                     // [buffer][tile][half]
-  u32x4 x[2][XS ? 1 : NT][2];             // operands ...
-  u32x4 xp[2][XS ? NXL : 1];              // ... or this thread's pieces of the chunk, on their way to LDS
-  float xs[2][XS ? 1 : NT];
-  // Loads go through buffer descriptors: scalar base and chunk offset, 32-bit lane offset, no vector
-  // address arithmetic; a chunk past the wave's last one is read through an empty descriptor,
-  // which touches no memory, so the loop needs no condition around a load (where two paths
-  // meet, the compiler waits as if the loads of the longer one had not been sent).
-  const uint32_t wbytes = (uint32_t)p.N * (uint32_t)K, xbytes = (uint32_t)p.a_rows * (uint32_t)K;
-  // A wave starts somewhere in its chunks and wraps around: if all started at the first one, all would
-  // ask for the same offsets of rows whose distance is a multiple of the channels' period.
-  const int skew = (int)((uint32_t)(tile.e * 5 + tile.nt * 3) % (uint32_t)max(nk, 1));
-  auto chunk_of = [&](int i) {
-    const int j = i + skew;
-    return kw + (j < nk ? j : j - nk) * KW;
-  };
-  auto load_w = [&](auto buf, int i) {
-    constexpr int B = decltype(buf)::value;
-    const auto rsrc = buffer_of(wbase, i < nk ? wbytes : 0u);
-    const int soff = chunk_of(i) * (WL ? 2048 : 128);
+    for (int ct = 0; ct < NCT; ++ct)
+      woff[ct] = WL ? (uint32_t)min(ncol(ct) >> 4, (p.N >> 4) - 1) * (uint32_t)KC * 2048u + (uint32_t)lane * 16u
+                    : (uint32_t)min(ncol(ct) + c, p.N - 1) * (uint32_t)K + 16u * g;
+    u32x4 w[2][NCT][2];                     // [buffer][tile][half]
+    u32x4 x[2][XS ? 1 : NT][2];             // operands ...
+    u32x4 xp[XS ? XD : 1][XS ? NXL : 1];    // ... or this thread's pieces of the chunk, on their way to LDS
+    float xs[2][XS ? 1 : NT];
+    // Loads go through buffer descriptors: scalar base and chunk offset, 32-bit lane offset, no vector
+    // address arithmetic; a chunk past the wave's last one is read through an empty descriptor,
+    // which touches no memory, so the loop needs no condition around a load (where two paths
+    // meet, the compiler waits as if the loads of the longer one had not been sent).
+    const uint32_t wbytes = (uint32_t)p.N * (uint32_t)K, xbytes = (uint32_t)p.a_rows * (uint32_t)K;
+    // A wave starts somewhere in its chunks and wraps around: if all started at the first one, all would
+    // ask for the same offsets of rows whose distance is a multiple of the channels' period.
+    const int skew = (int)((uint32_t)(tile.e * 5 + tile.nt * 3) % (uint32_t)max(nk, 1));
+    auto chunk_of = [&](int i) {
+      const int j = i + skew;
+      return kw + (j < nk ? j : j - nk) * KW;
+    };
+    auto load_w = [&](auto buf, int i) {
+      constexpr int B = decltype(buf)::value;
+      const auto rsrc = buffer_of(wbase, i < nk ? wbytes : 0u);
+      const int soff = chunk_of(i) * (WL ? 2048 : 128);
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-      // operand order: whole lines, non-temporal (8 - 10 % faster); row-major: half lines, kept for
-      // the load of the other half (non-temporal 8 - 10 % slower)
-      w[B][ct][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct], soff, WL ? 2 : 0);
-      w[B][ct][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct] + (WL ? 1024 : 64), soff, WL ? 2 : 0);
-    }
-  };
-  using B0 = std::integral_constant<int, 0>;
-  using B1 = std::integral_constant<int, 1>;
-  // Prologue: the loads go out in the order in which the loop waits for them (a wait in the loop
-  // serves both ways into it): everything that is needed once, then chunk by chunk weights,
-  // activations and their scales.
-  // rows whose activations this thread loads (rows past the tile repeat its last one): its operand
-  // rows, or the rows of its pieces and the row of its scale
-  const int xtid = threadIdx.x % (64 * CW);
-  constexpr int NR = XS ? NXL : NT;
-  auto row_of = [&](int t) { return min(XS ? (t * 64 * CW + xtid) >> 3 : 16 * t + c, tile.rows - 1); };
-  int sid[NR + 1];
+      for (int ct = 0; ct < NCT; ++ct) {
+        // operand order: whole lines, non-temporal (8 - 10 % faster) unless the expert's other row tiles
+        // are about to read them; row-major: half lines, kept for the load of the other half
+        // (non-temporal 8 - 10 % slower)
+        w[B][ct][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct], soff, kNonTemporal);
+        w[B][ct][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)woff[ct] + (WL ? 1024 : 64), soff, kNonTemporal);
+      }
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    // Prologue: the loads go out in the order in which the loop waits for them (a wait in the loop
+    // serves both ways into it): everything that is needed once, then chunk by chunk weights,
+    // activations and their scales.
+    // rows whose activations this thread loads (rows past the tile repeat its last one): its operand
+    // rows, or the rows of its pieces and the row of its scale
+    const int xtid = threadIdx.x % (64 * CW);
+    constexpr int NR = XS ? NXL : NT;
+    auto row_of = [&](int t) { return min(XS ? (t * 64 * CW + xtid) >> 3 : 16 * t + c, tile.rows - 1); };
+    int sid[NR + 1];
 #pragma unroll
-  for (int t = 0; t < NR; ++t) sid[t] = p.sorted_ids[tile.row0 + row_of(t)];
-  sid[NR] = 0;
-  if (XS && QT == 0) sid[NR] = p.sorted_ids[tile.row0 + min(xtid % kXRows, tile.rows - 1)];
-  // block scales of the weight tiles: chunk kc in lane kc % 64 of register kc / 64
-  float ws[NSB][2];
-  if (QT == 0) {
+    for (int t = 0; t < NR; ++t) sid[t] = p.sorted_ids[tile.row0 + row_of(t)];
+    sid[NR] = 0;
+    if (XS && QT == 0) sid[NR] = p.sorted_ids[tile.row0 + min(xtid % kXRows, tile.rows - 1)];
+    // block scales of the weight tiles: chunk kc in lane kc % 64 of register kc / 64
+    float ws[NSB][2];
+    if (QT == 0) {
 #pragma unroll
-    for (int b = 0; b < NSB; ++b) {
-      const int blk = min(ncol(b * NCT / 2) >> 7, (p.N >> 7) - 1);
-      const float* src = p.w_scale + ((int64_t)tile.e * (p.N >> 7) + blk) * KC;
-      ws[b][0] = src[min(lane, KC - 1)];
-      ws[b][1] = src[min(lane + 64, KC - 1)];
-    }
-  }
-  load_w(B0{}, 0);
-  __builtin_amdgcn_sched_barrier(0);
-
-  auto src_row = [&](int sid, int row) -> uint32_t {
-    if (GATED || p.gather_a) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
-    return (uint32_t)min((int64_t)(tile.row0 + row), p.a_rows - 1);
-  };
-  uint32_t xoff[NR], soff[NR];
-#pragma unroll
-  for (int t = 0; t < NR; ++t) {
-    const uint32_t src = src_row(sid[t], row_of(t));
-    xoff[t] = src * (uint32_t)K + 16u * (XS ? xtid & 7 : g);
-    soff[t] = src * (uint32_t)KC * 4u;
-  }
-  if (XS && QT == 0) soff[0] = src_row(sid[NR], min(xtid % kXRows, tile.rows - 1)) * (uint32_t)KC * 4u;
-  auto load_x = [&](auto buf, int i) {
-    constexpr int B = decltype(buf)::value;
-    const auto rsrc = buffer_of(p.a, i < nk ? xbytes : 0u);
-    const auto srsrc = buffer_of(p.a_scale, i < nk ? xbytes / 32u : 0u);  // 4 bytes per 128
-    const int kc = chunk_of(i);
-    if constexpr (XS) {
-#pragma unroll
-      for (int q = 0; q < NXL; ++q) xp[B][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[q], kc * 128, 0);
-      if (QT == 0) xs[B][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[0], kc * 4, 0));
-    } else {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        x[B][t][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t], kc * 128, 0);
-        x[B][t][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t] + 64, kc * 128, 0);
-        if (QT == 0) xs[B][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[t], kc * 4, 0));
+      for (int b = 0; b < NSB; ++b) {
+        const int blk = min(ncol(b * NCT / 2) >> 7, (p.N >> 7) - 1);
+        const float* src = p.w_scale + ((int64_t)tile.e * (p.N >> 7) + blk) * KC;
+        ws[b][0] = src[min(lane, KC - 1)];
+        ws[b][1] = src[min(lane + 64, KC - 1)];
       }
     }
-  };
-  // XS: piece (row, p) of a chunk sits at piece p ^ (row & 7) of its row, so that neither the
-  // writes (a row at a time) nor the operand reads (16 rows, one piece) meet in the banks
-  auto store_x = [&](auto buf) {
-    constexpr int B = decltype(buf)::value;
-    if constexpr (XS) {
-#pragma unroll
-      for (int q = 0; q < NXL; ++q) {
-        const int row = (q * 64 * CW + xtid) >> 3;
-        *(u32x4*)(x_lds[kw][B] + row * 128 + (((xtid ^ row) & 7) << 4)) = xp[B][q];
-      }
-      if (QT == 0) xs_lds[kw][B][xtid] = xs[B][0];  // (rows repeat past kXRows: no branch in the loop)
-    }
-  };
-  load_x(B0{}, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  load_w(B1{}, 1);
-  load_x(B1{}, 1);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (XS) {
-    store_x(B0{});
-    load_x(B0{}, 2);
-    __syncthreads();
-  }
+    load_w(B0{}, 0);
+    __builtin_amdgcn_sched_barrier(0);
 
-  f32x4 acc[NT][NCT];
+    auto src_row = [&](int sid, int row) -> uint32_t {
+      if (GATED || p.gather_a) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
+      return (uint32_t)min((int64_t)(tile.row0 + row), p.a_rows - 1);
+    };
+    uint32_t xoff[NR], soff[NR];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) acc[t][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto operand = [&](auto buf, int t, u32x4& x0, u32x4& x1) {
-    constexpr int B = decltype(buf)::value;
-    if constexpr (XS) {
-      const unsigned char* row = x_lds[kw][B] + (16 * t + c) * 128;
-      x0 = *(const u32x4*)(row + (((g ^ c) & 7) << 4));
-      x1 = *(const u32x4*)(row + ((((g + 4) ^ c) & 7) << 4));
-    } else {
-      x0 = x[B][t][0];
-      x1 = x[B][t][1];
+    for (int t = 0; t < NR; ++t) {
+      const uint32_t src = src_row(sid[t], row_of(t));
+      xoff[t] = src * (uint32_t)K + 16u * (XS ? xtid & 7 : g);
+      soff[t] = src * (uint32_t)KC * 4u;
     }
-  };
-  auto compute = [&](auto buf, int i) {
-    constexpr int B = decltype(buf)::value;
-    if constexpr (QT == 0) {
+    if (XS && QT == 0) soff[0] = src_row(sid[NR], min(xtid % kXRows, tile.rows - 1)) * (uint32_t)KC * 4u;
+    auto load_x = [&](auto buf, int i) {
+      constexpr int B = decltype(buf)::value;
+      const auto rsrc = buffer_of(p.a, i < nk ? xbytes : 0u);
+      const auto srsrc = buffer_of(p.a_scale, i < nk ? xbytes / 32u : 0u);  // 4 bytes per 128
       const int kc = chunk_of(i);
-      float sw[NSB];
+      if constexpr (XS) {
 #pragma unroll
-      for (int b = 0; b < NSB; ++b)
-        sw[b] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kc < 64 ? ws[b][0] : ws[b][1]), kc & 63));
-      // (one row tile's products at a time: all of them together do not fit the registers)
-      u32x4 xo[2][2];
-      operand(buf, 0, xo[0][0], xo[0][1]);
+        for (int q = 0; q < NXL; ++q) xp[B % XD][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[q], kc * 128, 0);
+        if (QT == 0) xs[B % XD][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[0], kc * 4, 0));
+      } else {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        if (t + 1 < NT) operand(buf, t + 1, xo[(t + 1) & 1][0], xo[(t + 1) & 1][1]);
-        if (XS) __builtin_amdgcn_sched_barrier(0);
-        const u32x4 x0 = xo[t & 1][0], x1 = xo[t & 1][1];
-        const float a = XS ? xs_lds[kw][B][16 * t + c] : xs[B][XS ? 0 : t];
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-          const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-          const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-              cat8(w[B][ct][0], w[B][ct][1]), cat8(x0, x1), zero, 0, 0, 0, 0, 0, 0);
-          const float f = a * sw[GATED ? ct / (NCT / 2) : 0];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[t][ct][r] = fmaf(pr[r], f, acc[t][ct][r]);
+        for (int t = 0; t < NT; ++t) {
+          x[B][t][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t], kc * 128, 0);
+          x[B][t][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t] + 64, kc * 128, 0);
+          if (QT == 0) xs[B][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[t], kc * 4, 0));
         }
       }
-    } else {
+    };
+    // XS: piece (row, p) of a chunk sits at piece p ^ (row & 7) of its row, so that neither the
+    // writes (a row at a time) nor the operand reads (16 rows, one piece) meet in the banks
+    auto store_x = [&](auto buf) {
+      constexpr int B = decltype(buf)::value;
+      if constexpr (XS) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        u32x4 xo[2];
-        operand(buf, t, xo[0], xo[1]);
-#pragma unroll
-        for (int half = 0; half < 2; ++half)
-#pragma unroll
-          for (int ct = 0; ct < NCT; ++ct) {
-            if constexpr (DT == DLB_DTYPE_BF16)
-              acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[B][ct][half]),
-                                                                   __builtin_bit_cast(bf16x8, xo[half]),
-                                                                   acc[t][ct], 0, 0, 0);
-            else
-              acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[B][ct][half]),
-                                                                  __builtin_bit_cast(f16x8, xo[half]),
-                                                                  acc[t][ct], 0, 0, 0);
-          }
+        for (int q = 0; q < NXL; ++q) {
+          const int row = (q * 64 * CW + xtid) >> 3;
+          *(u32x4*)(x_lds[kw][B] + row * 128 + (((xtid ^ row) & 7) << 4)) = xp[B % XD][q];
+        }
+        if (QT == 0) xs_lds[kw][B][xtid] = xs[B % XD][0];  // (rows repeat past kXRows: no branch in the loop)
+      }
+    };
+    load_x(B0{}, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(B1{}, 1);
+    if (!XS || XD == 2) load_x(B1{}, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kRowTable) {  // (published by the next barrier; behind the loads of the first chunks)
+      const int r = threadIdx.x;
+      if (r < kTileRows) {
+        const int slot = p.sorted_ids[tile.row0 + min(r, tile.rows - 1)];
+        const bool real = r < tile.rows && slot >= 0 && slot < p.numel;
+        dst_lds[r] = !real ? -1 : p.scatter_c ? slot : tile.row0 + r;
+        rw_lds[r] = real ? slot_weight(p, slot) : 0.0f;
       }
     }
-  };
-  // XS: while chunk i is multiplied from LDS buffer i % 2, chunk i + 1 goes from registers into the
-  // other one (whose readers passed the barrier that ended step i - 1), and chunk i + 3 is asked for.
-  auto step = [&](auto buf, int i) {
-    using Other = std::integral_constant<int, 1 - decltype(buf)::value>;
-    compute(buf, i);
-    __builtin_amdgcn_sched_barrier(0);
-    load_w(buf, i + 2);
     if constexpr (XS) {
-      store_x(Other{});
-      load_x(Other{}, i + 3);
+      store_x(B0{});
+      if constexpr (XD == 2) load_x(B0{}, 2);
+      else load_x(B1{}, 1);
       __syncthreads();
-    } else {
-      load_x(buf, i + 2);
     }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // (XS: all waves make the same number of steps; a wave past its last chunk multiplies zeros)
-  const int steps = XS ? (KC + KW - 1) / KW : nk;
-  int i = 0;
-#pragma nounroll
-  for (; i + 1 < steps; i += 2) {
-    step(B0{}, i);
-    step(B1{}, i + 1);
-  }
-  if (i < steps) compute(B0{}, i);
 
-  // ---- partial sums of the K split
-  if constexpr (KW > 1) {
-    f32x4* part = part_lds + ((kw - 1) * CW + cw) * (NT * NCT * 64);
-    if (kw > 0) {
+    f32x4 acc[NT][NCT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) part[(NCT * t + ct) * 64 + lane] = acc[t][ct];
+      for (int ct = 0; ct < NCT; ++ct) acc[t][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto operand = [&](auto buf, int t, u32x4& x0, u32x4& x1) {
+      constexpr int B = decltype(buf)::value;
+      if constexpr (XS) {
+        const unsigned char* row = x_lds[kw][B] + (16 * t + c) * 128;
+        x0 = *(const u32x4*)(row + (((g ^ c) & 7) << 4));
+        x1 = *(const u32x4*)(row + ((((g + 4) ^ c) & 7) << 4));
+      } else {
+        x0 = x[B][t][0];
+        x1 = x[B][t][1];
+      }
+    };
+    auto compute = [&](auto buf, int i) {
+      constexpr int B = decltype(buf)::value;
+      if constexpr (QT == 0) {
+        const int kc = chunk_of(i);
+        float sw[NSB];
+#pragma unroll
+        for (int b = 0; b < NSB; ++b)
+          sw[b] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kc < 64 ? ws[b][0] : ws[b][1]), kc & 63));
+        // (one row tile's products at a time: all of them together do not fit the registers)
+        u32x4 xo[2][2];
+        operand(buf, 0, xo[0][0], xo[0][1]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          if (t + 1 < NT) operand(buf, t + 1, xo[(t + 1) & 1][0], xo[(t + 1) & 1][1]);
+          if (XS) __builtin_amdgcn_sched_barrier(0);
+          const u32x4 x0 = xo[t & 1][0], x1 = xo[t & 1][1];
+          const float a = XS ? xs_lds[kw][B][16 * t + c] : xs[B][XS ? 0 : t];
+#pragma unroll
+          for (int ct = 0; ct < NCT; ++ct) {
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                cat8(w[B][ct][0], w[B][ct][1]), cat8(x0, x1), zero, 0, 0, 0, 0, 0, 0);
+            const float f = a * sw[GATED ? ct / (NCT / 2) : 0];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][ct][r] = fmaf(pr[r], f, acc[t][ct][r]);
+          }
+        }
+      } else {
+        u32x4 xo2[2][2];
+        operand(buf, 0, xo2[0][0], xo2[0][1]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          if (t + 1 < NT) operand(buf, t + 1, xo2[(t + 1) & 1][0], xo2[(t + 1) & 1][1]);
+          if (MAXNT == 8) __builtin_amdgcn_sched_barrier(0);
+          const u32x4 xo[2] = {xo2[t & 1][0], xo2[t & 1][1]};
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ++ct) {
+              if constexpr (DT == DLB_DTYPE_BF16)
+                acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[B][ct][half]),
+                                                                     __builtin_bit_cast(bf16x8, xo[half]),
+                                                                     acc[t][ct], 0, 0, 0);
+              else
+                acc[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[B][ct][half]),
+                                                                    __builtin_bit_cast(f16x8, xo[half]),
+                                                                    acc[t][ct], 0, 0, 0);
+            }
+        }
+      }
+    };
+    // XS: while chunk i is multiplied from LDS buffer i % 2, chunk i + 1 goes from registers into the
+    // other one (whose readers passed the barrier that ended step i - 1), and chunk i + 1 + XD is asked for.
+    auto step = [&](auto buf, int i) {
+      using Other = std::integral_constant<int, 1 - decltype(buf)::value>;
+      compute(buf, i);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(buf, i + 2);
+      if constexpr (XS) {
+        store_x(Other{});
+        if constexpr (XD == 2) load_x(Other{}, i + 3);
+        else load_x(buf, i + 2);
+        __syncthreads();
+      } else {
+        load_x(buf, i + 2);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // (XS: all waves make the same number of steps; a wave past its last chunk multiplies zeros)
+    const int steps = XS ? (KC + KW - 1) / KW : nk;
+    int i = 0;
+    // (as in the tiled kernel: a workgroup in its main loop goes before the CU's other one in its prologue)
+    if (MAXNT == 8) __builtin_amdgcn_s_setprio(3);
+#pragma nounroll
+    for (; i + 1 < steps; i += 2) {
+      step(B0{}, i);
+      step(B1{}, i + 1);
     }
-    __syncthreads();
-    if (kw == 0) {
-#pragma unroll
-      for (int q = 1; q < KW; ++q)
+    if (i < steps) compute(B0{}, i);
+    if (MAXNT == 8) __builtin_amdgcn_s_setprio(0);
+
+    // ---- partial sums of the K split
+    if constexpr (KW > 1) {
+      f32x4* part = part_lds + ((kw - 1) * CW + cw) * (NT * NCT * 64);
+      if (kw > 0) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int ct = 0; ct < NCT; ++ct) 
-            acc[t][ct] += part_lds[(((q - 1) * CW + cw) * NT * NCT + NCT * t + ct) * 64 + lane];
-    }
-  }
-
-  // ---- epilogues: lane holds token row 16 t + c, columns ncol(ct) + 4 g + r
-  if constexpr (GATED && QT == 0) {
-    f32x4 v[NT][NCT / 2];
-    if (kw == 0) {
+          for (int ct = 0; ct < NCT; ++ct) part[(NCT * t + ct) * 64 + lane] = acc[t][ct];
+      }
+      __syncthreads();
+      if (kw == 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        float amax = 0.0f;
+        for (int q = 1; q < KW; ++q)
 #pragma unroll
-        for (int ct = 0; ct < NCT / 2; ++ct)
+          for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float gate = acc[t][ct][r], up = acc[t][ct + NCT / 2][r];
-            v[t][ct][r] = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;  // 1-ulp reciprocal
-            amax = fmaxf(amax, fabsf(v[t][ct][r]));
-          }
-        amax = max_groups(amax);
-        if (g == 0) amax_lds[cw][16 * t + c] = amax;
+            for (int ct = 0; ct < NCT; ++ct) 
+              acc[t][ct] += part_lds[(((q - 1) * CW + cw) * NT * NCT + NCT * t + ct) * 64 + lane];
       }
     }
-    __syncthreads();
-    if (kw == 0) {
+
+    // 16-bit outputs of 128-row tiles leave through LDS as whole rows: with the tile's 8-byte pieces stored
+    // as they are held, every row is touched in 32-byte parts (4000 tokens, K 384: 278 against 240 us).
+    // values(t, ct): the two words of columns 4 g .. + 3 of MFMA tile ct, row 16 t + c.  row_ptr(r): where
+    // row r of the tile goes (null: nowhere); ncols: columns that exist.
+    auto store_rows = [&](auto values, auto row_ptr, int nct, int ncols) __attribute__((always_inline)) {
+      constexpr int kPieces = kCols / 8;            // 16-byte pieces of a row
+      constexpr int kRowsAt = 64 * CW / kPieces;    // rows stored at a time
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        float m = amax_lds[0][16 * t + c];
+      for (int pass = 0; pass < NT / 2; ++pass) {
+        unsigned char* stage = x_lds[0][pass & 1];
+        if (pass == 0) __syncthreads();  // (every wave has left the main loop)
 #pragma unroll
-        for (int q = 1; q < CW; ++q) m = fmaxf(m, amax_lds[q][16 * t + c]);
-        const float scale = fmaxf(m, kQuantEps) / kFp8Max;
-        const float inv = __builtin_amdgcn_rcpf(scale);  // the stored scale stays exact
-        if (16 * t + c < tile.rows) {
-          const int64_t row = tile.row0 + 16 * t + c;
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int ct = 0; ct < NCT; ++ct)
+            if (ct < nct)
+              *(u32x2*)(stage + (16 * tt + c) * kOutPitch + 2 * (kWaveCols * cw + 16 * ct + 4 * g)) =
+                  values(2 * pass + tt, ct);
+        __syncthreads();  // (buffer pass & 1 is written again behind the next pass's barrier)
+#pragma unroll
+        for (int q = 0; q < 32 / kRowsAt; ++q) {
+          const int r = q * kRowsAt + threadIdx.x / kPieces, pc = threadIdx.x % kPieces;
+          unsigned short* dst = row_ptr(32 * pass + r);
+          if (dst && 8 * pc < ncols)
+            __builtin_nontemporal_store(*(const u32x4*)(stage + r * kOutPitch + 16 * pc), (u32x4*)(dst + 8 * pc));
+        }
+      }
+    };
+
+    // ---- epilogues: lane holds token row 16 t + c, columns ncol(ct) + 4 g + r
+    if constexpr (GATED && QT == 0) {
+      f32x4 v[NT][NCT / 2];
+      if (kw == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          float amax = 0.0f;
 #pragma unroll
           for (int ct = 0; ct < NCT / 2; ++ct)
-            *(unsigned int*)(p.hq + row * p.I + col0 + 16 * ct + 4 * g) =
-                pack4_fp8(v[t][ct][0] * inv, v[t][ct][1] * inv, v[t][ct][2] * inv, v[t][ct][3] * inv);
-          if (cw == 0 && g == 0) p.hs[row * (p.I >> 7) + tile.nt] = scale;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float gate = acc[t][ct][r], up = acc[t][ct + NCT / 2][r];
+              v[t][ct][r] = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;  // 1-ulp reciprocal
+              amax = fmaxf(amax, fabsf(v[t][ct][r]));
+            }
+          amax = max_groups(amax);
+          if (g == 0) amax_lds[cw][16 * t + c] = amax;
         }
       }
-    }
-  } else if constexpr (GATED) {
-    // rounding points of the reference pipeline (fused_moe.py:166,351-352): GEMM result,
-    // silu(gate) and the product are each rounded to the activation type
-    if (kw == 0) {
+      __syncthreads();
+      if (kw == 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t) {
+          float m = amax_lds[0][16 * t + c];
 #pragma unroll
-        for (int ct = 0; ct < NCT / 2; ++ct) {
-          float v[4];
+          for (int q = 1; q < CW; ++q) m = fmaxf(m, amax_lds[q][16 * t + c]);
+          const float scale = fmaxf(m, kQuantEps) / kFp8Max;
+          const float inv = __builtin_amdgcn_rcpf(scale);  // the stored scale stays exact
+          const int64_t row = tile.row0 + 16 * t + c;
+          if (cw == 0 && g == 0 && 16 * t + c < tile.rows) p.hs[row * (p.I >> 7) + tile.nt] = scale;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const unsigned int gu = Elem<DT>::pack(acc[t][ct][r], acc[t][ct + NCT / 2][r]);
-            const float gate = Elem<DT>::lo(gu), up = Elem<DT>::hi(gu);
-            v[r] = Elem<DT>::lo(Elem<DT>::pack(gate / (1.0f + __expf(-gate)), 0.0f)) * up;
+          for (int ct = 0; ct < NCT / 2; ++ct) {
+            const unsigned int q4 = pack4_fp8(v[t][ct][0] * inv, v[t][ct][1] * inv, v[t][ct][2] * inv, v[t][ct][3] * inv);
+            if (16 * t + c < tile.rows) *(unsigned int*)(p.hq + row * p.I + col0 + 16 * ct + 4 * g) = q4;
           }
-          // (the last column tile may be partial)
-          if (16 * t + c < tile.rows && col0 + 16 * ct < p.I)
-            *(u32x2*)((unsigned short*)p.hq + (int64_t)(tile.row0 + 16 * t + c) * p.I + col0 + 16 * ct + 4 * g) =
-                u32x2{Elem<DT>::pack(v[0], v[1]), Elem<DT>::pack(v[2], v[3])};
         }
-    }
-  } else if (kw == 0) {
+      }
+    } else if constexpr (GATED) {
+      // rounding points of the reference pipeline (fused_moe.py:166,351-352): GEMM result,
+      // silu(gate) and the product are each rounded to the activation type
+      auto activated = [&](int t, int ct) __attribute__((always_inline)) -> u32x2 {
+        float v[4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (16 * t + c >= tile.rows) continue;
-      const int slot = p.sorted_ids[tile.row0 + 16 * t + c];
-      if (slot < 0 || slot >= p.numel) continue;
-      const float f = slot_weight(p, slot);
-      const int64_t dst = p.scatter_c ? slot : tile.row0 + 16 * t + c;
+        for (int r = 0; r < 4; ++r) {
+          const unsigned int gu = Elem<DT>::pack(acc[t][ct][r], acc[t][ct + NCT / 2][r]);
+          const float gate = Elem<DT>::lo(gu), up = Elem<DT>::hi(gu);
+          v[r] = Elem<DT>::lo(Elem<DT>::pack(gate / (1.0f + __expf(-gate)), 0.0f)) * up;
+        }
+        return u32x2{Elem<DT>::pack(v[0], v[1]), Elem<DT>::pack(v[2], v[3])};
+      };
+      // (the last column tile may be partial)
+      if constexpr (MAXNT == 8) {
+        store_rows(activated,
+                   [&](int r) -> unsigned short* {
+                     return r < tile.rows ? (unsigned short*)p.hq + (int64_t)(tile.row0 + r) * p.I + tile.nt * kCols
+                                          : nullptr;
+                   },
+                   NCT / 2, p.I - tile.nt * kCols);
+      } else if (kw == 0) {
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct)
-        if (col0 + 16 * ct + 4 * g < p.N)
-          *(u32x2*)((unsigned short*)p.out + dst * p.N + col0 + 16 * ct + 4 * g) =
-              u32x2{Elem<DT>::pack(acc[t][ct][0] * f, acc[t][ct][1] * f),
-                    Elem<DT>::pack(acc[t][ct][2] * f, acc[t][ct][3] * f)};
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int ct = 0; ct < NCT / 2; ++ct)
+            if (16 * t + c < tile.rows && col0 + 16 * ct < p.I)
+              *(u32x2*)((unsigned short*)p.hq + (int64_t)(tile.row0 + 16 * t + c) * p.I + col0 + 16 * ct + 4 * g) =
+                  activated(t, ct);
+      }
+    } else if constexpr (MAXNT == 8) {
+      float f[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) f[t] = rw_lds[16 * t + c];
+      store_rows([&](int t, int ct) __attribute__((always_inline)) -> u32x2 {
+                   return u32x2{Elem<DT>::pack(acc[t][ct][0] * f[t], acc[t][ct][1] * f[t]),
+                                Elem<DT>::pack(acc[t][ct][2] * f[t], acc[t][ct][3] * f[t])};
+                 },
+                 [&](int r) -> unsigned short* {
+                   const int dst = dst_lds[r];
+                   return dst < 0 ? nullptr : (unsigned short*)p.out + (int64_t)dst * p.N + tile.nt * kCols;
+                 },
+                 NCT, p.N - tile.nt * kCols);
+    } else if (kw == 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (16 * t + c >= tile.rows) continue;
+        const int slot = p.sorted_ids[tile.row0 + 16 * t + c];
+        if (slot < 0 || slot >= p.numel) continue;
+        const float f = slot_weight(p, slot);
+        const int64_t dst = p.scatter_c ? slot : tile.row0 + 16 * t + c;
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+          if (col0 + 16 * ct + 4 * g < p.N)
+            *(u32x2*)((unsigned short*)p.out + dst * p.N + col0 + 16 * ct + 4 * g) =
+                u32x2{Elem<DT>::pack(acc[t][ct][0] * f, acc[t][ct][1] * f),
+                      Elem<DT>::pack(acc[t][ct][2] * f, acc[t][ct][3] * f)};
+      }
     }
+  };
+  if constexpr (MAXNT == 8) {
+    if (tile.rows > 96) run(std::integral_constant<int, 8>{});
+    else if (tile.rows > 64) run(std::integral_constant<int, 6>{});
+    else run(std::integral_constant<int, 4>{});
+  } else {
+    run(std::integral_constant<int, MAXNT>{});
   }
 }
 
@@ -475,7 +578,8 @@ template <bool GATED, int DT, int QT>
 void launch_gemm(const MoeGemmParams& p, int w_layout, hipStream_t s) {
   if ((int64_t)p.numel <= 7 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 1>(p, w_layout, s);
   else if ((int64_t)p.numel <= 19 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 2>(p, w_layout, s);
-  else launch_nt<GATED, DT, QT, 4>(p, w_layout, s);
+  else if ((int64_t)p.numel <= 56 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 4>(p, w_layout, s);
+  else if constexpr (QT == 1) launch_shape<GATED, DT, QT, 4, 1, 8>(p, w_layout, s);
 }
 
 template <int DT>

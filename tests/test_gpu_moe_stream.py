@@ -1,6 +1,6 @@
-"""GPU parity of the grouped GEMMs where experts hold few rows: tile heights of 16, 32 and 64 rows, waves
+"""GPU parity of the grouped GEMMs from few rows per expert to many: tile heights of 16 to 128 rows, waves
 side by side or splitting K, chunk counts that do not divide by the waves, experts without rows, skewed
-routing (several row tiles of one expert), and the edge to the tiled kernel."""
+routing (several row tiles of one expert), rows just past a tile, and the edge to the tiled fp8 kernel."""
 import pytest
 import torch
 
@@ -21,7 +21,8 @@ def _routing(T, E, k, skew, g):
 # (T, H, I, E, k): mean rows per expert 0.2 .. 56 and just past both limits
 SHAPES = [(1, 128, 128, 8, 2), (3, 640, 384, 64, 6), (40, 2048, 256, 64, 6), (17, 256, 1408, 8, 2),
           (75, 384, 128, 8, 2), (100, 1152, 640, 16, 4), (168, 256, 256, 8, 2), (169, 256, 256, 8, 2),
-          (224, 192, 320, 8, 2), (225, 192, 320, 8, 2)]
+          (224, 192, 320, 8, 2), (225, 192, 320, 8, 2), (300, 64, 192, 4, 2), (333, 512, 128, 4, 2),
+          (420, 128, 384, 4, 3)]
 
 
 @pytest.mark.parametrize("T,H,I,E,k", SHAPES)
