@@ -133,7 +133,7 @@ __device__ __forceinline__ void write_block_experts(const AlignOut& o, const int
 // one over the experts turn ranks into positions.  The pad value is written everywhere first,
 // while the ids are on their way.  Router and alignment of 48 tokens x 6 of 64 experts (block 128):
 // 14.6 us a call in two launches, 5.8 us in this one; of 45 tokens x 8 of 256 experts, where the
-// pads used to be written by one workgroup expert by expert, 35.7 -> 11.0 us.
+// pads used to be written by one workgroup expert by expert, 35.7 -> 9.8 us.
 constexpr int kOneThreads = 1024;
 constexpr int kOneWaves = kOneThreads / kWave;
 constexpr int kOneGroups = 4;  // slots per lane
@@ -233,17 +233,25 @@ struct RouteParams {
   int renorm, vec_ok;
 };
 
-// Router, then the alignment of its own selections, in one workgroup: 64 tokens per pass.
-constexpr int kOneTokens = 256;
+// Router, then the alignment of its own selections, in one workgroup: 64 tokens per pass.  A pass keeps
+// the CU's SIMDs busy, so past one or two of them the second launch is the cheaper way (64 experts,
+// 128 tokens: 9.1 against 9.4 us, 256 tokens 14.9 against 9.2; 256 experts, 64 tokens: 11.1 against
+// 13.4, 100 tokens 14.8 against 13.1).
+constexpr int one_workgroup_tokens(int experts_per_lane) {
+  return experts_per_lane == 4 ? 128 : experts_per_lane == 8 ? 96 : 80;
+}
+constexpr int kRouteSlots = 128 * 16;
+static_assert(kRouteSlots <= kOneSlots, "the routed slots fit one workgroup's alignment");
 template <int VPL, int LT>
 __global__ __launch_bounds__(kOneThreads) void route_align_one_kernel(const RouteParams p, const AlignOut o) {
   __shared__ OneShared s;
-  __shared__ int32_t ids_s[kOneSlots];
+  __shared__ int32_t ids_s[kRouteSlots];
   const int row = threadIdx.x >> 4;
   float v[VPL];
   load_token_logits<VPL, LT>(p.logits, row, row < p.T, p.E, p.ld, p.vec_ok, v);
   align_one_begin(o, s);
-  for (int64_t first = 0; first < p.T; first += 64) {
+  // (a wave without a token leaves the SIMD to those that have one)
+  for (int64_t first = 0; first + 4 * (threadIdx.x / kWave) < p.T; first += 64) {
     const int64_t token = first + row;
     float next[VPL];
     load_token_logits<VPL, LT>(p.logits, token + 64, token + 64 < p.T, p.E, p.ld, p.vec_ok, next);
@@ -829,7 +837,7 @@ extern "C" int dlb_moe_align_block_size_static(const void* topk_ids, int ids_int
 }
 
 // ---------------------------------------------------------------------------------------
-// Router and alignment as one pipeline: one workgroup up to kOneTokens tokens, else the router with
+// Router and alignment as one pipeline: one workgroup up to one_workgroup_tokens, else the router with
 // per-chunk expert counts (a chunk = the K routing slots of route_chunk_tokens(T) consecutive
 // tokens) and the placement.
 // ---------------------------------------------------------------------------------------
@@ -842,7 +850,7 @@ int route_chunk_tokens(int64_t T) { return (T + 63) / 64 <= kFusedChunks ? 64 : 
 
 template <int VPL, int LT>
 void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table, hipStream_t s) {
-  if (p.T <= kOneTokens && o.numel <= kOneSlots) {
+  if (p.T <= one_workgroup_tokens(VPL)) {
     hipLaunchKernelGGL((route_align_one_kernel<VPL, LT>), dim3(1), dim3(kOneThreads), 0, s, p, o);
     return;
   }

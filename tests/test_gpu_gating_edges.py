@@ -1,5 +1,5 @@
 """GPU parity of the router + alignment around the sizes where the launch changes: one workgroup up to
-256 tokens / 4096 slots, 64- and 128-token chunks beyond."""
+80 to 128 tokens / 4096 slots, 64- and 128-token chunks beyond."""
 import pytest
 import torch
 
@@ -9,6 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,k,block", [(256, 256, 16, 128), (257, 256, 16, 128), (256, 13, 3, 16), (257, 13, 3, 16),
+                                         (128, 64, 16, 128), (129, 64, 16, 128), (96, 128, 8, 64), (97, 128, 8, 64), (80, 200, 8, 64), (81, 200, 8, 64),
                                          (192, 128, 8, 1), (16384, 255, 2, 128), (16448, 256, 16, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_router_and_alignment_at_launch_edges(dev, T, E, k, block, dtype):
