@@ -1079,7 +1079,13 @@ extern "C" int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const v
   const int64_t eids_cap = ceil_div(cap, block);
   int32_t* post = (int32_t*)(base + l.num_post);
   const size_t align_bytes = dlb_moe_align_ws_bytes(numel, num_experts);
-  if (quantised && aligned)
+  // a few rows per expert: gate_up quantises what it loads, and there is nothing to launch before it
+  if (quantised && aligned && numel <= (int64_t)kSmallMeanRows * num_experts && aligned16(x) && ld_x % 8 == 0 &&
+      T * ld_x * 2 < (int64_t)0xffffffffu) {
+    up.a = (const unsigned char*)x;
+    up.a_scale = nullptr;
+    up.lda = ld_x * 2;
+  } else if (quantised && aligned)
     st = dlb_per_token_group_quant_fp8(x, xq, xs, T, H, ld_x, H, H / 128, dtype, stream);
   else if (quantised)
     st = dlb_moe_align_quant_fp8(topk_ids, ids_int64, numel, num_experts, block, own_sorted, cap, eids, eids_cap,
@@ -1089,7 +1095,7 @@ extern "C" int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const v
     st = dlb_moe_align_block_size(topk_ids, ids_int64, numel, num_experts, block, own_sorted, cap, eids, eids_cap,
                                   own_counts, post, base + l.align_ws, align_bytes, stream);
   if (st != DLB_OK) return st;
-  st = quantised ? launch_moe_gemm<true, 0>(up, DLB_DTYPE_BF16, w_layout, s)
+  st = quantised ? launch_moe_gemm<true, 0>(up, dtype, w_layout, s)
                  : launch_moe_gemm<true, 1>(up, dtype, w_layout, s);
   if (st != DLB_OK) return st;
   st = quantised ? launch_moe_gemm<false, 0>(down, dtype, w_layout, s)

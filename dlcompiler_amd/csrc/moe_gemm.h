@@ -36,6 +36,7 @@ struct MoeGemmParams {
   // down flavour
   void* out;                  // [numel, N] bf16/f16
   const float* topk_w;        // [numel]
+  int64_t lda;                // gated fp8, few rows: `a` is 16-bit, rows of lda bytes (0: quantised)
   int renorm;                 // weights are divided by the sum of their token's
 };
 
@@ -78,5 +79,7 @@ int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dty
 // faster one (64 experts, 2048 x 1408: at 38 rows 118 vs 123 us, at 48 rows 130 vs 127).  16-bit
 // operands always take it.
 constexpr int kStreamMeanRows = 42;
+// ... and up to this many it runs tiles of 16 rows
+constexpr int kSmallMeanRows = 7;
 
 }  // namespace dlb

@@ -121,9 +121,15 @@ __device__ __forceinline__ float max_groups(float v) {
 constexpr int kWaveTiles = 4;  // MFMA tiles of 16 weight rows per wave
 // MAXNT: 16-row tiles of the largest row tile; 8 runs tiles of at most 64 or 96 rows on smaller copies of
 // the body (which share no registers).
+// QT: 0 fp8 operands with block scales, 1 16-bit operands, 2 fp8 weights and 16-bit activations that a wave
+// quantises as it loads them, to the quantiser's bytes.  With tiles of 16 rows that is little arithmetic
+// beside a weight stream, so three waves per SIMD instead of four cost less than the quantiser's launch
+// (64 experts of 2048 x 1408: 32 tokens 99.5 -> 96.5 us, 4 tokens 46.5 -> 43.6 us).
 template <bool GATED, int DT, int QT, int WL, int CW, int KW, int MAXNT>
-__global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) void moe_stream_kernel(const MoeGemmParams p, const int ntiles) {
-  static_assert(!GATED || QT == 1 || CW == 4, "fp8 intermediate: whole quantisation groups");
+__global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 && QT != 2 ? 4 : MAXNT <= 2 ? 3 : 2) void moe_stream_kernel(const MoeGemmParams p, const int ntiles) {
+  constexpr bool FP8 = QT != 1, XQ = QT == 2;  // fp8 weights; activations quantised here
+  static_assert(!XQ || (GATED && MAXNT == 1), "quantising is for tiles of 16 rows");
+  static_assert(!GATED || !FP8 || CW == 4, "fp8 intermediate: whole quantisation groups");
   constexpr int NCT = kWaveTiles;
   constexpr int kTileRows = 16 * MAXNT;
   constexpr int kWaveCols = GATED ? 8 * NCT : 16 * NCT;  // output columns of a wave
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
   constexpr int kOutPitch = 2 * kCols + 16;
   constexpr int kXBuf = MAXNT == 8 && 32 * kOutPitch > kTileRows * 128 ? 32 * kOutPitch : XS ? kTileRows * 128 : 16;
   __shared__ __attribute__((aligned(16))) unsigned char x_lds[XS ? KW : 1][XS ? 2 : 1][kXBuf];
-  __shared__ float xs_lds[XS && QT == 0 ? KW : 1][2][XS && QT == 0 ? 64 * CW : 1];
+  __shared__ float xs_lds[XS && FP8 ? KW : 1][2][XS && FP8 ? 64 * CW : 1];
   // down GEMM, 128-row tiles: destination row (-1: none) and routing weight of the tile's rows
   constexpr bool kRowTable = !GATED && MAXNT == 8;
   __shared__ int32_t dst_lds[kRowTable ? kTileRows : 1];
@@ -167,14 +173,14 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
       woff[ct] = WL ? (uint32_t)min(ncol(ct) >> 4, (p.N >> 4) - 1) * (uint32_t)KC * 2048u + (uint32_t)lane * 16u
                     : (uint32_t)min(ncol(ct) + c, p.N - 1) * (uint32_t)K + 16u * g;
     u32x4 w[2][NCT][2];                     // [buffer][tile][half]
-    u32x4 x[2][XS ? 1 : NT][2];             // operands ...
+    u32x4 x[2][XS ? 1 : NT][XQ ? 4 : 2];    // operands (XQ: 32 16-bit values of the chunk) ...
     u32x4 xp[XS ? XD : 1][XS ? NXL : 1];    // ... or this thread's pieces of the chunk, on their way to LDS
     float xs[2][XS ? 1 : NT];
     // Loads go through buffer descriptors: scalar base and chunk offset, 32-bit lane offset, no vector
     // address arithmetic; a chunk past the wave's last one is read through an empty descriptor,
     // which touches no memory, so the loop needs no condition around a load (where two paths
     // meet, the compiler waits as if the loads of the longer one had not been sent).
-    const uint32_t wbytes = (uint32_t)p.N * (uint32_t)K, xbytes = (uint32_t)p.a_rows * (uint32_t)K;
+    const uint32_t wbytes = (uint32_t)p.N * (uint32_t)K, xbytes = (uint32_t)p.a_rows * (uint32_t)(XQ ? p.lda : K);
     // A wave starts somewhere in its chunks and wraps around: if all started at the first one, all would
     // ask for the same offsets of rows whose distance is a multiple of the channels' period.
     const int skew = (int)((uint32_t)(tile.e * 5 + tile.nt * 3) % (uint32_t)max(nk, 1));
@@ -209,10 +215,10 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
 #pragma unroll
     for (int t = 0; t < NR; ++t) sid[t] = p.sorted_ids[tile.row0 + row_of(t)];
     sid[NR] = 0;
-    if (XS && QT == 0) sid[NR] = p.sorted_ids[tile.row0 + min(xtid % kXRows, tile.rows - 1)];
+    if (XS && FP8) sid[NR] = p.sorted_ids[tile.row0 + min(xtid % kXRows, tile.rows - 1)];
     // block scales of the weight tiles: chunk kc in lane kc % 64 of register kc / 64
     float ws[NSB][2];
-    if (QT == 0) {
+    if (FP8) {
 #pragma unroll
       for (int b = 0; b < NSB; ++b) {
         const int blk = min(ncol(b * NCT / 2) >> 7, (p.N >> 7) - 1);
@@ -232,10 +238,10 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
 #pragma unroll
     for (int t = 0; t < NR; ++t) {
       const uint32_t src = src_row(sid[t], row_of(t));
-      xoff[t] = src * (uint32_t)K + 16u * (XS ? xtid & 7 : g);
+      xoff[t] = XQ ? src * (uint32_t)p.lda + 32u * g : src * (uint32_t)K + 16u * (XS ? xtid & 7 : g);
       soff[t] = src * (uint32_t)KC * 4u;
     }
-    if (XS && QT == 0) soff[0] = src_row(sid[NR], min(xtid % kXRows, tile.rows - 1)) * (uint32_t)KC * 4u;
+    if (XS && FP8) soff[0] = src_row(sid[NR], min(xtid % kXRows, tile.rows - 1)) * (uint32_t)KC * 4u;
     auto load_x = [&](auto buf, int i) {
       constexpr int B = decltype(buf)::value;
       const auto rsrc = buffer_of(p.a, i < nk ? xbytes : 0u);
@@ -244,13 +250,19 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
       if constexpr (XS) {
 #pragma unroll
         for (int q = 0; q < NXL; ++q) xp[B % XD][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[q], kc * 128, 0);
-        if (QT == 0) xs[B % XD][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[0], kc * 4, 0));
+        if (FP8) xs[B % XD][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[0], kc * 4, 0));
       } else {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
+          if constexpr (XQ) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              x[B][t][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t] + 128 * (q >> 1) + 16 * (q & 1), kc * 256, 0);
+            continue;
+          }
           x[B][t][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t], kc * 128, 0);
           x[B][t][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)xoff[t] + 64, kc * 128, 0);
-          if (QT == 0) xs[B][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[t], kc * 4, 0));
+          if (FP8) xs[B][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, (int)soff[t], kc * 4, 0));
         }
       }
     };
@@ -264,7 +276,7 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
           const int row = (q * 64 * CW + xtid) >> 3;
           *(u32x4*)(x_lds[kw][B] + row * 128 + (((xtid ^ row) & 7) << 4)) = xp[B % XD][q];
         }
-        if (QT == 0) xs_lds[kw][B][xtid] = xs[B % XD][0];  // (rows repeat past kXRows: no branch in the loop)
+        if (FP8) xs_lds[kw][B][xtid] = xs[B % XD][0];  // (rows repeat past kXRows: no branch in the loop)
       }
     };
     load_x(B0{}, 0);
@@ -293,6 +305,34 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct) acc[t][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // 32 values of the lane's token row: pieces g of the chunk's halves, in fp8, and the row's scale
+    auto quantise = [&](const u32x4 (&v)[XQ ? 4 : 2], u32x4& x0, u32x4& x1, float& scale) {
+      if constexpr (XQ) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const unsigned int d = v[i >> 2][i & 3];
+          amax = fmaxf(fmaxf(amax, fabsf(Elem<DT>::lo(d))), fabsf(Elem<DT>::hi(d)));
+        }
+        scale = fmaxf(max_groups(amax), kQuantEps) / kFp8Max;
+        // f / scale, rounded as the division rounds (Markstein: one residual step from the rounded
+        // reciprocal); |f| <= 448 scale, up to a rounding, so there is nothing to clamp
+        const float inv = 1.0f / scale;
+        auto div = [&](float f) {
+          const float qt = f * inv;
+          return fmaf(fmaf(-qt, scale, f), inv, qt);
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          // (unpacked again: 32 floats over the reduction are registers that three waves per SIMD do not have)
+          unsigned int d0 = v[i >> 1][2 * (i & 1)], d1 = v[i >> 1][2 * (i & 1) + 1];
+          asm volatile("" : "+v"(d0), "+v"(d1));
+          int r = __builtin_amdgcn_cvt_pk_fp8_f32(div(Elem<DT>::lo(d0)), div(Elem<DT>::hi(d0)), 0, false);
+          r = __builtin_amdgcn_cvt_pk_fp8_f32(div(Elem<DT>::lo(d1)), div(Elem<DT>::hi(d1)), r, true);
+          (i < 4 ? x0 : x1)[i & 3] = (unsigned int)r;
+        }
+      }
+    };
     auto operand = [&](auto buf, int t, u32x4& x0, u32x4& x1) {
       constexpr int B = decltype(buf)::value;
       if constexpr (XS) {
@@ -306,7 +346,7 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
     };
     auto compute = [&](auto buf, int i) {
       constexpr int B = decltype(buf)::value;
-      if constexpr (QT == 0) {
+      if constexpr (FP8) {
         const int kc = chunk_of(i);
         float sw[NSB];
 #pragma unroll
@@ -314,13 +354,15 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
           sw[b] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kc < 64 ? ws[b][0] : ws[b][1]), kc & 63));
         // (one row tile's products at a time: all of them together do not fit the registers)
         u32x4 xo[2][2];
-        operand(buf, 0, xo[0][0], xo[0][1]);
+        float xscale = 0.0f;
+        if constexpr (XQ) quantise(x[B][0], xo[0][0], xo[0][1], xscale);
+        else operand(buf, 0, xo[0][0], xo[0][1]);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           if (t + 1 < NT) operand(buf, t + 1, xo[(t + 1) & 1][0], xo[(t + 1) & 1][1]);
           if (XS) __builtin_amdgcn_sched_barrier(0);
           const u32x4 x0 = xo[t & 1][0], x1 = xo[t & 1][1];
-          const float a = XS ? xs_lds[kw][B][16 * t + c] : xs[B][XS ? 0 : t];
+          const float a = XQ ? xscale : XS ? xs_lds[kw][B][16 * t + c] : xs[B][XS ? 0 : t];
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) {
             const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -436,7 +478,7 @@ __global__ __launch_bounds__(64 * CW * KW, MAXNT == 1 ? 4 : MAXNT == 2 ? 3 : 2) 
     };
 
     // ---- epilogues: lane holds token row 16 t + c, columns ncol(ct) + 4 g + r
-    if constexpr (GATED && QT == 0) {
+    if constexpr (GATED && FP8) {
       f32x4 v[NT][NCT / 2];
       if (kw == 0) {
 #pragma unroll
@@ -562,7 +604,7 @@ template <bool GATED, int DT, int QT, int NT>
 void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
   constexpr int kCols4 = (GATED ? 8 : 16) * kWaveTiles * 4;
   const int64_t tiles = ceil_div(GATED ? p.I : p.N, kCols4) * (p.numel < p.num_local ? p.numel : p.num_local);
-  if constexpr (GATED && QT == 0) {
+  if constexpr (GATED && QT != 1) {
     if (NT == 1 && tiles < 128) launch_shape<GATED, DT, QT, 4, NT == 1 ? 2 : 1, NT>(p, w_layout, s);
     else launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
   } else {
@@ -576,7 +618,7 @@ void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
 // weights come from L2 but pass through the CU again.
 template <bool GATED, int DT, int QT>
 void launch_gemm(const MoeGemmParams& p, int w_layout, hipStream_t s) {
-  if ((int64_t)p.numel <= 7 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 1>(p, w_layout, s);
+  if ((int64_t)p.numel <= kSmallMeanRows * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 1>(p, w_layout, s);
   else if ((int64_t)p.numel <= 19 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 2>(p, w_layout, s);
   else if ((int64_t)p.numel <= 56 * (int64_t)p.num_experts) launch_nt<GATED, DT, QT, 4>(p, w_layout, s);
   else if constexpr (QT == 1) launch_shape<GATED, DT, QT, 4, 1, 8>(p, w_layout, s);
@@ -584,7 +626,8 @@ void launch_gemm(const MoeGemmParams& p, int w_layout, hipStream_t s) {
 
 template <int DT>
 void launch_dt(const MoeGemmParams& p, bool gated, int quantised, int w_layout, hipStream_t s) {
-  if (gated && quantised) launch_gemm<true, DLB_DTYPE_BF16, 0>(p, w_layout, s);
+  if (gated && quantised && p.lda) launch_nt<true, DT, 2, 1>(p, w_layout, s);
+  else if (gated && quantised) launch_gemm<true, DLB_DTYPE_BF16, 0>(p, w_layout, s);
   else if (gated) launch_gemm<true, DT, 1>(p, w_layout, s);
   else if (quantised) launch_gemm<false, DT, 0>(p, w_layout, s);
   else launch_gemm<false, DT, 1>(p, w_layout, s);
