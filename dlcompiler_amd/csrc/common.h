@@ -226,14 +226,27 @@ __device__ __forceinline__ float max_xor32(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-// tanh for the logit soft-cap, relative error below 4e-7: odd polynomial near 0, 1 - 2 / (e^2x + 1)
-// elsewhere (saturates to +-1).  A third of tanhf's instructions, and no branch.
+// tanh for the logit soft-cap: no less accurate than tanhf, in half its instructions and without a branch.
+// Below 0.85 an odd polynomial (least squares on Chebyshev nodes, reweighted towards the smallest
+// largest relative error, 8e-9); from there on the term in 1 - 2 / (e^2|x| + 1), whose exponential and
+// reciprocal are each up to an ulp off, is at most a third of the result.  Against 64 bits over all
+// floats in [0.2, 1) and every seventh in [2^-10, 16), either sign: largest relative error 1.1e-7,
+// 1.30 ulp, root mean square 0.30 ulp; tanhf 1.5e-7, 1.41 and 0.32; a seam at 0.25 6.3e-7, 10.2 and 1.2.
+// 8 x 512 tokens over 4096, every tile capped: 645 us whatever the scores are, with tanhf 581 us where
+// they all stay under 0.6 of the cap and 804 us where they do not (waves walk both of its branches).
 __device__ __forceinline__ float softcap_tanh(float x) {
-  const float x2 = x * x;
-  const float poly = x * (1.0f + x2 * (-1.0f / 3.0f + x2 * (2.0f / 15.0f + x2 * (-17.0f / 315.0f + x2 * (62.0f / 2835.0f)))));
-  const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);
-  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
-  return fabsf(x) < 0.25f ? poly : big;
+  const float a = fabsf(x), z = x * x;
+  float c = 0.0014401802327483892f;
+  c = fmaf(z, c, -0.007142828777432442f);
+  c = fmaf(z, c, 0.02112109400331974f);
+  c = fmaf(z, c, -0.05379646271467209f);
+  c = fmaf(z, c, 0.13331478834152222f);
+  c = fmaf(z, c, -0.3333326578140259f);
+  const float poly = fmaf(x * z, c, x);
+  // e2 = 2 e^-2|x|: 1 - e2 / (1 + e2 / 2)
+  const float e2 = __builtin_amdgcn_exp2f(fmaf(a, -2.8853900817779268f, 1.0f));
+  const float big = fmaf(-e2, __builtin_amdgcn_rcpf(fmaf(0.5f, e2, 1.0f)), 1.0f);
+  return a < 0.85f ? poly : copysignf(big, x);
 }
 
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) {
