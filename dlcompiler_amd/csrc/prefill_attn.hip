@@ -38,9 +38,11 @@ struct PrefillParams {
   // PACK kernels: a workgroup's rows are those of 1 << pack_shift query heads of a KV group, the rows of
   // each being (kBlockM >> pack_shift) queries
   int pack_shift;
-  // nsplit > 1: a workgroup takes one of nsplit equal runs of its key tiles and leaves unnormalised
-  // rows in ws_o [nsplit][tokens][Hq][ws_d] and (maximum, denominator) in ws_ml [nsplit][tokens][Hq][2]
+  // nsplit > 1: the key tiles of a row tile may be shared out among up to nsplit workgroups, see
+  // tiles_per_part, which leave unnormalised rows in ws_o [nsplit][tokens][Hq][ws_d] and (maximum,
+  // denominator) in ws_ml [nsplit][tokens][Hq][2]
   int nsplit, ws_d;
+  int B;  // sequences
   int64_t tokens;
   float* ws_o;
   float* ws_ml;
@@ -87,8 +89,27 @@ struct Mma32<DLB_DTYPE_F16> {
   }
 };
 
-constexpr int kTileN = 64;    // keys per LDS tile
 constexpr int kThreads = 256;
+constexpr int kTileN = 64;    // keys per LDS tile
+constexpr int kPartTiles = 8;  // ... per part of a split row tile, at least
+
+// key tiles [first, end) that hold a key visible to one of the `rows` queries from q0 on
+struct TileRun {
+  int first, end;
+};
+__device__ __forceinline__ TileRun visible_tiles(int kv_total, int hist, int q0, int rows, int window) {
+  return TileRun{window > 0 ? max(hist + q0 - window, 0) / kTileN : 0,
+                 (min(kv_total, hist + q0 + rows) + kTileN - 1) / kTileN};
+}
+// Key tiles of a part.  The launch is cut for the longest context that the block table has room for, and
+// engines keep tables of a fixed width; how many parts there are follows from the context itself.
+// Parts past the last tile have no work, and where there is one part it writes the output itself.
+// 32 heads (8 kv) of 128, a table of 512 pages of 64: 32 queries over 100 keys 36.1 -> 11.4 us, over 1000
+// 42 -> 19, over 4000 58.8 -> 20.4; 4 x 100 over 600 27.2 -> 21.7 (in a table without room: 6.7, 15.9, 20.3, 14.6).
+__device__ __forceinline__ int tiles_per_part(const TileRun& run, int nsplit) {
+  const int tiles = run.end - run.first, parts = min(max(tiles / kPartTiles, 1), nsplit);
+  return (tiles + parts - 1) / parts;
+}
 
 template <int D>
 struct Smem {
@@ -138,11 +159,13 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   // the sequences are walked longest context first (blockIdx.z = rank, not index): the long
   // ones start in the first round and the short ones fill in behind them.  (The packed layout
   // has many workgroups per slot and gains nothing from the ranking: measured 1.5 % slower.)
-  int seq = blockIdx.z;
-  if (PAGED && gridDim.z > 1 && gridDim.z <= kThreads) {
+  // (PACK: the part is the slowest index, so that the parts that have keys start first and spread over the chip)
+  const int nb = PACK ? p.B : gridDim.z;
+  const int split = !PACK ? 0 : nb == 1 ? blockIdx.z : blockIdx.z / nb, rank_of = PACK ? blockIdx.z - split * nb : blockIdx.z;
+  int seq = rank_of;
+  if (PAGED && nb > 1 && nb <= kThreads) {
     __shared__ int32_t rank_key[kThreads];
     __shared__ int32_t rank_seq;
-    const int nb = gridDim.z;
     const int t = threadIdx.x;
     const int key = t < nb ? p.kv_len[t] : 0;
     rank_key[t] = key;
@@ -153,7 +176,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
         const int kj = rank_key[j];
         rank += (kj > key || (kj == key && j < t)) ? 1 : 0;
       }
-      if (rank == (int)blockIdx.z) rank_seq = t;  // ranks are a permutation: exactly one writer
+      if (rank == rank_of) rank_seq = t;  // ranks are a permutation: exactly one writer
     }
     __syncthreads();
     seq = __builtin_amdgcn_readfirstlane(rank_seq);
@@ -162,8 +185,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   const int L = __builtin_amdgcn_readfirstlane(p.seq_len[seq]);
   const int pack = PACK ? p.pack_shift : 0;
   const int kBlockQ = kBlockM >> pack;  // queries of a workgroup
-  const int qy = PACK ? blockIdx.y / p.nsplit : blockIdx.y, split = PACK ? blockIdx.y - qy * p.nsplit : 0;
-  const int qtile = (PACK ? gridDim.y / p.nsplit : gridDim.y) - 1 - qy;  // heaviest first
+  const int qtile = gridDim.y - 1 - blockIdx.y;  // heaviest first
   const int q0 = qtile * kBlockQ;
   if (q0 >= L) return;
   const int64_t tok0 = __builtin_amdgcn_readfirstlane(p.start_loc[seq]);
@@ -171,6 +193,17 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   const int kv_total = PAGED ? __builtin_amdgcn_readfirstlane(p.kv_len[seq]) : L;
   const int hist = kv_total - L;
   if (PAGED && hist < 0) return;  // inconsistent lengths: nothing sensible to compute
+  // sliding window (only the paged entry point exposes it; the packed kernel compiles it out)
+  const int window = PAGED ? p.window : -1;
+  TileRun run = visible_tiles(kv_total, hist, q0, kBlockQ, window);
+  bool parted = false;  // other workgroups have a part of these rows' keys
+  if (PACK && p.nsplit > 1) {
+    const int per = tiles_per_part(run, p.nsplit);
+    parted = run.end - run.first > per;
+    run.first += split * per;
+    if (run.first >= run.end) return;
+    run.end = min(run.end, run.first + per);
+  }
   int head = blockIdx.x;  // PACK: first of the workgroup's heads
   if (p.xcd_heads) head = (blockIdx.x & 7) * p.xcd_heads + (blockIdx.x >> 3);
   if (PACK) head <<= pack;
@@ -203,30 +236,19 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
     }
   }
 
-  const int kv_end = min(kv_total, hist + q0 + kBlockQ);  // keys this workgroup needs
-  int ntiles = (kv_end + kTileN - 1) / kTileN;
-  // window / soft-cap requests take the masked path for every tile
-  // (only the paged entry point exposes them; the packed kernel compiles them out)
-  const int window = PAGED ? p.window : -1;
+  const int jfirst = run.first, ntiles = run.end;
+  // (a soft-cap takes the masked path for every tile; only the paged entry point exposes it)
   const float softcap = PAGED ? p.softcap : -1.0f;
   // tiles below this index lie entirely under the diagonal for every wave of the workgroup
   // (all 64 keys <= position of row q0): no mask, no clamping of key rows
-  int nfull = softcap > 0.0f ? 0 : (hist + q0 + 1) / kTileN;
-  // first tile that can hold a visible key (sliding window), and the first whose keys every query
-  // of the workgroup sees
-  int jfirst = window > 0 ? max(hist + q0 - window, 0) / kTileN : 0;
+  const int nfull = softcap > 0.0f ? 0 : min((hist + q0 + 1) / kTileN, ntiles);
+  // first tile whose keys every query of the workgroup sees (sliding window)
   const int jopen = window > 0 ? max(hist + q0 + kBlockQ - 1 - window + kTileN - 1, 0) / kTileN : 0;
   const int qpos = hist + qrow;                          // context position of this lane's query
   // context positions of the wave's first and last query
   const int wave_q0 = PACK ? (32 * wave) & (kBlockQ - 1) : 32 * wave;
   const int wave_first_pos = hist + q0 + wave_q0;
   const int wave_last_pos = wave_first_pos + (PACK ? min(32, kBlockQ) : 32) - 1;
-  if (PACK && p.nsplit > 1) {  // this workgroup's run of the tiles
-    const int per = (ntiles - jfirst + p.nsplit - 1) / p.nsplit;
-    jfirst += split * per;
-    ntiles = min(ntiles, jfirst + per);
-    nfull = min(nfull, ntiles);
-  }
 
   // ---- global -> LDS staging of one K/V tile.  Per-thread base pointers are formed once; a
   // tile adds a workgroup-uniform offset.  CLAMP (tiles that may run past the sequence)
@@ -601,7 +623,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
 
   // ---- epilogue: normalise and store O (lane holds 4 consecutive dims per register quad)
   l_run += __shfl_xor(l_run, 32);
-  if (PACK && p.nsplit > 1) {
+  if (PACK && parted) {
     if (qrow < L) {
       const int64_t row = ((int64_t)split * p.tokens + tok0 + qrow) * p.Hq + head;
       float* wo = p.ws_o + row * p.ws_d;
@@ -635,30 +657,59 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   }
 }
 
-// Merge of the nsplit partial rows of every (query, head) of a sequence (blockIdx.y): one wave per row,
-// four rows per workgroup.  Rows without a visible key in any part become 0.
+// Merge of the partial rows of every (query, head) of a sequence (blockIdx.y): half a wave per row (at most
+// 128 dims), four rows per workgroup.  Rows without a visible key in any part become 0; rows in one part
+// are written already.  A chain of memory latencies: the lengths, all the (maximum, denominator) pairs of
+// a row in one load, then the parts eight at a time (3200 rows of 5 parts: 5.1 -> 4.5 us).
+constexpr int kCombineRows = 4;
 template <int DT>
-__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(32 * kCombineRows) void prefill_combine_kernel(const PrefillParams p) {
   const int seq = blockIdx.y;
-  const int idx = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int idx = blockIdx.x * kCombineRows + (threadIdx.x >> 5);
   const int qrow = idx / p.Hq, head = idx - qrow * p.Hq;
-  const int lane = threadIdx.x & 63;
-  const int L = p.seq_len[seq];
-  if (qrow >= L || p.kv_len[seq] < L) return;
-  const int64_t rows = p.tokens * p.Hq, tok = p.start_loc[seq] + qrow, row = tok * p.Hq + head;
-  float m = -__builtin_inff();
-  for (int s = 0; s < p.nsplit; ++s) m = fmaxf(m, p.ws_ml[2 * (s * rows + row)]);
-  float den = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s = 0; s < p.nsplit; ++s) {
-    const float ms = p.ws_ml[2 * (s * rows + row)];
-    const float w = ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(ms - m);
-    den += w * p.ws_ml[2 * (s * rows + row) + 1];
-    if (4 * lane < p.dv && w > 0.0f) {
-      const f32x4 v = *(const f32x4*)(p.ws_o + (s * rows + row) * p.ws_d + 4 * lane);
+  const int lane = threadIdx.x & 31;
+  const int L = p.seq_len[seq], kv_total = p.kv_len[seq], hist = kv_total - L;
+  const int64_t tok = p.start_loc[seq] + qrow;
+  if (qrow >= L || hist < 0) return;
+  const int block_q = 128 >> p.pack_shift;
+  const TileRun run = visible_tiles(kv_total, hist, qrow / block_q * block_q, block_q, p.window);
+  const int per = tiles_per_part(run, p.nsplit), parts = (run.end - run.first + per - 1) / per;
+  if (parts < 2) return;
+  const int64_t rows = p.tokens * p.Hq, row = tok * p.Hq + head;
+  const float NONE = -__builtin_inff();
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  // (loads are clamped, not conditional: behind a branch each would be waited for before the next)
+  auto pair_of = [&](int s) {
+    const f32x2 ml = *(const f32x2*)(p.ws_ml + 2 * (min(s, parts - 1) * rows + row));
+    return s < parts ? ml : f32x2{NONE, 0.0f};
+  };
+  f32x2 first = pair_of(lane);  // parts 0 .. 31; the rest below
+  float m = first[0];
+  for (int s0 = 32; s0 < parts; s0 += 32) m = fmaxf(m, pair_of(s0 + lane)[0]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += w * v[i];
+  for (int d = 16; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 32));
+  float den = 0.0f;
+  f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const float* mine = p.ws_o + row * p.ws_d + min(4 * lane, p.ws_d - 4);
+  for (int s0 = 0; s0 < parts; s0 += 32) {
+    const f32x2 ml = s0 == 0 ? first : pair_of(s0 + lane);
+    const float w = ml[0] == NONE ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - m);
+    den += w * ml[1];
+    const int n = min(parts - s0, 32);
+    for (int s = 0; s < n; s += 8) {
+      f32x4 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        v[u] = *(const f32x4*)(mine + min(s0 + s + u, parts - 1) * rows * p.ws_d);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float wu = __shfl(w, s + u, 32);  // (past the last part: 0)
+        if (wu > 0.0f) acc += wu * v[u];
+      }
     }
   }
+#pragma unroll
+  for (int d = 16; d >= 1; d >>= 1) den += __shfl_xor(den, d, 32);
   const float inv = den > 0.0f ? 1.0f / den : 0.0f;
   if (4 * lane < p.dv)
     *(u32x2*)((unsigned short*)p.o + tok * p.o_st + head * p.o_sh + 4 * lane) =
@@ -695,7 +746,7 @@ PackPlan pack_plan(int B, int Hq, int Hkv, int D, int max_len, int64_t max_keys,
     ++plan.pack_shift;
   const int64_t wgs = workgroups(plan.pack_shift);
   if (wgs <= 128 ? tiles >= 32 : wgs <= 256 && tiles >= 96) {
-    const int64_t most = tiles / 8;
+    const int64_t most = tiles / kPartTiles;
     plan.nsplit = (int)(512 / wgs < most ? 512 / wgs : most);
   }
   plan.use = plan.pack_shift > 0 || plan.nsplit > 1;
@@ -748,18 +799,19 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   }
   p.pack_shift = plan.pack_shift;
   p.nsplit = plan.nsplit;
+  p.B = B;
   p.ws_d = (Dv + 3) / 4 * 4;
   p.ws_o = (float*)ws;
   p.ws_ml = p.ws_o ? p.ws_o + (size_t)p.tokens * Hq * p.nsplit * p.ws_d : nullptr;
   const bool small = !plan.use && D <= 128 && Hq * ceil_div(max_len, 128) * B <= 240 && max_keys > 128;
   const int64_t qtiles = ceil_div(max_len, small ? 64 : 128 >> p.pack_shift);
-  if (qtiles * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
+  if (qtiles > 65535 || (int64_t)B * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
   const int head_groups = Hq >> p.pack_shift;
   // workgroups are dealt round-robin to the 8 XCDs by linear id; with Hq % 8 == 0 the
   // remap in the kernel puts heads {x, x+8, ...} -> consecutive heads on one XCD so a KV
   // group's four query heads hit the same L2.
   p.xcd_heads = head_groups % 8 == 0 && head_groups >= 16 ? head_groups >> 3 : 0;
-  const dim3 grid = dim3((uint32_t)head_groups, (uint32_t)(qtiles * p.nsplit), (uint32_t)B);
+  const dim3 grid = dim3((uint32_t)head_groups, (uint32_t)qtiles, (uint32_t)(B * p.nsplit));
 #define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_, PK_)                                                          \
   do {                                                                                                         \
     if (ragged)                                                                                                \
@@ -800,11 +852,11 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
 #undef DLB_LAUNCH_PREFILL
 #undef DLB_LAUNCH_PREFILL_RW
   if (p.nsplit > 1) {
-    const dim3 rows((uint32_t)ceil_div((int64_t)max_len * Hq, 4), (uint32_t)B);
+    const dim3 rows((uint32_t)ceil_div((int64_t)max_len * Hq, kCombineRows), (uint32_t)B);
     if (dtype == DLB_DTYPE_BF16)
-      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_BF16>, rows, dim3(256), 0, s, p);
+      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_BF16>, rows, dim3(32 * kCombineRows), 0, s, p);
     else
-      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_F16>, rows, dim3(256), 0, s, p);
+      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_F16>, rows, dim3(32 * kCombineRows), 0, s, p);
   }
   return launch_status();
 }
