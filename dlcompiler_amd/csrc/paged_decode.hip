@@ -596,7 +596,8 @@ __global__ __launch_bounds__(64 * W, RAGGED ? 1 : 2) void paged_decode_direct_ke
 // one sequence: 9.2 us, with four 10.7).
 int direct_waves(int B, int units, int max_ctx, int window, int D) {
   if (D > 128) return 0;
-  const bool windowed = window > 0 && window + 32 < max_ctx;
+  // (a window of any size up to 2^31 - 1 says "none" as well as -1 does)
+  const bool windowed = window > 0 && window < max_ctx - 32;
   const int keys = windowed ? window + 32 : max_ctx;
   const int64_t wgs = (int64_t)B * units;
   const bool few_keys = (int64_t)keys * D <= 700 * 128;

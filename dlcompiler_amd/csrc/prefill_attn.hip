@@ -750,7 +750,8 @@ PackPlan pack_plan(int B, int Hq, int Hkv, int D, int max_len, int64_t max_keys,
   PackPlan plan = {0, 1, false};
   if (D > 128) return plan;
   const int group = Hq / Hkv;
-  const int64_t seen = window > 0 && window + max_len < max_keys ? window + max_len : max_keys;
+  const int64_t reach = (int64_t)window + max_len;  // (windows of up to 2^31 - 1 come as "none")
+  const int64_t seen = window > 0 && reach < max_keys ? reach : max_keys;
   const int64_t tiles = ceil_div(seen, kTileN);
   auto workgroups = [&](int shift) { return (int64_t)(Hq >> shift) * ceil_div(max_len, 128 >> shift) * B; };
   while (group % (2 << plan.pack_shift) == 0 && (int64_t)max_len << (plan.pack_shift + 1) <= 128 &&
