@@ -1,7 +1,7 @@
 // fp8 (OCP e4m3fn) per-token-group quantisation of activations, shared by the stand-alone
 // quantiser and by the launch that runs it beside the expert alignment.
 // Rule: per group of 128 consecutive elements of a row, scale = max(absmax, 1e-10) / 448 and
-// q = rne_e4m3(clamp(x / scale, +-448)).
+// q = rne_e4m3(clamp(x / scale, +-448)); a NaN stays NaN and does not count for the absmax.
 #pragma once
 #include "common.h"
 
@@ -11,11 +11,9 @@ constexpr float kFp8Max = 448.0f;
 constexpr float kQuantEps = 1e-10f;
 
 __device__ __forceinline__ unsigned int pack4_fp8(float a, float b, float c, float d) {
-  // v_cvt_pk_fp8_f32 rounds to nearest even; values beyond +-464 would become NaN, so clamp.
-  a = fminf(fmaxf(a, -kFp8Max), kFp8Max);
-  b = fminf(fmaxf(b, -kFp8Max), kFp8Max);
-  c = fminf(fmaxf(c, -kFp8Max), kFp8Max);
-  d = fminf(fmaxf(d, -kFp8Max), kFp8Max);
+  // v_cvt_pk_fp8_f32 rounds to nearest even.  The scale is the group's own maximum / 448, so a finite
+  // quotient is at most 448 and a rounding, which rounds to 448 (only beyond 464 would it become NaN):
+  // there is nothing to clamp, and fminf / fmaxf would turn a NaN into -448.
   int r = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
   r = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, r, true);
   return (unsigned int)r;

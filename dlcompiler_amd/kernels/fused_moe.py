@@ -23,7 +23,7 @@ def per_token_group_quant_fp8(x: torch.Tensor, group_size: int = 128):
     """x [M, K] bf16/f16 -> (xq float8_e4m3fn [M, K], xs fp32 [M, K // 128]).
 
     Per group of 128 along K: ``scale = max(absmax, 1e-10) / 448``,
-    ``q = rne(clamp(x / scale, -448, 448))``.
+    ``q = rne(clamp(x / scale, -448, 448))``; a NaN stays NaN.
     """
     if group_size != 128:
         raise NotImplementedError("only groups of 128 are implemented")

@@ -269,7 +269,8 @@ int dlb_paged_prefill_attn_ws(const void* q, const void* k_cache, const void* v_
  * precedent: per-token int8 quant and scale-in-epilogue GEMM, kernels/w8a8.py:102-106,275-335.
  *
  * Quantisation rule (activations and the intermediate): for each group of 128 consecutive
- * elements of a row, scale = max(absmax, 1e-10) / 448 and q = rne_e4m3(clamp(x / scale, +-448)).
+ * elements of a row, scale = max(absmax, 1e-10) / 448 and q = rne_e4m3(clamp(x / scale, +-448)); a NaN
+ * stays NaN.
  * ---------------------------------------------------------------------------------------- */
 
 /* x [M, K] bf16/f16 (row stride ld_x) -> xq [M, K] fp8 (row stride ld_q, bytes),
