@@ -197,16 +197,6 @@ PyObject* rms_norm(PyObject*, PyObject* const* args, Py_ssize_t) {
     outs[i] = tensor(args[4 + i]);
     if (!like_x(outs[i])) NOT_HANDLED;
   }
-  // Two small results share one allocation, which costs the host about as much as the checks (a call of
-  // 8 tokens 4.5 -> 3.8 us); large ones do not, so that dropping one of them frees its memory.
-  constexpr int64_t kShared = 256 << 10;
-  const int64_t bytes = (x->nbytes() + 255) & ~(int64_t)255;
-  if (add && !outs[0] && !outs[1] && bytes <= kShared) {
-    const at::Tensor buf = empty({2 * bytes}, at::kByte, dev);
-    for (int i = 0; i < 2; ++i) made[i] = piece(buf, i * bytes, x->sizes(), x->scalar_type());
-    outs[0] = &made[0];
-    outs[1] = &made[1];
-  }
   for (int i = 0; i < (add ? 2 : 1); ++i)
     if (!outs[i]) {
       made[i] = empty(x->sizes(), x->scalar_type(), dev);
