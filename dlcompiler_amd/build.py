@@ -52,7 +52,8 @@ DEVICE_FLAGS = [
 ]
 
 # kernels whose loads and waits are issued by hand: no scratch, no spilled vector registers
-HAND_SCHEDULED = ("moe_gemm_kernel", "moe_stream_kernel", "prefill_attn_kernel", "paged_decode_split_kernel")
+HAND_SCHEDULED = ("moe_gemm_kernel", "moe_stream_kernel", "prefill_attn_kernel", "paged_decode_split_kernel",
+                  "paged_decode_direct_kernel")
 
 
 def _sources() -> list[Path]:

@@ -1,0 +1,38 @@
+"""The build stops when a kernel that issues its loads by hand spills or uses scratch memory (no GPU)."""
+import re
+
+import pytest
+
+from dlcompiler_amd.build import CSRC_DIR, check_hand_scheduled, kernel_resources
+
+# kernels that run the helpers of inline-assembly loads, or the key walk of the paged decode kernels, which
+# looks pages up with hand-issued scalar loads
+KERNELS = ["moe_gemm_kernel", "moe_stream_kernel", "prefill_attn_kernel", "paged_decode_split_kernel",
+           "paged_decode_direct_kernel"]
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_spills_and_scratch_are_refused(kernel):
+    name = f"_ZN3dlb12_GLOBAL__N_1{len(kernel)}{kernel}ILi0EEEv"
+    assert not check_hand_scheduled({name: {"scratch_bytes": 0, "vgpr_spills": 0}})
+    assert check_hand_scheduled({name: {"scratch_bytes": 8, "vgpr_spills": 0}})
+    assert check_hand_scheduled({name: {"scratch_bytes": 0, "vgpr_spills": 1}})
+    assert check_hand_scheduled({name: {"scratch_bytes": 0}})
+    assert check_hand_scheduled({}, f"void {kernel}(")
+
+
+def test_every_kernel_with_hand_issued_loads_is_named():
+    """Sources that issue loads by hand hold no kernel outside the gate but these, which use ordinary loads."""
+    ordinary = {"prefill_combine_kernel", "paged_decode_combine_kernel", "quant_fp8_group128_kernel",
+                "moe_topk_sum_kernel"}
+    for src in CSRC_DIR.glob("*.hip"):
+        text = src.read_text()
+        if re.search(r"dma\d+_global_to_lds|s_load_dword|buffer_of\(", text):
+            assert set(re.findall(r"void (\w+_kernel)\(", text)) - ordinary <= set(KERNELS), src.name
+
+
+def test_the_build_reports_every_gated_kernel():
+    built = kernel_resources()
+    for kernel in KERNELS:
+        reports = [r for name, r in built.items() if kernel in name]
+        assert reports and all(r["scratch_bytes"] == r["vgpr_spills"] == 0 for r in reports), kernel
