@@ -608,9 +608,9 @@ void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
     if (NT == 1 && tiles < 128) launch_shape<GATED, DT, QT, 4, NT == 1 ? 2 : 1, NT>(p, w_layout, s);
     else launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
   } else {
+    constexpr int CW = NT == 1 ? 1 : 2;
     if (tiles >= 512) launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
-    else if (NT == 1) launch_shape<GATED, DT, QT, NT == 1 ? 1 : 2, NT == 1 ? 4 : 2, NT>(p, w_layout, s);
-    else launch_shape<GATED, DT, QT, 2, 2, NT>(p, w_layout, s);
+    else launch_shape<GATED, DT, QT, CW, 4 / CW, NT>(p, w_layout, s);
   }
 }
 

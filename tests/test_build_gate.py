@@ -36,3 +36,11 @@ def test_the_build_reports_every_gated_kernel():
     for kernel in KERNELS:
         reports = [r for name, r in built.items() if kernel in name]
         assert reports and all(r["scratch_bytes"] == r["vgpr_spills"] == 0 for r in reports), kernel
+
+
+def test_no_instance_that_no_dispatch_reaches():
+    """Grouped GEMM with few rows: 16-row tiles split K over one column wave, taller ones over two."""
+    shapes = {m.groups() for m in (re.search(r"moe_stream_kernelILb\dELi\dELi\dELi\dELi(\d)ELi(\d)ELi(\d)E", name)
+                                   for name in kernel_resources()) if m}
+    assert shapes == {("4", "1", "1"), ("4", "2", "1"), ("1", "4", "1"), ("4", "1", "2"), ("2", "2", "2"),
+                      ("4", "1", "4"), ("2", "2", "4"), ("4", "1", "8")}
