@@ -599,4 +599,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dlb_host", "host side of the oper
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__dlb_host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__dlb_host(void) {
+  PyObject* m = PyModule_Create(&module);
+  // (of the header this module was built with: it calls the library by address)
+  if (m && PyModule_AddIntConstant(m, "abi_version", DLB_ABI_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -1,5 +1,6 @@
 """The C-ABI library loads and exports exactly what include/dlblas_hip.h declares (no GPU)."""
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -29,7 +30,7 @@ def test_every_declared_symbol_is_exported_and_bound():
 
 def test_version_and_status_strings():
     lib = _lib.load()
-    assert lib.dlb_version() == _lib.ABI_VERSION == 5
+    assert lib.dlb_version() == _lib.ABI_VERSION == 6
     assert lib.dlb_status_string(0) == b"ok"
     for code in (-1, -2, -3, -4, -99):
         assert lib.dlb_status_string(code)
@@ -40,6 +41,25 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     with pytest.raises(ImportError):
         _lib.load()
+
+
+def test_library_of_another_version_is_refused(monkeypatch, tmp_path):
+    # a library from before the entry points of version 6: nothing but a version to go by
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int dlb_version(void) { return 5; }")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setenv("DLBLAS_HIP_LIB", str(so))
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(ImportError, match="ABI version 5"):
+        _lib.load()
+
+
+def test_host_module_of_another_version_is_refused(monkeypatch):
+    assert _lib.host().abi_version == _lib.load().dlb_version()
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)   # (the library itself stays loaded)
+    with pytest.raises(ImportError, match="another ABI version"):
+        _lib.host()
 
 
 def test_cpu_tensor_is_rejected():
