@@ -114,7 +114,9 @@ shuffle_moe_weight_fp8 = shuffle_moe_weight
 
 # Operand-order copies made on behalf of callers that hand over the reference's row-major weights
 # on every call and cannot re-arrange them at load time themselves (a patched serving engine):
-# keyed by the weight tensor's storage, dropped when the tensor is modified in place.
+# keyed by where the weights lie, dropped when they are modified in place or their storage goes (an
+# address alone could be another tensor's by then).  The entry's weak reference keeps the storage
+# object, not its memory, from being reused: equal objects are the same storage.
 _OPERAND_ORDER_CACHE = {}
 _CACHE_ENV = "DLBLAS_HIP_CACHE_OPERAND_ORDER"
 
@@ -129,14 +131,19 @@ def _operand_order_cached(w: torch.Tensor) -> torch.Tensor:
     """The operand-order copy of ``w`` (see :func:`shuffle_moe_weight`), made on the first call
     and kept for as long as ``w`` keeps its storage and is not written through torch (its version
     counter).  Doubles the memory the weights take; one re-layout pass per weight tensor."""
+    from torch.multiprocessing.reductions import StorageWeakRef
+
+    storage = w.untyped_storage()
     key = (w.data_ptr(), tuple(w.shape), w.dtype, w.device)
     hit = _OPERAND_ORDER_CACHE.get(key)
-    if hit is not None and hit[0] == w._version:
+    if hit is not None and hit[0] == w._version and hit[2].cdata == storage._cdata:
         return hit[1]
+    for old in [k for k, v in _OPERAND_ORDER_CACHE.items() if v[2].expired()]:
+        del _OPERAND_ORDER_CACHE[old]
     if len(_OPERAND_ORDER_CACHE) > 256:
         _OPERAND_ORDER_CACHE.clear()
     sh = shuffle_moe_weight(w)
-    _OPERAND_ORDER_CACHE[key] = (w._version, sh)
+    _OPERAND_ORDER_CACHE[key] = (w._version, sh, StorageWeakRef(storage))
     return sh
 
 
