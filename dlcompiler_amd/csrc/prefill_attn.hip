@@ -18,6 +18,7 @@
 //   * the exponent runs in base 2 with the softmax scale folded into one FMA;
 //   * fully masked tiles are skipped per wave and only diagonal tiles pay for the mask; the
 //     heaviest query tiles are launched first.
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -769,6 +770,33 @@ size_t split_ws_bytes(int64_t tokens, int Hq, int Dv, int nsplit) {
   return nsplit > 1 ? (size_t)tokens * Hq * nsplit * ((Dv + 3) / 4 * 4 + 2) * sizeof(float) : 0;
 }
 
+// 64-row workgroups (half the chain of key tiles, RW = 2) or 128-row ones?  Counted in steps, one wave on one
+// key tile (about 0.95 us with D > 64, else 0.67 us): 128-row workgroups take the longest chain of key
+// tiles.  64-row ones take half of it, or a CU's share of the work where that is more, then half a step to merge,
+// and they wait for their turn.  With D > 64 a CU holds one of them (128 KB of LDS), and each further round puts
+// first loads that nothing hides, seven steps, in front of the chain; else it holds two, which hide most
+// of that and together take 1.5 times as long.  Host code knows the longest sequence only: the histories
+// of a batch count as half of the longest on average.
+// 64-row / 128-row us, D = 128: 32 heads x 512 tokens 11.2 / 13.8, 16 x 1536 22.0 / 28.4, 16 x 2560 49.3 / 46.7,
+// 8 x 4096 50.3 / 63.8, 8 heads x 8 x 300 15.4 / 10.7, 4 x 10 x 640 21.8 / 16.8; D = 64: 16 x 2048 19.5 / 26.6,
+// 32 x 1280 16.4 / 19.9, 8 x 8 x 300 8.5 / 7.8, 40 x 14 x 29 over up to 3355 60.2 / 88.0.  Over 1300 random batches of
+// up to 600 128-row workgroups the choice is 2 % above the better one on average ("up to 240 128-row workgroups":
+// 3 %), at worst 50 %, where all histories are long and equal.
+bool small_tiles(int Hq, int B, int D, int max_len, int64_t max_keys) {
+  if (D > 128) return false;
+  const double cus = current_device_cu_count();
+  const double rows = (double)ceil_div(max_len, 64), chain = (double)ceil_div(max_keys, kTileN);
+  const double history = chain > rows ? (chain - rows) * (B + 1) / (2.0 * B) : 0.0;
+  const double wgs = (double)Hq * B * rows, rounds = ceil(wgs / cus);
+  double share = 0.5 * rounds * history + 0.25 * (rows + 1.0) * wgs / cus, wait = 7.0 * (rounds - 1.0);
+  if (D <= 64) {
+    share /= 1.5;
+    wait = (rounds > 1.0 ? 1.0 : 0.0) + ceil(wgs / (2.0 * cus)) - 1.0;
+  }
+  const double half = ceil(0.5 * chain);
+  return chain > 2.0 && (share > half ? share : half) + 0.5 + wait < 0.95 * chain;
+}
+
 // Shared argument checks and launch of both entry points; the paged fields of `p` are already
 // filled in (or zeroed) by the caller.
 int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk, int Dv, int max_len,
@@ -800,8 +828,6 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.sm_scale = sm_scale;
 
   hipStream_t s = (hipStream_t)stream;
-  // 64-row workgroups where 128-row ones would leave CUs without any (of 256), unless there are so few
-  // keys that the merge costs more than it saves (40 heads, 4 x 49 tokens: 5.4 against 6.9 us)
   PackPlan plan = {0, 1, false};
   if (paged) plan = pack_plan(B, Hq, Hkv, D, max_len, max_keys, p.window);
   if (plan.nsplit > 1) {
@@ -816,7 +842,8 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.ws_d = (Dv + 3) / 4 * 4;
   p.ws_o = (float*)ws;
   p.ws_ml = p.ws_o ? p.ws_o + (size_t)p.tokens * Hq * p.nsplit * p.ws_d : nullptr;
-  const bool small = !plan.use && D <= 128 && Hq * ceil_div(max_len, 128) * B <= 240 && max_keys > 128;
+  const int64_t seen = p.window > 0 && (int64_t)p.window + max_len < max_keys ? (int64_t)p.window + max_len : max_keys;
+  const bool small = !plan.use && small_tiles(Hq, B, D, max_len, seen);
   const int64_t qtiles = ceil_div(max_len, small ? 64 : 128 >> p.pack_shift);
   if (qtiles > 65535 || (int64_t)B * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
   const int head_groups = Hq >> p.pack_shift;
