@@ -112,6 +112,13 @@ __device__ __forceinline__ int tiles_per_part(const TileRun& run, int nsplit) {
   return (tiles + parts - 1) / parts;
 }
 
+// ... and the most parts that a row tile of a sequence with kv_total keys has
+__device__ __forceinline__ int most_parts(int kv_total, const PrefillParams& p) {
+  int tiles = (kv_total + kTileN - 1) / kTileN;
+  if (p.window > 0 && p.window < kv_total) tiles = min(tiles, (p.window + (128 >> p.pack_shift)) / kTileN + 2);
+  return min(max(tiles / kPartTiles, 1), p.nsplit);
+}
+
 template <int D>
 struct Smem {
   static constexpr int kRowBytes = D * 2;           // K: [64][D], 16-byte chunks XOR-swizzled
@@ -160,27 +167,48 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   // the sequences are walked longest context first (blockIdx.z = rank, not index): the long
   // ones start in the first round and the short ones fill in behind them.  (The packed layout
   // has many workgroups per slot and gains nothing from the ranking: measured 1.5 % slower.)
-  // (PACK: the part is the slowest index, so that the parts that have keys start first and spread over the chip)
+  // Where key tiles are split, blockIdx.z counts the parts of one sequence after the other, in the same
+  // order; indexes past the last part have no work (the grid has room for nsplit parts of each).
   const int nb = PACK ? p.B : gridDim.z;
-  const int split = !PACK ? 0 : nb == 1 ? blockIdx.z : blockIdx.z / nb, rank_of = PACK ? blockIdx.z - split * nb : blockIdx.z;
-  int seq = rank_of;
+  const bool parts_too = PACK && p.nsplit > 1;
+  int seq = blockIdx.z, split = 0;
+  if (PACK && (nb == 1 || nb > kThreads)) {
+    split = nb == 1 ? seq : seq / nb;
+    seq -= split * nb;
+    if (nb == 1) seq = 0;
+  }
   if (PAGED && nb > 1 && nb <= kThreads) {
     __shared__ int32_t rank_key[kThreads];
-    __shared__ int32_t rank_seq;
+    __shared__ int32_t rank_parts[PACK ? kThreads : 1];
+    __shared__ int32_t rank_seq, rank_split;
     const int t = threadIdx.x;
     const int key = t < nb ? p.kv_len[t] : 0;
+    int parts = 1;
+    if (parts_too) {
+      parts = most_parts(key, p);
+      rank_parts[t] = parts;
+      if (t == 0) rank_seq = -1;
+    }
     rank_key[t] = key;
     __syncthreads();
     if (t < nb) {
-      int rank = 0;
+      int rank = 0;  // parts_too: in parts
       for (int j = 0; j < nb; ++j) {
         const int kj = rank_key[j];
-        rank += (kj > key || (kj == key && j < t)) ? 1 : 0;
+        rank += (kj > key || (kj == key && j < t)) ? (parts_too ? rank_parts[j] : 1) : 0;
       }
-      if (rank == rank_of) rank_seq = t;  // ranks are a permutation: exactly one writer
+      const int mine = (int)blockIdx.z - rank;
+      if (mine >= 0 && mine < parts) {  // exactly one writer, or none
+        rank_seq = t;
+        rank_split = mine;
+      }
     }
     __syncthreads();
     seq = __builtin_amdgcn_readfirstlane(rank_seq);
+    if (parts_too) {
+      if (seq < 0) return;
+      split = __builtin_amdgcn_readfirstlane(rank_split);
+    }
   }
   // (vector loads of wave-uniform values: saying that they are keeps loops and conditions scalar)
   const int L = __builtin_amdgcn_readfirstlane(p.seq_len[seq]);
