@@ -596,20 +596,21 @@ void launch_shape(const MoeGemmParams& p, int w_layout, hipStream_t s) {
 }
 
 // Workgroup shape.  Four waves side by side share most of their activations; where that leaves fewer
-// workgroups than two per CU (256 CUs), the waves of a workgroup split K instead, and there are
+// workgroups than two per CU, the waves of a workgroup split K instead, and there are
 // twice or four times as many: 16-bit, 8 experts of 4096 x 4096, 16 tokens, 184 -> 151 us; one
 // token 142 -> 57 us.  (64 experts, 2048 x 1408, 300 tokens: side by side 221 us, split 232 us.)
 // The fp8 gate_up GEMM always holds whole quantisation groups; its K split doubles the waves.
 template <bool GATED, int DT, int QT, int NT>
 void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
+  const int64_t cus = current_device_cu_count();
   constexpr int kCols4 = (GATED ? 8 : 16) * kWaveTiles * 4;
   const int64_t tiles = ceil_div(GATED ? p.I : p.N, kCols4) * (p.numel < p.num_local ? p.numel : p.num_local);
   if constexpr (GATED && QT != 1) {
-    if (NT == 1 && tiles < 128) launch_shape<GATED, DT, QT, 4, NT == 1 ? 2 : 1, NT>(p, w_layout, s);
+    if (NT == 1 && 2 * tiles < cus) launch_shape<GATED, DT, QT, 4, NT == 1 ? 2 : 1, NT>(p, w_layout, s);
     else launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
   } else {
     constexpr int CW = NT == 1 ? 1 : 2;
-    if (tiles >= 512) launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
+    if (tiles >= 2 * cus) launch_shape<GATED, DT, QT, 4, 1, NT>(p, w_layout, s);
     else launch_shape<GATED, DT, QT, CW, 4 / CW, NT>(p, w_layout, s);
   }
 }

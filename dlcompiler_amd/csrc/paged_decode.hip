@@ -599,11 +599,11 @@ int direct_waves(int B, int units, int max_ctx, int window, int D) {
   // (a window of any size up to 2^31 - 1 says "none" as well as -1 does)
   const bool windowed = window > 0 && window < max_ctx - 32;
   const int keys = windowed ? window + 32 : max_ctx;
-  const int64_t wgs = (int64_t)B * units;
+  const int64_t wgs = (int64_t)B * units, cus = current_device_cu_count();
   const bool few_keys = (int64_t)keys * D <= 700 * 128;
-  const bool busy = keys <= (windowed ? 2048 : 1024) && wgs >= (windowed ? 128 : 192);
+  const bool busy = keys <= (windowed ? 2048 : 1024) && wgs >= (windowed ? cus / 2 : 3 * cus / 4);
   if (!few_keys && !busy) return 0;
-  return D <= 64 && keys > 512 && wgs < 256 ? 8 : 4;
+  return D <= 64 && keys > 512 && wgs < cus ? 8 : 4;
 }
 
 // smallest piece a team may get, in 32-key units: 512 keys, less for small problems so that

@@ -765,12 +765,12 @@ namespace {
 
 // How a paged launch is cut.
 // Query runs that fill a fraction of 128 rows share a workgroup by heads of their KV group.  Where that
-// leaves few workgroups (up to 128, of 512 slots at two per CU) their key tiles are split, from 32
+// leaves few workgroups (up to half as many as CUs; the chip holds two per CU) their key tiles are split, from 32
 // tiles on, eight tiles per part at least; with more workgroups or fewer tiles the partial rows cost
 // more than the split saves (256 workgroups, 34 tiles: 43 us, split in two 49; 129 tiles: 156
 // against 110).  Where nothing is split, heads share a workgroup only while every CU still has one.
-// 32 heads (8 kv) of 128: 32 queries over 16000 keys 240 -> 38.6 us, 2 x 100 over 10000 156 -> 42.7,
-// 16 x 8 - 32 over up to 8000 174 -> 94.
+// 32 heads (8 kv) of 128, neither -> both: 32 queries over 16000 keys 254 -> 25.5 us, 2 x 100 over 10000
+// 166 -> 56, 16 x 8 - 32 over up to 8000 175 -> 95.
 struct PackPlan {
   int pack_shift, nsplit;
   bool use;
@@ -779,17 +779,18 @@ PackPlan pack_plan(int B, int Hq, int Hkv, int D, int max_len, int64_t max_keys,
   PackPlan plan = {0, 1, false};
   if (D > 128) return plan;
   const int group = Hq / Hkv;
+  const int64_t cus = current_device_cu_count();
   const int64_t reach = (int64_t)window + max_len;  // (windows of up to 2^31 - 1 come as "none")
   const int64_t seen = window > 0 && reach < max_keys ? reach : max_keys;
   const int64_t tiles = ceil_div(seen, kTileN);
   auto workgroups = [&](int shift) { return (int64_t)(Hq >> shift) * ceil_div(max_len, 128 >> shift) * B; };
   while (group % (2 << plan.pack_shift) == 0 && (int64_t)max_len << (plan.pack_shift + 1) <= 128 &&
-         (tiles >= 32 || workgroups(plan.pack_shift + 1) >= 256))
+         (tiles >= 32 || workgroups(plan.pack_shift + 1) >= cus))
     ++plan.pack_shift;
   const int64_t wgs = workgroups(plan.pack_shift);
-  if (wgs <= 128 ? tiles >= 32 : wgs <= 256 && tiles >= 96) {
+  if (2 * wgs <= cus ? tiles >= 32 : wgs <= cus && tiles >= 96) {
     const int64_t most = tiles / kPartTiles;
-    plan.nsplit = (int)(512 / wgs < most ? 512 / wgs : most);
+    plan.nsplit = (int)(2 * cus / wgs < most ? 2 * cus / wgs : most);
   }
   plan.use = plan.pack_shift > 0 || plan.nsplit > 1;
   return plan;

@@ -68,10 +68,10 @@ def paged_attention_fwd(
         assert q.dim() == 3 and o.dim() == 3
         (block_offsets, q_start_loc, q_seqlens, kv_seqlens), mask = _lib.index_arrays(
             block_offsets, q_start_loc.contiguous(), q_seqlens.contiguous(), kv_seqlens.contiguous())
-        ws_bytes = lib.dlb_paged_prefill_ws_bytes(q.size(0), batch, head, num_kv_heads, Lq, Lv, page, max_blocks,
-                                                  int(max_seqlen), int(window_size))
-        ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=q.device)
-        with _lib.device_guard(q.device):
+        with _lib.device_guard(q.device):   # (the plan follows the device's size)
+            ws_bytes = lib.dlb_paged_prefill_ws_bytes(q.size(0), batch, head, num_kv_heads, Lq, Lv, page, max_blocks,
+                                                      int(max_seqlen), int(window_size))
+            ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=q.device)
             st = lib.dlb_paged_prefill_attn_ws(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), block_offsets.data_ptr(),
                 q_start_loc.data_ptr(), q_seqlens.data_ptr(), kv_seqlens.data_ptr(), mask, batch, head,
