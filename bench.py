@@ -289,7 +289,7 @@ def wl_gating(dev, steps, warmup, cpu):
             "calls_per_graph": calls, "ms_per_call": ms_gpu, "value": bytes_ / ms_gpu / 1e6,
             "unit": "GB/s",
             "one_call_per_graph_ms": graph1_ms},
-        "roofline": {"kernel": "moe_topk_softmax_count_kernel + align_place_fused_kernel (the two "
+        "roofline": {"kernel": "route_count_kernel + route_place_kernel (the two "
                                "kernels of one call; GPU time per call from a graph of 20 calls)",
                      "bound": "hbm", "achieved": bytes_ / ms_gpu / 1e6, "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": bytes_ / ms_gpu / 1e6 / PEAK_HBM_GBS,
@@ -611,7 +611,7 @@ def wl_moe_bf16(dev, steps, warmup, cpu):
                                "reference's row-major [E, N, K] layout, seed 5",
                    "algorithmic_flops": flops},
         "weight_layouts": layouts,
-        "roofline": {"kernel": "moe_gemm_kernel<gate_up, bf16>", "bound": "mfma",
+        "roofline": {"kernel": "moe_stream_kernel<gate_up, bf16>", "bound": "mfma",
                      "achieved": gate_up_flops / ms_gate_up / 1e9, "peak": PEAK_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": gate_up_flops / ms_gate_up / 1e9 / PEAK_BF16_TFLOPS,
                      "traffic": _traffic("moe_gemm_bf16_gate_up")},

@@ -15,7 +15,7 @@
 // With many rows the matrix cores are the bound, and 16-bit operands stay here all the same: a 16-row
 // operand of row-major weights takes 16 cache lines per load, a 32-row one (which the tiled kernel
 // used for both types) 32, and the lines, not the bytes, limit the CU's load path.  64 experts,
-// 2048 x 1408, 4096 tokens: row-major 694 -> 623 us, operand order 504 -> 494; 768 tokens 277 -> 228.
+// 2048 x 1408, 4096 tokens: row-major 686 -> 611 us, operand order 508 -> 501; 768 tokens 277 -> 233.
 // (fp8 through this shape: products with a zero accumulator leave nothing to overlap the scaling
 // with, gate_up 201 against 171 us.)
 //
