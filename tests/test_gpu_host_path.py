@@ -65,6 +65,28 @@ def _prefill(idx):
     return call, (_r(75, 4, 64), _r(75, 2, 64), _r(75, 2, 64))
 
 
+def _moe(fp8, ids_type=torch.int64, aligned=False, shard=False, renorm=False, strided=False):
+    from dlcompiler_amd.kernels.fused_moe import ALIGN_BLOCK
+
+    T, H, I, E, k = 9, 256, 128, 4, 2
+    x = _r(T, 2 * H)[:, :H] if strided else _r(T, H)
+    weights, ids = torch.rand((T, k), device="cuda:0"), torch.randint(0, 8 if shard else E, (T, k), device="cuda:0")
+    ids = ids.to(ids_type)
+    experts = 8 if shard else None
+    alignment = None
+    if aligned:
+        slots, _, _, counts = d.moe_align_block_size(ids, ALIGN_BLOCK, experts or E, return_counts=True)
+        alignment = slots, counts
+    w1, w2 = _r(E, 2 * I, H) * 0.05, _r(E, H, I) * 0.05
+    if fp8:
+        quantised = [w.to(torch.float8_e4m3fn) for w in (w1, w2)]
+        s1, s2 = torch.rand((E, 2, 2), device="cuda:0"), torch.rand((E, 2, 1), device="cuda:0")
+        return (lambda x: d.fused_moe_fp8(x, quantised[0], s1, quantised[1], s2, weights, ids, k, 4 if shard else 0, experts,
+                                          renorm, alignment=alignment)), (x,)
+    return (lambda x: d.fused_moe(x, w1, w2, weights, ids, k, 4 if shard else 0, experts, renorm,
+                                  alignment=alignment)), (x,)
+
+
 CASES = {
     "silu": lambda: (d.silu_and_mul, (_r(3, 2 * 40),)),
     "silu_out": lambda: (d.silu_and_mul, (_r(3, 2 * 41, dtype=torch.float32), _r(3, 50, dtype=torch.float32)[:, :41])),
@@ -87,6 +109,14 @@ CASES = {
     "prefill_64": lambda: _prefill(torch.int64),
     "gate": lambda: (lambda x: d.moe_topk_softmax_align(x, 3, 16, return_counts=True), (_r(37, 12),)),
     "gate_one_token": lambda: (lambda x: d.moe_topk_softmax_align(x, 1, 128, 8, False), (_r(1, 8, dtype=torch.float32),)),
+    "moe": lambda: _moe(False),
+    "moe_aligned_renormalised": lambda: _moe(False, torch.int32, aligned=True, renorm=True),
+    "moe_shard": lambda: _moe(False, shard=True),
+    "moe_rows_strided": lambda: _moe(False, strided=True),   # copied by the general path
+    "moe_ids_16": lambda: _moe(False, torch.int16),          # converted by the general path
+    "moe_fp8": lambda: _moe(True),
+    "moe_fp8_aligned": lambda: _moe(True, torch.int32, aligned=True),
+    "moe_fp8_rows_strided_shard": lambda: _moe(True, shard=True, strided=True),
     "gate_columns_strided": lambda: (lambda x: d.moe_topk_softmax_align(x, 2, 64), (_r(12, 9).t(),)),
 }
 
