@@ -117,7 +117,7 @@ inline bool as_float(PyObject* o, double& v) {
   } else return false;
   return true;
 }
-// last dimension of unit stride (a dimension of one element counts whatever its stride says)
+// last dimension of unit stride (a dimension of one element may have another: the general path's to decide)
 inline bool unit_last(const at::Tensor& t) { return t.stride(-1) == 1; }
 
 // Other Python threads run while the launches are issued, as they do under ctypes.

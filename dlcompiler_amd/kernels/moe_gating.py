@@ -83,7 +83,8 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     * ``expert_ids[b]`` is the expert of block ``b`` (``-1`` past the padded total);
     * ``num_tokens_post_padded`` is a 1-element tensor; ``counts[e]`` the tokens of expert e.
 
-    Ids outside ``[0, num_experts)`` are dropped (experts held by another shard).
+    Ids outside ``[0, num_experts)`` are dropped (experts held by another shard).  The results are pieces
+    of one allocation, which is freed with the last of them.
     """
     _lib.require_cuda(topk_ids)
     if block_size < 1 or num_experts < 1:
@@ -121,7 +122,8 @@ def moe_topk_softmax_align(logits: torch.Tensor, k: int, block_size: int, num_ex
     native call of two launches (the router also produces the alignment's per-chunk expert
     counts).  Returns ``(weights, ids, sorted_token_ids, expert_ids, num_tokens_post_padded)``,
     bit for bit what the two functions return (plus the per-expert ``counts`` with
-    ``return_counts``).  More than 32768 tokens, no tokens at all, or ``num_experts``
+    ``return_counts``).  The results are pieces of one allocation, which is freed with the last of them;
+    clone one to resize it or to save it by itself.  More than 32768 tokens, no tokens at all, or ``num_experts``
     different from the router's expert count take the two separate calls.
     """
     if num_experts is None or num_experts == logits.shape[-1]:
