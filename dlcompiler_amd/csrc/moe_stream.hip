@@ -5,8 +5,8 @@
 // moe_fp8.hip (128 x 256 tiles, one barrier per chunk, two workgroups of four waves per CU) reads
 // them at 4.3 - 5.2 TB/s.  Here a wave owns 64 weight rows and every KW-th 128-byte chunk of them,
 // loads the weights straight into MFMA operands, two chunks ahead, and 8 - 16 waves per CU keep
-// 96 - 192 KB on their way: 5.3 - 6.2 TB/s (64 experts of 2048 x 1408 bf16, 300 tokens: layer
-// 265 -> 221 us; fp8, 32 tokens: 113 -> 101 us, 128 tokens 118 -> 109 us).
+// 96 - 192 KB on their way: 5.5 - 6.2 TB/s (64 experts of 2048 x 1408 bf16, 300 tokens: layer
+// 273 -> 214 us; fp8, 32 tokens: 113 -> 101 us, 128 tokens 118 -> 109 us).
 //
 // Activations: up to 16 rows they go straight into operands too.  With more rows they would pass
 // through the CU once per wave, as many bytes as the weights (300 tokens: 255 us); there each thread
@@ -598,7 +598,7 @@ void launch_shape(const MoeGemmParams& p, int w_layout, hipStream_t s) {
 // Workgroup shape.  Four waves side by side share most of their activations; where that leaves fewer
 // workgroups than two per CU, the waves of a workgroup split K instead, and there are
 // twice or four times as many: 16-bit, 8 experts of 4096 x 4096, 16 tokens, 184 -> 151 us; one
-// token 142 -> 57 us.  (64 experts, 2048 x 1408, 300 tokens: side by side 221 us, split 232 us.)
+// token 142 -> 57 us.  (64 experts, 2048 x 1408, 300 tokens: side by side 214 us, split 226 us.)
 // The fp8 gate_up GEMM always holds whole quantisation groups; its K split doubles the waves.
 template <bool GATED, int DT, int QT, int NT>
 void launch_nt(const MoeGemmParams& p, int w_layout, hipStream_t s) {
