@@ -490,12 +490,17 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
 #pragma unroll
       for (int i = 0; i < 16; ++i) top = fmaxf(top, fmaxf(fabsf(s[0][i]), fabsf(s[1][i])));
       // Mostly none of the wave's scores comes near the cap, and the polynomial is all there is: 8 x 512
-      // tokens over 4096, 645 -> 506 us; where some do in every tile the look costs 3 %.
+      // tokens over 4096, 645 -> 497 us; where some do in every tile the look costs nothing (646).
       if (__any(top * to_arg >= kSoftcapSmall)) {
+        // (a factor of its own: with the same one in both branches the compiler moves the polynomial in front
+        // of them, 32 more registers live, and calls of 64 dims without a cap lost a third of their waves:
+        // 64 heads, 8 x 66 - 134 tokens over 48, 14.9 us instead of 13.7)
+        float arg = to_arg;
+        asm volatile("" : "+v"(arg));
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[nt][i] = softcap_tanh(s[nt][i] * to_arg) * to_score;
+          for (int i = 0; i < 16; ++i) s[nt][i] = softcap_tanh(s[nt][i] * arg) * to_score;
       } else {
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt)

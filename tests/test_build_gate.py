@@ -31,6 +31,13 @@ def test_every_kernel_with_hand_issued_loads_is_named():
             assert set(re.findall(r"void (\w+_kernel)\(", text)) - ordinary <= set(KERNELS), src.name
 
 
+def test_short_head_dims_keep_their_waves():
+    """128-row prefill workgroups of 64 dims: three per CU, so 512 / 3 registers in steps of 8."""
+    reports = [r for name, r in kernel_resources().items()
+               if re.search(r"prefill_attn_kernelILi\dELi64ELi\dELb\dELi4E", name)]
+    assert reports and all(r["occupancy"] >= 3 and r["vgprs"] <= 168 for r in reports)
+
+
 def test_the_build_reports_every_gated_kernel():
     built = kernel_resources()
     for kernel in KERNELS:
