@@ -823,6 +823,7 @@ bool small_tiles(int Hq, int B, int D, int max_len, int64_t max_keys, int64_t to
   const double history = chain > rows ? (chain - rows) * (0.4 + 0.6 * B) / B : 0.0;
   double tiles = B * rows;  // row tiles of 64
   if (tokens > 0 && tokens / 64.0 + 0.7 * B < tiles) tiles = tokens / 64.0 + 0.7 * B;
+  if (tiles < B) tiles = B;  // (32 heads, 9 x up to 14 tokens over 151, D = 128: 64-row 14.0 us, 128-row 9.1)
   const double wgs = Hq * tiles, rounds = ceil(wgs / cus);
   double share = 0.5 * rounds * history + 0.25 * (rows + 1.0) * wgs / cus, wait = 7.0 * (rounds - 1.0);
   if (D <= 64) {
