@@ -809,13 +809,13 @@ size_t split_ws_bytes(int64_t tokens, int Hq, int Dv, int nsplit) {
 // tiles.  64-row ones take half of it, or a CU's share of the work where that is more, then half a step to merge,
 // and they wait for their turn.  With D > 64 a CU holds one of them (128 KB of LDS), and each further round puts
 // first loads that nothing hides, seven steps, in front of the chain; else it holds two, which hide most
-// of that and together take 1.5 times as long.  Host code knows the longest sequence and, if the caller
+// of that and together take 1.7 times as long.  Host code knows the longest sequence and, if the caller
 // says so, the tokens of all: a batch's other histories count as 0.6 of the longest.
 // 64-row / 128-row us, D = 128: 32 heads x 512 tokens 11.2 / 13.8, 16 x 1536 22.0 / 28.4, 16 x 2560 49.3 / 46.7,
 // 8 x 4096 50.3 / 63.8, 8 heads x 8 x 300 15.4 / 10.7, 4 x 10 x 640 21.8 / 16.8; D = 64: 16 x 2048 19.5 / 26.6,
-// 32 x 1280 16.4 / 19.9, 8 x 8 x 300 8.5 / 7.8, 40 x 14 x 29 over up to 3355 60.2 / 88.0.  Over 2300 random batches of
-// up to 600 128-row workgroups the choice is 1.3 % above the better one on average ("up to 240 128-row workgroups":
-// 2.7 %), at worst 50 %, where all histories are long and equal.
+// 32 x 1280 16.4 / 19.9, 8 x 8 x 300 8.5 / 7.8, paged 32 x 6 x up to 478 17.6 / 14.9, 40 x 14 x 29 over up to 3355
+// 33.8 / 46.4.  Over 1100 random batches of up to 2000 128-row workgroups the choice is 0.8 % above the better one on
+// average ("up to 240 128-row workgroups": 2.0 %), at worst 32 % (50 % has been seen), where all histories are long and equal.
 bool small_tiles(int Hq, int B, int D, int max_len, int64_t max_keys, int64_t tokens) {
   if (D > 128) return false;
   const double cus = current_device_cu_count();
@@ -827,7 +827,7 @@ bool small_tiles(int Hq, int B, int D, int max_len, int64_t max_keys, int64_t to
   const double wgs = Hq * tiles, rounds = ceil(wgs / cus);
   double share = 0.5 * rounds * history + 0.25 * (rows + 1.0) * wgs / cus, wait = 7.0 * (rounds - 1.0);
   if (D <= 64) {
-    share /= 1.5;
+    share /= 1.2;
     wait = (rounds > 1.0 ? 1.0 : 0.0) + ceil(wgs / (2.0 * cus)) - 1.0;
   }
   const double half = ceil(0.5 * chain);
