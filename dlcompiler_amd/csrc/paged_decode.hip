@@ -669,12 +669,14 @@ bool read_once(int B, int Hkv, int dims, int max_ctx, int window) {
 // the chip still sees a few thousand wavefronts.  64 keys, two steps of a wavefront, where that leaves each CU
 // at most four of them and a head at most 64 partials (128 / 64 keys: 8 kv heads of 128, 1 x 2000 11.1 / 9.4 us,
 // 8 x 2000 18.2 / 19.1, 1 x 8000 14.5 / 17.1; of 64, 1 x 4000 11.3 / 9.7).
-int pick_min_units(int B, int Hkv, int hchunks, int max_ctx) {
+// 64-key pieces need twice the scratch; a call that brings less, say what a larger batch or a wider table with its
+// longer pieces needs, gets 128-key ones.
+int pick_min_units(int B, int Hkv, int hchunks, int max_ctx, bool short_pieces) {
   const int64_t units = (int64_t)B * Hkv * hchunks;
   auto pieces = [&](int keys) { return ((int64_t)max_ctx + keys - 1) / keys; };
   int kps = 512;
   while (kps > 128 && units * pieces(kps) < 4096) kps >>= 1;
-  if (kps == 128 && pieces(64) <= 64 && units * pieces(64) <= 4 * (int64_t)current_device_cu_count()) kps = 64;
+  if (short_pieces && kps == 128 && pieces(64) <= 64 && units * pieces(64) <= 4 * (int64_t)current_device_cu_count()) kps = 64;
   return kps / 32;
 }
 
@@ -683,6 +685,10 @@ int pick_min_units(int B, int Hkv, int hchunks, int max_ctx) {
 int partial_slots(int max_ctx, int min_units) {
   const int t = (max_ctx + 31) / 32;
   return t / min_units + 2;
+}
+
+size_t scratch_bytes(int B, int Hq, int D, int max_ctx, int min_units) {
+  return (size_t)B * Hq * partial_slots(max_ctx, min_units) * (D + 2) * sizeof(float) + (size_t)B * sizeof(int32_t);
 }
 
 // teams that are resident together: wavefronts per CU (2 per SIMD, 1 in the masked variant) /
@@ -709,8 +715,7 @@ extern "C" size_t dlb_paged_decode_ws_bytes(int B, int Hq, int Hkv, int D, int p
   const int hchunks = (group + 15) / 16;
   const int64_t max_ctx = (int64_t)page * max_blocks;
   if (max_ctx > 0x7fffffff) return 0;
-  const int64_t ns = dlb::partial_slots((int)max_ctx, dlb::pick_min_units(B, Hkv, hchunks, (int)max_ctx));
-  return (size_t)B * Hq * ns * (D + 2) * sizeof(float) + (size_t)B * sizeof(int32_t);
+  return dlb::scratch_bytes(B, Hq, D, (int)max_ctx, dlb::pick_min_units(B, Hkv, hchunks, (int)max_ctx, true));
 }
 
 extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const void* v_cache,
@@ -743,10 +748,15 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
                              k_stride_head, v_stride_page, v_stride_tok,  v_stride_head};
   for (int64_t sd : strides)
     if (sd % 8 != 0) return DLB_ERR_UNSUPPORTED;
-  const size_t need = dlb_paged_decode_ws_bytes(B, Hq, Hkv, Dp, page, max_blocks);
-  if (!ws || ws_bytes < need) return DLB_ERR_WORKSPACE;
-
+  const int max_ctx = page * max_blocks;
   DecodeParams p;
+  p.group = Hq / Hkv;
+  p.hchunks = (p.group + 15) / 16;
+  p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, true);
+  if (ws_bytes < scratch_bytes(B, Hq, Dp, max_ctx, p.min_units))
+    p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, false);
+  if (!ws || ws_bytes < scratch_bytes(B, Hq, Dp, max_ctx, p.min_units)) return DLB_ERR_WORKSPACE;
+  p.nsplit_max = partial_slots(max_ctx, p.min_units);
   p.q = q;
   p.k = k_cache;
   p.v = v_cache;
@@ -768,16 +778,11 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
   p.B = B;
   p.Hq = Hq;
   p.Hkv = Hkv;
-  p.group = Hq / Hkv;
-  p.hchunks = (p.group + 15) / 16;
   p.page = page;
   p.page_shift = -1;
   for (int sh = 0; sh < 31; ++sh)
     if ((1 << sh) == page) p.page_shift = sh;
   p.max_blocks = max_blocks;
-  const int max_ctx = page * max_blocks;
-  p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx);
-  p.nsplit_max = partial_slots(max_ctx, p.min_units);
   p.scale_log2e = sm_scale * 1.4426950408889634f;
   p.sm_scale = sm_scale;
   p.window = window_size;

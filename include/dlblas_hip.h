@@ -181,7 +181,10 @@ int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights, int32_t* 
  * 256 with the extra dims masked, as the reference splits them into power-of-two blocks,
  * kernels/paged_attention.py:531-539; sizes above 128 run one wavefront per SIMD), page % 16 == 0, all strides multiples of 8 and base
  * pointers 16-byte aligned.  ws: dlb_paged_decode_ws_bytes(B, Hq, Hkv, max(D, Dv), page,
- * max_blocks) bytes of device scratch (split-KV partials), caller-owned.
+ * max_blocks) bytes of device scratch (split-KV partials), caller-owned.  The size is that of this call and does not
+ * grow with B and max_blocks throughout: a scratch for several calls is the largest of theirs.  (Few sequences also take
+ * what their split into pieces of 128 keys needs: B Hq (max_blocks page / 128 + 3) (D + 2) 4 + 4 B bytes are enough, with
+ * D rounded up to 64, 96, 128 or 256.)
  * ---------------------------------------------------------------------------------------- */
 size_t dlb_paged_decode_ws_bytes(int B, int Hq, int Hkv, int D, int page, int max_blocks);
 int dlb_paged_decode_attn(const void* q, const void* k_cache, const void* v_cache, void* o,
