@@ -148,6 +148,10 @@ struct DecodeSegment {
   // Addressing: a 16-key sub-tile never straddles a page (page % 16 == 0), so its physical
   // page comes from ONE wave-uniform block-table entry (a scalar load) and every lane adds a
   // 32-bit byte offset to a uniform 64-bit base.
+  // (uniform_ptr loses that a pointer is global, and a wait for LDS waits for every flat load in flight, here the half
+  // tile just asked for.  Flat / so, 8 kv heads of 128, contexts much shorter than the table: 1 x 4000 keys 26.9 / 23.3
+  // us, 8 x 500 - 8000 31.4 / 27.2; filling it, 64 x 512 - 8192 161.4 / 161.7, of 64 97.5 / 96.6)
+  typedef const __attribute__((address_space(1))) u32x4* gvec_t;
   const unsigned char* kbytes = (const unsigned char*)p.k + (int64_t)kvh * p.k_sh * 2;
   const unsigned char* vbytes = (const unsigned char*)p.v + (int64_t)kvh * p.v_sh * 2;
   const uint32_t k_tok_bytes = (uint32_t)p.k_st * 2u, v_tok_bytes = (uint32_t)p.v_st * 2u;
@@ -209,7 +213,7 @@ struct DecodeSegment {
             const unsigned char* from = uniform_ptr(base + (int64_t)((base_key & ~15) - page_key0 + 2 * pair) * k_tok_bytes);
 #pragma unroll
             for (int ln = 0; ln < KS / 2; ++ln)
-              f.kf[sub][KS / 2 * pair + ln] = __builtin_nontemporal_load((const u32x4*)(from + kl_off + 128 * ln));
+              f.kf[sub][KS / 2 * pair + ln] = __builtin_nontemporal_load((gvec_t)(from + kl_off + 128 * ln));
           }
         } else {
           // K rows are read as two half-line (64-byte) pieces by consecutive k-steps: keep them

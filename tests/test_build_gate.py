@@ -1,9 +1,11 @@
 """The build stops when a kernel that issues its loads by hand spills or uses scratch memory (no GPU)."""
 import re
+import subprocess
+from pathlib import Path
 
 import pytest
 
-from dlcompiler_amd.build import CSRC_DIR, check_hand_scheduled, kernel_resources
+from dlcompiler_amd.build import ARCH, CSRC_DIR, HIPCC, OBJ_DIR, check_hand_scheduled, kernel_resources
 
 # kernels that run the helpers of inline-assembly loads, or the key walk of the paged decode kernels, which
 # looks pages up with hand-issued scalar loads
@@ -51,3 +53,18 @@ def test_no_instance_that_no_dispatch_reaches():
                                    for name in kernel_resources()) if m}
     assert shapes == {("4", "1", "1"), ("4", "2", "1"), ("1", "4", "1"), ("4", "1", "2"), ("2", "2", "2"),
                       ("4", "1", "4"), ("2", "2", "4"), ("4", "1", "8")}
+
+
+@pytest.mark.parametrize("source", ["moe_fp8", "moe_stream", "paged_decode", "prefill_attn"])
+def test_pipelined_loads_are_global(source, tmp_path):
+    """A flat load counts as an LDS operation too: the next wait for LDS waits for every load in flight."""
+    tools = Path(HIPCC).resolve().parent.parent / "llvm" / "bin"
+    fat, code = tmp_path / "fat", tmp_path / "code"
+    subprocess.run([tools / "llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", OBJ_DIR / f"{source}.o",
+                    tmp_path / "unused"], check=True)
+    subprocess.run([tools / "clang-offload-bundler", "--unbundle", "--type=o", f"--input={fat}", f"--output={code}",
+                    f"--targets=hipv4-amdgcn-amd-amdhsa--{ARCH}"], check=True)
+    text = subprocess.run([tools / "llvm-objdump", "-d", code], check=True, capture_output=True, text=True).stdout
+    assert "global_load" in text or "buffer_load" in text
+    flat = {block.split(">", 1)[0] for block in re.split(r"^[0-9a-f]+ <", text, flags=re.M) if "flat_load" in block}
+    assert not flat, flat
