@@ -49,6 +49,7 @@ struct DecodeParams {
   int max_blocks;
   int min_units, nsplit_max;  // smallest piece (32-key units); partial slots per (sequence, head)
   int num_teams;
+  int once_units;  // K and V of more units than this go past the caches (CHOICE)
   float scale_log2e;
   float sm_scale;
   int dk, dv;      // real key / value head sizes (<= the padded size the kernel is built for)
@@ -96,7 +97,7 @@ constexpr int kVtRowBytes = 144;   // 64 keys * 2 B + 16 B pad
 // power-of-two blocks with masked loads (python/dlBLAS/dlblas/kernels/paged_attention.py:531-539).
 // (The masked variant keeps a few more per-lane offsets alive: it is built for one wavefront per
 // SIMD instead of two rather than spilling them.)
-// ONCE: K and V go past the caches (see read_once); without it, V alone.
+// ONCE: K and V go past the caches (see may_read_once); without it, V alone.
 template <int DT, int D, bool POW2, bool RAGGED, bool ONCE>
 struct DecodeSegment {
   static constexpr int KS = D / 32;  // MFMA k-steps over the head dim
@@ -130,6 +131,10 @@ struct DecodeSegment {
   kv_min = __builtin_amdgcn_readfirstlane(kv_min);
   const int32_t* bt = p.block_table.p + (((int64_t)b * p.bt_stride) << p.block_table.sh);
   const int bt_sh = p.block_table.sh;
+  // (what the loops use: arguments that are loaded again, see arguments_again, would be loaded in every step)
+  const int page = p.page, page_shift = p.page_shift;
+  const int64_t k_sp = p.k_sp, v_sp = p.v_sp;
+  const float softcap = p.softcap, sm_scale = p.sm_scale, scale_log2e = p.scale_log2e;
 
   // Q^T as the B operand: lane (n = query head c, k = dims 32*ks + 8g .. +8)
   u32x4 qf[KS];
@@ -184,7 +189,7 @@ struct DecodeSegment {
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int base_key = min(h0 + 16 * sub, ctx - 1);  // clamp: never look past the context
-      const int pi = POW2 ? (base_key >> p.page_shift) : (base_key / p.page);
+      const int pi = POW2 ? (base_key >> page_shift) : (base_key / page);
       entry[sub] = (const int32_t*)uniform_ptr((const unsigned char*)(bt + (pi << bt_sh)));
     }
     int p0, p1;
@@ -200,11 +205,11 @@ struct DecodeSegment {
     for (int sub = 0; sub < 2; ++sub) {
       const int base_key = min(h0 + 16 * sub, ctx - 1);  // uniform; clamp: never read past ctx
       const int pi =
-          __builtin_amdgcn_readfirstlane(POW2 ? (base_key >> p.page_shift) : (base_key / p.page));
+          __builtin_amdgcn_readfirstlane(POW2 ? (base_key >> page_shift) : (base_key / page));
       const int64_t pg = (int64_t)pg_now[sub];
-      const int page_key0 = pi * p.page;
+      const int page_key0 = pi * page;
       {
-        const unsigned char* base = kbytes + pg * p.k_sp * 2;
+        const unsigned char* base = kbytes + pg * k_sp * 2;
         if constexpr (KL) {
           // Operand row c = 2 k + half: half line of key 4 (k / 2) + 2 pair + k % 2 of the sub-tile that holds
           // base_key.  (Its keys past the context are slots of the same page, and masked.)
@@ -222,13 +227,12 @@ struct DecodeSegment {
           const uint32_t off = (uint32_t)(key - page_key0) * k_tok_bytes;
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) {
-            if (RAGGED) f.kf[sub][ks] = *(const u32x4*)(base + off + kdim_off[ks]);
-            else f.kf[sub][ks] = *(const u32x4*)(base + off + 16u * g + 64 * ks);
+            f.kf[sub][ks] = *(gvec_t)(base + off + (RAGGED ? kdim_off[ks] : 16u * g + 64 * ks));
           }
         }
       }
       {
-        const unsigned char* base = vbytes + pg * p.v_sp * 2;
+        const unsigned char* base = vbytes + pg * v_sp * 2;
 #pragma unroll
         for (int ps = 0; ps < VPASS; ++ps) {
           const int key0 = min(h0 + 16 * sub + 4 * (ps * VL + kgl), ctx - 1);
@@ -310,17 +314,17 @@ struct DecodeSegment {
 
     // ---- online softmax over these 32 keys (log2 domain) ----
     float mloc = -__builtin_inff();
-    if (p.softcap > 0.0f) {  // one uniform branch for the half tile, not one per element
+    if (softcap > 0.0f) {  // one uniform branch for the half tile, not one per element
 #pragma unroll
       for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          s[sub][i] = p.softcap * softcap_tanh(s[sub][i] * p.sm_scale / p.softcap) * 1.4426950408889634f;
+          s[sub][i] = softcap * softcap_tanh(s[sub][i] * sm_scale / softcap) * 1.4426950408889634f;
     } else {
 #pragma unroll
       for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[sub][i] *= p.scale_log2e;
+        for (int i = 0; i < 4; ++i) s[sub][i] *= scale_log2e;
     }
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
@@ -411,12 +415,23 @@ __device__ __forceinline__ int first_visible(const DecodeParams& p, int ctx) {
   return p.window > 0 ? max(ctx - 1 - p.window, 0) : 0;
 }
 
-template <int DT, int D, bool POW2, bool RAGGED, bool ONCE>
+// The kernel's arguments, to be loaded where they are used.  (For two walks of which one runs: what both need, kept
+// from before the branch, is more than the scalar registers, and those that spill go to lanes of vector registers that
+// are not there.)
+__device__ __forceinline__ const DecodeParams& arguments_again() {
+  typedef const __attribute__((address_space(4))) DecodeParams* args_t;
+  args_t args = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return *(const DecodeParams*)args;
+}
+
+// CHOICE: whether K and V go past the caches follows from the keys of the batch (see may_read_once).
+template <int DT, int D, bool POW2, bool RAGGED, bool CHOICE>
 __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(const DecodeParams p) {
   // grid: x = (kv head, head chunk) unit, y = team.  The unit is the fastest index, so the
   // wavefronts that start together read the 256-byte head slices of the SAME token rows at the
   // same time: whole 2 KB cache rows are in flight together and DRAM pages are hit while open.
-  using Segment = DecodeSegment<DT, D, POW2, RAGGED, ONCE>;
+  constexpr int kVtBytes = DecodeSegment<DT, D, POW2, RAGGED, false>::kVtBytes;
   const int unit = blockIdx.x;
   const int team = blockIdx.y;
   const int kvh = unit / p.hchunks;
@@ -424,7 +439,7 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
 
-  __shared__ __attribute__((aligned(16))) unsigned char vt[Segment::kVtBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char vt[kVtBytes];
   __shared__ int32_t seg_lds[3][64];  // (first unit, units, context) of the 64 sequences being walked
 
   const int hq_local = hchunk * 16 + c;
@@ -452,6 +467,8 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   const int hi = min(lo + upt, total);
 
   // ---- walk the sequences this piece overlaps ----
+  auto walk = [&](const DecodeParams& p, auto once) __attribute__((always_inline)) {
+  using Segment = DecodeSegment<DT, D, POW2, RAGGED, decltype(once)::value>;
   int carry = 0;  // units of all sequences before b0
   for (int b0 = 0; b0 < p.B; b0 += 64) {
     const int ctx_mine = context_of(b0 + lane);
@@ -491,6 +508,13 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
       }
     }
     if (carry >= hi) break;
+  }
+  };  // walk
+  if constexpr (CHOICE) {
+    if (total > p.once_units) walk(arguments_again(), std::true_type{});
+    else walk(arguments_again(), std::false_type{});
+  } else {
+    walk(p, std::false_type{});
   }
 }
 
@@ -659,15 +683,18 @@ int direct_waves(int B, int units, int max_ctx, int window, int D) {
   return D <= 64 && keys > 512 && wgs < cus ? 8 : 4;
 }
 
-// Do K and V go past the caches?  If the batch has room for more than the 256 MB behind the L2s: what a step
-// leaves there is of no use to the next one, or to the next layer.  As K lines come whole then, the stream is
-// faster (8 kv heads of 128, kept / past: 64 x 512 - 8192 keys 169.5 -> 161.5 us, 8 x 8000 (250 MB) 53.1 / 50.8,
-// 16 x 500 - 8000 48.1 / 45.9; of 64: 64 x 512 - 8192 101.5 / 94).  Smaller batches, timed behind each other, find
-// part of their keys there (8 x 500 - 8000 27.4 / 29.3, 1 x 4000 11.2 / 12.7).
-bool read_once(int B, int Hkv, int dims, int max_ctx, int window) {
+// Do K and V go past the caches, K in whole lines?  A table without room for more than the 256 MB behind the L2s keeps
+// them.  In a larger one it goes by the keys that the contexts have, which the kernel counts anyway: from half of that
+// on.  Kept / past, 8 kv heads of 128, each step on other caches, as the layers of a model are: 8 x 1500 keys 22.7 /
+// 24.8 us, 8 x 500 - 8000 (111 MB) 27.4 / 27.2, 32 x 500 - 2000 (145 MB) 37.4 / 34.9, 16 x 500 - 8000 48.2 / 45.9,
+// 64 x 512 - 8192 169.0 / 160.7.  On the same keys over and over, which the caches then partly hold, 111 MB 25.1 / 26.5,
+// 145 MB 33.2 / 33.3, 215 MB 44.3 / 45.4, and 256 x 100 - 300 52.3 / 57.5 (on others 63.2 / 58.5).
+constexpr int64_t kCacheBytes = (int64_t)256 << 20;
+bool may_read_once(int B, int Hkv, int dims, int max_ctx, int window) {
   const int64_t keys = window > 0 && window < max_ctx ? window : max_ctx;
-  return (int64_t)B * keys * Hkv * dims * 2 > ((int64_t)256 << 20);
+  return (int64_t)B * keys * Hkv * dims * 2 > kCacheBytes;
 }
+int once_units(int Hkv, int dims) { return (int)(kCacheBytes / 2 / ((int64_t)32 * Hkv * dims * 2)); }
 
 // Smallest piece a team may get, in 32-key units: 512 keys, less for small problems so that
 // the chip still sees a few thousand wavefronts.  64 keys, two steps of a wavefront, where that leaves each CU
@@ -804,14 +831,15 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
   const dim3 grid1((uint32_t)units, (uint32_t)p.num_teams);
   const dim3 grid2((uint32_t)Hq, (uint32_t)B), grid_direct((uint32_t)units, (uint32_t)B);
   const int direct = direct_waves(B, units, max_ctx, window_size, Dp);
-  const bool once = read_once(B, Hkv, D + Dv, max_ctx, window_size);
+  p.once_units = once_units(Hkv, D + Dv);
+  const bool choice = may_read_once(B, Hkv, D + Dv, max_ctx, window_size);
 #define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_)                                                                       \
   do {                                                                                                            \
     if (direct == 4)                                                                                              \
       hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, D_, P2_, RG_, 4>), grid_direct, dim3(256), 0, s, p);    \
     else if (D_ == 64 && direct == 8)                                                                             \
       hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, 64, P2_, RG_, 8>), grid_direct, dim3(512), 0, s, p);    \
-    else if (D_ % 64 == 0 && !RG_ && once)                                                                        \
+    else if (D_ % 64 == 0 && !RG_ && choice)                                                                        \
       hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, D_ % 64 == 0 && !RG_>), grid1, dim3(64), 0, s, p); \
     else                                                                                                          \
       hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false>), grid1, dim3(64), 0, s, p);        \
