@@ -20,11 +20,14 @@ __device__ __forceinline__ unsigned int pack4_fp8(float a, float b, float c, flo
 }
 
 // f / scale, rounded as the division rounds (Markstein: one residual step from the rounded reciprocal), for
-// |f| <= 448 scale, up to a rounding.  `by` is the scale, 0 if that is infinite: 0 for a finite f then, else NaN.
-// (The residual of -0 is +0, and so would be the sum.)
-__device__ __forceinline__ float divide_by_scale(float f, float by, float inv) {
+// |f| <= 448 scale, up to a rounding, and a finite scale; +0 for -0, whose residual is +0 as the sum then is.
+__device__ __forceinline__ float finite_quotient(float f, float scale, float inv) {
   const float q = f * inv;
-  return __builtin_copysignf(fmaf(fmaf(-q, by, f), inv, q), f);
+  return fmaf(fmaf(-q, scale, f), inv, q);
+}
+// ... with the sign of a zero, and `by` for the scale, 0 if that is infinite: 0 for a finite f then, else NaN.
+__device__ __forceinline__ float divide_by_scale(float f, float by, float inv) {
+  return __builtin_copysignf(finite_quotient(f, by, inv), f);
 }
 
 constexpr int kQuantThreads = 256;
