@@ -520,7 +520,7 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
 
 // Combine the partials of one (sequence, head): O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s
 // (paged_attention.py:238-285 with the exponent in base 2).  A row of D floats is read by D / 4 lanes
-// and the rows are spread over the workgroup, so up to 8 - 16 rows are in flight per round; the
+// and the rows are spread over the workgroup, which asks for 64 of them at once (D = 256: 32); the
 // kernel is a chain of memory latencies, so what does not depend on the number of partials (the
 // first 64 (m, l) pairs and the first round of rows: inside the scratch whether written or not,
 // and masked) is requested together with it.
@@ -572,7 +572,8 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(c
     const int n = min(64, ns - s0);
     // All 64 rows' loads at once (D <= 128), without a condition: rows past the last are the last one again and
     // count nothing.  Behind a branch each load was waited for before the next (8 kv heads of 128, 1 x 4000 keys,
-    // 32 - 63 partials: 11.6 -> 10.6 us; 1 x 32000, 250 partials: 36.0 -> 31.4).
+    // 32 - 63 partials: 11.6 -> 10.6 us; 1 x 32000, 250 partials: 36.0 -> 31.4).  Rows asked for twice cost nothing:
+    // with as many loads as D needs, four at 64, and v0 not asked for again 1 x 4000 keys of 64 took 8.6 us, so 8.5.
     constexpr int U = 8;
     if (row_lane) {
       for (int r0 = rg; r0 < n; r0 += U * RG) {
@@ -698,7 +699,7 @@ int once_units(int Hkv, int dims) { return (int)(kCacheBytes / 2 / ((int64_t)32 
 
 // Smallest piece a team may get, in 32-key units: 512 keys, less for small problems so that
 // the chip still sees a few thousand wavefronts.  64 keys, two steps of a wavefront, where that leaves each CU
-// at most four of them and a head at most 64 partials (128 / 64 keys: 8 kv heads of 128, 1 x 2000 11.1 / 9.4 us,
+// at most four of them and a head at most 64 partials, or 65 where pieces cross sequences (128 / 64 keys: 8 kv heads of 128, 1 x 2000 11.1 / 9.4 us,
 // 8 x 2000 18.2 / 19.1, 1 x 8000 14.5 / 17.1; of 64, 1 x 4000 11.3 / 9.7).
 // 64-key pieces need twice the scratch; a call that brings less, say what a larger batch or a wider table with its
 // longer pieces needs, gets 128-key ones.
