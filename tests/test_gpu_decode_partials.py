@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 # 64-key pieces up to 4096 keys of room and four wavefronts per CU, else 128: 1 .. 160 partials
-@pytest.mark.parametrize("lens", [[1100], [4095], [4096], [4033, 3], [8191], [8193], [20300], [64, 2300, 1, 700]])
+@pytest.mark.parametrize("lens", [[1100], [4095], [4096], [4033, 3], [3, 4096], [8191], [8193], [20300], [64, 2300, 1, 700]])
 @pytest.mark.parametrize("hq,hkv,d", [(4, 1, 128), (8, 4, 64), (2, 2, 96), (4, 2, 80), (2, 1, 256)])
 @pytest.mark.parametrize("window", [None, 900])
 def test_partials(dev, lens, hq, hkv, d, window):
