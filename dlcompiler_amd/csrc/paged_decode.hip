@@ -672,12 +672,12 @@ __global__ __launch_bounds__(64 * W, RAGGED ? 1 : 2) void paged_decode_direct_ke
 // What a sliding window leaves is about the same for every sequence.
 // Eight wavefronts pay where the rows are short and a few CUs read many keys (1000 keys of 64 dims,
 // one sequence: 9.2 us, with four 10.7).
-int direct_waves(int B, int units, int max_ctx, int window, int D) {
+int direct_waves(int B, int units, int max_ctx, int window, int D, int64_t cus) {
   if (D > 128) return 0;
   // (a window of any size up to 2^31 - 1 says "none" as well as -1 does)
   const bool windowed = window > 0 && window < max_ctx - 32;
   const int keys = windowed ? window + 32 : max_ctx;
-  const int64_t wgs = (int64_t)B * units, cus = current_device_cu_count();
+  const int64_t wgs = (int64_t)B * units;
   const bool few_keys = (int64_t)keys * D <= 700 * 128;
   const bool busy = keys <= (windowed ? 2048 : 1024) && wgs >= (windowed ? cus / 2 : 3 * cus / 4);
   if (!few_keys && !busy) return 0;
@@ -703,12 +703,12 @@ int once_units(int Hkv, int dims) { return (int)(kCacheBytes / 2 / ((int64_t)32 
 // 8 x 2000 18.2 / 19.1, 1 x 8000 14.5 / 17.1; of 64, 1 x 4000 11.3 / 9.7).
 // 64-key pieces need twice the scratch; a call that brings less, say what a larger batch or a wider table with its
 // longer pieces needs, gets 128-key ones.
-int pick_min_units(int B, int Hkv, int hchunks, int max_ctx, bool short_pieces) {
+int pick_min_units(int B, int Hkv, int hchunks, int max_ctx, bool short_pieces, int64_t cus) {
   const int64_t units = (int64_t)B * Hkv * hchunks;
   auto pieces = [&](int keys) { return ((int64_t)max_ctx + keys - 1) / keys; };
   int kps = 512;
   while (kps > 128 && units * pieces(kps) < 4096) kps >>= 1;
-  if (short_pieces && kps == 128 && pieces(64) <= 64 && units * pieces(64) <= 4 * (int64_t)current_device_cu_count()) kps = 64;
+  if (short_pieces && kps == 128 && pieces(64) <= 64 && units * pieces(64) <= 4 * cus) kps = 64;
   return kps / 32;
 }
 
@@ -725,8 +725,8 @@ size_t scratch_bytes(int B, int Hq, int D, int max_ctx, int min_units) {
 
 // teams that are resident together: wavefronts per CU (2 per SIMD, 1 in the masked variant) /
 // wavefronts per team
-int pick_num_teams(int units_per_team, bool ragged) {
-  return max(1, current_device_cu_count() * (ragged ? 4 : 8) / units_per_team);
+int pick_num_teams(int units_per_team, bool ragged, int cus) {
+  return max(1, cus * (ragged ? 4 : 8) / units_per_team);
 }
 
 // head size the kernel instance is built for; past 128 one instance, for 256, takes every size on
@@ -747,7 +747,8 @@ extern "C" size_t dlb_paged_decode_ws_bytes(int B, int Hq, int Hkv, int D, int p
   const int hchunks = (group + 15) / 16;
   const int64_t max_ctx = (int64_t)page * max_blocks;
   if (max_ctx > 0x7fffffff) return 0;
-  return dlb::scratch_bytes(B, Hq, D, (int)max_ctx, dlb::pick_min_units(B, Hkv, hchunks, (int)max_ctx, true));
+  return dlb::scratch_bytes(B, Hq, D, (int)max_ctx, dlb::pick_min_units(B, Hkv, hchunks, (int)max_ctx, true,
+                                                                         dlb::current_device_cu_count()));
 }
 
 extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const void* v_cache,
@@ -780,13 +781,13 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
                              k_stride_head, v_stride_page, v_stride_tok,  v_stride_head};
   for (int64_t sd : strides)
     if (sd % 8 != 0) return DLB_ERR_UNSUPPORTED;
-  const int max_ctx = page * max_blocks;
+  const int max_ctx = page * max_blocks, cus = current_device_cu_count();
   DecodeParams p;
   p.group = Hq / Hkv;
   p.hchunks = (p.group + 15) / 16;
-  p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, true);
+  p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, true, cus);
   if (ws_bytes < scratch_bytes(B, Hq, Dp, max_ctx, p.min_units))
-    p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, false);
+    p.min_units = pick_min_units(B, Hkv, p.hchunks, max_ctx, false, cus);
   if (!ws || ws_bytes < scratch_bytes(B, Hq, Dp, max_ctx, p.min_units)) return DLB_ERR_WORKSPACE;
   p.nsplit_max = partial_slots(max_ctx, p.min_units);
   p.q = q;
@@ -827,11 +828,11 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
 
   hipStream_t s = (hipStream_t)stream;
   const int units = Hkv * p.hchunks;
-  p.num_teams = pick_num_teams(units, ragged);
+  p.num_teams = pick_num_teams(units, ragged, cus);
   if (units > 65535 || p.num_teams > 65535 || B > 65535) return DLB_ERR_UNSUPPORTED;
   const dim3 grid1((uint32_t)units, (uint32_t)p.num_teams);
   const dim3 grid2((uint32_t)Hq, (uint32_t)B), grid_direct((uint32_t)units, (uint32_t)B);
-  const int direct = direct_waves(B, units, max_ctx, window_size, Dp);
+  const int direct = direct_waves(B, units, max_ctx, window_size, Dp, cus);
   p.once_units = once_units(Hkv, D + Dv);
   const bool choice = may_read_once(B, Hkv, D + Dv, max_ctx, window_size);
 #define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_)                                                                       \
