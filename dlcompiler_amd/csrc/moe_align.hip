@@ -406,11 +406,10 @@ __global__ __launch_bounds__(kThreads) void route_place_kernel(const IdxArray id
     if (e[g] >= 0)
       o.sorted_ids[wave_cnt[wave][e[g]] + rank[g]] = (int32_t)(begin + wave * per + g * kWave + lane);
   // (the blocks' experts, a binary search each, are shared out: by one workgroup they took longer than all the
-  // rest, 16384 tokens x 6 of 64 experts, 1600 blocks, 13.3 -> 10.3 us a call.  What one workgroup writes at once is left
-  // to the last chunk, which is the shortest: behind the first one's full chunk 147 tokens x 8 of 64 took 9.3 us, so
-  // 8.8.  More shares begin at the first chunk, whose workgroup starts first: 8192 x 8 of 256 14.7, else 14.9)
-  const int share = o.expert_ids_cap > kThreads ? me : chunks - 1 - me;
-  write_block_experts(o, base_s, share * kThreads + tid, chunks * kThreads);
+  // rest, 16384 tokens x 6 of 64 experts, 1600 blocks, 13.3 -> 10.3 us a call.  The last chunk, which is the shortest,
+  // has the first share, and few blocks need no other: behind the first one's full chunk 147 tokens x 8 of 64 took 9.2
+  // us, so 8.7, 1090 x 8 of 256 15.6 and 15.1, 8192 x 8 of 256 15.0 and 14.8)
+  write_block_experts(o, base_s, (chunks - 1 - me) * kThreads + tid, chunks * kThreads);
   if (me == chunks - 1 && tid < E && o.counts) o.counts[tid] = total_s[tid];
 }
 
