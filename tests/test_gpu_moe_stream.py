@@ -24,9 +24,9 @@ SHAPES = [(1, 128, 128, 8, 2), (3, 640, 384, 64, 6), (40, 2048, 256, 64, 6), (17
           (224, 192, 320, 8, 2), (225, 192, 320, 8, 2), (300, 64, 192, 4, 2), (333, 512, 128, 4, 2),
           (420, 128, 384, 4, 3)]
 # on either side of each limit: 7, 22, 32 (fp8: the tiled kernel from there on) and 52 rows per expert where waves split
-# K, 19 where they run side by side
+# K, 19 and 36 where they run side by side
 SHAPES += [(T, 256, 384, 8, 2) for T in (28, 29, 88, 89, 128, 129, 208, 209)]
-SHAPES += [(T, 128, 1088, 64, 4) for T in (304, 305)]
+SHAPES += [(T, 128, 1088, 64, 4) for T in (304, 305, 576, 577)]
 # rows of 4096 fp8 bytes, in either GEMM, where waves start at other chunks: tiles of 16, 32 and 64 rows
 SHAPES += [(T, H, I, 4, 2) for T in (6, 30, 60) for H, I in ((4096, 256), (256, 4096))]
 
