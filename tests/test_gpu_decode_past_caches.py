@@ -86,3 +86,36 @@ def test_the_keys_decide_and_not_the_table(dev, hq, hkv, d):
         wide[:, :table.shape[1]] = table
         results.append(_run(dev, q, kc, vc, wide, kv_len))
     assert torch.equal(*results)
+
+
+@pytest.mark.parametrize("hkv,d", [(2, 128), (4, 64)])
+def test_replays_follow_the_keys(dev, hkv, d):
+    """Captured with few keys and replayed with more than go through the caches, and back."""
+    from dlcompiler_amd.kernels.paged_attention import paged_attention_fwd
+
+    filling = 300 * 2**20 // (hkv * d * 4)
+    q, kc, vc, table, kv_len = (t.to(dev) for t in _inputs([1100, 40, 3000], 1, filling, 64, 4 * hkv, hkv, d, torch.bfloat16,
+                                                           "contiguous"))
+    start, new, o = torch.arange(5, device=dev), torch.ones(5, dtype=torch.int64, device=dev), torch.empty_like(q)
+
+    def call():
+        paged_attention_fwd(q, kc, vc, o, table, start, new, kv_len, 1)
+
+    kv_len[-1] = 500
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for keys in (filling, 500, filling // 2 - 40, filling // 3, filling):
+        kv_len[-1] = keys
+        call()
+        eager = o.clone()
+        o.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, eager), keys
