@@ -36,6 +36,10 @@ struct PrefillParams {
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;  // token / head strides (elements)
   int Hq, Hkv, group;
   int xcd_heads;  // heads (head groups) per XCD, != 0: remap blockIdx.x so a KV group's share an XCD
+  // kernels without PACK: query heads whose 32-query blocks share workgroups (group or 1), and what a block's
+  // number in their order is multiplied by for its quotient by them (0: 1)
+  int share;
+  unsigned int share_rcp;
   // PACK kernels: a workgroup's rows are those of 1 << pack_shift query heads of a KV group, the rows of
   // each being (kBlockM >> pack_shift) queries
   int pack_shift;
@@ -213,10 +217,38 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   // (vector loads of wave-uniform values: saying that they are keeps loops and conditions scalar)
   const int L = __builtin_amdgcn_readfirstlane(p.seq_len[seq]);
   const int pack = PACK ? p.pack_shift : 0;
-  const int kBlockQ = kBlockM >> pack;  // queries of a workgroup
   const int qtile = gridDim.y - 1 - blockIdx.y;  // heaviest first
-  const int q0 = qtile * kBlockQ;
+  // SHARE: a wave's rows are 32 queries of one head, and a workgroup takes the next four of the order
+  // (query block, head): with the heads of a KV group in that order its waves see the same keys, where those
+  // of 128 queries of one head reach the diagonal one after the other, and only a sequence's last workgroup
+  // has waves without rows.
+  constexpr bool SHARE = RW == 4 && !PACK;
+  int q0 = qtile * (kBlockM >> pack), span = kBlockM >> pack;  // queries of the workgroup: first, how many
+  int wave_q0 = 0, wave_head = 0;                              // of the wave: offset of its first query, head
+  int block_head = 0;                                          // head of the workgroup's first wave
+  if (SHARE) {
+    const int unit0 = qtile * RW;
+    const int first = p.share > 1 ? (int)__umulhi((unsigned)unit0, p.share_rcp) : unit0;
+    q0 = 32 * first;
+    block_head = unit0 - first * p.share;
+  }
   if (q0 >= L) return;
+  if (SHARE) {
+    auto block_of = [&](int w, int& dq, int& hd) {
+      dq = 0;
+      hd = block_head + w;
+#pragma unroll
+      for (int i = 1; i < RW; ++i)
+        if (hd >= p.share) {
+          hd -= p.share;
+          dq += 32;
+        }
+    };
+    int last_head;
+    block_of(RW - 1, span, last_head);
+    span += 32;
+    block_of(threadIdx.x >> 6, wave_q0, wave_head);
+  }
   const int64_t tok0 = __builtin_amdgcn_readfirstlane(p.start_loc[seq]);
   // context seen by this sequence: kv_total keys, the queries are its last L positions
   const int kv_total = PAGED ? __builtin_amdgcn_readfirstlane(p.kv_len[seq]) : L;
@@ -224,7 +256,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   if (PAGED && hist < 0) return;  // inconsistent lengths: nothing sensible to compute
   // sliding window (only the paged entry point exposes it; the packed kernel compiles it out)
   const int window = PAGED ? p.window : -1;
-  TileRun run = visible_tiles(kv_total, hist, q0, kBlockQ, window);
+  TileRun run = visible_tiles(kv_total, hist, q0, span, window);
   bool parted = false;  // other workgroups have a part of these rows' keys
   if (PACK && p.nsplit > 1) {
     const int per = tiles_per_part(run, p.nsplit);
@@ -236,6 +268,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   int head = blockIdx.x;  // PACK: first of the workgroup's heads
   if (p.xcd_heads) head = (blockIdx.x & 7) * p.xcd_heads + (blockIdx.x >> 3);
   if (PACK) head <<= pack;
+  else if (SHARE) head *= p.share;
   const int kvh = head / p.group;
 
   const int tid = threadIdx.x;
@@ -252,8 +285,9 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
 
   // ---- Q^T as B operand: lane (n = query, k = dims 16*ks + 8*hh .. +8), kept in registers
   const int brow = 32 * wave + col;  // row of the workgroup
-  const int qrow = q0 + (PACK ? brow & (kBlockQ - 1) : brow);
-  if (PACK) head += brow / kBlockQ;  // (by lane from here on)
+  const int qrow = q0 + (SHARE ? wave_q0 + col : PACK ? brow & (span - 1) : brow);
+  if (SHARE) head += __builtin_amdgcn_readfirstlane(wave_head);
+  if (PACK) head += brow / span;  // (by lane from here on)
   u32x4 qf[KS];
   {
     const unsigned short* qp =
@@ -272,12 +306,12 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   // (all 64 keys <= position of row q0): no mask, no clamping of key rows
   const int nfull = softcap > 0.0f ? 0 : min((hist + q0 + 1) / kTileN, ntiles);
   // first tile whose keys every query of the workgroup sees (sliding window)
-  const int jopen = window > 0 ? max(hist + q0 + kBlockQ - 1 - window + kTileN - 1, 0) / kTileN : 0;
+  const int jopen = window > 0 ? max(hist + q0 + span - 1 - window + kTileN - 1, 0) / kTileN : 0;
   const int qpos = hist + qrow;                          // context position of this lane's query
   // context positions of the wave's first and last query
-  const int wave_q0 = PACK ? (32 * wave) & (kBlockQ - 1) : 32 * wave;
+  if (!SHARE) wave_q0 = PACK ? (32 * wave) & (span - 1) : 32 * wave;
   const int wave_first_pos = hist + q0 + wave_q0;
-  const int wave_last_pos = wave_first_pos + (PACK ? min(32, kBlockQ) : 32) - 1;
+  const int wave_last_pos = wave_first_pos + (PACK ? min(32, span) : 32) - 1;
 
   // ---- global -> LDS staging of one K/V tile.  Per-thread base pointers are formed once; a
   // tile adds a workgroup-uniform offset.  CLAMP (tiles that may run past the sequence)
@@ -881,9 +915,23 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.ws_ml = p.ws_o ? p.ws_o + (size_t)p.tokens * Hq * p.nsplit * p.ws_d : nullptr;
   const int64_t seen = p.window > 0 && (int64_t)p.window + max_len < max_keys ? (int64_t)p.window + max_len : max_keys;
   const bool small = !plan.use && small_tiles(Hq, B, D, max_len, seen, p.tokens);
-  const int64_t qtiles = ceil_div(max_len, small ? 64 : 128 >> p.pack_shift);
+  // Heads of a KV group share workgroups in launches of more than two rounds (two workgroups on a CU, four with
+  // up to 64 dims), where the KV heads fall on the XCDs by themselves and the row tiles fit the grid.  32 heads
+  // (8 kv) of 128: 8 x 512 - 4096 tokens 284 -> 275 us, 8 x 100 - 1000 44 -> 41.3; 28 (4): 42 -> 39.8, 8 x 300 -
+  // 1000 over 2000 110 -> 99.  In one round the workgroups that finish early help their neighbours and it loses:
+  // 8 heads (1 kv), 3 x 1000 - 4000 55.5 -> 56.9; 32 (8) of 64 dims, 4 x 60 - 300 6.9 -> 7.5.  Over histories
+  // of unequal lengths 2.5 rounds are a matter of luck (8 x 300 - 600 over up to 4096, ten batches: 0.98 - 1.07).
+  const int row_waves = small ? 2 : 4;
+  const int64_t all_wgs = ceil_div(max_len, 128) * B * Hq, slots = (int64_t)current_device_cu_count() * (D <= 64 ? 4 : 2);
+  int64_t qtiles = ceil_div(ceil_div(max_len, 32) * p.group, row_waves);
+  p.share = !plan.use && !small && all_wgs > (paged ? 3 : 2) * slots && (8 % Hkv == 0 || Hkv % 8 == 0) && qtiles <= 65535 &&
+                    p.group <= 4096 ? p.group : 1;
+  // (exact: numbers below 2^18, at most 2^12 heads)
+  p.share_rcp = p.share > 1 ? (unsigned int)(0x100000000ull / p.share + 1) : 0;
+  if (p.share == 1) qtiles = ceil_div(max_len, 32 * row_waves);
+  if (plan.use) qtiles = ceil_div(max_len, 128 >> p.pack_shift);
   if (qtiles > 65535 || (int64_t)B * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
-  const int head_groups = Hq >> p.pack_shift;
+  const int head_groups = plan.use ? Hq >> p.pack_shift : Hq / p.share;
   // workgroups are dealt round-robin to the 8 XCDs by linear id; with Hq % 8 == 0 the
   // remap in the kernel puts heads {x, x+8, ...} -> consecutive heads on one XCD so a KV
   // group's four query heads hit the same L2.
