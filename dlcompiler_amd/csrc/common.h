@@ -217,14 +217,21 @@ __device__ __forceinline__ void dma4_global_to_lds_masked(const void* sbase, uns
                : "memory", "m0");
 }
 
-// max of a value and its partner 32 lanes away (v_permlane32_swap: a register-file exchange,
-// no trip through LDS as with ds_bpermute)
-__device__ __forceinline__ float max_xor32(float v) {
-  typedef __attribute__((ext_vector_type(2))) unsigned int u2;
-  const unsigned int u = __float_as_uint(v);
-  const u2 r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+// a value and its partner 16 / 32 lanes away combined (v_permlane16_swap, v_permlane32_swap: register-file
+// exchanges, no trip through LDS as with ds_bpermute)
+typedef __attribute__((ext_vector_type(2))) unsigned int permlane_pair;
+__device__ __forceinline__ permlane_pair lanes_xor16(float v) {
+  return __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
 }
+__device__ __forceinline__ permlane_pair lanes_xor32(float v) {
+  return __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+}
+__device__ __forceinline__ float max_of(permlane_pair r) { return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])); }
+__device__ __forceinline__ float sum_of(permlane_pair r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); }
+__device__ __forceinline__ float max_xor16(float v) { return max_of(lanes_xor16(v)); }
+__device__ __forceinline__ float max_xor32(float v) { return max_of(lanes_xor32(v)); }
+__device__ __forceinline__ float sum_xor16(float v) { return sum_of(lanes_xor16(v)); }
+__device__ __forceinline__ float sum_xor32(float v) { return sum_of(lanes_xor32(v)); }
 
 // tanh for the logit soft-cap: no less accurate than tanhf, in half its instructions and without a branch.
 // Below 0.85 an odd polynomial (least squares on Chebyshev nodes, reweighted towards the smallest

@@ -98,7 +98,12 @@ constexpr int kVtRowBytes = 144;   // 64 keys * 2 B + 16 B pad
 // (The masked variant keeps a few more per-lane offsets alive: it is built for one wavefront per
 // SIMD instead of two rather than spilling them.)
 // ONCE: K and V go past the caches (see may_read_once); without it, V alone.
-template <int DT, int D, bool POW2, bool RAGGED, bool ONCE>
+// HELD: page numbers come from a run of the block table that the lanes hold, else from scalar loads half a tile ahead.
+struct PageRun {
+  int entry;  // this lane's: page number of the sequence's page `first` + lane
+  int first;
+};
+template <int DT, int D, bool POW2, bool RAGGED, bool ONCE, bool HELD = false>
 struct DecodeSegment {
   static constexpr int KS = D / 32;  // MFMA k-steps over the head dim
   // K in whole 128-byte lines.  A load that brings 16 operand rows of one key each touches 16 half lines, so
@@ -116,7 +121,8 @@ struct DecodeSegment {
   // Keys [k_begin, k_end) of sequence b (context ctx, keys before kv_min masked), for one kv-head
   // unit; k_begin is a multiple of 32.  vt: this wavefront's V^T tile in LDS (kVtBytes).
   __device__ __forceinline__ void run(const DecodeParams& p, unsigned char* vt, int b, int ctx, int kvh, int head,
-                                      bool head_ok, int k_begin, int k_end, int kv_min) {
+                                      bool head_ok, int k_begin, int k_end, int kv_min,
+                                      const PageRun& pages = PageRun{0, 0}) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4;  // lane group 0..3
   const int c = lane & 15;  // column (query head) / row (key) inside a 16-tile
@@ -186,6 +192,15 @@ struct DecodeSegment {
   int pg_ahead[2];  // physical pages of the two 16-key sub-tiles of the next half tile to load
   auto lookup_pages = [&](int h0) {
     const int32_t* entry[2];
+    if constexpr (HELD) {
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) {
+        const int base_key = min(h0 + 16 * sub, ctx - 1);
+        const int pi = POW2 ? (base_key >> page_shift) : (base_key / page);
+        pg_ahead[sub] = __builtin_amdgcn_readlane(pages.entry, __builtin_amdgcn_readfirstlane(pi - pages.first));
+      }
+      return;
+    }
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int base_key = min(h0 + 16 * sub, ctx - 1);  // clamp: never look past the context
@@ -336,8 +351,7 @@ struct DecodeSegment {
         mloc = fmaxf(mloc, x);
       }
     }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+    mloc = max_xor32(max_xor16(mloc));
     const float m_new = fmaxf(m_run, mloc);
     // a half tile can be entirely masked (sliding window, chunk tail): keep exponents finite
     const float m_ref = (m_new == -__builtin_inff()) ? 0.0f : m_new;
@@ -404,8 +418,7 @@ struct DecodeSegment {
     if (second) compute_half(t0 + 32, hb, 1);
   }
 
-  l_run += __shfl_xor(l_run, 16);
-  l_run += __shfl_xor(l_run, 32);
+  l_run = sum_xor32(sum_xor16(l_run));
 
   }  // run
 };
@@ -426,7 +439,10 @@ __device__ __forceinline__ const DecodeParams& arguments_again() {
 }
 
 // CHOICE: whether K and V go past the caches follows from the keys of the batch (see may_read_once).
-template <int DT, int D, bool POW2, bool RAGGED, bool CHOICE>
+// ONE: one sequence, pieces of the smallest size (see one_sequence): where a team's piece starts does not depend on the
+// context, so the page numbers, the context and the query are asked for together.  A short run is a chain of loads (8 kv
+// heads of 128, 1 x 4000 keys: with one link fewer here and one in the merge 10.75 -> 9.3 us, of which the merge 0.7).
+template <int DT, int D, bool POW2, bool RAGGED, bool CHOICE, bool ONE>
 __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(const DecodeParams p) {
   // grid: x = (kv head, head chunk) unit, y = team.  The unit is the fastest index, so the
   // wavefronts that start together read the 256-byte head slices of the SAME token rows at the
@@ -446,21 +462,42 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   const bool head_ok = hq_local < p.group;
   const int head = kvh * p.group + hq_local;
 
+  if constexpr (ONE) {
+    using Segment = DecodeSegment<DT, D, POW2, RAGGED, false, true>;
+    const int max_ctx = p.max_blocks * p.page, k_begin = team * p.min_units * 32;
+    if (k_begin >= max_ctx) return;
+    PageRun pages;
+    pages.first = POW2 ? k_begin >> p.page_shift : k_begin / p.page;
+    pages.entry = p.block_table[min(pages.first + lane, p.max_blocks - 1)];
+    const int ctx = __builtin_amdgcn_readfirstlane(min(p.kv_len[0], max_ctx));
+    if (k_begin >= ctx) return;
+    if (team == 0 && unit == 0 && lane == 0) p.ws_np[0] = (ctx + 32 * p.min_units - 1) / (32 * p.min_units);
+    Segment seg;
+    seg.run(p, vt, 0, ctx, kvh, head, head_ok, k_begin, k_begin + 32 * p.min_units, 0, pages);
+    if (head_ok) {
+      const int64_t slot = (int64_t)head * p.nsplit_max + team;
+      float* wo = p.ws_o + slot * D;
+#pragma unroll
+      for (int mt = 0; mt < Segment::MT; ++mt) *(f32x4*)(wo + 16 * mt + 4 * g) = seg.o[mt];
+      if (g == 0) {
+        p.ws_ml[slot * 2 + 0] = seg.m_run;
+        p.ws_ml[slot * 2 + 1] = seg.l_run;
+      }
+    }
+    return;
+  }
+
   // ---- this team's piece of the concatenated KV streams (32-key units, visible keys only: with a
   // sliding window the teams share what the windows leave, not the whole contexts) ----
   auto context_of = [&](int bb) { return bb < p.B ? max(p.kv_len[bb], 0) : 0; };
   auto units_of = [&](int ctx) { return ((ctx + 31) >> 5) - (first_visible(p, ctx) >> 5); };
-  int total = 0;
-  for (int b0 = 0; b0 < p.B; b0 += 64) {
-    int t = units_of(context_of(b0 + lane));
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) t += __shfl_xor(t, d);
-    total += t;
-  }
-  // (the reduction leaves the same value in every lane; say so, or every address derived from
-  // it is treated as lane-dependent and the block-table lookups become vector loads that
-  // share the in-order return queue of the K/V stream)
-  total = __builtin_amdgcn_readfirstlane(total);
+  // (the first 64 sequences' values serve the walk as well: of a short run's chain of loads and scans every link
+  // counts)
+  const int first_ctx = context_of(lane);
+  const int first_incl = wave_inclusive_scan(units_of(first_ctx));
+  int total = __builtin_amdgcn_readlane(first_incl, 63);
+  for (int b0 = 64; b0 < p.B; b0 += 64)
+    total += __builtin_amdgcn_readlane(wave_inclusive_scan(units_of(context_of(b0 + lane))), 63);
   const int upt = max((total + p.num_teams - 1) / p.num_teams, p.min_units);  // units per team
   const int lo = team * upt;
   if (lo >= total) return;
@@ -471,16 +508,16 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
   using Segment = DecodeSegment<DT, D, POW2, RAGGED, decltype(once)::value>;
   int carry = 0;  // units of all sequences before b0
   for (int b0 = 0; b0 < p.B; b0 += 64) {
-    const int ctx_mine = context_of(b0 + lane);
+    const int ctx_mine = b0 == 0 ? first_ctx : context_of(b0 + lane);
     const int t = units_of(ctx_mine);
-    const int incl = wave_inclusive_scan(t);
+    const int incl = b0 == 0 ? first_incl : wave_inclusive_scan(t);
     const int excl = carry + incl - t;
     uint64_t hit = __ballot(t > 0 && excl < hi && excl + t > lo);
     // park the per-sequence values in LDS: nothing per-lane stays live across a segment
     seg_lds[0][lane] = excl;
     seg_lds[1][lane] = t;
     seg_lds[2][lane] = ctx_mine;
-    carry = __builtin_amdgcn_readfirstlane(carry + __shfl(incl, 63));
+    carry += __builtin_amdgcn_readlane(incl, 63);
     while (hit) {  // wave-uniform
       const int l = __builtin_ctzll(hit);
       hit &= hit - 1;
@@ -525,10 +562,13 @@ __global__ __launch_bounds__(64, RAGGED ? 1 : 2) void paged_decode_split_kernel(
 // first 64 (m, l) pairs and the first round of rows: inside the scratch whether written or not,
 // and masked) is requested together with it.
 constexpr int kCombineThreads = 256;
-template <int DT, int D>
+// EARLY: the first 64 rows are all requested with the number of partials instead of after it: for launches of up to a
+// workgroup per CU (2 x 1500 - 3000 keys 10.8 -> 10.0 us); larger ones would read rows that no partial was written to.
+template <int DT, int D, bool EARLY>
 __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(const DecodeParams p) {
   constexpr int RL = D / 4;                    // lanes per row
   constexpr int RG = kCombineThreads / RL;     // rows per round
+  constexpr int E = EARLY ? (64 + RG - 1) / RG : 1;  // rows per lane requested early
   __shared__ float acc_lds[RG][D];
   __shared__ float w_lds[kCombineThreads / 64][64];
   const int head = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
@@ -543,21 +583,18 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(c
     m0 = p.ws_ml[(slot0 + lane) * 2];
     l0 = p.ws_ml[(slot0 + lane) * 2 + 1];
   }
-  f32x4 v0 = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (row_lane && rg < p.nsplit_max) v0 = *(const f32x4*)(p.ws_o + (slot0 + rg) * D + 4 * d4);
+  f32x4 early[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u)  // (clamped: inside the scratch, masked below)
+    early[u] = *(const f32x4*)(p.ws_o + (slot0 + min(rg + u * RG, p.nsplit_max - 1)) * D + 4 * d4);
   if (ctx <= 0) ns = 0;
   if (lane >= ns) {
     m0 = -__builtin_inff();
     l0 = 0.0f;
   }
-  auto wave_max = [](float v) {
-#pragma unroll
-    for (int x = 32; x >= 1; x >>= 1) v = fmaxf(v, __shfl_xor(v, x));
-    return v;
-  };
   float m = m0;
   for (int s0 = 64; s0 < ns; s0 += 64) m = fmaxf(m, s0 + lane < ns ? p.ws_ml[(slot0 + s0 + lane) * 2] : m);
-  m = wave_max(m);
+  m = max_xor32(max_xor16(row16_max(m)));
   float den = 0.0f;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < ns; s0 += 64) {
@@ -570,6 +607,16 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(c
     den += w * ls;
     w_lds[wave][lane] = w;  // (each wave its own copy: no barrier)
     const int n = min(64, ns - s0);
+    if (EARLY && s0 == 0) {
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        const int r = rg + u * RG;
+        const float wr = w_lds[wave][min(r, 63)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += r < n ? wr * early[u][i] : 0.0f;
+      }
+      continue;
+    }
     // All 64 rows' loads at once (D <= 128), without a condition: rows past the last are the last one again and
     // count nothing.  Behind a branch each load was waited for before the next (8 kv heads of 128, 1 x 4000 keys,
     // 32 - 63 partials: 11.6 -> 10.6 us; 1 x 32000, 250 partials: 36.0 -> 31.4).  Rows asked for twice cost nothing:
@@ -581,7 +628,7 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(c
 #pragma unroll
         for (int u = 0; u < U; ++u)
           v[u] = *(const f32x4*)(p.ws_o + (slot0 + s0 + min(r0 + u * RG, n - 1)) * D + 4 * d4);
-        if (s0 == 0 && r0 == rg) v[0] = v0;
+        if (s0 == 0 && r0 == rg) v[0] = early[0];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int r = r0 + u * RG;
@@ -592,8 +639,7 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(c
       }
     }
   }
-#pragma unroll
-  for (int x = 32; x >= 1; x >>= 1) den += __shfl_xor(den, x);
+  den = row16_sum(sum_xor16(sum_xor32(den)));
   if (row_lane) *(f32x4*)&acc_lds[rg][4 * d4] = acc;
   __syncthreads();
   if (tid < p.dv) {
@@ -664,21 +710,22 @@ __global__ __launch_bounds__(64 * W, RAGGED ? 1 : 2) void paged_decode_direct_ke
 
 // Wavefronts per workgroup of the one-launch kernel, 0: the split kernel.
 // One workgroup per (sequence, kv-head unit) reads a CU's share of the bandwidth at best, so with few
-// workgroups the split is the faster one from about 700 keys of 128 dims on (one sequence, 8 kv
-// heads: 100 keys 17.1 -> 4.7 us, 300 keys 17.1 -> 6.8, 700 keys 10.1 either way, 1400 keys 15.7
-// against 10.4).  With most CUs busy it wins up to the lengths where one long context among short
+// workgroups the split is the faster one from about 700 keys of 128 dims on, with its 64-key pieces from about
+// 500 keys on (640 of up to 64 dims; direct / split, one sequence of 8 kv heads: 100 keys 4.4 / 7, 320 keys 6.5 /
+// 7.1, 448 6.7 / 7.3, 576 8.7 / 7.2, 704 9.0 / 7.2; eight: 448 9.4 / 9.6, 576 10.4 / 9.9; sixteen, for which pieces have
+// 128 keys: 576 10.9 / 12.9; 4 kv heads of 64: 576 7.2 / 7.3, 704 7.4 / 7.3).  With most CUs busy it wins up to the lengths where one long context among short
 // ones would be the whole time (20 sequences of 16 kv heads, 64 - 1024 keys: 22.7 -> 22.0 us; 250
 // of one kv head 23.9 -> 16.3; 128 x 100 keys 20.1 -> 13.4); past 1024 keys mixed lengths cost 3 - 6 %.
 // What a sliding window leaves is about the same for every sequence.
 // Eight wavefronts pay where the rows are short and a few CUs read many keys (1000 keys of 64 dims,
 // one sequence: 9.2 us, with four 10.7).
-int direct_waves(int B, int units, int max_ctx, int window, int D, int64_t cus) {
+int direct_waves(int B, int units, int max_ctx, int window, int D, bool short_pieces, int64_t cus) {
   if (D > 128) return 0;
   // (a window of any size up to 2^31 - 1 says "none" as well as -1 does)
   const bool windowed = window > 0 && window < max_ctx - 32;
   const int keys = windowed ? window + 32 : max_ctx;
   const int64_t wgs = (int64_t)B * units;
-  const bool few_keys = (int64_t)keys * D <= 700 * 128;
+  const bool few_keys = short_pieces ? keys <= (D <= 64 ? 640 : 512) : (int64_t)keys * D <= 700 * 128;
   const bool busy = keys <= (windowed ? 2048 : 1024) && wgs >= (windowed ? cus / 2 : 3 * cus / 4);
   if (!few_keys && !busy) return 0;
   return D <= 64 && keys > 512 && wgs < cus ? 8 : 4;
@@ -699,8 +746,9 @@ int once_units(int Hkv, int dims) { return (int)(kCacheBytes / 2 / ((int64_t)32 
 
 // Smallest piece a team may get, in 32-key units: 512 keys, less for small problems so that
 // the chip still sees a few thousand wavefronts.  64 keys, two steps of a wavefront, where that leaves each CU
-// at most four of them and a head at most 64 partials, or 65 where pieces cross sequences (128 / 64 keys: 8 kv heads of 128, 1 x 2000 11.1 / 9.4 us,
-// 8 x 2000 18.2 / 19.1, 1 x 8000 14.5 / 17.1; of 64, 1 x 4000 11.3 / 9.7).
+// at most four of them and a head at most 64 partials, or 65 where pieces cross sequences (128 / 64 keys, measured with
+// another merge: 8 kv heads of 128, 1 x 2000 11.1 / 9.4 us, 8 x 2000 18.2 / 19.1, 1 x 8000 14.5 / 17.1; of 64, 1 x 4000
+// 11.3 / 9.7).
 // 64-key pieces need twice the scratch; a call that brings less, say what a larger batch or a wider table with its
 // longer pieces needs, gets 128-key ones.
 int pick_min_units(int B, int Hkv, int hchunks, int max_ctx, bool short_pieces, int64_t cus) {
@@ -717,6 +765,11 @@ int pick_min_units(int B, int Hkv, int hchunks, int max_ctx, bool short_pieces, 
 int partial_slots(int max_ctx, int min_units) {
   const int t = (max_ctx + 31) / 32;
   return t / min_units + 2;
+}
+
+// One sequence whose teams all have pieces of min_units units, whatever its context is, and at most 64 pages per piece
+bool one_sequence(int B, int max_ctx, int min_units, int num_teams, int window) {
+  return B == 1 && window <= 0 && (max_ctx + 31) / 32 <= (int64_t)num_teams * min_units && min_units <= 16;
 }
 
 size_t scratch_bytes(int B, int Hq, int D, int max_ctx, int min_units) {
@@ -832,8 +885,10 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
   if (units > 65535 || p.num_teams > 65535 || B > 65535) return DLB_ERR_UNSUPPORTED;
   const dim3 grid1((uint32_t)units, (uint32_t)p.num_teams);
   const dim3 grid2((uint32_t)Hq, (uint32_t)B), grid_direct((uint32_t)units, (uint32_t)B);
-  const int direct = direct_waves(B, units, max_ctx, window_size, Dp, cus);
+  const int direct = direct_waves(B, units, max_ctx, window_size, Dp, p.min_units == 2, cus);
   p.once_units = once_units(Hkv, D + Dv);
+  const bool one = one_sequence(B, max_ctx, p.min_units, p.num_teams, window_size);
+  const bool early = (int64_t)B * Hq <= cus;
   const bool choice = may_read_once(B, Hkv, D + Dv, max_ctx, window_size);
 #define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_)                                                                       \
   do {                                                                                                            \
@@ -841,10 +896,12 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
       hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, D_, P2_, RG_, 4>), grid_direct, dim3(256), 0, s, p);    \
     else if (D_ == 64 && direct == 8)                                                                             \
       hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, 64, P2_, RG_, 8>), grid_direct, dim3(512), 0, s, p);    \
-    else if (D_ % 64 == 0 && !RG_ && choice)                                                                        \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, D_ % 64 == 0 && !RG_>), grid1, dim3(64), 0, s, p); \
+    else if (D_ % 64 == 0 && !RG_ && choice)                                                                      \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, D_ % 64 == 0 && !RG_, false>), grid1, dim3(64), 0, s, p); \
+    else if (one)                                                                                                 \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, true>), grid1, dim3(64), 0, s, p);  \
     else                                                                                                          \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false>), grid1, dim3(64), 0, s, p);        \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, false>), grid1, dim3(64), 0, s, p); \
   } while (0)
 #define DLB_LAUNCH_DECODE(DT_, D_)                                                                           \
   do {                                                                                                       \
@@ -855,16 +912,18 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
       if (ragged) DLB_LAUNCH_SPLIT(DT_, D_, false, true);                                                    \
       else DLB_LAUNCH_SPLIT(DT_, D_, false, false);                                                          \
     }                                                                                                        \
-    if (!direct)                                                                                             \
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_>), grid2, dim3(kCombineThreads), 0, s, p);      \
+    if (!direct && early)                                                                                    \
+      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_, true>), grid2, dim3(kCombineThreads), 0, s, p); \
+    else if (!direct)                                                                                        \
+      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_, false>), grid2, dim3(kCombineThreads), 0, s, p); \
   } while (0)
 #define DLB_LAUNCH_DECODE_256(DT_)                                                                           \
   do {                                                                                                       \
     if (p.page_shift >= 0)                                                                                   \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, true, true, false>), grid1, dim3(64), 0, s, p);        \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, true, true, false, false>), grid1, dim3(64), 0, s, p);        \
     else                                                                                                     \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, false, true, false>), grid1, dim3(64), 0, s, p);       \
-    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, 256>), grid2, dim3(kCombineThreads), 0, s, p);       \
+      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, false, true, false, false>), grid1, dim3(64), 0, s, p);       \
+    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, 256, false>), grid2, dim3(kCombineThreads), 0, s, p);       \
   } while (0)
 #define DLB_DISPATCH_DECODE(DT_)                        \
   do {                                                  \
