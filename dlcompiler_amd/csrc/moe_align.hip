@@ -75,15 +75,23 @@ __device__ __forceinline__ uint64_t same_expert(int32_t e) {
   return peers;
 }
 
+// n / block by the block's reciprocal (2^32 / block, rounded down), whose estimate is at most one too small.  (A
+// division by a number that only the host knows is 20 instructions, and a workgroup waits for these.)
+__device__ __forceinline__ uint32_t blocks_of(uint32_t n, uint32_t block, uint32_t rcp) {
+  const uint32_t q = __umulhi(n, rcp);
+  return n - q * block >= block ? q + 1 : q;
+}
+
 // totals (0 past E, 16-byte aligned) -> padded expert bases base_s[0 .. E], by one wave: four
 // experts per lane
-__device__ __forceinline__ void scan_bases(const int32_t* total_s, int32_t* base_s, int E, int block, int lane) {
+__device__ __forceinline__ void scan_bases(const int32_t* total_s, int32_t* base_s, int E, int block, uint32_t rcp,
+                                           int lane) {
   typedef __attribute__((ext_vector_type(4))) int i32x4;
   const i32x4 total = ((const i32x4*)total_s)[lane];
   int32_t pad[4], sum = 0;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    pad[c] = (int32_t)(((uint32_t)total[c] + (uint32_t)block - 1u) / (uint32_t)block * (uint32_t)block);
+    pad[c] = (int32_t)(blocks_of((uint32_t)total[c] + (uint32_t)block - 1u, block, rcp) * (uint32_t)block);
     sum += pad[c];
   }
   int32_t run = wave_inclusive_scan(sum) - sum;
@@ -95,17 +103,6 @@ __device__ __forceinline__ void scan_bases(const int32_t* total_s, int32_t* base
   if (lane == 63) base_s[E] = run;
 }
 
-// expert whose padded run holds position p (base_s[E] > p): the last one that starts at or before p
-__device__ __forceinline__ int expert_at(const int32_t* base_s, int E, int32_t p) {
-  int lo = 0, hi = E;  // base_s[lo] <= p < base_s[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (base_s[mid] <= p) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
-
 struct AlignOut {
   int32_t* sorted_ids;
   int64_t sorted_cap;
@@ -115,15 +112,25 @@ struct AlignOut {
   int32_t* num_post_pad;
   int64_t numel;
   int E, block;
+  uint32_t block_rcp;  // 2^32 / block, rounded down (block 1: 2^32 - 1)
 };
-// block -> expert ids (-1 past the last block) and the padded total, as thread t of nt
+uint32_t reciprocal_of(int block) { return block > 1 ? (uint32_t)(0x100000000ull / (uint32_t)block) : 0xffffffffu; }
+// block -> expert ids (-1 past the last block) and the padded total, as thread t of nt (at least kMaxE): every thread
+// takes blocks of one expert.  (Looking up a block's expert takes six or eight dependent reads of base_s.  With this
+// and blocks_of, 48 tokens x 6 of 64 experts 5.58 -> 5.28 us a call, 64 x 8 of 256 10.9 -> 10.5, 16384 x 6 of 64
+// 10.3 -> 10.05.)
 __device__ __forceinline__ void write_block_experts(const AlignOut& o, const int32_t* base_s, int t, int nt) {
   const int32_t total_padded = base_s[o.E];
   if (t == 0) *o.num_post_pad = total_padded;
-  for (int64_t b = t; b < o.expert_ids_cap; b += nt) {
-    const int64_t p = b * o.block;
-    o.expert_ids[b] = p < total_padded ? expert_at(base_s, o.E, (int32_t)p) : -1;
+  const int shift = o.E > 1 ? 32 - __builtin_clz(o.E - 1) : 0;  // experts, rounded up to a power of two
+  const int e = t & ((1 << shift) - 1);
+  if (e < o.E) {
+    const uint32_t first = blocks_of((uint32_t)base_s[e], o.block, o.block_rcp);
+    const uint32_t end = blocks_of((uint32_t)base_s[e + 1], o.block, o.block_rcp);
+    for (uint32_t b = first + (uint32_t)(t >> shift); b < end; b += (uint32_t)(nt >> shift)) o.expert_ids[b] = e;
   }
+  for (int64_t b = blocks_of((uint32_t)total_padded, o.block, o.block_rcp) + t; b < o.expert_ids_cap; b += nt)
+    o.expert_ids[b] = -1;
 }
 
 // ---- everything in one workgroup ------------------------------------------------------------
@@ -192,7 +199,7 @@ __device__ __forceinline__ void align_one_workgroup(const AlignOut& o, OneShared
     if (tid < E && o.counts) o.counts[tid] = run;
   }
   __syncthreads();
-  if (wave == 0) scan_bases(s.total, s.base, E, o.block, lane);
+  if (wave == 0) scan_bases(s.total, s.base, E, o.block, o.block_rcp, lane);
   __syncthreads();
 #pragma unroll
   for (int g = 0; g < kOneGroups; ++g)
@@ -389,7 +396,7 @@ __global__ __launch_bounds__(kThreads) void route_place_kernel(const IdxArray id
     atomicAdd(&before_s[e0 + 3], (int)(bef_hi >> 16));
   }
   __syncthreads();
-  if (wave == 0) scan_bases(total_s, base_s, E, o.block, lane);
+  if (wave == 0) scan_bases(total_s, base_s, E, o.block, o.block_rcp, lane);
   __syncthreads();
   if (tid < E) {  // first position of each wave's slots of expert tid
     int32_t run = base_s[tid] + before_s[tid];
@@ -405,10 +412,10 @@ __global__ __launch_bounds__(kThreads) void route_place_kernel(const IdxArray id
   for (int g = 0; g < kRouteGroups; ++g)
     if (e[g] >= 0)
       o.sorted_ids[wave_cnt[wave][e[g]] + rank[g]] = (int32_t)(begin + wave * per + g * kWave + lane);
-  // (the blocks' experts, a binary search each, are shared out: by one workgroup they took longer than all the
-  // rest, 16384 tokens x 6 of 64 experts, 1600 blocks, 13.3 -> 10.3 us a call.  The last chunk, which is the shortest,
-  // has the first share, and few blocks need no other: behind the first one's full chunk 147 tokens x 8 of 64 took 9.2
-  // us, so 8.7, 1090 x 8 of 256 15.6 and 15.1, 8192 x 8 of 256 15.0 and 14.8)
+  // (the blocks' experts are shared out: by one workgroup, which looked up one after the other, they took longer than
+  // all the rest, 16384 tokens x 6 of 64 experts, 1600 blocks, 13.3 us a call against 10.3.  The last chunk, which is
+  // the shortest, has the first share, and few blocks need no other: behind the first one's full chunk, measured with
+  // look-ups too, 147 tokens x 8 of 64 took 9.2 us, so 8.7, 1090 x 8 of 256 15.6 and 15.1, 8192 x 8 of 256 15.0 and 14.8)
   write_block_experts(o, base_s, (chunks - 1 - me) * kThreads + tid, chunks * kThreads);
   if (me == chunks - 1 && tid < E && o.counts) o.counts[tid] = total_s[tid];
 }
@@ -470,7 +477,7 @@ __global__ __launch_bounds__(kScanThreads) void align_scan_kernel(
     total_s[tid] = 0;
   }
   __syncthreads();
-  if (tid < 64) scan_bases(total_s, base_s, E, block, tid);
+  if (tid < 64) scan_bases(total_s, base_s, E, block, o.block_rcp, tid);
   __syncthreads();
   if (live) {
     // chunk start offsets of this slice for the placement pass
@@ -621,7 +628,7 @@ __device__ __forceinline__ void align_place_fused_block(const PlaceParams& pp, c
   __syncthreads();
   for (int i = tid; i < kWaves * kMaxE; i += kThreads) (&wave_cnt[0][0])[i] = 0;
   __syncthreads();
-  if (tid < 64) scan_bases(total_s, base_s, E, pp.out.block, tid);
+  if (tid < 64) scan_bases(total_s, base_s, E, pp.out.block, pp.out.block_rcp, tid);
   __syncthreads();
   if (tid < E) cursor[tid] = base_s[tid] + before;
   if (me == chunks) {  // the extra workgroup: what the scan kernel emits besides offsets
@@ -707,7 +714,8 @@ int launch_align(const IdxArray topk_ids, int64_t numel, int E, int block, int32
                  int64_t sorted_cap, int32_t* expert_ids, int64_t expert_ids_cap, int32_t* counts,
                  int32_t* num_post_pad, int32_t* chunk_counts, hipStream_t s,
                  const QuantParams* quant = nullptr, int quant_dtype = DLB_DTYPE_BF16) {
-  const AlignOut out = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block};
+  const AlignOut out = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block,
+                      reciprocal_of(block)};
   if (numel <= kOneSlots) {
     if (quant && quant->total_groups > 0) {
       const uint32_t grid = (uint32_t)(1 + ceil_div(quant->total_groups, kQuantGroupsPerBlock * kOneQuantBlocks));
@@ -907,7 +915,8 @@ extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights
   hipStream_t s = (hipStream_t)stream;
   const RouteParams p = {logits, weights, ids, T, E, K, ld_logits, renormalize,
                          (int)(logits_vector_ok(logits, logits_dtype, ld_logits) && (E == 64 || E == 128 || E == 256))};
-  const AlignOut o = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block};
+  const AlignOut o = {sorted_ids, sorted_cap, expert_ids, expert_ids_cap, counts, num_post_pad, numel, E, block,
+                      reciprocal_of(block)};
   uint32_t* table = (uint32_t*)ws;
 #define DLB_LAUNCH_ROUTE_ALIGN(VPL_)                                                                   \
   do {                                                                                                 \

@@ -34,3 +34,19 @@ def test_alignment_of_given_ids_at_launch_edges(dev, numel, E, block):
     rs, re_, rn, rc = og.align_block_size(ids, block, E)
     assert torch.equal(slots.cpu(), rs) and torch.equal(experts.cpu(), re_)
     assert int(total.item()) == int(rn.item()) and torch.equal(counts.cpu(), rc.to(torch.int32))
+
+
+# block sizes whose reciprocal is exact, inexact and the smallest; one expert with more blocks than threads, in one
+# launch, in two and in three
+@pytest.mark.parametrize("block", [1, 3, 7, 127, 1 << 16])
+@pytest.mark.parametrize("numel", [300, 4000, 30000, 530000])
+@pytest.mark.parametrize("E", [1, 3, 256])
+def test_blocks_of_one_expert(dev, block, numel, E):
+    from dlcompiler_amd.kernels.moe_gating import moe_align_block_size
+
+    ids = torch.full((numel, 1), E // 2, dtype=torch.int32)
+    ids[::11] = E - 1
+    slots, experts, total, counts = moe_align_block_size(ids.to(dev), block, E, return_counts=True)
+    rs, re_, rn, rc = og.align_block_size(ids, block, E)
+    assert torch.equal(slots.cpu(), rs) and torch.equal(experts.cpu(), re_)
+    assert int(total.item()) == int(rn.item()) and torch.equal(counts.cpu(), rc.to(torch.int32))
