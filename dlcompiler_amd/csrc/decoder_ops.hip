@@ -419,8 +419,8 @@ extern "C" int dlb_fill_kv_cache(const void* k_states, const void* v_states, voi
           mult16(p.k_row_bytes) && mult16(p.v_row_bytes) && mult16(p.ks_tok) && mult16(p.ks_head) &&
           mult16(p.vs_tok) && mult16(p.vs_head) && mult16(p.kc_page) && mult16(p.kc_slot) &&
           mult16(p.kc_head) && mult16(p.vc_page) && mult16(p.vc_slot) && mult16(p.vc_head);
-  hipLaunchKernelGGL(fill_kv_cache_kernel, dim3((uint32_t)ceil_div(num_tokens, kFillTokens)),
-                     dim3(64 * kFillTokens), 0, (hipStream_t)stream, p);
+  launch(fill_kv_cache_kernel, dim3((uint32_t)ceil_div(num_tokens, kFillTokens)),
+                     dim3(64 * kFillTokens), (hipStream_t)stream, p);
   return launch_status();
 }
 
@@ -450,10 +450,10 @@ extern "C" int dlb_rms_norm(const void* x, const void* weight, const void* resid
 #define DLB_LAUNCH_NORM_ANY(DT_)                                                                   \
   do {                                                                                             \
     if (residual)                                                                                  \
-      hipLaunchKernelGGL((rms_norm_any_kernel<DT_, true>), grid, block, 0, s, x, weight, residual, \
+      launch((rms_norm_any_kernel<DT_, true>), grid, block, s, x, weight, residual, \
                          out, out_residual, N, ld_x, ld_res, ld_out, ld_out_res, eps);             \
     else                                                                                           \
-      hipLaunchKernelGGL((rms_norm_any_kernel<DT_, false>), grid, block, 0, s, x, weight, residual, \
+      launch((rms_norm_any_kernel<DT_, false>), grid, block, s, x, weight, residual, \
                          out, out_residual, N, ld_x, ld_res, ld_out, ld_out_res, eps);             \
   } while (0)
     if (dtype == DLB_DTYPE_F32) DLB_LAUNCH_NORM_ANY(DLB_DTYPE_F32);
@@ -465,17 +465,17 @@ extern "C" int dlb_rms_norm(const void* x, const void* weight, const void* resid
   static_assert(kMaxVecF32 * 4 == kMaxVec * 8, "same row length limit for every element type");
   if (dtype == DLB_DTYPE_F32) {
     if (residual)
-      hipLaunchKernelGGL(rms_norm_f32_kernel<true>, grid, block, 0, s, (const float*)x,
+      launch(rms_norm_f32_kernel<true>, grid, block, s, (const float*)x,
                          (const float*)weight, (const float*)residual, (float*)out,
                          (float*)out_residual, N, ld_x, ld_res, ld_out, ld_out_res, eps);
     else
-      hipLaunchKernelGGL(rms_norm_f32_kernel<false>, grid, block, 0, s, (const float*)x,
+      launch(rms_norm_f32_kernel<false>, grid, block, s, (const float*)x,
                          (const float*)weight, (const float*)residual, (float*)out,
                          (float*)out_residual, N, ld_x, ld_res, ld_out, ld_out_res, eps);
     return launch_status();
   }
 #define DLB_LAUNCH_NORM(DT_, ADD_)                                                            \
-  hipLaunchKernelGGL((rms_norm_kernel<DT_, ADD_>), grid, block, 0, s, (const unsigned short*)x, \
+  launch((rms_norm_kernel<DT_, ADD_>), grid, block, s, (const unsigned short*)x, \
                      (const unsigned short*)weight, (const unsigned short*)residual,          \
                      (unsigned short*)out, (unsigned short*)out_residual, N, ld_x, ld_res,    \
                      ld_out, ld_out_res, eps)
@@ -515,7 +515,7 @@ extern "C" int dlb_apply_rotary_pos_emb(const void* q, const void* k, const void
   const dim3 grid((uint32_t)num_tokens), block(256);
   if (!vector_ok) {  // any even head size, any strides: one element pair per thread and step
 #define DLB_LAUNCH_ROTARY_ANY(DT_)                                                               \
-  hipLaunchKernelGGL(rotary_any_kernel<DT_>, grid, block, 0, s, q, k, cos, sin, q_out, k_out, Hq, \
+  launch(rotary_any_kernel<DT_>, grid, block, s, q, k, cos, sin, q_out, k_out, Hq, \
                      Hk, D, q_stride_tok, q_stride_head, k_stride_tok, k_stride_head,            \
                      qo_stride_tok, qo_stride_head, ko_stride_tok, ko_stride_head, cs_stride_tok)
     if (dtype == DLB_DTYPE_F32) DLB_LAUNCH_ROTARY_ANY(DLB_DTYPE_F32);
@@ -525,18 +525,18 @@ extern "C" int dlb_apply_rotary_pos_emb(const void* q, const void* k, const void
     return launch_status();
   }
   if (dtype == DLB_DTYPE_F32)
-    hipLaunchKernelGGL(rotary_f32_kernel, grid, block, 0, s, (const float*)q, (const float*)k,
+    launch(rotary_f32_kernel, grid, block, s, (const float*)q, (const float*)k,
                        (const float*)cos, (const float*)sin, (float*)q_out, (float*)k_out, Hq, Hk,
                        D, q_stride_tok, q_stride_head, k_stride_tok, k_stride_head, qo_stride_tok,
                        qo_stride_head, ko_stride_tok, ko_stride_head, cs_stride_tok);
   else if (dtype == DLB_DTYPE_BF16)
-    hipLaunchKernelGGL(rotary_kernel<DLB_DTYPE_BF16>, grid, block, 0, s, (const unsigned short*)q,
+    launch(rotary_kernel<DLB_DTYPE_BF16>, grid, block, s, (const unsigned short*)q,
                        (const unsigned short*)k, (const unsigned short*)cos,
                        (const unsigned short*)sin, (unsigned short*)q_out, (unsigned short*)k_out,
                        Hq, Hk, D, q_stride_tok, q_stride_head, k_stride_tok, k_stride_head,
                        qo_stride_tok, qo_stride_head, ko_stride_tok, ko_stride_head, cs_stride_tok);
   else
-    hipLaunchKernelGGL(rotary_kernel<DLB_DTYPE_F16>, grid, block, 0, s, (const unsigned short*)q,
+    launch(rotary_kernel<DLB_DTYPE_F16>, grid, block, s, (const unsigned short*)q,
                        (const unsigned short*)k, (const unsigned short*)cos,
                        (const unsigned short*)sin, (unsigned short*)q_out, (unsigned short*)k_out,
                        Hq, Hk, D, q_stride_tok, q_stride_head, k_stride_tok, k_stride_head,

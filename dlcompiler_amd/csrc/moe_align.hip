@@ -720,36 +720,36 @@ int launch_align(const IdxArray topk_ids, int64_t numel, int E, int block, int32
     if (quant && quant->total_groups > 0) {
       const uint32_t grid = (uint32_t)(1 + ceil_div(quant->total_groups, kQuantGroupsPerBlock * kOneQuantBlocks));
       if (quant_dtype == DLB_DTYPE_BF16)
-        hipLaunchKernelGGL(align_one_quant_kernel<DLB_DTYPE_BF16>, dim3(grid), dim3(kOneThreads), 0, s, out,
+        launch(align_one_quant_kernel<DLB_DTYPE_BF16>, dim3(grid), dim3(kOneThreads), s, out,
                            topk_ids, *quant);
       else
-        hipLaunchKernelGGL(align_one_quant_kernel<DLB_DTYPE_F16>, dim3(grid), dim3(kOneThreads), 0, s, out,
+        launch(align_one_quant_kernel<DLB_DTYPE_F16>, dim3(grid), dim3(kOneThreads), s, out,
                            topk_ids, *quant);
     } else {
-      hipLaunchKernelGGL(align_one_kernel, dim3(1), dim3(kOneThreads), 0, s, out, topk_ids);
+      launch(align_one_kernel, dim3(1), dim3(kOneThreads), s, out, topk_ids);
     }
     return launch_status();
   }
   const int64_t chunks = num_chunks(numel);
   const int chunk_ids = chunk_ids_for(numel);
-  hipLaunchKernelGGL(align_count_kernel, dim3((uint32_t)chunks), dim3(kThreads), 0, s, topk_ids,
+  launch(align_count_kernel, dim3((uint32_t)chunks), dim3(kThreads), s, topk_ids,
                      numel, E, chunk_ids, chunk_counts, sorted_ids, sorted_cap);
   if (chunks <= kFusedChunks) {
     const PlaceParams pp = {topk_ids, chunk_counts, (int)chunks, chunk_ids, out};
     if (quant && quant->total_groups > 0) {
       const uint32_t grid = (uint32_t)(chunks + 1 + ceil_div(quant->total_groups, kQuantGroupsPerBlock));
       if (quant_dtype == DLB_DTYPE_BF16)
-        hipLaunchKernelGGL(align_place_quant_kernel<DLB_DTYPE_BF16>, dim3(grid), dim3(kThreads), 0, s, pp, *quant);
+        launch(align_place_quant_kernel<DLB_DTYPE_BF16>, dim3(grid), dim3(kThreads), s, pp, *quant);
       else
-        hipLaunchKernelGGL(align_place_quant_kernel<DLB_DTYPE_F16>, dim3(grid), dim3(kThreads), 0, s, pp, *quant);
+        launch(align_place_quant_kernel<DLB_DTYPE_F16>, dim3(grid), dim3(kThreads), s, pp, *quant);
     } else {
-      hipLaunchKernelGGL(align_place_fused_kernel, dim3((uint32_t)chunks + 1), dim3(kThreads), 0, s, pp);
+      launch(align_place_fused_kernel, dim3((uint32_t)chunks + 1), dim3(kThreads), s, pp);
     }
     return launch_status();
   }
   if (quant) return DLB_ERR_UNSUPPORTED;  // (the caller launches the quantiser on its own then)
-  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_counts, chunks, out);
-  hipLaunchKernelGGL(align_place_kernel, dim3((uint32_t)chunks), dim3(kThreads), 0, s, topk_ids, numel, E,
+  launch(align_scan_kernel, dim3(1), dim3(kScanThreads), s, chunk_counts, chunks, out);
+  launch(align_place_kernel, dim3((uint32_t)chunks), dim3(kThreads), s, topk_ids, numel, E,
                      chunk_counts, sorted_ids);
   return launch_status();
 }
@@ -866,16 +866,16 @@ int route_chunk_tokens(int64_t T) { return (T + 63) / 64 <= kFusedChunks ? 64 : 
 template <int VPL, int LT>
 void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table, hipStream_t s) {
   if (p.T <= one_workgroup_tokens(VPL)) {
-    hipLaunchKernelGGL((route_align_one_kernel<VPL, LT>), dim3(1), dim3(kOneThreads), 0, s, p, o);
+    launch((route_align_one_kernel<VPL, LT>), dim3(1), dim3(kOneThreads), s, p, o);
     return;
   }
   const int chunk_tokens = route_chunk_tokens(p.T);
   const int chunks = (int)ceil_div(p.T, chunk_tokens);
   if (chunk_tokens == 64)
-    hipLaunchKernelGGL((route_count_kernel<VPL, 1, LT>), dim3(chunks), dim3(kOneThreads), 0, s, p, o, table);
+    launch((route_count_kernel<VPL, 1, LT>), dim3(chunks), dim3(kOneThreads), s, p, o, table);
   else
-    hipLaunchKernelGGL((route_count_kernel<VPL, 2, LT>), dim3(chunks), dim3(kOneThreads), 0, s, p, o, table);
-  hipLaunchKernelGGL(route_place_kernel, dim3(chunks), dim3(kThreads), 0, s, IdxArray{p.ids, 0}, o, table, chunks,
+    launch((route_count_kernel<VPL, 2, LT>), dim3(chunks), dim3(kOneThreads), s, p, o, table);
+  launch(route_place_kernel, dim3(chunks), dim3(kThreads), s, IdxArray{p.ids, 0}, o, table, chunks,
                      chunk_tokens * p.K);
 }
 

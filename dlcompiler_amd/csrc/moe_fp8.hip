@@ -699,9 +699,9 @@ extern "C" int dlb_per_token_group_quant_fp8(const void* x, void* xq, float* xs,
   const dim3 grid((uint32_t)ceil_div(q.total_groups, kQuantGroupsPerBlock));
   hipStream_t s = (hipStream_t)stream;
   if (dtype == DLB_DTYPE_BF16)
-    hipLaunchKernelGGL(quant_fp8_group128_kernel<DLB_DTYPE_BF16>, grid, dim3(kQuantThreads), 0, s, q);
+    launch(quant_fp8_group128_kernel<DLB_DTYPE_BF16>, grid, dim3(kQuantThreads), s, q);
   else
-    hipLaunchKernelGGL(quant_fp8_group128_kernel<DLB_DTYPE_F16>, grid, dim3(kQuantThreads), 0, s, q);
+    launch(quant_fp8_group128_kernel<DLB_DTYPE_F16>, grid, dim3(kQuantThreads), s, q);
   return launch_status();
 }
 
@@ -724,11 +724,11 @@ int launch_moe_gemm(const MoeGemmParams& p, int dtype, int w_layout, hipStream_t
 #define DLB_LAUNCH_GEMM(DT_)                                                               \
   do {                                                                                   \
     if (w_layout && once)                                                                       \
-      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, 1, true>), dim3(grid), dim3(256), 0, s, p);  \
+      launch((moe_gemm_kernel<GATED, DT_, 1, true>), dim3(grid), dim3(256), s, p);  \
     else if (w_layout)                                                                          \
-      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, 1, false>), dim3(grid), dim3(256), 0, s, p); \
+      launch((moe_gemm_kernel<GATED, DT_, 1, false>), dim3(grid), dim3(256), s, p); \
     else                                                                                        \
-      hipLaunchKernelGGL((moe_gemm_kernel<GATED, DT_, 0, false>), dim3(grid), dim3(256), 0, s, p); \
+      launch((moe_gemm_kernel<GATED, DT_, 0, false>), dim3(grid), dim3(256), s, p); \
   } while (0)
     if (dtype == DLB_DTYPE_BF16) DLB_LAUNCH_GEMM(DLB_DTYPE_BF16);
     else DLB_LAUNCH_GEMM(DLB_DTYPE_F16);
@@ -942,10 +942,10 @@ int launch_topk_sum(const void* in, void* out, int64_t num_tokens, int topk, int
 #define DLB_LAUNCH_SUM(DT_, TK_)                                                                       \
   do {                                                                                                 \
     if (shard)                                                                                         \
-      hipLaunchKernelGGL((moe_topk_sum_kernel<DT_, TK_, true>), grid, dim3(256), 0, s, (const u32x4*)in, \
+      launch((moe_topk_sum_kernel<DT_, TK_, true>), grid, dim3(256), s, (const u32x4*)in, \
                          (u32x4*)out, total, (int)(N / 8), topk, *shard);                              \
     else                                                                                               \
-      hipLaunchKernelGGL((moe_topk_sum_kernel<DT_, TK_, false>), grid, dim3(256), 0, s,                \
+      launch((moe_topk_sum_kernel<DT_, TK_, false>), grid, dim3(256), s,                \
                          (const u32x4*)in, (u32x4*)out, total, (int)(N / 8), topk, none);              \
   } while (0)
 #define DLB_DISPATCH_SUM(DT_)                 \

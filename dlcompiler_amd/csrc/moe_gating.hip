@@ -48,13 +48,13 @@ extern "C" int dlb_moe_topk_softmax_f32(const void* logits, float* weights, int3
 #define DLB_LAUNCH_ROUTE(LT_)                                                                      \
   do {                                                                                             \
     if (E <= 64)                                                                                   \
-      hipLaunchKernelGGL((moe_topk_softmax_kernel<4, LT_>), grid, block, 0, s, logits, weights, ids, \
+      launch((moe_topk_softmax_kernel<4, LT_>), grid, block, s, logits, weights, ids, \
                          T, E, K, ld_logits, renormalize, (int)(a16 && E == 64), probs, masks);    \
     else if (E <= 128)                                                                             \
-      hipLaunchKernelGGL((moe_topk_softmax_kernel<8, LT_>), grid, block, 0, s, logits, weights, ids, \
+      launch((moe_topk_softmax_kernel<8, LT_>), grid, block, s, logits, weights, ids, \
                          T, E, K, ld_logits, renormalize, (int)(a16 && E == 128), probs, masks);   \
     else                                                                                           \
-      hipLaunchKernelGGL((moe_topk_softmax_kernel<16, LT_>), grid, block, 0, s, logits, weights,   \
+      launch((moe_topk_softmax_kernel<16, LT_>), grid, block, s, logits, weights,   \
                          ids, T, E, K, ld_logits, renormalize, (int)(a16 && E == 256), probs,      \
                          masks);                                                                   \
   } while (0)

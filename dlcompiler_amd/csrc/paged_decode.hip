@@ -893,15 +893,15 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
 #define DLB_LAUNCH_SPLIT(DT_, D_, P2_, RG_)                                                                       \
   do {                                                                                                            \
     if (direct == 4)                                                                                              \
-      hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, D_, P2_, RG_, 4>), grid_direct, dim3(256), 0, s, p);    \
+      launch((paged_decode_direct_kernel<DT_, D_, P2_, RG_, 4>), grid_direct, dim3(256), s, p);    \
     else if (D_ == 64 && direct == 8)                                                                             \
-      hipLaunchKernelGGL((paged_decode_direct_kernel<DT_, 64, P2_, RG_, 8>), grid_direct, dim3(512), 0, s, p);    \
+      launch((paged_decode_direct_kernel<DT_, 64, P2_, RG_, 8>), grid_direct, dim3(512), s, p);    \
     else if (D_ % 64 == 0 && !RG_ && choice)                                                                      \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, D_ % 64 == 0 && !RG_, false>), grid1, dim3(64), 0, s, p); \
+      launch((paged_decode_split_kernel<DT_, D_, P2_, RG_, D_ % 64 == 0 && !RG_, false>), grid1, dim3(64), s, p); \
     else if (one)                                                                                                 \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, true>), grid1, dim3(64), 0, s, p);  \
+      launch((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, true>), grid1, dim3(64), s, p);  \
     else                                                                                                          \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, false>), grid1, dim3(64), 0, s, p); \
+      launch((paged_decode_split_kernel<DT_, D_, P2_, RG_, false, false>), grid1, dim3(64), s, p); \
   } while (0)
 #define DLB_LAUNCH_DECODE(DT_, D_)                                                                           \
   do {                                                                                                       \
@@ -913,17 +913,17 @@ extern "C" int dlb_paged_decode_attn(const void* q, const void* k_cache, const v
       else DLB_LAUNCH_SPLIT(DT_, D_, false, false);                                                          \
     }                                                                                                        \
     if (!direct && early)                                                                                    \
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_, true>), grid2, dim3(kCombineThreads), 0, s, p); \
+      launch((paged_decode_combine_kernel<DT_, D_, true>), grid2, dim3(kCombineThreads), s, p); \
     else if (!direct)                                                                                        \
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, D_, false>), grid2, dim3(kCombineThreads), 0, s, p); \
+      launch((paged_decode_combine_kernel<DT_, D_, false>), grid2, dim3(kCombineThreads), s, p); \
   } while (0)
 #define DLB_LAUNCH_DECODE_256(DT_)                                                                           \
   do {                                                                                                       \
     if (p.page_shift >= 0)                                                                                   \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, true, true, false, false>), grid1, dim3(64), 0, s, p);        \
+      launch((paged_decode_split_kernel<DT_, 256, true, true, false, false>), grid1, dim3(64), s, p);        \
     else                                                                                                     \
-      hipLaunchKernelGGL((paged_decode_split_kernel<DT_, 256, false, true, false, false>), grid1, dim3(64), 0, s, p);       \
-    hipLaunchKernelGGL((paged_decode_combine_kernel<DT_, 256, false>), grid2, dim3(kCombineThreads), 0, s, p);       \
+      launch((paged_decode_split_kernel<DT_, 256, false, true, false, false>), grid1, dim3(64), s, p);       \
+    launch((paged_decode_combine_kernel<DT_, 256, false>), grid2, dim3(kCombineThreads), s, p);       \
   } while (0)
 #define DLB_DISPATCH_DECODE(DT_)                        \
   do {                                                  \

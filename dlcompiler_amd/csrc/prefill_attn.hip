@@ -940,9 +940,9 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
 #define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_, PK_)                                                          \
   do {                                                                                                         \
     if (ragged)                                                                                                \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, true, RW_, PK_>), grid, dim3(kThreads), 0, s, p);   \
+      launch((prefill_attn_kernel<DT_, D_, PG_, true, RW_, PK_>), grid, dim3(kThreads), s, p);   \
     else                                                                                                       \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, D_, PG_, false, RW_, PK_>), grid, dim3(kThreads), 0, s, p);  \
+      launch((prefill_attn_kernel<DT_, D_, PG_, false, RW_, PK_>), grid, dim3(kThreads), s, p);  \
   } while (0)
 #define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                                          \
   do {                                                                            \
@@ -953,7 +953,7 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
 #define DLB_DISPATCH_PREFILL_DT(DT_, PG_)                                                               \
   do {                                                                                                  \
     if (D == 256)                                                                                       \
-      hipLaunchKernelGGL((prefill_attn_kernel<DT_, 256, PG_, true, 4, false>), grid, dim3(kThreads), 0, s, p); \
+      launch((prefill_attn_kernel<DT_, 256, PG_, true, 4, false>), grid, dim3(kThreads), s, p); \
     else if (D == 128) DLB_LAUNCH_PREFILL(DT_, 128, PG_);                                               \
     else if (D == 96) DLB_LAUNCH_PREFILL(DT_, 96, PG_);                                                 \
     else DLB_LAUNCH_PREFILL(DT_, 64, PG_);                                                              \
@@ -979,9 +979,9 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   if (p.nsplit > 1) {
     const dim3 rows((uint32_t)ceil_div((int64_t)max_len * Hq, kCombineRows), (uint32_t)B);
     if (dtype == DLB_DTYPE_BF16)
-      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_BF16>, rows, dim3(32 * kCombineRows), 0, s, p);
+      launch(prefill_combine_kernel<DLB_DTYPE_BF16>, rows, dim3(32 * kCombineRows), s, p);
     else
-      hipLaunchKernelGGL(prefill_combine_kernel<DLB_DTYPE_F16>, rows, dim3(32 * kCombineRows), 0, s, p);
+      launch(prefill_combine_kernel<DLB_DTYPE_F16>, rows, dim3(32 * kCombineRows), s, p);
   }
   return launch_status();
 }

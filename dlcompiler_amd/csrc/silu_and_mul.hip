@@ -106,13 +106,13 @@ int launch_16bit(const void* x, void* out, int64_t M, int64_t N, int64_t ldx, in
                       M * (ldx / VEC) < (int64_t)0xffffffffu && M * (ldo / VEC) < (int64_t)0xffffffffu;
   if (vec_ok) {
     const uint32_t blocks = (uint32_t)ceil_div(total_vec, 256 * UNROLL);
-    hipLaunchKernelGGL((silu_and_mul_vec16<DT, UNROLL>), dim3(blocks), dim3(256), 0, s,
+    launch((silu_and_mul_vec16<DT, UNROLL>), dim3(blocks), dim3(256), s,
                        (const u32x4*)x, (u32x4*)out, (uint32_t)total_vec, (uint32_t)(N / VEC),
                        (uint32_t)(ldx / VEC), (uint32_t)(ldo / VEC));
   } else {
     const int64_t blocks = ceil_div(M * N, 256);
-    hipLaunchKernelGGL((silu_and_mul_scalar<DT>), dim3((uint32_t)(blocks < 65536 ? blocks : 65536)),
-                       dim3(256), 0, s, x, out, M, N, ldx, ldo);
+    launch((silu_and_mul_scalar<DT>), dim3((uint32_t)(blocks < 65536 ? blocks : 65536)),
+                       dim3(256), s, x, out, M, N, ldx, ldo);
   }
   return launch_status();
 }
@@ -138,13 +138,13 @@ extern "C" int dlb_silu_and_mul(const void* x, void* out, int64_t M, int64_t N, 
                           aligned16(out) && total_vec < (int64_t)0xffffff00u &&
                           M * (ld_x / 4) < (int64_t)0xffffffffu;
       if (vec_ok) {
-        hipLaunchKernelGGL(silu_and_mul_f32_vec16, dim3((uint32_t)ceil_div(total_vec, 256)),
-                           dim3(256), 0, s, (const f32x4*)x, (f32x4*)out, (uint32_t)total_vec,
+        launch(silu_and_mul_f32_vec16, dim3((uint32_t)ceil_div(total_vec, 256)),
+                           dim3(256), s, (const f32x4*)x, (f32x4*)out, (uint32_t)total_vec,
                            (uint32_t)(N / 4), (uint32_t)(ld_x / 4), (uint32_t)(ld_out / 4));
       } else {
         const int64_t blocks = ceil_div(M * N, 256);
-        hipLaunchKernelGGL((silu_and_mul_scalar<DLB_DTYPE_F32>),
-                           dim3((uint32_t)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, s, x,
+        launch((silu_and_mul_scalar<DLB_DTYPE_F32>),
+                           dim3((uint32_t)(blocks < 65536 ? blocks : 65536)), dim3(256), s, x,
                            out, M, N, ld_x, ld_out);
       }
       return launch_status();
