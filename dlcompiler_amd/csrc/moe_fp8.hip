@@ -787,6 +787,7 @@ int fill_gemm_params(MoeGemmParams& p, bool gated, int elem, const void* a, cons
   p.K = Kel * elem;
   p.N = N;
   p.KC = p.K / 128;
+  p.kc_rcp = p.KC > 1 ? (uint32_t)(0x100000000ull / (uint32_t)p.KC) : 0;
   p.topk = topk;
   p.numel = num_tokens * topk;
   p.num_tokens = num_tokens;
@@ -1083,8 +1084,16 @@ extern "C" int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const v
   const int64_t eids_cap = ceil_div(cap, block);
   int32_t* post = (int32_t*)(base + l.num_post);
   const size_t align_bytes = dlb_moe_align_ws_bytes(numel, num_experts);
+  const bool few = quantised && numel <= (int64_t)kSmallMeanRows * num_experts;
+  // (the scratch of the fp8 intermediate has whole blocks of rows for every expert)
+  if (few && moe_hands_over_f32(up) && 4 * numel <= l.used_mblocks * block) {
+    up.h32 = down.h32 = (float*)h;
+    down.a_scale = nullptr;
+    down.a_rows = numel;
+    down.lda = (int64_t)I * 4;
+  }
   // a few rows per expert: gate_up quantises what it loads, and there is nothing to launch before it
-  if (quantised && aligned && numel <= (int64_t)kSmallMeanRows * num_experts && aligned16(x) && ld_x % 8 == 0 &&
+  if (few && aligned && aligned16(x) && ld_x % 8 == 0 &&
       T * ld_x * 2 < (int64_t)0xffffffffu) {
     up.a = (const unsigned char*)x;
     up.a_scale = nullptr;

@@ -37,6 +37,10 @@ struct MoeGemmParams {
   void* out;                  // [numel, N] bf16/f16
   const float* topk_w;        // [numel]
   int64_t lda;                // gated fp8, few rows: `a` is 16-bit, rows of lda bytes (0: quantised)
+  uint32_t kc_rcp;            // 2^32 / KC, rounded down (KC > 1)
+  // fp8, very few rows (see moe_hands_over_f32): the intermediate is [numel, I] fp32, by routing slot, which
+  // gate_up leaves in h32 and the down GEMM, whose `a` it is, quantises as it loads it
+  float* h32;
   int renorm;                 // weights are divided by the sum of their token's
 };
 
@@ -73,6 +77,8 @@ struct TileId {
   int rows;  // real (unpadded) rows of the tile
 };
 
+// Do a layer's GEMMs hand the intermediate over in fp32?  (up: of the gate_up GEMM, with 16-bit activations)
+bool moe_hands_over_f32(const MoeGemmParams& up);
 // Launches the streaming kernel.  gated / quantised as the entry points; N_out checks are done.
 int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dtype, int w_layout, hipStream_t s);
 // fp8: up to this many rows per expert, on average over the routed slots, the streaming kernel is the

@@ -34,6 +34,41 @@ constexpr int kQuantThreads = 256;
 constexpr int kQuantUnroll = 4;  // groups per DPP row and workgroup pass (loads issued together)
 constexpr int kQuantGroupsPerBlock = (kQuantThreads / 16) * kQuantUnroll;
 
+// One group by a DPP row, eight 16-bit values a lane: the lane's eight bytes, and the group's scale in every lane.
+template <int DT>
+__device__ __forceinline__ u32x2 quantise_group(const u32x4& raw, float& scale) {
+  float v[8];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    v[2 * w] = Elem<DT>::lo(raw[w]);
+    v[2 * w + 1] = Elem<DT>::hi(raw[w]);
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+  amax = row16_max(amax);
+  scale = fmaxf(amax, kQuantEps) / kFp8Max;
+  const float inv = 1.0f / scale, by = scale == __builtin_inff() ? 0.0f : scale;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = divide_by_scale(v[j], by, inv);
+  return u32x2{pack4_fp8(v[0], v[1], v[2], v[3]), pack4_fp8(v[4], v[5], v[6], v[7])};
+}
+
+// ... of eight fp32 values a lane, to the bytes that the epilogue of the gate_up GEMM gives
+__device__ __forceinline__ u32x2 quantise_group_f32(const u32x4& lo, const u32x4& hi, float& scale) {
+  float v[8], amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    v[j] = __uint_as_float(j < 4 ? lo[j] : hi[j - 4]);
+    amax = fmaxf(amax, fabsf(v[j]));
+  }
+  scale = fmaxf(row16_max(amax), kQuantEps) / kFp8Max;
+  const float inv = __builtin_amdgcn_rcpf(scale);  // the stored scale stays exact
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] *= inv;
+  return u32x2{pack4_fp8(v[0], v[1], v[2], v[3]), pack4_fp8(v[4], v[5], v[6], v[7])};
+}
+
 struct QuantParams {
   const unsigned short* x;
   unsigned char* xq;
@@ -73,24 +108,9 @@ __device__ __forceinline__ void quant_fp8_group128_block(const QuantParams& q, i
   }
 #pragma unroll
   for (int u = 0; u < kQuantUnroll; ++u) {
-    float v[8];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      v[2 * w] = Elem<DT>::lo(raw[u][w]);
-      v[2 * w + 1] = Elem<DT>::hi(raw[u][w]);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    amax = row16_max(amax);
-    const float scale = fmaxf(amax, kQuantEps) / kFp8Max;
-    const float inv = 1.0f / scale, by = scale == __builtin_inff() ? 0.0f : scale;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = divide_by_scale(v[j], by, inv);
+    float scale;
+    const u32x2 o = quantise_group<DT>(raw[u], scale);
     if (live[u]) {
-      u32x2 o;
-      o[0] = pack4_fp8(v[0], v[1], v[2], v[3]);
-      o[1] = pack4_fp8(v[4], v[5], v[6], v[7]);
       *(u32x2*)(q.xq + row[u] * q.ldq + gc[u] * 128 + lane16 * 8) = o;
       if (lane16 == 0) q.xs[row[u] * q.lds + gc[u]] = scale;
     }
