@@ -36,10 +36,6 @@ struct PrefillParams {
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;  // token / head strides (elements)
   int Hq, Hkv, group;
   int xcd_heads;  // heads (head groups) per XCD, != 0: remap blockIdx.x so a KV group's share an XCD
-  // kernels without PACK: query heads whose 32-query blocks share workgroups (group or 1), and what a block's
-  // number in their order is multiplied by for its quotient by them (0: 1)
-  int share;
-  unsigned int share_rcp;
   // PACK kernels: a workgroup's rows are those of 1 << pack_shift query heads of a KV group, the rows of
   // each being (kBlockM >> pack_shift) queries
   int pack_shift;
@@ -63,6 +59,7 @@ struct PrefillParams {
   // generic masking (both layouts): sliding window (> 0) and logit soft-cap (> 0)
   int window;
   float softcap, sm_scale;
+  unsigned int share_rcp;  // SHARE kernels: a block's number in their order times this is its quotient by the heads
 };
 
 template <int DT>
@@ -151,7 +148,7 @@ struct Smem {
 // PACK: short query runs over a history (every run fits a fraction of the rows): the heads of a KV
 // group share a workgroup, so the rows are filled and K/V is staged once for all of them; and the
 // key tiles may be split over workgroups.
-template <int DT, int D, int PAGED, bool RAGGED, int RW, bool PACK>
+template <int DT, int D, int PAGED, bool RAGGED, int RW, bool PACK, bool SHARE = false>
 __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefill_attn_kernel(const PrefillParams p) {
   constexpr int KG = 4 / RW;
   constexpr int kBlockM = 32 * RW;  // query rows per workgroup
@@ -219,18 +216,18 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   const int pack = PACK ? p.pack_shift : 0;
   const int qtile = gridDim.y - 1 - blockIdx.y;  // heaviest first
   // SHARE: a wave's rows are 32 queries of one head, and a workgroup takes the next four of the order
-  // (query block, head): with the heads of a KV group in that order its waves see the same keys, where those
+  // (query block, head) of a KV group: with the heads of a KV group in that order its waves see the same keys, where those
   // of 128 queries of one head reach the diagonal one after the other, and only a sequence's last workgroup
   // has waves without rows.
-  constexpr bool SHARE = RW == 4 && !PACK;
+  static_assert(!SHARE || (RW == 4 && !PACK), "");
   int q0 = qtile * (kBlockM >> pack), span = kBlockM >> pack;  // queries of the workgroup: first, how many
   int wave_q0 = 0, wave_head = 0;                              // of the wave: offset of its first query, head
   int block_head = 0;                                          // head of the workgroup's first wave
   if (SHARE) {
     const int unit0 = qtile * RW;
-    const int first = p.share > 1 ? (int)__umulhi((unsigned)unit0, p.share_rcp) : unit0;
+    const int first = (int)__umulhi((unsigned)unit0, p.share_rcp);
     q0 = 32 * first;
-    block_head = unit0 - first * p.share;
+    block_head = unit0 - first * p.group;
   }
   if (q0 >= L) return;
   if (SHARE) {
@@ -239,8 +236,8 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
       hd = block_head + w;
 #pragma unroll
       for (int i = 1; i < RW; ++i)
-        if (hd >= p.share) {
-          hd -= p.share;
+        if (hd >= p.group) {
+          hd -= p.group;
           dq += 32;
         }
     };
@@ -268,7 +265,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : RW == 2 ? 1 : 2) void prefi
   int head = blockIdx.x;  // PACK: first of the workgroup's heads
   if (p.xcd_heads) head = (blockIdx.x & 7) * p.xcd_heads + (blockIdx.x >> 3);
   if (PACK) head <<= pack;
-  else if (SHARE) head *= p.share;
+  else if (SHARE) head *= p.group;
   const int kvh = head / p.group;
 
   const int tid = threadIdx.x;
@@ -924,39 +921,43 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   const int row_waves = small ? 2 : 4;
   const int64_t all_wgs = ceil_div(max_len, 128) * B * Hq, slots = (int64_t)current_device_cu_count() * (D <= 64 ? 4 : 2);
   int64_t qtiles = ceil_div(ceil_div(max_len, 32) * p.group, row_waves);
-  p.share = !plan.use && !small && all_wgs > (paged ? 3 : 2) * slots && (8 % Hkv == 0 || Hkv % 8 == 0) && qtiles <= 65535 &&
-                    p.group <= 4096 ? p.group : 1;
+  // (A kernel of its own: where heads do not share, its longer start costs 1 %, 16 heads, 16 kv, of 64: 176.2 / 178.7.)
+  const bool share = !plan.use && !small && all_wgs > (paged ? 3 : 2) * slots && (8 % Hkv == 0 || Hkv % 8 == 0) &&
+                     qtiles <= 65535 && p.group > 1 && p.group <= 4096;
   // (exact: numbers below 2^18, at most 2^12 heads)
-  p.share_rcp = p.share > 1 ? (unsigned int)(0x100000000ull / p.share + 1) : 0;
-  if (p.share == 1) qtiles = ceil_div(max_len, 32 * row_waves);
+  p.share_rcp = share ? (unsigned int)(0x100000000ull / p.group + 1) : 0;
+  if (!share) qtiles = ceil_div(max_len, 32 * row_waves);
   if (plan.use) qtiles = ceil_div(max_len, 128 >> p.pack_shift);
   if (qtiles > 65535 || (int64_t)B * p.nsplit > 65535) return DLB_ERR_UNSUPPORTED;
-  const int head_groups = plan.use ? Hq >> p.pack_shift : Hq / p.share;
+  const int head_groups = plan.use ? Hq >> p.pack_shift : share ? Hkv : Hq;
   // workgroups are dealt round-robin to the 8 XCDs by linear id; with Hq % 8 == 0 the
   // remap in the kernel puts heads {x, x+8, ...} -> consecutive heads on one XCD so a KV
   // group's four query heads hit the same L2.
   p.xcd_heads = head_groups % 8 == 0 && head_groups >= 16 ? head_groups >> 3 : 0;
   const dim3 grid = dim3((uint32_t)head_groups, (uint32_t)qtiles, (uint32_t)(B * p.nsplit));
-#define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_, PK_)                                                          \
-  do {                                                                                                         \
-    if (ragged)                                                                                                \
-      launch((prefill_attn_kernel<DT_, D_, PG_, true, RW_, PK_>), grid, dim3(kThreads), s, p);   \
-    else                                                                                                       \
-      launch((prefill_attn_kernel<DT_, D_, PG_, false, RW_, PK_>), grid, dim3(kThreads), s, p);  \
+#define DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, RW_, PK_, SH_)                                                    \
+  do {                                                                                                        \
+    if (ragged)                                                                                               \
+      launch((prefill_attn_kernel<DT_, D_, PG_, true, RW_, PK_, SH_>), grid, dim3(kThreads), s, p);           \
+    else                                                                                                      \
+      launch((prefill_attn_kernel<DT_, D_, PG_, false, RW_, PK_, SH_>), grid, dim3(kThreads), s, p);          \
   } while (0)
-#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                                          \
-  do {                                                                            \
-    if (PG_ != 0 && plan.use) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, (PG_ != 0)); \
-    else if (small) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 2, false);                \
-    else DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, false);                           \
+#define DLB_LAUNCH_PREFILL(DT_, D_, PG_)                                                 \
+  do {                                                                                   \
+    if (PG_ != 0 && plan.use) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, (PG_ != 0), false); \
+    else if (small) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 2, false, false);                \
+    else if (share) DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, false, true);                 \
+    else DLB_LAUNCH_PREFILL_RW(DT_, D_, PG_, 4, false, false);                           \
   } while (0)
-#define DLB_DISPATCH_PREFILL_DT(DT_, PG_)                                                               \
-  do {                                                                                                  \
-    if (D == 256)                                                                                       \
-      launch((prefill_attn_kernel<DT_, 256, PG_, true, 4, false>), grid, dim3(kThreads), s, p); \
-    else if (D == 128) DLB_LAUNCH_PREFILL(DT_, 128, PG_);                                               \
-    else if (D == 96) DLB_LAUNCH_PREFILL(DT_, 96, PG_);                                                 \
-    else DLB_LAUNCH_PREFILL(DT_, 64, PG_);                                                              \
+#define DLB_DISPATCH_PREFILL_DT(DT_, PG_)                                                                       \
+  do {                                                                                                          \
+    if (D == 256 && share)                                                                                      \
+      launch((prefill_attn_kernel<DT_, 256, PG_, true, 4, false, true>), grid, dim3(kThreads), s, p);           \
+    else if (D == 256)                                                                                          \
+      launch((prefill_attn_kernel<DT_, 256, PG_, true, 4, false, false>), grid, dim3(kThreads), s, p);          \
+    else if (D == 128) DLB_LAUNCH_PREFILL(DT_, 128, PG_);                                                       \
+    else if (D == 96) DLB_LAUNCH_PREFILL(DT_, 96, PG_);                                                         \
+    else DLB_LAUNCH_PREFILL(DT_, 64, PG_);                                                                      \
   } while (0)
 #define DLB_DISPATCH_PREFILL(PG_)                                               \
   if (dtype == DLB_DTYPE_BF16) DLB_DISPATCH_PREFILL_DT(DLB_DTYPE_BF16, PG_);    \
