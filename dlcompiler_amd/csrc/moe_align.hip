@@ -122,6 +122,10 @@ uint32_t reciprocal_of(int block) { return block > 1 ? (uint32_t)(0x100000000ull
 __device__ __forceinline__ void write_block_experts(const AlignOut& o, const int32_t* base_s, int t, int nt) {
   const int32_t total_padded = base_s[o.E];
   if (t == 0) *o.num_post_pad = total_padded;
+  // (no more threads than blocks: a workgroup without a share, which has a full chunk behind it where the first ones
+  // have the short last one's, leaves at once; 1220 tokens x 8 of 64, 9.7 -> 9.5 us)
+  if (o.expert_ids_cap < nt) nt = (int)(o.expert_ids_cap + kMaxE - 1) / kMaxE * kMaxE;
+  if (t >= nt) return;
   const int shift = o.E > 1 ? 32 - __builtin_clz(o.E - 1) : 0;  // experts, rounded up to a power of two
   const int e = t & ((1 << shift) - 1);
   if (e < o.E) {
