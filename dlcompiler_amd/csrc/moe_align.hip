@@ -250,13 +250,13 @@ struct RouteParams {
 };
 
 // Router, then the alignment of its own selections, in one workgroup: 64 tokens per pass.  A pass keeps
-// the CU's SIMDs busy, so past one or two of them the second launch is the cheaper way (64 experts,
-// 128 tokens: 9.1 against 9.4 us, 256 tokens 14.9 against 9.2; 256 experts, 64 tokens: 11.1 against
-// 13.4, 100 tokens 14.8 against 13.1).
+// the CU's SIMDs busy, so past some tokens the second launch, whose router has 16 of them on a CU, is the
+// cheaper way (one / two launches, fp32, us: 64 experts, 80 tokens 6.8 / 7.3, 96 7.35 / 7.3, 128 9.0 / 7.4; 128
+// experts, 48 tokens 7.6 / 8.1, 64 8.6 / 8.1; 256 experts, 32 tokens 9.2 / 10.0, 48 11.2 / 9.8).
 constexpr int one_workgroup_tokens(int experts_per_lane) {
-  return experts_per_lane == 4 ? 128 : experts_per_lane == 8 ? 96 : 80;
+  return experts_per_lane == 4 ? 96 : experts_per_lane == 8 ? 56 : 36;
 }
-constexpr int kRouteSlots = 128 * 16;
+constexpr int kRouteSlots = one_workgroup_tokens(4) * 16;
 static_assert(kRouteSlots <= kOneSlots, "the routed slots fit one workgroup's alignment");
 template <int VPL, int LT>
 __global__ __launch_bounds__(kOneThreads) void route_align_one_kernel(const RouteParams p, const AlignOut o) {
@@ -280,31 +280,33 @@ __global__ __launch_bounds__(kOneThreads) void route_align_one_kernel(const Rout
   align_one_workgroup(o, s, [&](int, int i) { return ids_s[i]; });
 }
 
-// More tokens: two launches.  First the router, 64 * PASSES tokens per workgroup, which also
+// More tokens: two launches.  First the router, THREADS / 16 * PASSES tokens per workgroup, which also
 // writes a row of the [chunks, E] count table: the experts selected by exactly those tokens.  A
 // token selects an expert at most once, so a count fits a byte, and the table the second launch
 // reduces in every workgroup is a quarter of what 32-bit counts take.  The pad value goes
 // everywhere meanwhile (the second launch scatters the slots over it).  Both launches are bound by
 // latency: 16384 tokens x 6 of 64 experts 15.7 -> 12.8 us a call, 9336 x 8 of 256 43.9 -> 16.6 us.
-template <int VPL, int PASSES, int LT>
-__global__ __launch_bounds__(kOneThreads) void route_count_kernel(const RouteParams p, const AlignOut o,
+template <int VPL, int THREADS, int PASSES, int LT>
+__global__ __launch_bounds__(THREADS) void route_count_kernel(const RouteParams p, const AlignOut o,
                                                                   uint32_t* __restrict__ table) {
-  static_assert(64 * PASSES < 256, "counts are bytes");
+  constexpr int kRows = THREADS / 16;  // tokens per pass
+  static_assert(kRows * PASSES < 256, "counts are bytes");
+  static_assert(THREADS >= kMaxE, "a thread per expert");
   __shared__ int32_t hist[kMaxE];
   if (threadIdx.x < kMaxE) hist[threadIdx.x] = 0;
-  const int64_t first = (int64_t)blockIdx.x * (64 * PASSES);
+  const int64_t first = (int64_t)blockIdx.x * (kRows * PASSES);
   float v[PASSES][VPL];
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {  // all loads first: one memory round trip
-    const int64_t token = first + pass * 64 + (threadIdx.x >> 4);
+    const int64_t token = first + pass * kRows + (threadIdx.x >> 4);
     load_token_logits<VPL, LT>(p.logits, token, token < p.T, p.E, p.ld, p.vec_ok, v[pass]);
   }
-  fill_words(o.sorted_ids, o.sorted_cap, (int32_t)o.numel, (int64_t)blockIdx.x * kOneThreads + threadIdx.x,
-             (int64_t)gridDim.x * kOneThreads);
+  fill_words(o.sorted_ids, o.sorted_cap, (int32_t)o.numel, (int64_t)blockIdx.x * THREADS + threadIdx.x,
+             (int64_t)gridDim.x * THREADS);
   __syncthreads();
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
-    const int64_t token = first + pass * 64 + (threadIdx.x >> 4);
+    const int64_t token = first + pass * kRows + (threadIdx.x >> 4);
     const int32_t e = route_token<VPL, LT>(v[pass], p.weights, p.ids, token, token < p.T, p.E, p.K, p.renorm);
     if (e >= 0) atomicAdd(&hist[e], 1);  // integer add: order-insensitive
   }
@@ -857,28 +859,44 @@ extern "C" int dlb_moe_align_block_size_static(const void* topk_ids, int ids_int
 
 // ---------------------------------------------------------------------------------------
 // Router and alignment as one pipeline: one workgroup up to one_workgroup_tokens, else the router with
-// per-chunk expert counts (a chunk = the K routing slots of route_chunk_tokens(T) consecutive
+// per-chunk expert counts (a chunk = the K routing slots of route_chunk_tokens consecutive
 // tokens) and the placement.
 // ---------------------------------------------------------------------------------------
 namespace dlb {
 namespace {
 
-// tokens per workgroup of the router: 64 (one pass) while that keeps the count table within
-// kFusedChunks rows, else 128 (two passes)
-int route_chunk_tokens(int64_t T) { return (T + 63) / 64 <= kFusedChunks ? 64 : 128; }
+// Tokens per workgroup of the router.  Its arg-max rounds keep the SIMDs busy, so the fewer tokens a CU has the
+// better, but every placing workgroup reduces the whole count table: 16 tokens while it reads that at once, 32
+// while the table stays within kFusedChunks rows, as 64 (one pass) after that, else 128 (two passes).  64 / 32 / 16
+// tokens, us in fp32: 256 experts, 8 each, 1024 tokens 14.9 / 10.9 / 10.2, 4096 15.4 / 12.3 / 13.7; 128 experts,
+// 2048 tokens 11.1 / 8.9 / 8.7, 4096 11.4 / 9.3 / 9.9; 64 experts, 6 each, 200 tokens 8.5 / 7.4 / 7.3, 4096 9.1 / 7.9 /
+// 7.9, 6000 9.1 / 8.0.
+int route_chunk_tokens(int64_t T, int E) {
+  const int at_once = 16 * kThreads / (E <= 64 ? 16 : E <= 128 ? 32 : 64);
+  if (ceil_div(T, 16) <= at_once) return 16;
+  for (int tokens = 32; tokens < 128; tokens *= 2)
+    if (ceil_div(T, tokens) <= kFusedChunks) return tokens;
+  return 128;
+}
+size_t route_ws_bytes(int64_t T, int E, int chunk_tokens) {
+  return (size_t)(T > 0 ? ceil_div(T, chunk_tokens) : 1) * (size_t)((E + 3) / 4) * sizeof(uint32_t);
+}
 
 template <int VPL, int LT>
-void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table, hipStream_t s) {
+void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table, int chunk_tokens, hipStream_t s) {
   if (p.T <= one_workgroup_tokens(VPL)) {
     launch((route_align_one_kernel<VPL, LT>), dim3(1), dim3(kOneThreads), s, p, o);
     return;
   }
-  const int chunk_tokens = route_chunk_tokens(p.T);
   const int chunks = (int)ceil_div(p.T, chunk_tokens);
-  if (chunk_tokens == 64)
-    launch((route_count_kernel<VPL, 1, LT>), dim3(chunks), dim3(kOneThreads), s, p, o, table);
+  if (chunk_tokens == 16)
+    launch((route_count_kernel<VPL, 256, 1, LT>), dim3(chunks), dim3(256), s, p, o, table);
+  else if (chunk_tokens == 32)
+    launch((route_count_kernel<VPL, 512, 1, LT>), dim3(chunks), dim3(512), s, p, o, table);
+  else if (chunk_tokens == 64)
+    launch((route_count_kernel<VPL, 1024, 1, LT>), dim3(chunks), dim3(1024), s, p, o, table);
   else
-    launch((route_count_kernel<VPL, 2, LT>), dim3(chunks), dim3(kOneThreads), s, p, o, table);
+    launch((route_count_kernel<VPL, 1024, 2, LT>), dim3(chunks), dim3(1024), s, p, o, table);
   launch(route_place_kernel, dim3(chunks), dim3(kThreads), s, IdxArray{p.ids, 0}, o, table, chunks,
                      chunk_tokens * p.K);
 }
@@ -888,8 +906,7 @@ void launch_route_align(const RouteParams& p, const AlignOut& o, uint32_t* table
 
 extern "C" size_t dlb_moe_topk_softmax_align_ws_bytes(int64_t T, int E) {
   if (T < 0 || E < 1) return 0;
-  const int64_t chunks = T > 0 ? dlb::ceil_div(T, dlb::route_chunk_tokens(T)) : 1;
-  return (size_t)chunks * (size_t)((E + 3) / 4) * sizeof(uint32_t);
+  return dlb::route_ws_bytes(T, E, dlb::route_chunk_tokens(T, E));
 }
 
 extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights, int32_t* ids,
@@ -907,15 +924,16 @@ extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights
     return DLB_ERR_UNSUPPORTED;
   const int64_t numel = T * K;
   if (numel + (int64_t)E * block >= (int64_t)0x7fffffff) return DLB_ERR_UNSUPPORTED;
-  const int chunk_tokens = route_chunk_tokens(T);
-  const int64_t chunks = T > 0 ? ceil_div(T, chunk_tokens) : 1;
   // larger inputs take the two separate entry points (their scan runs as its own launch)
-  if (chunks > kFusedChunks) return DLB_ERR_UNSUPPORTED;
+  int chunk_tokens = route_chunk_tokens(T, E);
+  if (T > (int64_t)kFusedChunks * chunk_tokens) return DLB_ERR_UNSUPPORTED;
+  // (a scratch for chunks of 64 tokens is enough)
+  while (chunk_tokens < 64 && ws_bytes < route_ws_bytes(T, E, chunk_tokens)) chunk_tokens *= 2;
   if (!sorted_ids || !expert_ids || !num_post_pad || (T > 0 && (!logits || !weights || !ids)))
     return DLB_ERR_BAD_ARG;
   if (sorted_cap < numel + (int64_t)E * (block - 1)) return DLB_ERR_BAD_ARG;
   if (expert_ids_cap < ceil_div(sorted_cap, block)) return DLB_ERR_BAD_ARG;
-  if (!ws || ws_bytes < dlb_moe_topk_softmax_align_ws_bytes(T, E)) return DLB_ERR_WORKSPACE;
+  if (!ws || ws_bytes < route_ws_bytes(T, E, chunk_tokens)) return DLB_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   const RouteParams p = {logits, weights, ids, T, E, K, ld_logits, renormalize,
                          (int)(logits_vector_ok(logits, logits_dtype, ld_logits) && (E == 64 || E == 128 || E == 256))};
@@ -924,9 +942,9 @@ extern "C" int dlb_moe_topk_softmax_align_f32(const void* logits, float* weights
   uint32_t* table = (uint32_t*)ws;
 #define DLB_LAUNCH_ROUTE_ALIGN(VPL_)                                                                   \
   do {                                                                                                 \
-    if (logits_dtype == DLB_DTYPE_F32) launch_route_align<VPL_, DLB_DTYPE_F32>(p, o, table, s);        \
-    else if (logits_dtype == DLB_DTYPE_BF16) launch_route_align<VPL_, DLB_DTYPE_BF16>(p, o, table, s); \
-    else launch_route_align<VPL_, DLB_DTYPE_F16>(p, o, table, s);                                      \
+    if (logits_dtype == DLB_DTYPE_F32) launch_route_align<VPL_, DLB_DTYPE_F32>(p, o, table, chunk_tokens, s);        \
+    else if (logits_dtype == DLB_DTYPE_BF16) launch_route_align<VPL_, DLB_DTYPE_BF16>(p, o, table, chunk_tokens, s); \
+    else launch_route_align<VPL_, DLB_DTYPE_F16>(p, o, table, chunk_tokens, s);                                      \
   } while (0)
   if (E <= 64) DLB_LAUNCH_ROUTE_ALIGN(4);
   else if (E <= 128) DLB_LAUNCH_ROUTE_ALIGN(8);
