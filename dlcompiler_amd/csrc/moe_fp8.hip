@@ -228,6 +228,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   const int nrt_real = (tile.rows + 31) >> 5;  // row tiles that hold real rows (<= NRT)
   const int row0 = tile.row0;
   const int K = p.K, KC = p.KC;
+  const bool weights_by_slot = p.topk_w && !p.renorm;  // down: rows' routing weights are what stands at their slot
   const bool stager = wave < nrt_real;  // this wave's row tile is real: it stages those rows
 
   // ---- weight fragments: column tile ct of this wave covers 32 output columns
@@ -264,27 +265,40 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   using H1 = std::integral_constant<int, 1>;
 
   u32x4 wr[2][2][2][2];  // weight units [chunk parity][chunk half][column tile][piece]
-  // the first unit goes out before the routing slots are even known: it only needs the expert
-  issue_w(H0{}, 0, wr[0][0]);
-
-  // ---- routing slots.  Gated: the rows this lane stages (four) and the row whose scale it
-  // fetches.  Down: thread t < 128 keeps slot and routing weight of row t for the epilogue.
+  // ---- routing slots.  Gated: the rows this lane stages (four) and the row whose scale it fetches; asked for
+  // first, since the activations' addresses wait for them, and loads are waited for in their order.
   int sid_x[4] = {0, 0, 0, 0};
   int sid_s = 0;
   // (positions past the tile's real rows hold the pad sentinel or another tile's slots: the last real
   // row is read instead, unconditionally -- behind a branch each load would be waited for)
   auto slot_at = [&](int r) -> int { return p.sorted_ids[row0 + min(r, tile.rows - 1)]; };
-  if (GATED && stager) {
+  if (GATED) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) sid_x[i] = slot_at(32 * wave + 8 * i + drow);
     sid_s = slot_at(32 * wave + j);
   }
-  int sid_out = -1;  // down: slot of the tile's row `tid`
-  if (!GATED) sid_out = slot_at(tid & 127);
+  __builtin_amdgcn_sched_barrier(0);
+  // the first weights, which only need the expert
+  issue_w(H0{}, 0, wr[0][0]);
+  // Block scales of the wave's two column tiles for all chunks, and (down) the tile's routing slots: straight into
+  // LDS, nobody waits for them before the first activations are there.
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    const int sblk = min(ncol[ct] >> 7, (p.N >> 7) - 1);
+    const float* src = p.w_scale + ((int64_t)e * (p.N >> 7) + sblk) * KC;
+    for (int i = 0; i < KC; i += 64) dma4_global_to_lds(src + min(lane + i, KC - 1), lds_addr(ws_lds[wave][ct]) + 4 * i);
+  }
+  if (!GATED && wave < 2) {
+    const IdxArray& ids = p.sorted_ids;
+    dma4_global_to_lds(ids.p + ((int64_t)(row0 + min(tid, tile.rows - 1)) << ids.sh), lds_addr(sid_lds) + 256 * wave);
+  }
   // source row of the tile's row r whose routing slot is sid (gated: the slot's token; pad
   // slots read a valid row)
   auto src_row_of = [&](int sid, int r) -> uint32_t {
-    if (GATED) return (uint32_t)min(max(sid, 0) / p.topk, p.num_tokens - 1);
+    if (GATED) {
+      const uint32_t n = (uint32_t)max(sid, 0), q = p.topk > 1 ? __umulhi(n, p.topk_rcp) : n;
+      return min(n - q * p.topk >= (uint32_t)p.topk ? q + 1 : q, (uint32_t)p.num_tokens - 1);  // (q: at most one too small)
+    }
     return (uint32_t)min((int64_t)(row0 + r), p.a_rows - 1);
   };
   // ---- activation staging: per chunk 16 instructions of 8 rows x 128 bytes, four per wave
@@ -302,22 +316,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     *(u32x4*)xoff_lds[tid] = xo;  // read back by the same lane only: no barrier needed
   }
   // activation scales: one 4-byte copy per wave and chunk with 32 lanes active, lane l fetching
-  // the scale of the wave's staging row l.  The block scales of the wave's two column tiles for
-  // all chunks are fetched once, here, and parked in LDS.
-  uint32_t sc_voff = 0;
-  {
-    if (stager && lane < 32) sc_voff = src_row_of(sid_s, 32 * wave + j) * (uint32_t)KC * 4u;
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int sblk = min(ncol[ct] >> 7, (p.N >> 7) - 1);
-      const float* src = p.w_scale + ((int64_t)e * (p.N >> 7) + sblk) * KC;
-#pragma unroll
-      for (int i = 0; i < kMaxKC / 64; ++i) {
-        const int kc = lane + 64 * i;
-        if (kc < KC) ws_lds[wave][ct][kc] = src[kc];
-      }
-    }
-  }
+  // the scale of the wave's staging row l
+  const uint32_t sc_voff = stager && lane < 32 ? src_row_of(sid_s, 32 * wave + j) * (uint32_t)KC * 4u : 0u;
 
   const unsigned int x_dst0 = lds_addr(x_lds) + wave * 4096;
   const unsigned int sc_dst0 = lds_addr(sc_lds) + wave * kScWave;
@@ -385,17 +385,13 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   issue_w(H0{}, 1, wr[1][0]);
   issue_x(1, 1);
   issue_w(H1{}, 1, wr[1][1]);
-  if (!GATED) {
-    // destination row of the tile's row `tid` (-1: none) and its routing weight, published by the
-    // barrier that opens the main loop; here, behind the loads that the first chunks wait for
-    if (tid < 128) {
-      const bool real = tid < tile.rows && sid_out >= 0 && sid_out < p.numel;
-      sid_lds[tid] = real ? sid_out : -1;
-      rw_lds[tid] = real ? slot_weight(p, sid_out) : 0.0f;
-    }
-  }
-  wait_vm<12 + D>();  // X(0) landed
+  wait_vm<12 + D>();  // X(0) landed, and everything before it
   __syncthreads();
+  if (!GATED && wave < 2 && weights_by_slot) {
+    // (one operation more on its way than the waits of the first chunk assume: they wait for one more)
+    const int slot = min(max(sid_lds[tid], 0), p.numel - 1);
+    dma4_global_to_lds(p.topk_w + slot, lds_addr(rw_lds) + 256 * wave);
+  }
 
   u32x4 xa[2], xb[2];  // fragment buffers, taken in turn by the 2 * NRT steps of a chunk
   read_x(0, 0, 0, xa);
@@ -557,6 +553,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     constexpr int kPitch = 512 + 16;  // staging row pitch: rows 16 bytes apart in the banks
     static_assert(64 * kPitch <= NX * kXSlot, "output staging fits the activation slots");
     const int ncols = min(256, p.N - nt * 256);
+    if (!weights_by_slot && tid_e < 128) rw_lds[tid_e] = slot_weight(p, min(max(sid_lds[tid_e], 0), p.numel - 1));
     __syncthreads();  // every wave has left the main loop
 #pragma unroll
     for (int half = 0; half < (NRT + 1) / 2; ++half) {
@@ -592,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
         for (int i = 0; i < 8; ++i) {
           const int r = (tid_e >> 5) + 8 * i, pc = tid_e & 31;
           const int sid = sid_lds[64 * half + r];  // destination row
-          if (sid >= 0 && 8 * pc < ncols)
+          if (64 * half + r < tile.rows && (unsigned)sid < (unsigned)p.numel && 8 * pc < ncols)
             // (cached: the sum over the slots finds them behind the L2s, 4096 tokens x 6 of 64 experts, 100 MB: 21.4 ->
             // 18.3 us; past the caches, this kernel is no faster, 114.5 us and 113.6 so)
             *(u32x4*)((unsigned short*)p.out + (int64_t)sid * p.N + nt * 256 + 8 * pc) =
@@ -789,6 +786,7 @@ int fill_gemm_params(MoeGemmParams& p, bool gated, int elem, const void* a, cons
   p.KC = p.K / 128;
   p.kc_rcp = p.KC > 1 ? (uint32_t)(0x100000000ull / (uint32_t)p.KC) : 0;
   p.topk = topk;
+  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0;
   p.numel = num_tokens * topk;
   p.num_tokens = num_tokens;
   p.expert_offset = expert_offset;
@@ -917,6 +915,7 @@ extern "C" int dlb_moe_gemm_16bit_launcher(const void* a, const void* b, void* c
   p.N = N;
   p.KC = p.K / 128;
   p.topk = topk;
+  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0;
   p.numel = (int)num_slots;
   // gathered rows are slot / topk; the caller says how many rows `a` has
   p.num_tokens = a_rows < 0x7fffffff ? (int)a_rows : 0x7fffffff;
