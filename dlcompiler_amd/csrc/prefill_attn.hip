@@ -194,7 +194,7 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   const int row_waves = small ? 2 : 4;
   const int64_t all_wgs = ceil_div(max_len, 128) * B * Hq, slots = (int64_t)current_device_cu_count() * (D <= 64 ? 4 : 2);
   int64_t qtiles = ceil_div(ceil_div(max_len, 32) * p.group, row_waves);
-  // Not with a soft-cap, whose kernel has no such form: with tanh in front of it the 3 % are less than that.
+  // (A soft-cap has kernels of its own, which have no such form.)
   // (A kernel of its own: where heads do not share, its longer start costs 1 %, 16 heads, 16 kv, of 64: 176.2 / 178.7.)
   const bool share = !plan.use && !small && all_wgs > (paged ? 3 : 2) * slots && (8 % Hkv == 0 || Hkv % 8 == 0) &&
                      qtiles <= 65535 && p.group > 1 && p.group <= 4096 && !(paged && p.softcap > 0.0f);
