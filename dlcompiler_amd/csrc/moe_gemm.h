@@ -78,7 +78,7 @@ struct TileId {
   int rows;  // real (unpadded) rows of the tile
 };
 
-// Do a layer's GEMMs hand the intermediate over in fp32?  (up: of the gate_up GEMM, with 16-bit activations)
+// Do a layer's GEMMs hand the intermediate over in fp32 (fp8, up to kSmallMeanRows; see fp8_few_rows)?  up: of gate_up
 bool moe_hands_over_f32(const MoeGemmParams& up);
 // Launches the streaming kernel.  gated / quantised as the entry points; N_out checks are done.
 int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dtype, int w_layout, hipStream_t s);

@@ -1,5 +1,5 @@
 """A few tokens through the fp8 MoE layer: the intermediate handed over in fp32 and quantised by the down GEMM (one
-token's experts, and between one and two column tiles per CU), activations quantised ahead of the main loop, and the
+token's experts, and about one column tile with rows per CU), activations quantised ahead of the main loop, and the
 sizes next to either rule.  The alignment handed over or not, the result has the same bits."""
 import pytest
 import torch
@@ -56,11 +56,17 @@ def test_few_column_tiles(dev, T, H, I, E, k, shuffled, dtype):
     _layer(dev, T, H, I, E, k, shuffled, dtype)
 
 
-# 256 CUs: 320 to 512 tiles with up to 1.5 rows per expert, then more tiles, of rows of up to 2048 and of 4096
+# 256 CUs, 257 to 548 tiles with rows: quantised ahead of the main loop, rows of up to 2048 and of 4096
 @pytest.mark.parametrize("T,H,I,E,k", [(10, 384, 1024, 40, 6), (8, 384, 1024, 64, 8), (12, 256, 1024, 64, 8),
                                        (30, 2048, 640, 128, 8), (20, 2304, 640, 64, 8)])
 def test_more_column_tiles(dev, T, H, I, E, k):
     _layer(dev, T, H, I, E, k, True, torch.bfloat16)
+
+
+# rows of 1536 and more: 256 tiles with rows, fp32 intermediate, and 224, quantised in every step
+@pytest.mark.parametrize("T,H", [(12, 1536), (12, 2304), (9, 1536)])
+def test_a_tile_per_cu(dev, T, H):
+    _layer(dev, T, H, 1280, 32, 4, True, torch.bfloat16)
 
 
 @pytest.mark.parametrize("T,E", [(20, 64), (33, 16), (7, 8)])

@@ -1,0 +1,65 @@
+"""Which form of a kernel a launch takes, by sizes alone: the rules' headers, compiled for the host (no GPU).  For each
+size the form that was measured to be the faster one, by more than the runs differ."""
+import subprocess
+
+import pytest
+
+from dlcompiler_amd.build import CSRC_DIR
+
+PROGRAM = """
+#include <cstdio>
+#include <cstring>
+#include "moe_rules.h"
+using namespace dlb;
+int main() {
+  char what[32];
+  long long a[9];
+  while (scanf("%31s", what) == 1) {
+    for (int i = 0; i < 9; ++i) a[i] = 0;
+    int n = 0;
+    while (n < 9 && scanf("%lld", &a[n]) == 1) ++n;
+    if (!strcmp(what, "few")) {  // experts, local, topk, tokens, hidden, inter, cus
+      const MoeLaunch up = {true, a[3] * a[2], a[3], a[2], a[0], a[1], a[5], a[4], a[6]};
+      const FewRows f = fp8_few_rows(up);
+      puts(f == FewRows::kInSteps ? "steps" : f == FewRows::kAhead ? "ahead" : "f32");
+    }
+    scanf("%*[;\\n ]");
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rules")
+    (folder / "rules.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", f"-I{CSRC_DIR}", str(folder / "rules.cpp"), "-o", str(folder / "rules")],
+                   check=True)
+
+    def ask(what, *sizes):
+        line = " ".join([what, *map(str, sizes)]) + " ;\n"
+        return subprocess.run([folder / "rules"], input=line, text=True, capture_output=True, check=True).stdout.strip()
+
+    return ask
+
+
+# us a layer: in the steps of the main loop, ahead of it, ahead of it with an fp32 intermediate
+@pytest.mark.parametrize("E,local,k,T,H,I,us", [
+    (128, 128, 8, 10, 1152, 512, (34.3, 34.5, 40.9)), (128, 128, 8, 23, 1152, 512, (48.3, 45.9, 51.8)),
+    (256, 128, 8, 7, 1280, 1152, (33.2, 34.0, 39.3)), (128, 64, 8, 16, 1536, 768, (38.8, 39.0, 44.5)),
+    (32, 32, 4, 8, 1536, 1280, (34.4, 34.1, 38.1)), (64, 64, 8, 3, 4096, 1024, (56.6, 56.5, 58.6)),
+    (64, 64, 6, 8, 3584, 640, (52.9, 53.0, 54.9)), (128, 128, 8, 14, 4096, 256, (55.9, 57.0, 57.4)),
+    (64, 64, 8, 6, 4096, 1024, (100.6, 99.3, 88.6)), (128, 128, 8, 8, 2048, 768, (60.4, 57.0, 53.7)),
+    (64, 64, 6, 1, 2048, 1408, (28.6, 27.0, 25.3)), (64, 64, 6, 8, 2048, 1408, (63.5, 60.7, 65.7)),
+    (256, 64, 8, 4, 2688, 896, (33.5, 33.3, 25.8)), (8, 8, 2, 1, 4096, 4096, (43.5, 43.0, 32.8)),
+])
+def test_fp8_few_rows(rule, E, local, k, T, H, I, us):
+    chosen = us[("steps", "ahead", "f32").index(rule("few", E, local, k, T, H, I, 256))]
+    assert chosen <= 1.02 * min(us)
+
+
+@pytest.mark.parametrize("E,local,k,T,H,I", [(1, 1, 1, 1, 128, 128), (8, 8, 8, 3, 4224, 128), (4, 1, 4, 100, 4096, 4224),
+                                             (256, 256, 8, 10 ** 6, 16384, 128)])
+def test_fp8_few_rows_at_the_ends(rule, E, local, k, T, H, I):
+    form = rule("few", E, local, k, T, H, I, 256)
+    assert form in ("steps", "ahead", "f32") and (H <= 4096 or form == "steps") and (I <= 4096 or form != "f32")
