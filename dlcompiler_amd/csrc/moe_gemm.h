@@ -4,6 +4,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "moe_rules.h"
 
 namespace dlb {
 
@@ -87,8 +88,6 @@ int launch_moe_stream(const MoeGemmParams& p, bool gated, int quantised, int dty
 // 2048 x 1408, 15 rows 110 / 112, 36 rows 119 / 116; 128 of 2048 x 768, 30 rows 134.7 / 135.6, 42 rows 147 / 140).
 // 16-bit operands always take it.
 constexpr int kStreamMeanRows = 32;
-// ... and up to this many it runs tiles of 16 rows
-constexpr int kSmallMeanRows = 7;
 // While an expert mostly has one tile of up to 128 rows its weights are read once, and go past the caches: 64
 // experts of 2048 x 1408, kept / not kept: 16 bit, 75 rows 234 / 210 us, 105 rows 254 / 224, 140 rows 316 / 387;
 // fp8, 50 rows 125.7 / 119.7, 105 rows 145.2 / 140.9, 125 rows 176 / 187.  Not so weights that the 256 MB behind

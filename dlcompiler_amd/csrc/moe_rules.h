@@ -5,6 +5,9 @@
 
 namespace dlb {
 
+// Up to this many rows per expert, on average over the routed slots, the streaming kernel runs tiles of 16 rows.
+constexpr int kSmallMeanRows = 7;
+
 // Sizes of one grouped GEMM.  (Not the routing, which the host does not know: where a rule needs the experts or the row
 // tiles that have rows, it takes them for a routing that spreads the tokens evenly.)
 struct MoeLaunch {
@@ -20,6 +23,81 @@ struct MoeLaunch {
     return (double)local * (1.0 - std::pow(miss, (double)tokens));
   }
 };
+
+// 16 bit, side by side.  down: tiles of up to 128 rows, which store whole rows, take over from those of 32 at once
+// (64-row tiles / 128-row ones, in both layouts alike: 128 experts of 2048 x 768, 28 rows 219.4 / 211.7 us; 64 of 3072 x
+// 2048, 28 rows 411 / 390; 64 of 4096 x 1024, 28 rows 275.5 / 270.7; 64 of 2048 x 1408 188.9 / 188.3; 21 rows 183.9 /
+// 183.6; 32-row ones there 199 / 185).  gate_up, which writes half as much: 64-row tiles, with two chunks of activations
+// on their way, up to 36 rows (64-row / 128-row: 64 of 2048 x 1408, 28 rows 188.3 / 191.2, 37 rows 194.1 / 195.8, 43 rows
+// 197.9 / 197.6; 64 of 1024 x 1408, 28 rows 105.6 / 109.9; 128 of 1536 x 512, 28 rows 120.6 / 122.2; 128 of 2048 x 768,
+// 36 rows 217.3 / 216.3; 64 of 3072 x 2048, 28 rows 390.2 / 390.1, 37 rows 402.9 / 397.8).
+// A launch of few column tiles (few experts, or a rank's share of them) is bound by the CUs that it leaves idle, and by
+// those that get one workgroup more than the others.  Where four waves side by side give more workgroups than every other
+// CU but fewer than one each, splitting K gives most CUs two of half the size, which is no less for the busiest, and the
+// partial sums on top (layer, split / side by side: 16 experts of 2176 x 1536, 192 and 144 tiles, 25 rows 83.0 / 78.0 us,
+// 50 rows, then of 128, 90.3 / 82.5; 32 of 2048 x 768, 192 and 256, 37 rows 76.2 / 69.0; but gate_up of 8 of 4096 x 2048,
+// 128 tiles, 25 rows 78.7 / 91.1, and of 8 of 4096 x 4096, 256 tiles, 141.4 / 150.6).  The down GEMM's tall tiles, which
+// store whole rows, pay up to twice as many (32 of 2816 x 704, 352 tiles, 22 rows 95.4 / 85.9; gate_up, 384 tiles, 128 of
+// 1792 x 384, 40 rows 116.9 / 122.3).
+// With fewer tiles the shape is the first in this order that has a workgroup for somewhat more than every other CU: 128
+// rows, 64 side by side, 64 with K split in two, 32, 16 with K split in four, which has to fit the CUs once.  us of a
+// layer with gate_up in each:
+//                                                     128    64   64/2  32/2  16/4
+//   8 of 2816 x 896, 4 of them here (28 tiles)  15 rows                 37.0  29.8
+//                                               32             42.6  40.6  37.4
+//                                               63      68.8  65.5  49.7  45.5  45.6
+//                                              125      79.9  68.6  53.2  48.8  64.7
+//   8 of 2048 x 1024 (64 tiles)                 32             39.7  38.7  44.1
+//                                               64      61.1  56.2  46.0  53.0  59.6
+//                                              128      71.3  60.2  62.4  66.9  83.6
+//   16 of 2048 x 1408, 8 here (88 tiles)       125      79.9  68.9  72.7  88.8
+//   16 of 1024 x 512, 4 here (16 tiles)         25             27.8  26.6  23.2
+//                                               75      39.4  38.1  32.8  30.2  30.1
+// (4000 tokens through the last, 1000 rows: 133 workgroups of 128 rows 53.8 us, 258 of 64, one CU with two, 58.8.)
+// Above 52 rows two more things count.  gate_up, 62 to 84 rows, with K split in two: half of the experts have a second
+// tile of 64 rows, and where some CUs get two such workgroups that way and none gets two of 32 rows side by side, those
+// are faster (128 / 64 / 64 in two / 32 side by side: 8 experts of 1408 x 1280, 67 rows 44.8 / 45.1 / 48.0 / 42.6; 16 of
+// 1536 x 640, 77 rows 50.7 / 52.0 / 55.0 / 50.2; 8 of 2816 x 2816, 4 of them here, 69 rows 78.2 / 74.9 / 80.5 / 71.5).
+// down: tall tiles store whole rows, and 64-row ones gain by what K is long enough to hide (128 / 64: 16 experts of 1792 x
+// 1280, 68 rows 65.5 / 73.5; 1536 x 640, 77 rows 51.7 / 55.0; 1408 x 512, 85 rows 37.7 / 39.8; but 1408 x 3968, 106 rows
+// 144.7 / 134.7, 1664 x 1152, 95 rows 70.5 / 65.9).
+// Of 840 GEMMs (7 to 320 rows) the shape is 0.7 % above the best of the seven on average and 5 % at worst above what
+// the rows alone would choose (K split in two up to 52, else 128-row tiles), which is 6.5 % above the best.
+struct StreamShape { int cw, nt; };  // (four waves, cw of them side by side; rows 16 nt)
+inline StreamShape stream_shape_16bit(const MoeLaunch& p) {
+  const int64_t wave_columns = p.gated ? 32 : 64, experts = p.most_experts(), cus = p.cus;
+  const auto column_tiles = [&](int cw) { return (p.columns + cw * wave_columns - 1) / (cw * wave_columns) * experts; };
+  const int64_t tiles = column_tiles(4);
+  // Workgroups with rows: on average an expert's last row tile is half full, and an expert of
+  // up to 0.72 of a tile seldom has a second one.
+  const auto blocks = [&](int cw, int nt) {
+    const double full = (double)p.slots / ((double)p.experts * 16 * nt);
+    return (double)column_tiles(cw) * (full <= 0.72 ? 1.0 : full + 0.5);
+  };
+  const bool one_round = 2 * tiles > cus && 10 * tiles <= 9 * cus, beside = tiles >= 2 * cus;
+  if (p.mean_up_to(kSmallMeanRows)) return {beside ? 4 : 1, 1};
+  if (one_round || beside) {
+    if (p.mean_up_to(19)) return {4, 2};
+    return {4, p.gated && p.mean_up_to(36) ? 4 : 8};
+  }
+  if (!p.mean_up_to(52) && (2 * tiles >= cus || blocks(4, 4) > cus)) return {4, 8};
+  if (!p.mean_up_to(22)) {
+    if (!p.gated && tiles > cus / 2) return {4, 8};
+    if (!p.mean_up_to(52)) {
+      const bool tall = blocks(4, 4) >= 0.55 * cus;
+      const bool short_k = p.row_bytes < 2048 || p.slots < 80 * p.experts;
+      if (!p.gated && 16 * tiles >= 5 * cus && short_k && (tall || !p.mean_up_to(60))) return {4, 8};
+      if (p.gated && !p.mean_up_to(62) && p.mean_up_to(84) && blocks(2, 4) > 0.95 * cus && blocks(4, 2) <= 0.95 * cus)
+        return {4, 2};
+      if (tall) return {4, 4};
+    }
+    // (up to 28 rows 32-row tiles seldom have a second one either: 8 experts of 1152 x 1152, 26 rows 32.5 / 31.2, 47 rows
+    // 33.5 / 35.6)
+    if (blocks(2, 4) >= (!p.mean_up_to(28) && p.mean_up_to(52) ? 0.55 : 0.65) * cus) return {2, 4};
+  }
+  if (blocks(2, 2) >= 0.55 * cus || blocks(1, 1) > 1.1 * cus) return {2, 2};
+  return {1, 1};
+}
 
 // fp8, up to kSmallMeanRows rows per expert: where the activations and the intermediate are quantised.
 //   kInSteps    activations by every wave in every step of its main loop, the intermediate by gate_up's epilogue, whose

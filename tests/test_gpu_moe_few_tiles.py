@@ -18,6 +18,9 @@ SIZES += [(T, 64, 640, 1552, 32, 4) for T in (57, 150, 153, 288, 290, 416, 420)]
 # 288 and 448, where the down GEMM alone goes to 128 rows, and 144 and 224
 SIZES += [(T, 64, 1152, 3336, 32, 4) for T in (170, 190, 300)]
 
+# half the experts: 80 gate_up tiles of 32 rows side by side, 112 down tiles of 128 rows, then of 64, which a long K hides
+SIZES += [(540, 64, 640, 1552, 32, 4), (700, 64, 640, 1552, 32, 4), (700, 64, 1024, 1552, 32, 4)]
+
 
 @pytest.mark.parametrize("T,H,I,O,E,k", SIZES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -23,6 +23,10 @@ int main() {
       const FewRows f = fp8_few_rows(up);
       puts(f == FewRows::kInSteps ? "steps" : f == FewRows::kAhead ? "ahead" : "f32");
     }
+    if (!strcmp(what, "shape")) {  // gated, experts, local, slots, columns, row bytes, cus
+      const StreamShape f = stream_shape_16bit({a[0] != 0, a[3], a[3], 1, a[1], a[2], a[4], a[5], a[6]});
+      printf("%d%d\\n", f.cw, f.nt);
+    }
     scanf("%*[;\\n ]");
   }
 }
@@ -63,3 +67,31 @@ def test_fp8_few_rows(rule, E, local, k, T, H, I, us):
 def test_fp8_few_rows_at_the_ends(rule, E, local, k, T, H, I):
     form = rule("few", E, local, k, T, H, I, 256)
     assert form in ("steps", "ahead", "f32") and (H <= 4096 or form == "steps") and (I <= 4096 or form != "f32")
+
+
+# us a layer with this GEMM's waves side by side and its rows in tiles of 16: 48 44 24 42 22 41 11
+SHAPES = ("48", "44", "24", "42", "22", "41", "11")
+
+
+@pytest.mark.parametrize("gated,E,local,rows,columns,K,us", [
+    (0, 8, 8, 43.75, 2432, 2560, (86.1, 88.7, 80.9, 88.3, 91.1, 104.8, 95.4)),
+    (0, 16, 16, 67.5, 1792, 1280, (65.5, 73.5, 74.6, 84.2, 78.9, 102.3, 87.9)),
+    (0, 16, 16, 77.25, 1536, 640, (51.7, 55.0, 56.2, 59.0, 56.6, 62.1, 61.4)),
+    (0, 16, 16, 85, 1408, 512, (37.7, 39.8, 41.2, 41.3, 40.7, 45.8, 45.2)),
+    (0, 16, 16, 106.25, 1408, 3968, (144.7, 134.7, 143.0, 174.9, 165.4, 231.4, 208.8)),
+    (1, 8, 8, 47, 1152, 1152, (36.2, 37.6, 33.5, 35.6, 35.6, 35.6, 36.4)),
+    (1, 16, 16, 77.25, 640, 1536, (50.7, 52.0, 55.0, 50.2, 52.6, 66.2, 65.1)),
+    (1, 8, 4, 69.25, 2816, 2816, (78.2, 74.9, 80.5, 71.5, 74.5, 105.9, 97.6)),
+    (1, 8, 8, 117.5, 896, 3200, (82.9, 73.5, 57.3, 67.7, 72.5, 107.9, 100.1)),
+    (1, 16, 16, 273.75, 1664, 1536, (139.1, 164.5, 162.8, 219.1, 208.7, 338.5, 317.8)),
+    (1, 8, 8, 26.25, 1152, 1152, (35.8, 36.9, 32.5, 36.1, 31.2, 35.3, 34.3)),
+])
+def test_16bit_shapes(rule, gated, E, local, rows, columns, K, us):
+    chosen = us[SHAPES.index(rule("shape", gated, E, local, int(rows * E), columns, 2 * K, 256))]
+    assert chosen <= 1.02 * min(us)
+
+
+def test_16bit_shapes_have_kernels(rule):
+    seen = {rule("shape", g, E, E, int(r * E), c, 2048, 256) for g in (0, 1) for E in (1, 4, 16, 256)
+            for r in (0.1, 5, 12, 21, 26, 40, 58, 66, 83, 100, 1000) for c in (64, 704, 2816)}
+    assert seen == set(SHAPES)
