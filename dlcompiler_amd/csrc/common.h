@@ -217,6 +217,10 @@ __device__ __forceinline__ void dma4_global_to_lds_masked(const void* sbase, uns
                : "memory", "m0");
 }
 
+// Around non-temporal stores on one side of a condition whose other side makes the same stores through the caches:
+// the compiler would make them one, without the hint.
+__device__ __forceinline__ void keep_apart() { asm volatile("" ::: "memory"); }
+
 // a value and its partner 16 / 32 lanes away combined (v_permlane16_swap, v_permlane32_swap: register-file
 // exchanges, no trip through LDS as with ds_bpermute)
 typedef __attribute__((ext_vector_type(2))) unsigned int permlane_pair;

@@ -585,16 +585,29 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
         }
         __syncthreads();
         // 64 rows x 32 pieces; thread t takes piece t % 32 of rows t / 32 + 8 i
+        auto store_rows = [&](auto past) __attribute__((always_inline)) {
+          constexpr bool PAST = decltype(past)::value;
+          if (PAST) keep_apart();
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int r = (tid_e >> 5) + 8 * i, pc = tid_e & 31;
-          const int sid = sid_lds[64 * half + r];  // destination row
-          if (64 * half + r < tile.rows && (unsigned)sid < (unsigned)p.numel && 8 * pc < ncols)
-            // (cached: the sum over the slots finds them behind the L2s, 4096 tokens x 6 of 64 experts, 100 MB: 21.4 ->
-            // 18.3 us; past the caches, this kernel is no faster, 114.5 us and 113.6 so)
-            *(u32x4*)((unsigned short*)p.out + (int64_t)sid * p.N + nt * 256 + 8 * pc) =
-                *(const u32x4*)(x_lds + r * kPitch + 16 * pc);
-        }
+          for (int i = 0; i < 8; ++i) {
+            const int r = (tid_e >> 5) + 8 * i, pc = tid_e & 31;
+            const int sid = sid_lds[64 * half + r];  // destination row
+            if (64 * half + r < tile.rows && (unsigned)sid < (unsigned)p.numel && 8 * pc < ncols) {
+              const u32x4 piece = *(const u32x4*)(x_lds + r * kPitch + 16 * pc);
+              u32x4* to = (u32x4*)((unsigned short*)p.out + (int64_t)sid * p.N + nt * 256 + 8 * pc);
+              if (PAST) __builtin_nontemporal_store(piece, to);
+              else *to = piece;
+            }
+          }
+          if (PAST) keep_apart();
+        };
+        // Past the caches, rows do not push weights out of the L2s; but the sum over the slots, where it follows at
+        // once, finds cached rows behind them (past / through the caches, us, operand order: 4096 tokens x 6 of 64
+        // experts of 2048 x 1408 this kernel 104.4 / 106.9, with buffers that stay the same 89.6 / 104.0, with the
+        // sum 125.9 / 122.0; 2000 x 8 of 128 of 2048 x 768 67.6 / 71.0, 55.2 / 61.1, 81.0 / 78.9; 1500 x 4 of 16 of
+        // 4096 x 1024 40.6 / 47.7, 40.0 / 41.5, 51.4 / 52.9, but in the layer 130.0 / 128.0)
+        if (p.summed) store_rows(std::false_type{});
+        else store_rows(std::true_type{});
         if (half + 1 < (NRT + 1) / 2) __syncthreads();  // the second half reuses the staging rows
       }
     }
@@ -1078,6 +1091,7 @@ extern "C" int dlb_fused_moe(int quantised, const void* x, int64_t ld_x, const v
   down.out = base + l.slots;
   down.topk_w = topk_weights;
   down.renorm = renormalize ? 1 : 0;
+  down.summed = 1;
 
   int32_t* eids = (int32_t*)(base + l.expert_ids);
   const int64_t eids_cap = ceil_div(cap, block);

@@ -44,6 +44,7 @@ struct MoeGemmParams {
   // gate_up leaves in h32 and the down GEMM, whose `a` it is, quantises as it loads it
   float* h32;
   int renorm;                 // weights are divided by the sum of their token's
+  int summed;                 // the sum over the slots follows: fp8, many rows, `out` goes through the caches
 };
 
 // routing weight of a slot (1 without weights)

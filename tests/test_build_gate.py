@@ -55,9 +55,8 @@ def test_no_instance_that_no_dispatch_reaches():
                       ("4", "1", "4"), ("2", "2", "4"), ("4", "1", "8")}
 
 
-@pytest.mark.parametrize("source", ["moe_fp8", "moe_stream", "paged_decode", "prefill_attn"])
-def test_pipelined_loads_are_global(source, tmp_path):
-    """A flat load counts as an LDS operation too: the next wait for LDS waits for every load in flight."""
+def _code_of(source, tmp_path):
+    """The assembly of each function that an object built here holds."""
     tools = Path(HIPCC).resolve().parent.parent / "llvm" / "bin"
     fat, code = tmp_path / "fat", tmp_path / "code"
     subprocess.run([tools / "llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", OBJ_DIR / f"{source}.o",
@@ -65,6 +64,24 @@ def test_pipelined_loads_are_global(source, tmp_path):
     subprocess.run([tools / "clang-offload-bundler", "--unbundle", "--type=o", f"--input={fat}", f"--output={code}",
                     f"--targets=hipv4-amdgcn-amd-amdhsa--{ARCH}"], check=True)
     text = subprocess.run([tools / "llvm-objdump", "-d", code], check=True, capture_output=True, text=True).stdout
-    assert "global_load" in text or "buffer_load" in text
-    flat = {block.split(">", 1)[0] for block in re.split(r"^[0-9a-f]+ <", text, flags=re.M) if "flat_load" in block}
+    return dict(block.split(">", 1) for block in re.split(r"^[0-9a-f]+ <", text, flags=re.M)[1:])
+
+
+@pytest.mark.parametrize("source", ["moe_fp8", "moe_stream", "paged_decode", "prefill_attn"])
+def test_pipelined_loads_are_global(source, tmp_path):
+    """A flat load counts as an LDS operation too: the next wait for LDS waits for every load in flight."""
+    code = _code_of(source, tmp_path)
+    assert any("global_load" in text or "buffer_load" in text for text in code.values())
+    flat = {name for name, text in code.items() if "flat_load" in text}
     assert not flat, flat
+
+
+def test_down_gemm_stores_past_the_caches_too(tmp_path):
+    """fp8 down GEMM: slot rows go through the caches where the sum over the slots follows, past them where it is called
+    alone.  (Both stores on either side of a condition, the compiler would make them one.)"""
+    down = {name: text for name, text in _code_of("moe_fp8", tmp_path).items() if "moe_gemm_kernelILb0E" in name}
+    assert down
+    for name, text in down.items():
+        stores = re.findall(r"global_store_dwordx4 .*", text)
+        past = [" nt" in store.split("//")[0] for store in stores]
+        assert any(past) and not all(past), name
