@@ -266,7 +266,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
 
   u32x4 wr[2][2][2][2];  // weight units [chunk parity][chunk half][column tile][piece]
   // ---- routing slots.  Gated: the rows this lane stages (four) and the row whose scale it fetches; asked for
-  // first, since the activations' addresses wait for them, and loads are waited for in their order.
+  // first, since the activations' addresses wait for them and loads are waited for in their order: the first weights
+  // stay on their way.
   int sid_x[4] = {0, 0, 0, 0};
   int sid_s = 0;
   // (positions past the tile's real rows hold the pad sentinel or another tile's slots: the last real
@@ -280,8 +281,39 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   __builtin_amdgcn_sched_barrier(0);
   // the first weights, which only need the expert
   issue_w(H0{}, 0, wr[0][0]);
+  // source row of the tile's row r whose routing slot is sid (gated: the slot's token; pad
+  // slots read a valid row)
+  // (read once: a load of an argument between the uses of the slots would be waited for in every row)
+  const uint32_t topk = (uint32_t)p.topk, topk_rcp = p.topk_rcp, last_token = (uint32_t)p.num_tokens - 1;
+  auto src_row_of = [&](int sid, int r) -> uint32_t {
+    if (GATED) {
+      const uint32_t n = (uint32_t)max(sid, 0), q = __umulhi(n, topk_rcp);
+      return min(n - q * topk >= topk ? q + 1 : q, last_token);  // (q: at most one too small)
+    }
+    return (uint32_t)min((int64_t)(row0 + r), p.a_rows - 1);
+  };
+  // ---- activation staging: per chunk 16 instructions of 8 rows x 128 bytes, four per wave
+  // (its own row tile); lane -> (row, physical piece), the logical piece it fetches undoes the
+  // swizzle.  A wave whose row tile is padding copies the same 16 bytes with every lane.
+  // (the four byte offsets of a lane are parked in LDS and re-read for every chunk: they would
+  // otherwise occupy four registers for the whole kernel)
+  const uint32_t mine = stager ? ~0u : 0u;  // (no branch: behind one a slot is waited for once more)
+  {
+    u32x4 xo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 32 * wave + 8 * i + drow;
+      xo[i] = (src_row_of(sid_x[i], r) * (uint32_t)K + (uint32_t)((dpc ^ ((r >> 1) & 7)) << 4)) & mine;
+    }
+    *(u32x4*)xoff_lds[tid] = xo;  // read back by the same lane only: no barrier needed
+  }
+  // activation scales: one 4-byte copy per wave and chunk with 32 lanes active, lane l fetching
+  // the scale of the wave's staging row l
+  const uint32_t sc_voff = (src_row_of(sid_s, 32 * wave + j) * (uint32_t)KC * 4u) & mine;
+
   // Block scales of the wave's two column tiles for all chunks, and (down) the tile's routing slots: straight into
-  // LDS, nobody waits for them before the first activations are there.
+  // LDS, and waited for with the first activations.  Behind the last use of the gated slots: the compiler does not
+  // count these copies, and with them between, its wait for a slot would be one for the first weights too.
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct) {
     const int sblk = min(ncol[ct] >> 7, (p.N >> 7) - 1);
@@ -292,32 +324,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     const IdxArray& ids = p.sorted_ids;
     dma4_global_to_lds(ids.p + ((int64_t)(row0 + min(tid, tile.rows - 1)) << ids.sh), lds_addr(sid_lds) + 256 * wave);
   }
-  // source row of the tile's row r whose routing slot is sid (gated: the slot's token; pad
-  // slots read a valid row)
-  auto src_row_of = [&](int sid, int r) -> uint32_t {
-    if (GATED) {
-      const uint32_t n = (uint32_t)max(sid, 0), q = p.topk > 1 ? __umulhi(n, p.topk_rcp) : n;
-      return min(n - q * p.topk >= (uint32_t)p.topk ? q + 1 : q, (uint32_t)p.num_tokens - 1);  // (q: at most one too small)
-    }
-    return (uint32_t)min((int64_t)(row0 + r), p.a_rows - 1);
-  };
-  // ---- activation staging: per chunk 16 instructions of 8 rows x 128 bytes, four per wave
-  // (its own row tile); lane -> (row, physical piece), the logical piece it fetches undoes the
-  // swizzle.  A wave whose row tile is padding copies the same 16 bytes with every lane.
-  // (the four byte offsets of a lane are parked in LDS and re-read for every chunk: they would
-  // otherwise occupy four registers for the whole kernel)
-  {
-    u32x4 xo;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 32 * wave + 8 * i + drow;
-      xo[i] = stager ? src_row_of(sid_x[i], r) * (uint32_t)K + (uint32_t)((dpc ^ ((r >> 1) & 7)) << 4) : 0u;
-    }
-    *(u32x4*)xoff_lds[tid] = xo;  // read back by the same lane only: no barrier needed
-  }
-  // activation scales: one 4-byte copy per wave and chunk with 32 lanes active, lane l fetching
-  // the scale of the wave's staging row l
-  const uint32_t sc_voff = stager && lane < 32 ? src_row_of(sid_s, 32 * wave + j) * (uint32_t)KC * 4u : 0u;
 
   const unsigned int x_dst0 = lds_addr(x_lds) + wave * 4096;
   const unsigned int sc_dst0 = lds_addr(sc_lds) + wave * kScWave;
@@ -799,7 +805,7 @@ int fill_gemm_params(MoeGemmParams& p, bool gated, int elem, const void* a, cons
   p.KC = p.K / 128;
   p.kc_rcp = p.KC > 1 ? (uint32_t)(0x100000000ull / (uint32_t)p.KC) : 0;
   p.topk = topk;
-  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0;
+  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0xffffffffu;
   p.numel = num_tokens * topk;
   p.num_tokens = num_tokens;
   p.expert_offset = expert_offset;
@@ -928,7 +934,7 @@ extern "C" int dlb_moe_gemm_16bit_launcher(const void* a, const void* b, void* c
   p.N = N;
   p.KC = p.K / 128;
   p.topk = topk;
-  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0;
+  p.topk_rcp = topk > 1 ? (uint32_t)(0x100000000ull / (uint32_t)topk) : 0xffffffffu;
   p.numel = (int)num_slots;
   // gathered rows are slot / topk; the caller says how many rows `a` has
   p.num_tokens = a_rows < 0x7fffffff ? (int)a_rows : 0x7fffffff;

@@ -39,7 +39,7 @@ struct MoeGemmParams {
   const float* topk_w;        // [numel]
   int64_t lda;                // gated fp8, few rows: `a` is 16-bit, rows of lda bytes (0: quantised)
   uint32_t kc_rcp;            // 2^32 / KC, rounded down (KC > 1)
-  uint32_t topk_rcp;          // 2^32 / topk, rounded down (topk > 1)
+  uint32_t topk_rcp;          // 2^32 / topk, rounded down (topk 1: 2^32 - 1)
   // fp8, very few rows (see moe_hands_over_f32): the intermediate is [numel, I] fp32, by routing slot, which
   // gate_up leaves in h32 and the down GEMM, whose `a` it is, quantises as it loads it
   float* h32;

@@ -76,6 +76,18 @@ def test_pipelined_loads_are_global(source, tmp_path):
     assert not flat, flat
 
 
+def test_gate_up_waits_for_its_slots_alone(tmp_path):
+    """fp8 gate_up GEMM: the first activations' addresses (which one 16-byte LDS store parks) wait for the routing slots.  A
+    copy into LDS in front of them, which the compiler does not count, would have that wait cover the first weights."""
+    gated = {name: text for name, text in _code_of("moe_fp8", tmp_path).items() if "moe_gemm_kernelILb1E" in name}
+    assert gated
+    for name, text in gated.items():
+        start = text[:text.index("ds_write_b128")]
+        slots, weights = start.rindex("global_load_dword "), start.index("global_load_dwordx4")
+        assert slots < weights and "global_load_lds" not in start, name
+        assert min(int(n) for n in re.findall(r"vmcnt\((\d+)\)", start[weights:])) >= 4, name
+
+
 def test_down_gemm_stores_past_the_caches_too(tmp_path):
     """fp8 down GEMM: slot rows go through the caches where the sum over the slots follows, past them where it is called
     alone.  (Both stores on either side of a condition, the compiler would make them one.)"""
