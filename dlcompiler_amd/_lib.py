@@ -14,7 +14,7 @@ _PKG_DIR = Path(__file__).resolve().parent
 DEFAULT_LIB_PATH = _PKG_DIR / "lib" / "libdlblas_hip.so"
 
 DLB_OK = 0
-ABI_VERSION = 6  # DLB_ABI_VERSION of include/dlblas_hip.h this binding was written against
+ABI_VERSION = 7  # DLB_ABI_VERSION of include/dlblas_hip.h this binding was written against
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
 
 # name -> (restype, argtypes); must list every symbol include/dlblas_hip.h declares
@@ -46,6 +46,8 @@ SIGNATURES = {
                               + [c_float, c_int, c_float, c_int, c_void_p, c_size_t, c_void_p]),
     "dlb_prefill_attn_varlen": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_int64] * 8
                                 + [c_float, c_int, c_void_p]),
+    "dlb_prefill_attn_varlen_tokens": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_int64] * 8
+                                       + [c_float, c_int, c_int64, c_void_p]),
     "dlb_paged_prefill_attn": (c_int, [c_void_p] * 8 + [c_int] * 9 + [c_int64] * 11
                                + [c_float, c_int, c_float, c_int, c_void_p]),
     "dlb_paged_prefill_attn_ws": (c_int, [c_void_p] * 8 + [c_int] * 9 + [c_int64] * 11

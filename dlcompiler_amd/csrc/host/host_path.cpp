@@ -33,7 +33,7 @@ namespace {
   X(dlb_fill_kv_cache)            \
   X(dlb_moe_topk_softmax_align_ws_bytes) \
   X(dlb_moe_topk_softmax_align_f32) \
-  X(dlb_prefill_attn_varlen)      \
+  X(dlb_prefill_attn_varlen_tokens) \
   X(dlb_paged_prefill_ws_bytes)   \
   X(dlb_paged_prefill_attn_ws)    \
   X(dlb_paged_decode_ws_bytes)    \
@@ -388,11 +388,11 @@ PyObject* context_attention_fwd(PyObject*, PyObject* const* args, Py_ssize_t) {
   int st;
   {
     NoGil nogil;
-    st = abi.dlb_prefill_attn_varlen(
+    st = abi.dlb_prefill_attn_varlen_tokens(
         q->data_ptr(), k->data_ptr(), v->data_ptr(), o->data_ptr(), start->data_ptr(), len->data_ptr(), mask,
         (int)len->size(0), (int)Hq, (int)k->size(1), (int)D, (int)max_len, q->stride(0), q->stride(1), k->stride(0),
         k->stride(1), v->stride(0), v->stride(1), o->stride(0), o->stride(1), (float)(1.0 / std::sqrt((double)D)),
-        dtype_code(*q), stream_of(dev));
+        dtype_code(*q), q->size(0), stream_of(dev));
   }
   if (st != DLB_OK) NOT_HANDLED;
   Py_RETURN_TRUE;

@@ -3,6 +3,7 @@
 #include <cmath>
 
 #include "prefill_attn.h"
+#include "prefill_rules.h"
 
 namespace dlb {
 namespace {
@@ -139,8 +140,8 @@ bool small_tiles(int Hq, int B, int D, int max_len, int64_t max_keys, int64_t to
 }
 
 // Shared argument checks and launch of both entry points; the paged fields of `p` are already
-// filled in (or zeroed) by the caller.
-int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk, int Dv, int max_len,
+// filled in (or zeroed) by the caller.  tokens: rows of q, 0 if the caller does not say.
+int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk, int Dv, int max_len, int64_t tokens,
                    int64_t max_keys, float sm_scale, int dtype, void* ws, size_t ws_bytes, void* stream) {
   if (Dk % 8 != 0 || Dv % 8 != 0 || Dk > 256 || Dv > 256) return DLB_ERR_UNSUPPORTED;
   // head size the kernel instance is built for; past 128 there is one instance, for 256, that
@@ -185,19 +186,14 @@ int launch_prefill(PrefillParams& p, bool paged, int B, int Hq, int Hkv, int Dk,
   p.ws_ml = p.ws_o ? p.ws_o + (size_t)p.tokens * Hq * p.nsplit * p.ws_d : nullptr;
   const int64_t seen = p.window > 0 && (int64_t)p.window + max_len < max_keys ? (int64_t)p.window + max_len : max_keys;
   const bool small = !plan.use && small_tiles(Hq, B, D, max_len, seen, p.tokens);
-  // Heads of a KV group share workgroups in launches of more than two rounds (two workgroups on a CU, four with
-  // up to 64 dims), where the KV heads fall on the XCDs by themselves and the row tiles fit the grid.  32 heads
-  // (8 kv) of 128: 8 x 512 - 4096 tokens 284 -> 275 us, 8 x 100 - 1000 44 -> 41.3; 28 (4): 42 -> 39.8, 8 x 300 -
-  // 1000 over 2000 110 -> 99.  In one round the workgroups that finish early help their neighbours and it loses:
-  // 8 heads (1 kv), 3 x 1000 - 4000 55.5 -> 56.9; 32 (8) of 64 dims, 4 x 60 - 300 6.9 -> 7.5.  Over histories
-  // of unequal lengths 2.5 rounds are a matter of luck (8 x 300 - 600 over up to 4096, ten batches: 0.98 - 1.07).
+  // Heads of a KV group share workgroups where the KV heads fall on the XCDs by themselves and the row tiles fit the grid.
   const int row_waves = small ? 2 : 4;
-  const int64_t all_wgs = ceil_div(max_len, 128) * B * Hq, slots = (int64_t)current_device_cu_count() * (D <= 64 ? 4 : 2);
   int64_t qtiles = ceil_div(ceil_div(max_len, 32) * p.group, row_waves);
   // (A soft-cap has kernels of its own, which have no such form.)
   // (A kernel of its own: where heads do not share, its longer start costs 1 %, 16 heads, 16 kv, of 64: 176.2 / 178.7.)
-  const bool share = !plan.use && !small && all_wgs > (paged ? 3 : 2) * slots && (8 % Hkv == 0 || Hkv % 8 == 0) &&
-                     qtiles <= 65535 && p.group > 1 && p.group <= 4096 && !(paged && p.softcap > 0.0f);
+  const bool share = !plan.use && !small && (8 % Hkv == 0 || Hkv % 8 == 0) && qtiles <= 65535 && p.group > 1 &&
+                     p.group <= 4096 && !(paged && p.softcap > 0.0f) &&
+                     heads_share_workgroups(paged, D, B, Hq, max_len, tokens, current_device_cu_count());
   // (exact: numbers below 2^18, at most 2^12 heads)
   p.share_rcp = share ? (unsigned int)(0x100000000ull / p.group + 1) : 0;
   if (!share) qtiles = ceil_div(max_len, 32 * row_waves);
@@ -237,6 +233,19 @@ extern "C" int dlb_prefill_attn_varlen(const void* q, const void* k, const void*
                                        int64_t v_stride_head, int64_t o_stride_tok,
                                        int64_t o_stride_head, float sm_scale, int dtype,
                                        void* stream) {
+  return dlb_prefill_attn_varlen_tokens(q, k, v, o, start_loc, seq_len, index64_mask, B, Hq, Hkv, D, max_len, q_stride_tok,
+                                        q_stride_head, k_stride_tok, k_stride_head, v_stride_tok, v_stride_head,
+                                        o_stride_tok, o_stride_head, sm_scale, dtype, 0, stream);
+}
+
+extern "C" int dlb_prefill_attn_varlen_tokens(const void* q, const void* k, const void* v, void* o,
+                                       const void* start_loc, const void* seq_len,
+                                       int index64_mask, int B, int Hq, int Hkv, int D, int max_len, int64_t q_stride_tok,
+                                       int64_t q_stride_head, int64_t k_stride_tok,
+                                       int64_t k_stride_head, int64_t v_stride_tok,
+                                       int64_t v_stride_head, int64_t o_stride_tok,
+                                       int64_t o_stride_head, float sm_scale, int dtype, int64_t tokens,
+                                       void* stream) {
   using namespace dlb;
   if (B < 0 || Hq < 1 || Hkv < 1 || D < 1 || max_len < 0) return DLB_ERR_BAD_ARG;
   if (Hq % Hkv != 0) return DLB_ERR_BAD_ARG;
@@ -262,7 +271,7 @@ extern "C" int dlb_prefill_attn_varlen(const void* q, const void* k, const void*
   p.page_shift = 0;
   p.window = -1;
   p.softcap = -1.0f;
-  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, max_len, sm_scale, dtype, nullptr, 0, stream);
+  return launch_prefill(p, false, B, Hq, Hkv, D, D, max_len, tokens, max_len, sm_scale, dtype, nullptr, 0, stream);
 }
 
 extern "C" size_t dlb_paged_prefill_ws_bytes(int64_t tokens, int B, int Hq, int Hkv, int D, int Dv, int page,
@@ -335,6 +344,6 @@ extern "C" int dlb_paged_prefill_attn_ws(const void* q, const void* k_cache, con
   p.page_shift = (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1;
   p.window = window_size;
   p.softcap = logit_softcapping;
-  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, (int64_t)page * max_blocks, sm_scale, dtype, ws,
+  return launch_prefill(p, true, B, Hq, Hkv, D, Dv, max_q_len, tokens, (int64_t)page * max_blocks, sm_scale, dtype, ws,
                         ws_bytes, stream);
 }

@@ -33,10 +33,10 @@ def context_attention_fwd(q, k, v, o, b_start_loc, b_seq_len, max_input_len):
     # prefill_attention.py:155-181)
     (start, lens), mask = _lib.index_arrays(b_start_loc.contiguous(), b_seq_len.contiguous())
     with _lib.device_guard(q.device):
-        st = lib.dlb_prefill_attn_varlen(
+        st = lib.dlb_prefill_attn_varlen_tokens(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), start.data_ptr(),
             lens.data_ptr(), mask, batch, head, k.shape[1], Lq, int(max_input_len),
             q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
             o.stride(0), o.stride(1), float(sm_scale), _lib.torch_dtype_code(q.dtype),
-            _lib.current_stream_ptr(q.device))
-    _lib.check(st, "dlb_prefill_attn_varlen")
+            q.size(0), _lib.current_stream_ptr(q.device))
+    _lib.check(st, "dlb_prefill_attn_varlen_tokens")

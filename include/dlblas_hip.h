@@ -38,7 +38,7 @@ extern "C" {
 /* ABI version: bumped whenever a signature below changes or an entry point is added; dlb_version()
  * returns the value the library was built with, and a binding should refuse a library whose version
  * differs. */
-#define DLB_ABI_VERSION 6
+#define DLB_ABI_VERSION 7
 int dlb_version(void);
 
 /* Index arrays (block tables, sequence lengths, start offsets) are read in the integer width the
@@ -219,6 +219,15 @@ int dlb_prefill_attn_varlen(const void* q, const void* k, const void* v, void* o
                             int64_t q_stride_head, int64_t k_stride_tok, int64_t k_stride_head,
                             int64_t v_stride_tok, int64_t v_stride_head, int64_t o_stride_tok,
                             int64_t o_stride_head, float sm_scale, int dtype, void* stream);
+
+/* The same with the rows of q and o (0: not known), by which a launch is cut where they say more than the longest
+ * sequence does: a long prompt among short ones.  The results are the same. */
+int dlb_prefill_attn_varlen_tokens(const void* q, const void* k, const void* v, void* o,
+                                   const void* start_loc, const void* seq_len, int index64_mask, int B,
+                                   int Hq, int Hkv, int D, int max_len, int64_t q_stride_tok,
+                                   int64_t q_stride_head, int64_t k_stride_tok, int64_t k_stride_head,
+                                   int64_t v_stride_tok, int64_t v_stride_head, int64_t o_stride_tok,
+                                   int64_t o_stride_head, float sm_scale, int dtype, int64_t tokens, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Causal attention of new query tokens over a paged KV cache that already holds them and

@@ -30,7 +30,7 @@ def test_every_declared_symbol_is_exported_and_bound():
 
 def test_version_and_status_strings():
     lib = _lib.load()
-    assert lib.dlb_version() == _lib.ABI_VERSION == 6
+    assert lib.dlb_version() == _lib.ABI_VERSION == 7
     assert lib.dlb_status_string(0) == b"ok"
     for code in (-1, -2, -3, -4, -99):
         assert lib.dlb_status_string(code)

@@ -10,6 +10,7 @@ PROGRAM = """
 #include <cstdio>
 #include <cstring>
 #include "moe_rules.h"
+#include "prefill_rules.h"
 using namespace dlb;
 int main() {
   char what[32];
@@ -27,6 +28,8 @@ int main() {
       const StreamShape f = stream_shape_16bit({a[0] != 0, a[3], a[3], 1, a[1], a[2], a[4], a[5], a[6]});
       printf("%d%d\\n", f.cw, f.nt);
     }
+    if (!strcmp(what, "share"))  // paged, head size, heads, sequences, longest, tokens, cus
+      puts(heads_share_workgroups(a[0] != 0, (int)a[1], a[3], a[2], a[4], a[5], a[6]) ? "shared" : "single");
     scanf("%*[;\\n ]");
   }
 }
@@ -95,3 +98,26 @@ def test_16bit_shapes_have_kernels(rule):
     seen = {rule("shape", g, E, E, int(r * E), c, 2048, 256) for g in (0, 1) for E in (1, 4, 16, 256)
             for r in (0.1, 5, 12, 21, 26, 40, 58, 66, 83, 100, 1000) for c in (64, 704, 2816)}
     assert seen == set(SHAPES)
+
+
+FIFTEEN = [137, 211, 84, 125, 190, 249, 66, 173, 228, 101, 152, 97, 240, 118, 77]  # short prompts
+CHATS = [42, 26, 28, 20, 57, 50, 26, 39, 40, 35, 58, 55, 48, 16, 18]                # short turns
+
+
+# us with a head per workgroup and with heads that share them
+@pytest.mark.parametrize("paged,D,heads,lens,us", [
+    (0, 128, 8, [2000, 1500] + FIFTEEN[:14], (35.2, 36.8)), (0, 128, 8, [4000] + FIFTEEN, (63.2, 64.7)),
+    (0, 64, 16, [8000] + CHATS, (162.8, 164.9)), (0, 256, 8, [1900, 1500] + CHATS[:14], (58.0, 59.2)),
+    (0, 128, 32, [672, 180, 145, 416, 574, 213, 541, 376, 214, 121, 533, 308, 557, 591, 544, 399], (55.5, 51.1)),
+    (0, 128, 28, [4000] + FIFTEEN, (133.5, 128.6)), (0, 256, 28, [1024] * 8, (214.7, 201.4)),
+    (1, 64, 32, [1000] + CHATS, (78.8, 86.4)), (1, 256, 16, [1000] + CHATS, (215.2, 235.6)),
+    (1, 128, 28, [2000] + FIFTEEN, (97.0, 87.0)), (1, 256, 16, [700] * 8, (289.7, 276.0)),
+])
+def test_heads_that_share_workgroups(rule, paged, D, heads, lens, us):
+    form = rule("share", paged, D, heads, len(lens), max(lens), sum(lens), 256)
+    assert us[("single", "shared").index(form)] == min(us)
+
+
+def test_unknown_tokens_count_as_part_of_the_longest(rule):
+    ask = lambda n, tokens: rule("share", 0, 128, 32, n, 1024, tokens, 256)  # noqa: E731
+    assert ask(2, 2 * 1024) == ask(2, 0) == "single" and ask(8, 8 * 1024) == ask(8, 0) == "shared"
