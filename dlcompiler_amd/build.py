@@ -96,16 +96,27 @@ def parse_resource_remarks(stderr: str) -> dict[str, dict[str, int]]:
     return kernels
 
 
+def text_with_headers(src: Path, seen: set[Path] | None = None) -> str:
+    """The text of a source and of the headers of this project that it includes, each once."""
+    seen = set() if seen is None else seen
+    if src.resolve() in seen:
+        return ""
+    seen.add(src.resolve())
+    text = src.read_text()
+    return text + "".join(text_with_headers(src.parent / name, seen)
+                          for name in re.findall(r'^#include "([^"]+)"', text, flags=re.M))
+
+
 def check_hand_scheduled(kernels: dict[str, dict[str, int]], source_text: str = "") -> list[str]:
     """Names (with the offending figures) of hand-scheduled kernels that use scratch or spill.
 
-    The check fails closed: a source that defines a hand-scheduled kernel (its tag appears in
-    ``source_text``) must yield at least one parsed report for it, and every such report must
-    carry both figures -- a compiler that prints the remarks differently, or not at all, stops
-    the build instead of passing it."""
+    The check fails closed: a source that defines a hand-scheduled kernel (``source_text``, its own
+    text and that of the headers it includes, does) must yield at least one parsed report for it,
+    and every such report must carry both figures -- a compiler that prints the remarks differently,
+    or not at all, stops the build instead of passing it."""
     bad = []
     for tag in HAND_SCHEDULED:
-        if tag in source_text and not any(tag in name for name in kernels):
+        if f"void {tag}(" in source_text and not any(tag in name for name in kernels):
             bad.append(f"{tag}: defined in the source but no resource report was parsed for it")
     for name, r in kernels.items():
         if any(tag in name for tag in HAND_SCHEDULED):
@@ -137,7 +148,7 @@ def _compile_one(src: Path, obj: Path, verbose: bool) -> None:
     kernels = parse_resource_remarks(proc.stderr)
     report = obj.with_suffix(".resources.json")
     report.write_text(json.dumps(kernels, indent=1, sort_keys=True))
-    bad = check_hand_scheduled(kernels, src.read_text())
+    bad = check_hand_scheduled(kernels, text_with_headers(src))
     if bad:
         obj.unlink(missing_ok=True)
         raise RuntimeError(f"{src.name}: hand-scheduled kernels must not spill or use scratch:\n  "

@@ -5,7 +5,7 @@ from pathlib import Path
 
 import pytest
 
-from dlcompiler_amd.build import ARCH, CSRC_DIR, HIPCC, OBJ_DIR, check_hand_scheduled, kernel_resources
+from dlcompiler_amd.build import ARCH, CSRC_DIR, HIPCC, OBJ_DIR, check_hand_scheduled, kernel_resources, text_with_headers
 
 # kernels that run the helpers of inline-assembly loads, or the key walk of the paged decode kernels, which
 # looks pages up with hand-issued scalar loads
@@ -27,10 +27,26 @@ def test_every_kernel_with_hand_issued_loads_is_named():
     """Sources that issue loads by hand hold no kernel outside the gate but these, which use ordinary loads."""
     ordinary = {"prefill_combine_kernel", "paged_decode_combine_kernel", "quant_fp8_group128_kernel",
                 "moe_topk_sum_kernel"}
-    for src in CSRC_DIR.glob("*.hip"):
+    named = set()
+    for src in [*CSRC_DIR.glob("*.hip"), *CSRC_DIR.glob("*.h")]:
         text = src.read_text()
         if re.search(r"dma\d+_global_to_lds|s_load_dword|buffer_of\(", text):
-            assert set(re.findall(r"void (\w+_kernel)\(", text)) - ordinary <= set(KERNELS), src.name
+            found = set(re.findall(r"__global__[^;{]*void (\w+_kernel)\(", text)) - ordinary
+            assert found <= set(KERNELS), src.name
+            named |= found
+    assert named == set(KERNELS)
+
+
+@pytest.mark.parametrize("source,kernels", [("moe_fp8", {"moe_gemm_kernel"}), ("moe_stream", {"moe_stream_kernel"}),
+                                            ("paged_decode", {"paged_decode_split_kernel", "paged_decode_direct_kernel"}),
+                                            ("prefill_attn", {"prefill_attn_kernel"}),
+                                            ("prefill_attn_cap", {"prefill_attn_kernel"}),
+                                            ("silu_and_mul", set())])
+def test_missing_reports_stop_the_build(source, kernels):
+    """Kernels count as a source's where it or a header of its defines them, comments aside."""
+    text = re.sub(r"//.*", "", text_with_headers(CSRC_DIR / f"{source}.hip"))
+    assert {m.split(":")[0] for m in check_hand_scheduled({}, text)} == kernels
+    assert not check_hand_scheduled({}, "// " + " ".join(KERNELS))
 
 
 def test_short_head_dims_keep_their_waves():
@@ -67,7 +83,7 @@ def _code_of(source, tmp_path):
     return dict(block.split(">", 1) for block in re.split(r"^[0-9a-f]+ <", text, flags=re.M)[1:])
 
 
-@pytest.mark.parametrize("source", ["moe_fp8", "moe_stream", "paged_decode", "prefill_attn"])
+@pytest.mark.parametrize("source", ["moe_fp8", "moe_stream", "paged_decode", "prefill_attn", "prefill_attn_cap"])
 def test_pipelined_loads_are_global(source, tmp_path):
     """A flat load counts as an LDS operation too: the next wait for LDS waits for every load in flight."""
     code = _code_of(source, tmp_path)
