@@ -489,6 +489,14 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
   }
   if (k < KC) chunk(std::integral_constant<int, 0>{}, k);
   __builtin_amdgcn_s_setprio(0);
+  // The lane coordinates are derived afresh for the epilogue: carried across the main loop they
+  // would hold four registers that the loop needs.
+  int tid_e = threadIdx.x;
+  asm volatile("" : "+v"(tid_e));
+  const int j_e = tid_e & 31, h_e = (tid_e >> 5) & 1;
+  // (routing weights that are divided by their token's sum: asked for while the copies past the end are on their way)
+  if (!GATED && !weights_by_slot && tid_e < 128)
+    rw_lds[tid_e] = slot_weight(p, min(max(sid_lds[tid_e], 0), p.numel - 1));
   // the clamped copies past the end are still in flight and will write the LDS slots
   wait_vm<0>();
   // the accumulators hold sum / s(last chunk), whose scales are still in their LDS slot (x_tgt
@@ -497,11 +505,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     return read_as(x_tgt, rt) * read_ws(KC - 1, ct);
   };
 
-  // The lane coordinates are derived afresh for the epilogue: carried across the main loop they
-  // would hold four registers that the loop needs.
-  int tid_e = threadIdx.x;
-  asm volatile("" : "+v"(tid_e));
-  const int j_e = tid_e & 31, h_e = (tid_e >> 5) & 1;
   // ---- epilogues: lane holds token (32*rt + j_e), columns ncol[ct] + 8*(r/4) + 4*h_e + r%4.
   // A swap between the lane halves turns two 4-column runs into one 8-column run per lane.
   // Output tiles leave through LDS (the activation slots, free once every wave has left the
@@ -559,7 +562,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeGemmParams p)
     constexpr int kPitch = 512 + 16;  // staging row pitch: rows 16 bytes apart in the banks
     static_assert(64 * kPitch <= NX * kXSlot, "output staging fits the activation slots");
     const int ncols = min(256, p.N - nt * 256);
-    if (!weights_by_slot && tid_e < 128) rw_lds[tid_e] = slot_weight(p, min(max(sid_lds[tid_e], 0), p.numel - 1));
     __syncthreads();  // every wave has left the main loop
 #pragma unroll
     for (int half = 0; half < (NRT + 1) / 2; ++half) {

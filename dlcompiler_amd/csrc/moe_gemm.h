@@ -52,9 +52,23 @@ __device__ __forceinline__ float slot_weight(const MoeGemmParams& p, int slot) {
   if (!p.topk_w) return 1.0f;
   const float w = p.topk_w[slot];
   if (!p.renorm) return w;
-  const float* mine = p.topk_w + (slot - slot % p.topk);
+  const uint32_t n = (uint32_t)slot, q = __umulhi(n, p.topk_rcp), token = n - q * p.topk >= (uint32_t)p.topk ? q + 1 : q;
+  const float* mine = p.topk_w + token * (uint32_t)p.topk;
   float sum = 0.0f;
-  for (int j = 0; j < p.topk; ++j) sum += mine[j];
+  // Four or eight weights on their way at once: one after the other is a chain of topk loads (fp8, us a layer: 64 experts of
+  // 1024 x 512, 6000 tokens x 8, 196.9 -> 190.5; 32 of 2048 x 256, 2500 x 4, 77.0 -> 72.6).  Eight for two alone cost 1 %.
+  auto add = [&](auto ahead) __attribute__((always_inline)) {
+    constexpr int N = decltype(ahead)::value;
+    for (int j0 = 0; j0 < p.topk; j0 += N) {
+      float v[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) v[j] = mine[min(j0 + j, p.topk - 1)];
+#pragma unroll
+      for (int j = 0; j < N; ++j) sum += j0 + j < p.topk ? v[j] : 0.0f;
+    }
+  };
+  if (p.topk <= 4) add(std::integral_constant<int, 4>{});
+  else add(std::integral_constant<int, 8>{});
   return w / sum;
 }
 

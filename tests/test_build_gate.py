@@ -113,3 +113,13 @@ def test_down_gemm_stores_past_the_caches_too(tmp_path):
         stores = re.findall(r"global_store_dwordx4 .*", text)
         past = [" nt" in store.split("//")[0] for store in stores]
         assert any(past) and not all(past), name
+
+
+def test_routing_weights_of_a_token_are_asked_for_together(tmp_path):
+    """Renormalised weights: a loop that loads, waits and adds is a chain of as many loads as a token has slots."""
+    for source, kernel in (("moe_fp8", "moe_gemm_kernelILb0E"), ("moe_stream", "moe_stream_kernelILb0E")):
+        down = {name: text for name, text in _code_of(source, tmp_path).items() if kernel in name}
+        assert down
+        for name, text in down.items():
+            runs = re.split(r"s_waitcnt[^\n]*vmcnt|s_cbranch", text)
+            assert max(len(re.findall(r"global_load_dword ", run)) for run in runs) >= 8, name
