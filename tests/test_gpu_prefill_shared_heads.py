@@ -55,7 +55,7 @@ def test_paged_head_sizes(dev, D, window, page):
 def _paged(dev, Hq, Hkv, D, window, page):
     from dlcompiler_amd.kernels.paged_attention import paged_attention_fwd
 
-    new = _repeated([150, 65, 97, 131], Hq, 2, D, paged=True)
+    new = _repeated([150, 65, 97, 131], Hq, 2.2, D, paged=True)  # (lengths that differ: more than 2.1)
     history = [70, 0, 333, 64] * (len(new) // 4)
     g = torch.Generator().manual_seed(Hq)
     ctx = [a + b for a, b in zip(new, history)]

@@ -112,6 +112,8 @@ CHATS = [42, 26, 28, 20, 57, 50, 26, 39, 40, 35, 58, 55, 48, 16, 18]            
     (0, 128, 28, [4000] + FIFTEEN, (133.5, 128.6)), (0, 256, 28, [1024] * 8, (214.7, 201.4)),
     (1, 64, 32, [1000] + CHATS, (78.8, 86.4)), (1, 256, 16, [1000] + CHATS, (215.2, 235.6)),
     (1, 128, 28, [2000] + FIFTEEN, (97.0, 87.0)), (1, 256, 16, [700] * 8, (289.7, 276.0)),
+    (1, 128, 32, [430, 483, 571, 314, 538, 427, 326, 380], (185.4, 190.6)), (1, 128, 32, [512] * 8, (222.1, 219.0)),
+    (1, 128, 32, [38, 53, 106, 97, 45, 59, 57, 39, 99, 65, 93, 80, 68, 101, 98, 72, 46, 94], (29.0, 30.9)),
 ])
 def test_heads_that_share_workgroups(rule, paged, D, heads, lens, us):
     form = rule("share", paged, D, heads, len(lens), max(lens), sum(lens), 256)
