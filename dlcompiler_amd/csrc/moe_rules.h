@@ -54,25 +54,29 @@ struct MoeLaunch {
 //   16 of 1024 x 512, 4 here (16 tiles)         25             27.8  26.6  23.2
 //                                               75      39.4  38.1  32.8  30.2  30.1
 // (4000 tokens through the last, 1000 rows: 133 workgroups of 128 rows 53.8 us, 258 of 64, one CU with two, 58.8.)
-// Above 52 rows two more things count.  gate_up, 62 to 84 rows, with K split in two: half of the experts have a second
-// tile of 64 rows, and where some CUs get two such workgroups that way and none gets two of 32 rows side by side, those
-// are faster (128 / 64 / 64 in two / 32 side by side: 8 experts of 1408 x 1280, 67 rows 44.8 / 45.1 / 48.0 / 42.6; 16 of
-// 1536 x 640, 77 rows 50.7 / 52.0 / 55.0 / 50.2; 8 of 2816 x 2816, 4 of them here, 69 rows 78.2 / 74.9 / 80.5 / 71.5).
-// down: tall tiles store whole rows, and 64-row ones gain by what K is long enough to hide (128 / 64: 16 experts of 1792 x
-// 1280, 68 rows 65.5 / 73.5; 1536 x 640, 77 rows 51.7 / 55.0; 1408 x 512, 85 rows 37.7 / 39.8; but 1408 x 3968, 106 rows
-// 144.7 / 134.7, 1664 x 1152, 95 rows 70.5 / 65.9).
-// Of 840 GEMMs (7 to 320 rows) the shape is 0.7 % above the best of the seven on average and 5 % at worst above what
-// the rows alone would choose (K split in two up to 52, else 128-row tiles), which is 6.5 % above the best.
+// Three more things count (us of a layer with one GEMM in each shape, other weights at each step).
+// Above 52 rows, gate_up, 62 to 84 rows, with K split in two: half of the experts have a second tile of 64 rows, and where
+// some CUs get two such workgroups that way and none gets two of 32 rows side by side, those are faster (128 / 64 / 64 in
+// two / 32 side by side: 16 experts of 3840 x 640, 66 rows 86.9 / 84.0 / 85.7 / 79.8; 16 of 1280 x 1408, 8 of them here, 72
+// rows 60.3 / 56.4 / 60.3 / 54.1; but 8 of 2048 x 2816, 4 here, 72 rows 87.0 / 81.5 / 86.9 / 90.2).
+// down, up to 76 rows, where 64-row tiles would have one for most CUs: few experts have a second one, and a tall tile reads
+// the weights once (128 / 64 rows, 53 - 76 rows per expert: K from 1280 on 0.975 on average, of 768 and less 1.00; 78 - 120
+// rows 1.01 - 1.06; 16 of 1792 x 1280, 68 rows 65.5 / 73.5; but 16 of 3584 x 2688, 8 here, 75 rows 114.6 / 113.7).
+// 35 to 44 rows, where 32-row tiles have second ones and 64-row ones do not: 64 in two from 0.55 of the CUs on (64 / 32 in
+// two: 16 of 1024 x 1280, 8 here, 42 rows 41.0 / 44.7; down, 16 of 1280 x 1792, 36 rows 55.5 / 60.6; but 30 rows 48.0 / 46.8,
+// 48 rows 62.0 / 57.3 and 84.9 / 81.8).
+// Of 900 GEMMs (7 to 330 rows, few column tiles, half of them where the three apply) four are more than 1 % slower than
+// without them, one of them 11 %, 2.1 % and 1.3 % less on average where they apply (gate_up, down).
 struct StreamShape { int cw, nt; };  // (four waves, cw of them side by side; rows 16 nt)
 inline StreamShape stream_shape_16bit(const MoeLaunch& p) {
   const int64_t wave_columns = p.gated ? 32 : 64, experts = p.most_experts(), cus = p.cus;
   const auto column_tiles = [&](int cw) { return (p.columns + cw * wave_columns - 1) / (cw * wave_columns) * experts; };
   const int64_t tiles = column_tiles(4);
   // Workgroups with rows: on average an expert's last row tile is half full, and an expert of
-  // up to 0.72 of a tile seldom has a second one.
+  // up to three quarters of a tile seldom has a second one.
   const auto blocks = [&](int cw, int nt) {
     const double full = (double)p.slots / ((double)p.experts * 16 * nt);
-    return (double)column_tiles(cw) * (full <= 0.72 ? 1.0 : full + 0.5);
+    return (double)column_tiles(cw) * (full <= 0.75 ? 1.0 : full + 0.5);
   };
   const bool one_round = 2 * tiles > cus && 10 * tiles <= 9 * cus, beside = tiles >= 2 * cus;
   if (p.mean_up_to(kSmallMeanRows)) return {beside ? 4 : 1, 1};
@@ -85,15 +89,11 @@ inline StreamShape stream_shape_16bit(const MoeLaunch& p) {
     if (!p.gated && tiles > cus / 2) return {4, 8};
     if (!p.mean_up_to(52)) {
       const bool tall = blocks(4, 4) >= 0.55 * cus;
-      const bool short_k = p.row_bytes < 2048 || p.slots < 80 * p.experts;
-      if (!p.gated && 16 * tiles >= 5 * cus && short_k && (tall || !p.mean_up_to(60))) return {4, 8};
       if (p.gated && !p.mean_up_to(62) && p.mean_up_to(84) && blocks(2, 4) > 0.95 * cus && blocks(4, 2) <= 0.95 * cus)
         return {4, 2};
-      if (tall) return {4, 4};
+      if (tall) return {4, !p.gated && p.row_bytes >= 2560 && p.mean_up_to(76) ? 8 : 4};
     }
-    // (up to 28 rows 32-row tiles seldom have a second one either: 8 experts of 1152 x 1152, 26 rows 32.5 / 31.2, 47 rows
-    // 33.5 / 35.6)
-    if (blocks(2, 4) >= (!p.mean_up_to(28) && p.mean_up_to(52) ? 0.55 : 0.65) * cus) return {2, 4};
+    if (blocks(2, 4) >= (!p.mean_up_to(34) && p.mean_up_to(44) ? 0.55 : 0.65) * cus) return {2, 4};
   }
   if (blocks(2, 2) >= 0.55 * cus || blocks(1, 1) > 1.1 * cus) return {2, 2};
   return {1, 1};

@@ -79,13 +79,20 @@ SHAPES = ("48", "44", "24", "42", "22", "41", "11")
 @pytest.mark.parametrize("gated,E,local,rows,columns,K,us", [
     (0, 8, 8, 43.75, 2432, 2560, (86.1, 88.7, 80.9, 88.3, 91.1, 104.8, 95.4)),
     (0, 16, 16, 67.5, 1792, 1280, (65.5, 73.5, 74.6, 84.2, 78.9, 102.3, 87.9)),
-    (0, 16, 16, 77.25, 1536, 640, (51.7, 55.0, 56.2, 59.0, 56.6, 62.1, 61.4)),
-    (0, 16, 16, 85, 1408, 512, (37.7, 39.8, 41.2, 41.3, 40.7, 45.8, 45.2)),
     (0, 16, 16, 106.25, 1408, 3968, (144.7, 134.7, 143.0, 174.9, 165.4, 231.4, 208.8)),
-    (1, 8, 8, 47, 1152, 1152, (36.2, 37.6, 33.5, 35.6, 35.6, 35.6, 36.4)),
     (1, 16, 16, 77.25, 640, 1536, (50.7, 52.0, 55.0, 50.2, 52.6, 66.2, 65.1)),
     (1, 8, 4, 69.25, 2816, 2816, (78.2, 74.9, 80.5, 71.5, 74.5, 105.9, 97.6)),
     (1, 8, 8, 117.5, 896, 3200, (82.9, 73.5, 57.3, 67.7, 72.5, 107.9, 100.1)),
+    (1, 16, 8, 42.5, 1280, 1024, (48.7, 44.5, 41.0, 43.6, 44.7, 45.7, 46.1)),
+    (1, 16, 8, 48.5, 1024, 3840, (82.9, 80.7, 62.0, 74.2, 57.3, 80.6, 82.2)),
+    (1, 16, 8, 30.0, 1152, 2432, (62.6, 59.8, 48.0, 58.0, 46.8, 59.1, 54.3)),
+    (1, 16, 16, 66.0, 640, 3840, (86.9, 84.0, 85.7, 79.8, 86.0, 131.1, 110.2)),
+    (0, 16, 16, 36.0, 1280, 1792, (59.3, 63.3, 55.5, 62.0, 60.6, 62.4, 62.3)),
+    (0, 8, 8, 48.0, 2048, 3840, (93.1, 104.6, 84.9, 98.9, 81.8, 105.3, 106.0)),
+    (0, 16, 8, 61.25, 2688, 2176, (88.6, 89.7, 78.6, 85.4, 87.3, 111.3, 100.1)),
+    (0, 16, 8, 89.75, 2944, 896, (82.1, 78.9, 81.2, 85.3, 82.2, 95.9, 91.2)),
+    (0, 32, 16, 102.875, 1408, 768, (62.3, 58.3, 61.1, 64.5, 61.6, 74.0, 71.7)),
+    (0, 16, 8, 120.0, 2432, 384, (66.8, 64.9, 67.0, 67.0, 65.6, 71.0, 73.5)),
     (1, 16, 16, 273.75, 1664, 1536, (139.1, 164.5, 162.8, 219.1, 208.7, 338.5, 317.8)),
     (1, 8, 8, 26.25, 1152, 1152, (35.8, 36.9, 32.5, 36.1, 31.2, 35.3, 34.3)),
 ])
