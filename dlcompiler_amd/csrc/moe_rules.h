@@ -108,7 +108,9 @@ inline StreamShape stream_shape_16bit(const MoeLaunch& p) {
 // What counts is how many of gate_up's 128-column tiles have rows.  With fewer than every other CU one, the shorter tiles
 // use the CUs that these leave idle.  With more, up to one for each, nothing helps; and with up to 1.4 for each, some
 // CUs have twice the weights of others and short tiles even that out, if rows are long enough that their start does
-// not cost more.  us a layer, 64 experts of 2048 x 1408, 6 per token: 1 token (66 tiles) 28.6 / 27.0 / 25.3, 2 (126)
+// not cost more.  (Short rows, fewer than 0.45 of the CUs: 16 experts of 1152 x 1664, 4 per token, 3 tokens (120) 20.2 / 20.7 /
+// 21.9; 64 of 1152 x 256, 8 per token, 18 tokens (116) 22.8 / 23.1 / 25.0; 16 of 1408 x 896, 24 tokens (112) 0.95 of
+// kInSteps.)  us a layer, 64 experts of 2048 x 1408, 6 per token: 1 token (66 tiles) 28.6 / 27.0 / 25.3, 2 (126)
 // 33.9 / 32.4 / 31.5, 4 (230) 44.1 / 44.9 / 46.2, 8 (386) 63.5 / 60.7 / 65.7; 128 of 1152 x 512, 8 per token: 10 tokens
 // (243) 34.3 / 34.5 / 40.9, 14 (305) 43.9 / 41.3 / 43.8, 23 (396) 48.3 / 45.9 / 51.8; 64 of 4096 x 1024, 8 per token:
 // 6 tokens (282) 100.6 / 99.3 / 88.6, 8 (336) 103.9 / 103.2 / 95.9, 16 (452) 125.8 / 124.4 / 126.4; 32 of 1536 x 1280, 4
@@ -122,7 +124,7 @@ inline FewRows fp8_few_rows(const MoeLaunch& up) {
   const double busy = (double)groups * up.hit_experts(), cus = (double)up.cus;
   const bool long_rows = up.row_bytes >= 1536;
   if (up.columns <= 4096) {
-    const bool idle = busy <= 0.48 * cus || (long_rows && 2 * groups * up.most_experts() <= up.cus);
+    const bool idle = busy <= (long_rows ? 0.48 : 0.45) * cus || (long_rows && 2 * groups * up.most_experts() <= up.cus);
     const bool uneven = long_rows && busy >= 0.98 * cus && busy <= 1.4 * cus && 2 * up.slots <= 3 * up.experts;
     if (idle || uneven) return FewRows::kHandedOver;
   }

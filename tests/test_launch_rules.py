@@ -57,6 +57,7 @@ def rule(tmp_path_factory):
     (32, 32, 4, 8, 1536, 1280, (34.4, 34.1, 38.1)), (64, 64, 8, 3, 4096, 1024, (56.6, 56.5, 58.6)),
     (64, 64, 6, 8, 3584, 640, (52.9, 53.0, 54.9)), (128, 128, 8, 14, 4096, 256, (55.9, 57.0, 57.4)),
     (64, 64, 8, 6, 4096, 1024, (100.6, 99.3, 88.6)), (128, 128, 8, 8, 2048, 768, (60.4, 57.0, 53.7)),
+    (16, 16, 4, 3, 1152, 1664, (20.2, 20.7, 21.9)), (64, 64, 8, 18, 1152, 256, (22.8, 23.1, 25.0)),
     (64, 64, 6, 1, 2048, 1408, (28.6, 27.0, 25.3)), (64, 64, 6, 8, 2048, 1408, (63.5, 60.7, 65.7)),
     (256, 64, 8, 4, 2688, 896, (33.5, 33.3, 25.8)), (8, 8, 2, 1, 4096, 4096, (43.5, 43.0, 32.8)),
 ])
