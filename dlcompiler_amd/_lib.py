@@ -14,7 +14,7 @@ _PKG_DIR = Path(__file__).resolve().parent
 DEFAULT_LIB_PATH = _PKG_DIR / "lib" / "libdlblas_hip.so"
 
 DLB_OK = 0
-ABI_VERSION = 7  # DLB_ABI_VERSION of include/dlblas_hip.h this binding was written against
+ABI_VERSION = 6  # DLB_ABI_VERSION of include/dlblas_hip.h this binding was written against
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
 
 # name -> (restype, argtypes); must list every symbol include/dlblas_hip.h declares
@@ -98,12 +98,14 @@ def load() -> ctypes.CDLL:
             f"{path} not found: build it with `python -m dlcompiler_amd.build` "
             "(there is no fallback implementation)")
     lib = ctypes.CDLL(str(path))
-    # the version first: a library of another version lacks entry points, or has them with other arguments
+    # the version first: a library of another version has entry points with other arguments
     if lib.dlb_version() != ABI_VERSION:
         raise ImportError(f"{path} has ABI version {lib.dlb_version()}, this binding needs "
                           f"{ABI_VERSION}: rebuild it with `python -m dlcompiler_amd.build`")
     for name, (restype, argtypes) in SIGNATURES.items():
-        fn = getattr(lib, name)  # AttributeError if the symbol is missing
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise ImportError(f"{path} lacks {name}: rebuild it with `python -m dlcompiler_amd.build`")
         fn.restype = restype
         fn.argtypes = argtypes
     _lib = lib

@@ -35,10 +35,10 @@ extern "C" {
 #define DLB_DTYPE_F16 1
 #define DLB_DTYPE_F32 2
 
-/* ABI version: bumped whenever a signature below changes or an entry point is added; dlb_version()
+/* ABI version: bumped whenever a signature below changes or an entry point goes; dlb_version()
  * returns the value the library was built with, and a binding should refuse a library whose version
- * differs. */
-#define DLB_ABI_VERSION 7
+ * differs, or that lacks an entry point it needs. */
+#define DLB_ABI_VERSION 6
 int dlb_version(void);
 
 /* Index arrays (block tables, sequence lengths, start offsets) are read in the integer width the

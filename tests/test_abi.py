@@ -30,7 +30,7 @@ def test_every_declared_symbol_is_exported_and_bound():
 
 def test_version_and_status_strings():
     lib = _lib.load()
-    assert lib.dlb_version() == _lib.ABI_VERSION == 7
+    assert lib.dlb_version() == _lib.ABI_VERSION == 6
     assert lib.dlb_status_string(0) == b"ok"
     for code in (-1, -2, -3, -4, -99):
         assert lib.dlb_status_string(code)
@@ -125,3 +125,15 @@ def test_launcher_and_fused_prepare_argument_checks_need_no_gpu():
                                        one, one, one, 32, 256, 256, 256, 2, 0, None) == -1  # sorted_cap too small
     assert lib.dlb_moe_align_quant_fp8(one, 0, 64, 8, 128, one, 64 + 8 * 127, one, 9, one, one, one, 1 << 20,
                                        one, one, one, 32, 200, 200, 200, 1, 0, None) == -2  # K % 128
+
+
+def test_library_that_lacks_an_entry_point_is_refused(monkeypatch, tmp_path):
+    # a library from before dlb_prefill_attn_varlen_tokens: the version alone does not tell
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    names = sorted(set(_lib.SIGNATURES) - {"dlb_version", "dlb_prefill_attn_varlen_tokens"})
+    src.write_text(f"int dlb_version(void) {{ return {_lib.ABI_VERSION}; }}\n" + "".join(f"void {n}(void) {{}}\n" for n in names))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setenv("DLBLAS_HIP_LIB", str(so))
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(ImportError, match="lacks dlb_prefill_attn_varlen_tokens"):
+        _lib.load()
